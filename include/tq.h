@@ -83,8 +83,8 @@ int tq_nearest_centroid(const double *values, int64_t n, const double *centroids
 int tq_quantize_indices(const tq_handle *h, const void *x, int64_t n, int in_dtype, uint8_t *idx, double *norms,
                         double *rotated, void *stream);
 
-/* polar_quant.py:87-119 PolarQuant.dequantize -> out [n,d] float64.  When x is not
- * NULL also writes residual = x - out (polar_quant.py:121-132). */
+/* polar_quant.py:87-119 PolarQuant.dequantize -> out [n,d] float64.  When residual is not
+ * NULL also writes residual = x - out (polar_quant.py:121-132); out may then be NULL. */
 int tq_dequantize_indices(const tq_handle *h, const uint8_t *idx, const double *norms, int64_t n, double *out,
                           const void *x, int x_dtype, double *residual, void *stream);
 
@@ -95,6 +95,11 @@ int tq_qjl_quantize(const tq_handle *h, const void *r, int64_t n, int in_dtype, 
 /* qjl.py:96-134 QJL.dequantize: out = S^T z * (projection_scale * norm * shrinkage). */
 int tq_qjl_dequantize(const tq_handle *h, const int8_t *signs, const double *norms, double shrinkage, int64_t n,
                       double *out, void *stream);
+
+/* tq_qjl_dequantize added to what out holds: the two halves of TurboQuant.dequantize (turboquant.py:102-124) in one
+ * buffer. */
+int tq_qjl_dequantize_add(const tq_handle *h, const int8_t *signs, const double *norms, double shrinkage, int64_t n,
+                          double *out, void *stream);
 
 /* utils.py:20-49 pack_bits / utils.py:52-68 unpack_bits on [n,d] int8 signs. */
 int tq_pack_bits(const int8_t *signs, int64_t n, int32_t d, uint8_t *packed, void *stream);

@@ -1,0 +1,62 @@
+"""The float64 dense products (rotation, reconstruction, projections) at the edges of their tiles.
+
+Tolerance: a sum of d products in any order is off by at most d * 2^-53 * sum |m||x| <= d * 2^-53 * ||x|| for rows of an
+orthogonal matrix, on each of the two sides compared; a few further roundings (norm, division, scale) add a constant."""
+import numpy as np
+import pytest
+
+import tq_oracle as O
+import turboquant_plus_amd as tqa
+
+pytestmark = pytest.mark.gpu
+
+
+def bound(d):
+    return 2 * (d + 16) * 2.0 ** -53
+
+
+# one vector and up to 16 (single tiles), one tile row more, several rows and a remainder; dimensions below, at and past a
+# chunk of 16 values, a tile of 16 columns and the eight column blocks that are dealt to the XCDs
+@pytest.mark.parametrize("n,d", [(1, 1), (3, 2), (16, 16), (17, 15), (2, 17), (33, 31), (16, 130), (31, 33), (65, 64), (5, 250),
+                                 (40, 257), (700, 129), (2100, 200), (4500, 272)])
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+def test_dense_products_at_tile_edges(n, d, dtype):
+    x = (np.random.default_rng(n * 1000 + d).standard_normal((n, d)) * np.logspace(-3, 3, n)[:, None]).astype(dtype)
+    if n > 2:
+        x[n // 2] = 0.0
+    g, o = tqa.PolarQuant(d, 3, seed=7), O.PolarRef(d, 3, seed=7)
+    idx, norms = g.quantize(x)
+    y, no = o.rotated(x)
+    np.testing.assert_allclose(norms, no, rtol=bound(d))
+    mid = (o.centroids[:-1] + o.centroids[1:]) / 2
+    want = np.searchsorted(mid, y.ravel(), side="left").reshape(y.shape)
+    near = np.abs(y[..., None] - mid).min(axis=-1) <= bound(d)
+    assert idx.dtype == np.int64 and np.array_equal(idx[~near], want[~near])
+    i2, n2, res = g.quantize_and_residual(x)
+    assert np.array_equal(i2, idx) and np.array_equal(n2, norms)
+    xh = g.dequantize(idx, norms)
+    tol = 4 * bound(d) * norms[:, None] + 1e-300
+    assert np.all(np.abs(xh - o.dequantize(idx, norms)) <= tol)
+    assert np.all(np.abs(res - (x.astype(np.float64) - xh)) <= tol)
+    q, qo = tqa.QJL(d, seed=5), O.QJLRef(d, seed=5)
+    s, rn = q.quantize(x)
+    proj = qo.project(x.astype(np.float64))
+    clear = np.abs(proj) > bound(d) * no[:, None]
+    assert s.dtype == np.int8 and np.array_equal(s[clear], np.where(proj < 0, -1, 1)[clear])
+    np.testing.assert_allclose(rn, no, rtol=bound(d))
+    # signs have norm sqrt(d): the sums are that much larger than the result's scale * norm
+    assert np.all(np.abs(q.dequantize(s, rn) - qo.dequantize(s, rn)) <= 4 * bound(d) * np.sqrt(d) * q.scale * rn[:, None] + 1e-300)
+
+
+@pytest.mark.parametrize("bits", [1, 5, 8])
+def test_level_search_at_every_width(bits):
+    """The level of a value is the number of midpoints below it; midpoints themselves and NaN included."""
+    g = tqa.PolarQuant(64, bits, seed=3)
+    x = np.random.default_rng(bits).standard_normal((300, 64))
+    idx, norms = g.quantize(x)
+    y, _ = O.PolarRef(64, bits, seed=3).rotated(x)
+    mid = (g.centroids[:-1] + g.centroids[1:]) / 2
+    near = np.abs(y[..., None] - mid).min(axis=-1) <= bound(64)
+    assert np.array_equal(idx[~near], np.searchsorted(mid, y.ravel(), side="left").reshape(y.shape)[~near])
+    w = tqa.PolarQuant(64, bits, seed=3, rotation="wht")
+    assert np.array_equal(w.quantize(x)[0], O.PolarRef(64, bits, seed=3, rotation="wht").quantize(x)[0])

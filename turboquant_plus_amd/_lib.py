@@ -54,6 +54,7 @@ PROTOTYPES = {
     "tq_dequantize_indices": (_I, [_P, _P, _P, _L, _P, _P, _I, _P, _P]),
     "tq_qjl_quantize": (_I, [_P, _P, _L, _I, _P, _P, _P]),
     "tq_qjl_dequantize": (_I, [_P, _P, _P, _D, _L, _P, _P]),
+    "tq_qjl_dequantize_add": (_I, [_P, _P, _P, _D, _L, _P, _P]),
     "tq_pack_bits": (_I, [_P, _L, C.c_int32, _P, _P]),
     "tq_unpack_bits": (_I, [_P, _L, C.c_int32, _P, _P]),
     "tq_pack_indices": (_I, [_P, _L, C.c_int32, _P, _P]),

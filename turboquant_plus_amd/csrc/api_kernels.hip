@@ -2,17 +2,288 @@
 //
 // These back the Python classes that keep the reference's signatures
 // (PolarQuant, QJL, the rotation and codebook free functions, pack helpers).
-// One workgroup of 128 threads handles VB = 8 vectors (4 or 2 for dimensions above 1024 / 2048) staged in LDS; the
-// rotation is either a dense d x d product read from L2 (matrix stored so
-// that consecutive threads read consecutive addresses) or the sign-diagonal
-// Walsh-Hadamard butterfly done in LDS with the reference's stage order, which
-// makes the float64 WHT results bit-identical to NumPy's.
+// Dense rotations and projections run as one float64 matrix-core product per
+// call with the per-vector work in its prologue and epilogue (k_dense64).  The
+// sign-diagonal Walsh-Hadamard rotation is a butterfly in LDS, one workgroup of
+// 128 threads per VB = 8 vectors (4 or 2 for dimensions above 1024 / 2048), in
+// the reference's stage order, which makes the float64 WHT results
+// bit-identical to NumPy's.
 #include "tq_internal.h"
 #include "tq_device64.h"
+
+#include <type_traits>
 
 namespace {
 
 using namespace tq64;
+
+// number of midpoints strictly below v: nb = 2^bits - 1 of them, ascending (NaN: 0)
+__device__ __forceinline__ int level_of(double v, const double *bounds, int bits) {
+    int c = 0;
+    for (int b = bits - 1; b >= 0; --b) {
+        const int t = c + (1 << b);
+        if (bounds[t - 1] < v) c = t;
+    }
+    return c;
+}
+
+// ---- dense products: out[row][j] = sum_k f(in[row][k]) M[k][j], float64 matrix cores -----------------------------
+// One thread per (output, vector) read the whole matrix from L2 once per VB vectors and an LDS operand per multiply:
+// 1.56 ms per product for 256 vectors of 1536 (0.8 of 75 TFLOP/s), 92 us for 32 768 of 128.  Here a wavefront owns RT x
+// CT tiles of 16 x 16 outputs of v_mfma_f64_16x16x4_f64 and a share of the contraction: 31 and 33 us for the same.  What
+// bounds it is the matrix instruction (64 clocks; 22 and 20 us of them at the 1.7 GHz the part holds here), then the
+// uneven last round of workgroups.  The order of the contraction is free, so in a chunk of 16 values lane quarter q takes
+// values 4q .. 4q+3 for the chunk's four steps: the A operand of four steps is one vector load, the B operand of a step
+// four runs of 128 bytes.  Nothing is staged in LDS during the product.
+// `ks` wavefronts of a workgroup split the contraction (the chunks in turn) and add their tiles in LDS in a fixed
+// order at the end; the other wavefronts work on further rows.  Column blocks are dealt to the XCDs in turn, so that
+// each XCD's L2 holds only its eighth of the matrix (an 18.9 MB matrix at d = 1536 against 4 MB of L2).
+// The vectors' norms are row properties that the contraction's own operands give (one multiply-add per operand
+// beside the tiles' matrix instructions) and divide the finished sums, so nothing passes over the input twice.
+enum DenseOp { DENSE_ROTATE, DENSE_QUANTIZE, DENSE_DEQUANTIZE, DENSE_QJL_QUANTIZE, DENSE_QJL_DEQUANTIZE };
+
+struct DenseArgs {
+    int d;
+    int64_t n;
+    const double *mat;        // M, row-major [d][d]
+    const void *in;           // [n][d]: vectors, indices or signs
+    int ks;                   // wavefronts that share a tile's contraction
+    unsigned n_row, n_col;    // row and column blocks of the launch
+    // quantize: bounds, bits; dequantize: centroids, norm_correction
+    const double *bounds, *centroids;
+    int bits, norm_correction;
+    const double *norms_in;   // dequantize, QJL dequantize
+    double *norms_out;        // quantize, QJL quantize
+    void *out;                // ROTATE: values; QUANTIZE: indices; (QJL_)DEQUANTIZE: float64; QJL_QUANTIZE: int8 signs
+    double *rotated;          // quantize: rotated unit vectors or NULL
+    const void *x;            // dequantize: the vectors that `residual` is taken against
+    double *residual;
+    double proj_scale, shrinkage;
+    int accumulate;           // QJL dequantize: add to out
+};
+
+typedef double double4_t __attribute__((ext_vector_type(4)));
+
+// OP, element type of the input, and of the output (of x: DEQUANTIZE)
+template <DenseOp OP, typename TI, typename TO, int RT, int CT, int NW>
+__global__ __launch_bounds__(64 * NW) void k_dense64(DenseArgs a) {
+    constexpr bool NORMS = OP == DENSE_QUANTIZE || OP == DENSE_QJL_QUANTIZE || OP == DENSE_DEQUANTIZE;
+    constexpr int NT_ = RT * CT;
+    extern __shared__ double sm[];   // [NW][NT_][4][64] partial tiles when ks > 1
+    __shared__ double table[OP == DENSE_DEQUANTIZE || OP == DENSE_QUANTIZE ? 256 : 1];
+    __shared__ double sq_s[NW][RT * 16];
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int c16 = lane & 15, q = lane >> 4;
+    const int kslice = wave % a.ks, rgroup = wave / a.ks, rgs = NW / a.ks;
+    unsigned row_b, col_b;
+    if (a.n_col >= 8) {   // column block % 8 = blockIdx % 8 = the XCD
+        const unsigned i = blockIdx.x >> 3;
+        row_b = i % a.n_row;
+        col_b = (i / a.n_row) * 8 + (blockIdx.x & 7);
+        if (col_b >= a.n_col) return;
+    } else {
+        col_b = blockIdx.x % a.n_col;
+        row_b = blockIdx.x / a.n_col;
+    }
+    const int d = a.d;
+    const int64_t row0 = ((int64_t)row_b * rgs + rgroup) * (RT * 16);
+    const int col0 = (int)col_b * (CT * 16);
+    if constexpr (OP == DENSE_DEQUANTIZE) {
+        for (int e = tid; e < 256; e += 64 * NW) table[e] = e < (1 << a.bits) ? a.centroids[e] : 0.0;
+        __syncthreads();
+    }
+    if constexpr (OP == DENSE_QUANTIZE)
+        for (int e = tid; e < (1 << a.bits) - 1; e += 64 * NW) table[e] = a.bounds[e];
+
+    // Addresses are a wave-uniform part, which moves with the chunk, and a lane's own offset.  Rows and columns past the
+    // end repeat the last one; their sums are not stored.
+    const int64_t rbase = row0 < a.n ? row0 : a.n - 1;
+    const TI *in = reinterpret_cast<const TI *>(a.in) + rbase * d;
+    uint32_t aoff[RT], boff[CT];
+#pragma unroll
+    for (int rt = 0; rt < RT; ++rt) aoff[rt] = (uint32_t)min((int64_t)(16 * rt + c16), a.n - 1 - rbase) * d + 4 * q;
+#pragma unroll
+    for (int ct = 0; ct < CT; ++ct) boff[ct] = 4 * q * d + min(col0 + 16 * ct + c16, d - 1);
+
+    struct Operands {
+        TI x[RT][4];
+        double b[CT][4];
+    };
+    auto load = [&](int chunk, Operands &o) {
+#pragma unroll
+        for (int rt = 0; rt < RT; ++rt) __builtin_memcpy(o.x[rt], in + 16 * chunk + aoff[rt], 4 * sizeof(TI));
+#pragma unroll
+        for (int s = 0; s < 4; ++s) {
+            const double *mrow = a.mat + (int64_t)(16 * chunk + s) * d;
+#pragma unroll
+            for (int ct = 0; ct < CT; ++ct) o.b[ct][s] = mrow[boff[ct]];
+        }
+    };
+    double4_t acc[RT][CT];
+    double sq[RT][2];
+#pragma unroll
+    for (int rt = 0; rt < RT; ++rt) {
+        sq[rt][0] = sq[rt][1] = 0.0;
+#pragma unroll
+        for (int ct = 0; ct < CT; ++ct) acc[rt][ct] = double4_t{0.0, 0.0, 0.0, 0.0};
+    }
+    auto value = [&](TI e) {
+        if constexpr (OP == DENSE_DEQUANTIZE) return table[e];   // 256 entries, those past the codebook 0
+        else return ldd(&e, 0);
+    };
+    auto multiply = [&](const Operands &o) {
+#pragma unroll
+        for (int s = 0; s < 4; ++s) {
+#pragma unroll
+            for (int rt = 0; rt < RT; ++rt) {
+                const double v = value(o.x[rt][s]);
+                if constexpr (NORMS) sq[rt][s & 1] = fma(v, v, sq[rt][s & 1]);
+#pragma unroll
+                for (int ct = 0; ct < CT; ++ct) acc[rt][ct] = __builtin_amdgcn_mfma_f64_16x16x4f64(v, o.b[ct][s], acc[rt][ct], 0, 0, 0);
+            }
+        }
+    };
+    // whole chunks; the request past this wavefront's last one repeats it, so that what has to be waited for is the same on
+    // every path (a branch around the request made the compiler wait for the newest one everywhere: 59 against 32 us for
+    // 256 vectors of 1536; holding the request in front of the products with scheduling barriers changed nothing)
+    const int full = d >> 4;
+    int left = (full - kslice + a.ks - 1) / a.ks;
+    if (left > 0) {
+        Operands o0, o1;
+        int c = kslice;
+        load(c, o0);
+        while (true) {
+            c = left > 1 ? c + a.ks : c;
+            load(c, o1);
+            multiply(o0);
+            if (--left == 0) break;
+            c = left > 1 ? c + a.ks : c;
+            load(c, o0);
+            multiply(o1);
+            if (--left == 0) break;
+        }
+    }
+    if ((d & 15) && kslice == full % a.ks) {   // the rest of the contraction, value by value
+        const int k0 = 16 * full + 4 * q;
+#pragma unroll
+        for (int s = 0; s < 4; ++s) {
+            const bool in_row = k0 + s < d;
+            double bv[CT];
+#pragma unroll
+            for (int ct = 0; ct < CT; ++ct) bv[ct] = a.mat[(int64_t)min(k0 + s, d - 1) * d + min(col0 + 16 * ct + c16, d - 1)];
+#pragma unroll
+            for (int rt = 0; rt < RT; ++rt) {
+                const double v = in_row ? value(in[aoff[rt] - 4 * q + min(k0 + s, d - 1)]) : 0.0;
+                if constexpr (NORMS) sq[rt][s & 1] = fma(v, v, sq[rt][s & 1]);
+#pragma unroll
+                for (int ct = 0; ct < CT; ++ct) acc[rt][ct] = __builtin_amdgcn_mfma_f64_16x16x4f64(v, bv[ct], acc[rt][ct], 0, 0, 0);
+            }
+        }
+    }
+    // norms: this wavefront's share of a row's squares, summed over the lane quarters, then over the wavefronts
+    if constexpr (NORMS) {
+#pragma unroll
+        for (int rt = 0; rt < RT; ++rt) {
+            double s = sq[rt][0] + sq[rt][1];
+            s += __shfl_xor(s, 16);
+            s += __shfl_xor(s, 32);
+            if (q == 0) sq_s[wave][16 * rt + c16] = s;
+        }
+    }
+    if (a.ks > 1) {
+        double *mine = sm + (size_t)wave * NT_ * 256 + lane;
+#pragma unroll
+        for (int t = 0; t < NT_; ++t)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) mine[(t * 4 + i) * 64] = acc[t / CT][t % CT][i];
+    }
+    __syncthreads();
+    auto norm_of = [&](int r) {   // row r of this wavefront's rows
+        double s = 0.0;
+        for (int w = 0; w < a.ks; ++w) s += sq_s[rgroup * a.ks + w][r];
+        return sqrt(s);
+    };
+    if constexpr (OP == DENSE_QUANTIZE || OP == DENSE_QJL_QUANTIZE) {
+        if (col_b == 0 && kslice == 0)
+            for (int r = lane; r < RT * 16; r += 64)
+                if (row0 + r < a.n) a.norms_out[row0 + r] = norm_of(r);
+    }
+#pragma unroll
+    for (int t = 0; t < NT_; ++t) {
+        if (t % a.ks != kslice) continue;   // the tile's wavefronts share out its tiles
+        const int rt = t / CT, ct = t % CT, col = col0 + 16 * ct + c16;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int r = 16 * rt + 4 * i + q;
+            const int64_t row = row0 + r;
+            double y;
+            if (a.ks > 1) {
+                y = 0.0;
+                const double *part = sm + (size_t)(rgroup * a.ks) * NT_ * 256 + (t * 4 + i) * 64 + lane;
+                for (int w = 0; w < a.ks; ++w) y += part[(size_t)w * NT_ * 256];
+            } else {
+                y = acc[rt][ct][i];
+            }
+            if (row >= a.n || col >= d) continue;
+            const int64_t at = row * d + col;
+            if constexpr (OP == DENSE_ROTATE) {
+                std_(reinterpret_cast<TO *>(a.out), at, y);
+            } else if constexpr (OP == DENSE_QUANTIZE) {
+                const double nv = norm_of(r);
+                y /= nv > 0.0 ? nv : 1.0;
+                reinterpret_cast<uint8_t *>(a.out)[at] = (uint8_t)level_of(y, table, a.bits);
+                if (a.rotated) a.rotated[at] = y;
+            } else if constexpr (OP == DENSE_DEQUANTIZE) {
+                if (a.norm_correction) {
+                    const double cn = norm_of(r);
+                    y /= cn > 1e-10 ? cn : 1.0;
+                }
+                const double v = y * a.norms_in[row];
+                if (a.out) reinterpret_cast<double *>(a.out)[at] = v;
+                if (a.residual) a.residual[at] = ldd(reinterpret_cast<const TO *>(a.x), at) - v;
+            } else if constexpr (OP == DENSE_QJL_QUANTIZE) {
+                reinterpret_cast<int8_t *>(a.out)[at] = y < 0.0 ? (int8_t)-1 : (int8_t)1;
+            } else {
+                const double v = y * ((a.proj_scale * a.norms_in[row]) * a.shrinkage);
+                double *o = reinterpret_cast<double *>(a.out) + at;
+                *o = a.accumulate ? *o + v : v;
+            }
+        }
+    }
+}
+
+template <DenseOp OP, typename TI, typename TO, int RT, int CT, int NW>
+void launch_dense_tiles(DenseArgs a, int ks, hipStream_t s) {
+    a.ks = ks;
+    const int rows = NW / ks * RT * 16;
+    a.n_row = (unsigned)((a.n + rows - 1) / rows);
+    a.n_col = (unsigned)((a.d + CT * 16 - 1) / (CT * 16));
+    const unsigned grid = a.n_col >= 8 ? a.n_row * ((a.n_col + 7) / 8 * 8) : a.n_row * a.n_col;
+    const size_t lds = ks > 1 ? (size_t)NW * RT * CT * 256 * sizeof(double) : 0;
+    if (lds > 48 * 1024)
+        (void)hipFuncSetAttribute((const void *)k_dense64<OP, TI, TO, RT, CT, NW>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+    k_dense64<OP, TI, TO, RT, CT, NW><<<grid, 64 * NW, lds, s>>>(a);
+}
+
+// Tiles and split of the contraction (us per product, splits of 8 / 4 / 2 / 1):
+//   4096 and more 2 x 2 tiles: no split (32 768 vectors of 128: 54 / 40 / 35 / 33); twice the split for half the tiles, so
+//   that a launch has about 4096 wavefronts (4096 of 128: 8.5 / 8.6 / 12.5 / 20; 1000 of 384: 12.6 / 13.0 / 22 / 38);
+//   fewer than 256 of them: 1 x 2 tiles, so that more CUs get a workgroup (100 of 768: 9.1 against 12.2);
+//   up to 16 vectors: single tiles over sixteen wavefronts - what counts is how many wavefronts stream the matrix (one
+//   vector of 1536: 7.9 against 11.0, sixteen: 10.4 against 12.9).
+template <DenseOp OP, typename TI, typename TO>
+int launch_dense(const DenseArgs &a, const char *what, hipStream_t s) {
+    const int64_t tiles = ((a.n + 31) / 32) * ((a.d + 31) / 32);
+    const int chunks = (a.d + 15) / 16;
+    auto split = [&](int most) {   // at least one chunk for every wavefront
+        while (most > 1 && most > chunks) most >>= 1;
+        return most;
+    };
+    if (a.n <= 16) launch_dense_tiles<OP, TI, TO, 1, 1, 16>(a, split(16), s);
+    else if (tiles < 256) launch_dense_tiles<OP, TI, TO, 1, 2, 8>(a, split(8), s);
+    else launch_dense_tiles<OP, TI, TO, 2, 2, 8>(a, split(tiles < 1024 ? 8 : tiles < 2048 ? 4 : tiles < 4096 ? 2 : 1), s);
+    return tq_check_launch(what);
+}
 
 template <int VB, typename TI, typename TO>
 __global__ __launch_bounds__(NT) void k_rotate64(const TI *x, TO *y, int64_t n, RotArgs r) {
@@ -28,7 +299,7 @@ __global__ __launch_bounds__(NT) void k_rotate64(const TI *x, TO *y, int64_t n, 
 }
 
 template <int VB, typename T>
-__global__ __launch_bounds__(NT) void k_quantize64(const T *x, int64_t n, RotArgs r, const double *bounds, int nb,
+__global__ __launch_bounds__(NT) void k_quantize64(const T *x, int64_t n, RotArgs r, const double *bounds, int bits,
                                                   uint8_t *idx, double *norms, double *rotated) {
     extern __shared__ double sm[];
     __shared__ double nrm[VB];
@@ -46,9 +317,7 @@ __global__ __launch_bounds__(NT) void k_quantize64(const T *x, int64_t n, RotArg
         const int v = i / r.d, j = i % r.d;
         if (v0 + v >= n) continue;
         const double yv = ys[v * r.pd + j];
-        int c = 0;
-        for (int k = 0; k < nb; ++k) c += (bounds[k] < yv) ? 1 : 0;
-        idx[(v0 + v) * r.d + j] = (uint8_t)c;
+        idx[(v0 + v) * r.d + j] = (uint8_t)level_of(yv, bounds, bits);
         if (rotated) rotated[(v0 + v) * r.d + j] = yv;
     }
     if (threadIdx.x < VB && v0 + threadIdx.x < n) norms[v0 + threadIdx.x] = nrm[threadIdx.x];
@@ -56,7 +325,7 @@ __global__ __launch_bounds__(NT) void k_quantize64(const T *x, int64_t n, RotArg
 
 template <int VB, typename T>
 __global__ __launch_bounds__(NT) void k_dequantize64(const uint8_t *idx, const double *norms, int64_t n, RotArgs r,
-                                                    const double *centroids, int norm_correction, double *out,
+                                                    const double *centroids, int n_centroids, int norm_correction, double *out,
                                                     const T *x, double *residual) {
     extern __shared__ double sm[];
     __shared__ double nrm[VB];
@@ -64,7 +333,7 @@ __global__ __launch_bounds__(NT) void k_dequantize64(const uint8_t *idx, const d
     const int64_t v0 = (int64_t)blockIdx.x * VB;
     for (int i = threadIdx.x; i < VB * r.pd; i += NT) {
         const int v = i / r.pd, j = i % r.pd;
-        xs[i] = (v0 + v < n && j < r.d) ? centroids[idx[(v0 + v) * r.d + j]] : 0.0;
+        xs[i] = (v0 + v < n && j < r.d) ? centroids[min((int)idx[(v0 + v) * r.d + j], n_centroids - 1)] : 0.0;
     }
     __syncthreads();
     if (norm_correction) {
@@ -80,40 +349,8 @@ __global__ __launch_bounds__(NT) void k_dequantize64(const uint8_t *idx, const d
         const int v = i / r.d, j = i % r.d;
         if (v0 + v >= n) continue;
         const double o = ys[v * r.pd + j] * norms[v0 + v];
-        out[(v0 + v) * r.d + j] = o;
+        if (out) out[(v0 + v) * r.d + j] = o;
         if (residual) residual[(v0 + v) * r.d + j] = ldd(x, (v0 + v) * r.d + j) - o;
-    }
-}
-
-template <int VB, typename T>
-__global__ __launch_bounds__(NT) void k_qjl_quantize64(const T *x, int64_t n, RotArgs r, int8_t *signs, double *norms) {
-    extern __shared__ double sm[];
-    __shared__ double nrm[VB];
-    double *xs = sm, *ys = sm + VB * r.pd;
-    const int64_t v0 = (int64_t)blockIdx.x * VB;
-    load_block<VB>(x, n, v0, r.d, r.pd, xs);
-    norms_block<VB>(xs, r.d, r.pd, nrm);
-    rotate_block<VB>(r, xs, ys);
-    for (int i = threadIdx.x; i < VB * r.d; i += NT) {
-        const int v = i / r.d, j = i % r.d;
-        if (v0 + v < n) signs[(v0 + v) * r.d + j] = ys[v * r.pd + j] < 0.0 ? (int8_t)-1 : (int8_t)1;
-    }
-    if (threadIdx.x < VB && v0 + threadIdx.x < n) norms[v0 + threadIdx.x] = nrm[threadIdx.x];
-}
-
-template <int VB>
-__global__ __launch_bounds__(NT) void k_qjl_dequantize64(const int8_t *signs, const double *norms, int64_t n, RotArgs r,
-                                                        double proj_scale, double shrinkage, double *out) {
-    extern __shared__ double sm[];
-    double *xs = sm, *ys = sm + VB * r.pd;
-    const int64_t v0 = (int64_t)blockIdx.x * VB;
-    load_block<VB>(signs, n, v0, r.d, r.pd, xs);
-    rotate_block<VB>(r, xs, ys);
-    for (int i = threadIdx.x; i < VB * r.d; i += NT) {
-        const int v = i / r.d, j = i % r.d;
-        if (v0 + v >= n) continue;
-        const double sc = (proj_scale * norms[v0 + v]) * shrinkage;
-        out[(v0 + v) * r.d + j] = ys[v * r.pd + j] * sc;
     }
 }
 
@@ -190,14 +427,26 @@ inline unsigned nblocks(int64_t n, int pd) {
 RotArgs rot_args(const tq_handle *h, int transpose) {
     RotArgs r;
     r.d = h->d;
-    r.pd = h->rotation == TQ_ROT_WHT ? h->pd : h->d;
-    r.mode = h->rotation;
-    // forward dense: out[j] = sum_k Pi[j][k] in[k]  -> M[k*d+j] = Pi^T row-major
-    r.mat = transpose ? h->rot64 : h->rot64_t;
+    r.pd = h->pd;
     r.sa = transpose ? h->s2_64 : h->s1_64;
     r.sb = transpose ? h->s1_64 : h->s2_64;
     return r;
 }
+
+// dense rotation: forward out[j] = sum_k Pi[j][k] in[k], i.e. M = Pi^T row-major
+DenseArgs dense_args(const tq_handle *h, const double *mat, const void *in, int64_t n) {
+    DenseArgs a = {};
+    a.d = h->d;
+    a.n = n;
+    a.mat = mat;
+    a.in = in;
+    a.bits = h->bits;
+    a.bounds = h->bounds64;
+    a.centroids = h->centroids64;
+    a.norm_correction = h->norm_correction;
+    return a;
+}
+inline const double *rotation_matrix(const tq_handle *h, int transpose) { return transpose ? h->rot64 : h->rot64_t; }
 
 #define DISPATCH_IN(dt, F)          \
     switch (dt) {                   \
@@ -224,21 +473,33 @@ int launch_rotate(const void *x, void *y, int64_t n, int out_dtype, const RotArg
     }
 }
 
+template <typename TI> int launch_rotate_dense(const DenseArgs &a, int out_dtype, hipStream_t s) {
+    switch (out_dtype) {
+    case TQ_F16: return launch_dense<DENSE_ROTATE, TI, __half>(a, "rotate64", s);
+    case TQ_F32: return launch_dense<DENSE_ROTATE, TI, float>(a, "rotate64", s);
+    case TQ_F64: return launch_dense<DENSE_ROTATE, TI, double>(a, "rotate64", s);
+    default: tq_set_error("bad dtype %d", out_dtype); return TQ_ERR_ARG;
+    }
+}
+
 }  // namespace
 
 int tqk_fwht(const void *x, void *y, int64_t n, int len, int in_dtype, int out_dtype, hipStream_t s) {
     RotArgs r;
     r.d = r.pd = len;
-    r.mode = TQ_ROT_WHT;
-    r.mat = nullptr;
     r.sa = r.sb = nullptr;
     DISPATCH_IN(in_dtype, return launch_rotate<TI>(x, y, n, out_dtype, r, s));
 }
 
 int tqk_rotate64(const tq_handle *h, const void *x, void *y, int64_t n, int in_dtype, int out_dtype, int transpose,
                  hipStream_t s) {
-    const RotArgs r = rot_args(h, transpose);
-    DISPATCH_IN(in_dtype, return launch_rotate<TI>(x, y, n, out_dtype, r, s));
+    if (h->rotation == TQ_ROT_WHT) {
+        const RotArgs r = rot_args(h, transpose);
+        DISPATCH_IN(in_dtype, return launch_rotate<TI>(x, y, n, out_dtype, r, s));
+    }
+    DenseArgs a = dense_args(h, rotation_matrix(h, transpose), x, n);
+    a.out = y;
+    DISPATCH_IN(in_dtype, return launch_rotate_dense<TI>(a, out_dtype, s));
 }
 
 int tqk_nearest(const double *values, int64_t n, const double *bounds_host, int nb, int32_t *idx, hipStream_t s) {
@@ -248,49 +509,69 @@ int tqk_nearest(const double *values, int64_t n, const double *bounds_host, int 
     return tq_check_launch("nearest");
 }
 
+template <typename TI>
+static int quantize_from(const tq_handle *h, const void *x, int64_t n, uint8_t *idx, double *norms, double *rotated, hipStream_t s) {
+    if (h->rotation == TQ_ROT_WHT) {
+        const RotArgs r = rot_args(h, 0);
+        DISPATCH_VB(r.pd, (allow_lds(k_quantize64<VB, TI>, lds_bytes(r.pd)),
+                           k_quantize64<VB, TI><<<nblocks(n, r.pd), NT, lds_bytes(r.pd), s>>>((const TI *)x, n, r, h->bounds64, h->bits,
+                                                                                            idx, norms, rotated)));
+        return tq_check_launch("quantize64");
+    }
+    DenseArgs a = dense_args(h, rotation_matrix(h, 0), x, n);
+    a.out = idx;
+    a.norms_out = norms;
+    a.rotated = rotated;
+    return launch_dense<DENSE_QUANTIZE, TI, uint8_t>(a, "quantize64", s);
+}
+
 int tqk_quantize_indices(const tq_handle *h, const void *x, int64_t n, int in_dtype, uint8_t *idx, double *norms,
                          double *rotated, hipStream_t s) {
-    const RotArgs r = rot_args(h, 0);
-    DISPATCH_IN(in_dtype, DISPATCH_VB(r.pd, (allow_lds(k_quantize64<VB, TI>, lds_bytes(r.pd)),
-                                             k_quantize64<VB, TI><<<nblocks(n, r.pd), NT, lds_bytes(r.pd), s>>>(
-                                                 (const TI *)x, n, r, h->bounds64, h->n_centroids - 1, idx, norms, rotated))));
-    return tq_check_launch("quantize64");
+    DISPATCH_IN(in_dtype, return quantize_from<TI>(h, x, n, idx, norms, rotated, s));
+}
+
+template <typename TX>
+static int dequantize_to(const tq_handle *h, const uint8_t *idx, const double *norms, int64_t n, double *out, const void *x,
+                         double *residual, hipStream_t s) {
+    if (h->rotation == TQ_ROT_WHT) {
+        const RotArgs r = rot_args(h, 1);
+        DISPATCH_VB(r.pd, (allow_lds(k_dequantize64<VB, TX>, lds_bytes(r.pd)),
+                           k_dequantize64<VB, TX><<<nblocks(n, r.pd), NT, lds_bytes(r.pd), s>>>(
+                               idx, norms, n, r, h->centroids64, h->n_centroids, h->norm_correction, out, (const TX *)x, residual)));
+        return tq_check_launch("dequantize64");
+    }
+    DenseArgs a = dense_args(h, rotation_matrix(h, 1), idx, n);
+    a.norms_in = norms;
+    a.out = out;
+    a.x = x;
+    a.residual = residual;
+    return launch_dense<DENSE_DEQUANTIZE, uint8_t, TX>(a, "dequantize64", s);
 }
 
 int tqk_dequantize_indices(const tq_handle *h, const uint8_t *idx, const double *norms, int64_t n, double *out,
                            const void *x, int x_dtype, double *residual, hipStream_t s) {
-    const RotArgs r = rot_args(h, 1);
     if (!residual) x_dtype = TQ_F64;
-    DISPATCH_IN(x_dtype, DISPATCH_VB(r.pd, (allow_lds(k_dequantize64<VB, TI>, lds_bytes(r.pd)),
-                                            k_dequantize64<VB, TI><<<nblocks(n, r.pd), NT, lds_bytes(r.pd), s>>>(
-                                                idx, norms, n, r, h->centroids64, h->norm_correction, out, (const TI *)x, residual))));
-    return tq_check_launch("dequantize64");
+    DISPATCH_IN(x_dtype, return dequantize_to<TI>(h, idx, norms, n, out, x, residual, s));
 }
 
+// projections: out[j] = sum_k S[j][k] in[k] with M = S^T, and sum_k S[k][j] z[k] with M = S
 int tqk_qjl_quantize(const tq_handle *h, const void *rr, int64_t n, int in_dtype, int8_t *signs, double *norms,
                      hipStream_t s) {
-    RotArgs r;
-    r.d = r.pd = h->d;
-    r.mode = TQ_ROT_DENSE;
-    r.mat = h->proj64_t;  // out[j] = sum_k S[j][k] in[k]
-    r.sa = r.sb = nullptr;
-    DISPATCH_IN(in_dtype, DISPATCH_VB(r.pd, (allow_lds(k_qjl_quantize64<VB, TI>, lds_bytes(r.pd)),
-                                             k_qjl_quantize64<VB, TI><<<nblocks(n, r.pd), NT, lds_bytes(r.pd), s>>>(
-                                                 (const TI *)rr, n, r, signs, norms))));
-    return tq_check_launch("qjl_quantize64");
+    DenseArgs a = dense_args(h, h->proj64_t, rr, n);
+    a.out = signs;
+    a.norms_out = norms;
+    DISPATCH_IN(in_dtype, return (launch_dense<DENSE_QJL_QUANTIZE, TI, int8_t>(a, "qjl_quantize64", s)));
 }
 
 int tqk_qjl_dequantize(const tq_handle *h, const int8_t *signs, const double *norms, double shrinkage, int64_t n,
-                       double *out, hipStream_t s) {
-    RotArgs r;
-    r.d = r.pd = h->d;
-    r.mode = TQ_ROT_DENSE;
-    r.mat = h->proj64;  // out[j] = sum_k S[k][j] z[k]
-    r.sa = r.sb = nullptr;
-    DISPATCH_VB(r.pd, (allow_lds(k_qjl_dequantize64<VB>, lds_bytes(r.pd)),
-                       k_qjl_dequantize64<VB><<<nblocks(n, r.pd), NT, lds_bytes(r.pd), s>>>(signs, norms, n, r, h->proj_scale,
-                                                                                          shrinkage, out)));
-    return tq_check_launch("qjl_dequantize64");
+                       double *out, int accumulate, hipStream_t s) {
+    DenseArgs a = dense_args(h, h->proj64, signs, n);
+    a.norms_in = norms;
+    a.out = out;
+    a.proj_scale = h->proj_scale;
+    a.shrinkage = shrinkage;
+    a.accumulate = accumulate;
+    return launch_dense<DENSE_QJL_DEQUANTIZE, int8_t, double>(a, "qjl_dequantize64", s);
 }
 
 int tqk_pack_bits(const int8_t *signs, int64_t n, int d, uint8_t *packed, hipStream_t s) {

@@ -450,7 +450,7 @@ int tq_quantize_indices(const tq_handle *h, const void *x, int64_t n, int in_dty
 
 int tq_dequantize_indices(const tq_handle *h, const uint8_t *idx, const double *norms, int64_t n, double *out,
                           const void *x, int x_dtype, double *residual, void *stream) {
-    REQUIRE(h && idx && norms && out && n >= 0, TQ_ERR_ARG, "tq_dequantize_indices: bad argument");
+    REQUIRE(h && idx && norms && (out || residual) && n >= 0, TQ_ERR_ARG, "tq_dequantize_indices: bad argument");
     REQUIRE(!residual || x, TQ_ERR_ARG, "tq_dequantize_indices: residual needs x");
     if (n == 0) return TQ_OK;
     return tqk_dequantize_indices(h, idx, norms, n, out, x, x_dtype, residual, (hipStream_t)stream);
@@ -469,7 +469,15 @@ int tq_qjl_dequantize(const tq_handle *h, const int8_t *signs, const double *nor
     REQUIRE(h && signs && norms && out && n >= 0, TQ_ERR_ARG, "tq_qjl_dequantize: bad argument");
     REQUIRE(h->has_proj, TQ_ERR_ARG, "tq_qjl_dequantize: handle has no projection");
     if (n == 0) return TQ_OK;
-    return tqk_qjl_dequantize(h, signs, norms, shrinkage, n, out, (hipStream_t)stream);
+    return tqk_qjl_dequantize(h, signs, norms, shrinkage, n, out, 0, (hipStream_t)stream);
+}
+
+int tq_qjl_dequantize_add(const tq_handle *h, const int8_t *signs, const double *norms, double shrinkage, int64_t n,
+                          double *out, void *stream) {
+    REQUIRE(h && signs && norms && out && n >= 0, TQ_ERR_ARG, "tq_qjl_dequantize_add: bad argument");
+    REQUIRE(h->has_proj, TQ_ERR_ARG, "tq_qjl_dequantize_add: handle has no projection");
+    if (n == 0) return TQ_OK;
+    return tqk_qjl_dequantize(h, signs, norms, shrinkage, n, out, 1, (hipStream_t)stream);
 }
 
 int tq_pack_bits(const int8_t *signs, int64_t n, int32_t d, uint8_t *packed, void *stream) {

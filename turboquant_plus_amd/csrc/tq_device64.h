@@ -1,6 +1,6 @@
 // float64 block helpers shared by the reference-API kernels and the QJL store
-// kernel: VB vectors staged in LDS, rotated by a dense matrix read from L2 or
-// by the sign-diagonal Walsh-Hadamard butterfly in the reference's stage order.
+// kernel: VB vectors staged in LDS, rotated by the sign-diagonal Walsh-Hadamard
+// butterfly in the reference's stage order.
 #pragma once
 #include "tq_internal.h"
 
@@ -17,32 +17,15 @@ template <typename T> __device__ inline void std_(T *p, int64_t i, double v) { p
 template <> __device__ inline void std_<__half>(__half *p, int64_t i, double v) { p[i] = __float2half_rn((float)v); }
 
 struct RotArgs {
-    int d, pd, mode;        // mode: TQ_ROT_DENSE / TQ_ROT_WHT
-    const double *mat;      // dense: matrix M with out[j] = sum_k M[k*d+j] * in[k]
-    const double *sa, *sb;  // wht: signs applied before / after the butterfly (NULL = ones)
+    int d, pd;
+    const double *sa, *sb;  // signs applied before / after the butterfly (NULL = ones)
 };
 
-// in: xs[VB][pd] (entries >= d zero in WHT mode); out: ys[VB][pd].  All threads call.
+// in: xs[VB][pd] (entries >= d zero); out: ys[VB][pd].  All threads call.
 template <int VB>
 __device__ void rotate_block(const RotArgs &r, double *xs, double *ys) {
     const int tid = threadIdx.x;
-    const int d = r.d, pd = r.pd;
-    if (r.mode == TQ_ROT_DENSE) {
-        for (int j = tid; j < d; j += NT) {
-            double acc[VB];
-#pragma unroll
-            for (int v = 0; v < VB; ++v) acc[v] = 0.0;
-            for (int k = 0; k < d; ++k) {
-                const double m = r.mat[(int64_t)k * d + j];
-#pragma unroll
-                for (int v = 0; v < VB; ++v) acc[v] = fma(m, xs[v * pd + k], acc[v]);
-            }
-#pragma unroll
-            for (int v = 0; v < VB; ++v) ys[v * pd + j] = acc[v];
-        }
-        __syncthreads();
-        return;
-    }
+    const int pd = r.pd;
     if (r.sa) {
         for (int i = tid; i < VB * pd; i += NT) xs[i] *= r.sa[i % pd];
         __syncthreads();

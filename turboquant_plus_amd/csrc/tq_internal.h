@@ -75,7 +75,7 @@ int tqk_dequantize_indices(const tq_handle *h, const uint8_t *idx, const double 
 int tqk_qjl_quantize(const tq_handle *h, const void *r, int64_t n, int in_dtype, int8_t *signs, double *norms,
                      hipStream_t s);
 int tqk_qjl_dequantize(const tq_handle *h, const int8_t *signs, const double *norms, double shrinkage, int64_t n,
-                       double *out, hipStream_t s);
+                       double *out, int accumulate, hipStream_t s);
 int tqk_pack_bits(const int8_t *signs, int64_t n, int d, uint8_t *packed, hipStream_t s);
 int tqk_unpack_bits(const uint8_t *packed, int64_t n, int d, int8_t *signs, hipStream_t s);
 int tqk_pack_indices(const uint8_t *idx, int64_t count, int bits, uint8_t *packed, hipStream_t s);
