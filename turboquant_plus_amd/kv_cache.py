@@ -11,6 +11,7 @@ from dataclasses import dataclass, field
 
 import numpy as np
 
+from . import _lib as lib
 from .turboquant import CompressedVector, TurboQuant, TurboQuantMSE
 
 
@@ -26,6 +27,20 @@ class CompressedKVCache:
     head_dim: int = 0
     k_bit_width: int = 0
     v_bit_width: int = 0
+
+
+def _joined(pieces):
+    """The (layer, head) arrays one after another.  compress() hands out views that follow each other in one array: pieces
+    of one base whose memory is adjacent are taken as the stretch they are, others are copied together."""
+    pieces = [np.asarray(p) for p in pieces]
+    first = pieces[0]
+    at = first.__array_interface__["data"][0]
+    for p in pieces:
+        if (first.base is None or p.base is not first.base or p.dtype != first.dtype or p.shape != first.shape
+                or not p.flags.c_contiguous or p.__array_interface__["data"][0] != at):
+            return np.concatenate(pieces, axis=0)
+        at += p.nbytes
+    return np.lib.stride_tricks.as_strided(first, (len(pieces) * first.shape[0],) + first.shape[1:], first.strides)
 
 
 class KVCacheCompressor:
@@ -44,13 +59,14 @@ class KVCacheCompressor:
         assert v_cache.shape == k_cache.shape
         out = CompressedKVCache(num_layers=L, num_heads=H, seq_len=S, head_dim=D,
                                 k_bit_width=self.k_bits, v_bit_width=self.v_bits)
-        kc = self.k_quantizer.quantize(np.asarray(k_cache).reshape(L * H * S, D))
-        vi, vn = self.v_quantizer.quantize(np.asarray(v_cache).reshape(L * H * S, D))
-        k_idx = kc.mse_indices.reshape(L, H, S, D)
-        k_nrm = kc.vector_norms.reshape(L, H, S)
-        k_sgn = kc.qjl_signs.reshape(L, H, S, D)
-        k_rn = kc.residual_norms.reshape(L, H, S)
-        vi, vn = vi.reshape(L, H, S, D), vn.reshape(L, H, S)
+        # both tensors are on their way before the first results are waited for
+        kq, vq = self.k_quantizer, self.v_quantizer.polar_quant
+        k_block = kq._launch_quantize(lib.to_device(np.asarray(k_cache).reshape(L * H * S, D)))
+        v_block = vq._start_quantize(np.asarray(v_cache).reshape(L * H * S, D))
+        k_idx, k_nrm, k_sgn, k_rn = kq._fetch(k_block)
+        vi, vn = vq._fetch(v_block)
+        k_idx, k_sgn, vi = (a.reshape(L, H, S, D) for a in (k_idx, k_sgn, vi))
+        k_nrm, k_rn, vn = (a.reshape(L, H, S) for a in (k_nrm, k_rn, vn))
         for l in range(L):
             out.k_compressed.append([CompressedVector(k_idx[l, h], k_nrm[l, h], k_sgn[l, h], k_rn[l, h], self.k_bits)
                                      for h in range(H)])
@@ -60,16 +76,15 @@ class KVCacheCompressor:
 
     def decompress(self, compressed: CompressedKVCache):
         L, H, S, D = compressed.num_layers, compressed.num_heads, compressed.seq_len, compressed.head_dim
-        cat = lambda rows: np.concatenate([np.asarray(r).reshape(-1, *np.shape(r)[1:]) for r in rows], axis=0)
         flat = [compressed.k_compressed[l][h] for l in range(L) for h in range(H)]
         if not flat or S == 0:
             z = np.zeros((L, H, S, D))
             return z, z.copy()
-        kc = CompressedVector(cat([c.mse_indices for c in flat]), cat([c.vector_norms for c in flat]),
-                              cat([c.qjl_signs for c in flat]), cat([c.residual_norms for c in flat]), self.k_bits)
+        kc = CompressedVector(_joined([c.mse_indices for c in flat]), _joined([c.vector_norms for c in flat]),
+                              _joined([c.qjl_signs for c in flat]), _joined([c.residual_norms for c in flat]), self.k_bits)
         k = self.k_quantizer.dequantize(kc).reshape(L, H, S, D)
-        vi = cat([compressed.v_indices[l][h] for l in range(L) for h in range(H)])
-        vn = cat([compressed.v_norms[l][h] for l in range(L) for h in range(H)])
+        vi = _joined([compressed.v_indices[l][h] for l in range(L) for h in range(H)])
+        vn = _joined([compressed.v_norms[l][h] for l in range(L) for h in range(H)])
         v = self.v_quantizer.dequantize(vi, vn).reshape(L, H, S, D)
         return k, v
 

@@ -51,6 +51,30 @@ class PolarQuant:
         if a.shape[-1] != self.d:
             raise ValueError(f"{what}: last dimension must be {self.d}, got {a.shape[-1]}")
 
+    def _launch_quantize(self, xd, idx, norms):
+        """Device vectors [n, d] -> uint8 indices and float64 norms (tq_quantize_indices)."""
+        L.check(L.lib().tq_quantize_indices(self.handle.h, L.ptr(xd), xd.shape[0], L.dtype_code(xd), L.ptr(idx), L.ptr(norms),
+                                            None, L.stream_ptr()))
+
+    def _launch_residual(self, xd, idx, norms, res):
+        """xd minus the reconstruction of (uint8 idx, norms), float64."""
+        L.check(L.lib().tq_dequantize_indices(self.handle.h, L.ptr(idx), L.ptr(norms), xd.shape[0], None, L.ptr(xd),
+                                              L.dtype_code(xd), L.ptr(res), L.stream_ptr()))
+
+    def _start_quantize(self, x2):
+        """Host vectors [n, d] -> (block, indices, norms) on the device, nothing waited for after the upload."""
+        tt = L.torch()
+        xd = L.to_device(x2)
+        n = xd.shape[0]
+        buf, (idx, norms) = L.device_block(((n, self.d), tt.uint8), ((n,), tt.float64))
+        self._launch_quantize(xd, idx, norms)
+        return buf, idx, norms
+
+    @staticmethod
+    def _fetch(block):
+        buf, idx, norms = block
+        return L.fetch(buf, (idx, np.int64), (norms, np.float64))
+
     def quantize(self, x):
         """(indices int64, norms float64); 1-D input gives 1-D indices and a
         scalar norm (turboquant/polar_quant.py:56-85)."""
@@ -58,32 +82,13 @@ class PolarQuant:
         single = x.ndim == 1
         x2 = x[None, :] if single else x
         self._check(x2, "quantize")
-        tt = L.torch()
-        xd = L.to_device(x2)
-        n = xd.shape[0]
-        idx = tt.empty((n, self.d), dtype=tt.uint8, device=xd.device)
-        norms = tt.empty((n,), dtype=tt.float64, device=xd.device)
-        L.check(L.lib().tq_quantize_indices(self.handle.h, L.ptr(xd), n, L.dtype_code(xd), L.ptr(idx), L.ptr(norms),
-                                            None, L.stream_ptr()))
-        idx_h = idx.cpu().numpy().astype(np.int64)
-        norms_h = norms.cpu().numpy()
+        idx_h, norms_h = self._fetch(self._start_quantize(x2))
         return (idx_h[0], norms_h[0]) if single else (idx_h, norms_h)
 
-    def _dequantize_device(self, indices, norms, x=None):
-        tt = L.torch()
-        dev = L.require_gpu()
-        idx = tt.from_numpy(np.ascontiguousarray(indices, dtype=np.uint8)).to(dev)
-        nd = tt.from_numpy(np.ascontiguousarray(norms, dtype=np.float64)).to(dev)
-        n = idx.shape[0]
-        out = tt.empty((n, self.d), dtype=tt.float64, device=dev)
-        res = xd = None
-        if x is not None:
-            xd = L.to_device(x)
-            res = tt.empty_like(out)
-        L.check(L.lib().tq_dequantize_indices(self.handle.h, L.ptr(idx), L.ptr(nd), n, L.ptr(out), L.ptr(xd),
-                                              L.dtype_code(xd) if xd is not None else L.TQ_F64, L.ptr(res),
-                                              L.stream_ptr()))
-        return out.cpu().numpy(), (res.cpu().numpy() if res is not None else None)
+    def _launch_dequantize(self, idx, norms, out):
+        """uint8 indices and norms on the device -> float64 reconstruction."""
+        L.check(L.lib().tq_dequantize_indices(self.handle.h, L.ptr(idx), L.ptr(norms), idx.shape[0], L.ptr(out), None, L.TQ_F64,
+                                              None, L.stream_ptr()))
 
     def dequantize(self, indices, norms):
         """Reconstruction, float64 (turboquant/polar_quant.py:87-119)."""
@@ -93,18 +98,24 @@ class PolarQuant:
             indices = indices[None, :]
             norms = np.array([norms])
         self._check(indices, "dequantize")
-        if indices.size and (indices.min() < 0 or indices.max() >= self.n_centroids):
-            raise ValueError("indices out of range for this codebook")
-        out, _ = self._dequantize_device(indices, np.asarray(norms, dtype=np.float64).reshape(-1))
-        return out[0] if single else out
+        tt = L.torch()
+        idx, nrm = L.upload(L.narrow_indices(indices, self.n_centroids), L.host_norms(norms, indices.shape[0]))
+        buf, (out,) = L.device_block(((idx.shape[0], self.d), tt.float64))
+        self._launch_dequantize(idx, nrm, out)
+        out_h = L.fetch(buf, (out, np.float64))[0]
+        return out_h[0] if single else out_h
 
     def quantize_and_residual(self, x):
         """(indices, norms, x - dequantize(indices, norms)) (turboquant/polar_quant.py:121-132)."""
         x = np.asarray(x)
         single = x.ndim == 1
-        idx, norms = self.quantize(x)
         x2 = x[None, :] if single else x
-        i2 = idx[None, :] if single else idx
-        n2 = np.array([norms]) if single else norms
-        _, res = self._dequantize_device(i2, n2, x=x2)
-        return idx, norms, (res[0] if single else res)
+        self._check(x2, "quantize")
+        tt = L.torch()
+        xd = L.to_device(x2)
+        n = xd.shape[0]
+        buf, (idx, norms, res) = L.device_block(((n, self.d), tt.uint8), ((n,), tt.float64), ((n, self.d), tt.float64))
+        self._launch_quantize(xd, idx, norms)
+        self._launch_residual(xd, idx, norms, res)
+        idx_h, norms_h, res_h = L.fetch(buf, (idx, np.int64), (norms, np.float64), (res, np.float64))
+        return (idx_h[0], norms_h[0], res_h[0]) if single else (idx_h, norms_h, res_h)

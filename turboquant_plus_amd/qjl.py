@@ -44,6 +44,16 @@ class QJL:
                                     projection_scale=self.scale)
         return self._handle
 
+    def _launch_quantize(self, rd, signs, norms):
+        """Device vectors [n, d] -> int8 signs and float64 norms (tq_qjl_quantize)."""
+        L.check(L.lib().tq_qjl_quantize(self.handle.h, L.ptr(rd), rd.shape[0], L.dtype_code(rd), L.ptr(signs), L.ptr(norms),
+                                        L.stream_ptr()))
+
+    def _launch_dequantize(self, signs, norms, shrinkage, out, add=False):
+        """scale * norm * shrinkage * S^T signs into `out`, or added to what it holds."""
+        fn = L.lib().tq_qjl_dequantize_add if add else L.lib().tq_qjl_dequantize
+        L.check(fn(self.handle.h, L.ptr(signs), L.ptr(norms), float(shrinkage), signs.shape[0], L.ptr(out), L.stream_ptr()))
+
     def quantize(self, r):
         """(signs int8 in {+1,-1}, norms float64) (turboquant/qjl.py:72-94)."""
         r = np.asarray(r)
@@ -54,11 +64,9 @@ class QJL:
         tt = L.torch()
         rd = L.to_device(r2)
         n = rd.shape[0]
-        signs = tt.empty((n, self.d), dtype=tt.int8, device=rd.device)
-        norms = tt.empty((n,), dtype=tt.float64, device=rd.device)
-        L.check(L.lib().tq_qjl_quantize(self.handle.h, L.ptr(rd), n, L.dtype_code(rd), L.ptr(signs), L.ptr(norms),
-                                        L.stream_ptr()))
-        s, nn = signs.cpu().numpy(), norms.cpu().numpy()
+        buf, (signs, norms) = L.device_block(((n, self.d), tt.int8), ((n,), tt.float64))
+        self._launch_quantize(rd, signs, norms)
+        s, nn = L.fetch(buf, (signs, np.int8), (norms, np.float64))
         return (s[0], nn[0]) if single else (s, nn)
 
     def dequantize(self, signs, norms, shrinkage: float = 1.0):
@@ -68,13 +76,11 @@ class QJL:
         if single:
             signs = signs[None, :]
             norms = np.array([norms])
+        if signs.shape[-1] != self.d:
+            raise ValueError(f"dequantize: last dimension must be {self.d}")
         tt = L.torch()
-        dev = L.require_gpu()
-        sd = tt.from_numpy(np.ascontiguousarray(signs, dtype=np.int8)).to(dev)
-        nd = tt.from_numpy(np.ascontiguousarray(np.asarray(norms, dtype=np.float64).reshape(-1))).to(dev)
-        n = sd.shape[0]
-        out = tt.empty((n, self.d), dtype=tt.float64, device=dev)
-        L.check(L.lib().tq_qjl_dequantize(self.handle.h, L.ptr(sd), L.ptr(nd), float(shrinkage), n, L.ptr(out),
-                                          L.stream_ptr()))
-        res = out.cpu().numpy()
+        sd, nd = L.upload(np.ascontiguousarray(signs, dtype=np.int8), L.host_norms(norms, signs.shape[0]))
+        buf, (out,) = L.device_block(((sd.shape[0], self.d), tt.float64))
+        self._launch_dequantize(sd, nd, shrinkage, out)
+        res = L.fetch(buf, (out, np.float64))[0]
         return res[0] if single else res

@@ -6,6 +6,7 @@ from dataclasses import dataclass
 
 import numpy as np
 
+from . import _lib as L
 from .polar_quant import PolarQuant
 from .qjl import QJL
 
@@ -32,15 +33,54 @@ class TurboQuant:
                                       rotation=rotation)
         self.qjl = QJL(d, seed=seed + 1000, projection=projection)  # turboquant/turboquant.py:77
 
+    # Both directions stay on the device between the stages: indices, norms and the residual are handed over there, and
+    # only what the caller gets crosses to the host.
+    def _launch_quantize(self, xd):
+        """Device vectors [n, d] -> (block, indices uint8, norms, signs, residual norms) on the device."""
+        tt = L.torch()
+        n = xd.shape[0]
+        buf, (idx, norms, signs, rnorms) = L.device_block(((n, self.d), tt.uint8), ((n,), tt.float64), ((n, self.d), tt.int8),
+                                                          ((n,), tt.float64))
+        res = tt.empty((n, self.d), dtype=tt.float64, device=xd.device)
+        self.polar_quant._launch_quantize(xd, idx, norms)
+        self.polar_quant._launch_residual(xd, idx, norms, res)
+        self.qjl._launch_quantize(res, signs, rnorms)
+        return buf, idx, norms, signs, rnorms
+
+    @staticmethod
+    def _fetch(block):
+        buf, idx, norms, signs, rnorms = block
+        return L.fetch(buf, (idx, np.int64), (norms, np.float64), (signs, np.int8), (rnorms, np.float64))
+
     def quantize(self, x) -> CompressedVector:
-        idx, norms, residual = self.polar_quant.quantize_and_residual(x)
-        signs, rnorms = self.qjl.quantize(residual)
+        x = np.asarray(x)
+        single = x.ndim == 1
+        x2 = x[None, :] if single else x
+        self.polar_quant._check(x2, "quantize")
+        idx, norms, signs, rnorms = self._fetch(self._launch_quantize(L.to_device(x2)))
+        if single:
+            idx, norms, signs, rnorms = idx[0], norms[0], signs[0], rnorms[0]
         return CompressedVector(mse_indices=idx, vector_norms=norms, qjl_signs=signs, residual_norms=rnorms,
                                 bit_width=self.bit_width)
 
     def dequantize(self, compressed: CompressedVector, shrinkage: float = 1.0):
-        return (self.polar_quant.dequantize(compressed.mse_indices, compressed.vector_norms)
-                + self.qjl.dequantize(compressed.qjl_signs, compressed.residual_norms, shrinkage=shrinkage))
+        idx, signs = np.asarray(compressed.mse_indices), np.asarray(compressed.qjl_signs)
+        norms, rnorms = compressed.vector_norms, compressed.residual_norms
+        single = idx.ndim == 1
+        if single:
+            idx, signs, norms, rnorms = idx[None, :], signs[None, :], np.array([norms]), np.array([rnorms])
+        self.polar_quant._check(idx, "dequantize")
+        if signs.shape != idx.shape:
+            raise ValueError(f"dequantize: indices are {idx.shape} and signs {signs.shape}")
+        n = idx.shape[0]
+        tt = L.torch()
+        idx_d, norms_d, signs_d, rnorms_d = L.upload(L.narrow_indices(idx, self.polar_quant.n_centroids), L.host_norms(norms, n),
+                                                     np.ascontiguousarray(signs, dtype=np.int8), L.host_norms(rnorms, n))
+        buf, (out,) = L.device_block(((n, self.d), tt.float64))
+        self.polar_quant._launch_dequantize(idx_d, norms_d, out)
+        self.qjl._launch_dequantize(signs_d, rnorms_d, shrinkage, out, add=True)
+        out_h = L.fetch(buf, (out, np.float64))[0]
+        return out_h[0] if single else out_h
 
     def compressed_size_bits(self, n_vectors: int) -> int:
         """b bits per coordinate plus one 32-bit norm per vector (turboquant/turboquant.py:126-136)."""
