@@ -4016,7 +4016,9 @@ int tqk_store_kv(const tq_handle *hk, const tq_handle *hv, const void *k, const 
     const bool ragged = tokens != bps * TQ_ROWS_PER_BLOCK || out_bps != bps;
     // one workgroup of 12 wavefronts per CU
     const unsigned wg = 768;
-    const unsigned grid = (unsigned)((va.n_units + 11) / 12 < 256 ? (va.n_units + 11) / 12 : 256);
+    // ... as many of them as there are V tiles (a V tile occupies one wavefront for 4 to 13 us, so a short prompt takes a
+    // CU per tile, not a twelfth of one: 8 x 777 tokens ran on 10 workgroups) or rounds of K units, up to one per CU
+    const unsigned grid = (unsigned)std::min<uint32_t>(std::max(va.n_units, (ka.n_units + 11) / 12), 256u);
     if (in_dtype != TQ_F16) {  // fp32 rows
         if (hk->bits == hv->bits) {
 #define TQ_KV32(B)                                                                                                            \
