@@ -1,0 +1,61 @@
+"""Appends whose first and last token fall on, before and behind the edges of the append kernels' units: the 16-token
+groups of a V tile (a thread per row and group), the four tokens of a 16-lane row, the 128-token block.  The oracle is the
+store of the whole sequence with the same arithmetic (float64 rows for the turbo formats), byte for byte."""
+import numpy as np
+import pytest
+
+import tq_oracle as O
+import turboquant_plus_amd as tqa
+from turboquant_plus_amd import _lib as L
+from test_gpu_turbo import np_
+
+pytestmark = pytest.mark.gpu
+SPANS = [(0, 1), (0, 16), (0, 127), (1, 15), (15, 1), (15, 2), (16, 16), (17, 30), (31, 33), (47, 81), (63, 1), (63, 66), (64, 63),
+         (79, 49), (112, 16), (113, 15), (126, 3), (127, 1), (127, 130), (130, 256)]
+N_SEQS, CAPACITY, D = 2, 512, 128
+
+
+@pytest.mark.parametrize("bits", [2, 3, 4])
+@pytest.mark.parametrize("kind", ["k", "v"])
+def test_turbo_rows(bits, kind):
+    codec = tqa.TurboCodec(bits, seed=3)
+    x = np.random.default_rng(bits).standard_normal((N_SEQS, 400, D))
+    x[0, 20] = 0
+    for pos, n_new in SPANS:
+        cache = L.torch().full((tqa.packed_bytes(bits, N_SEQS, CAPACITY),), 0xA5, dtype=L.torch().uint8, device="cuda")
+        if pos:
+            codec.append(x[:, 200:200 + pos], cache, 0, CAPACITY, kind=kind)
+        codec.append(x[:, :n_new], cache, pos, CAPACITY, kind=kind)
+        want = np_(codec.store(np.concatenate([x[:, 200:200 + pos], x[:, :n_new]], axis=1), kind=kind)).reshape(N_SEQS, -1, O.block_bytes(bits))
+        got = np_(cache).reshape(N_SEQS, -1, O.block_bytes(bits))
+        assert np.array_equal(got[:, :want.shape[1]], want), (pos, n_new)
+        assert (got[:, want.shape[1]:] == 0xA5).all(), (pos, n_new)
+
+
+@pytest.mark.parametrize("kind", ["k", "v"])
+@pytest.mark.parametrize("dtype", ["float16", "float32", "float64"])
+@pytest.mark.parametrize("shift", [0, 1])
+def test_q8_0_rows(kind, dtype, shift):
+    """shift: rows that start one value behind a 16-byte boundary."""
+    tt = L.torch()
+    row = 128 * 136
+    flat = tt.randn(N_SEQS * 400 * D, generator=tt.Generator("cuda").manual_seed(5), device="cuda", dtype=tt.float32).to(getattr(tt, dtype))
+    x = flat.reshape(N_SEQS, 400, D)
+    x[0, 20] = 0
+    x[1, 3, 40] = float("inf")
+
+    def rows(lo, n):
+        buf = tt.empty(N_SEQS * n * D + 8, dtype=x.dtype, device="cuda")
+        out = buf[shift:shift + N_SEQS * n * D].view(N_SEQS, n, D)
+        out.copy_(x[:, lo:lo + n])
+        assert (out.data_ptr() % 16 != 0) == bool(shift and x.element_size() * shift % 16)
+        return out
+    for pos, n_new in SPANS:
+        cache = tt.full((N_SEQS * CAPACITY // 128 * row,), 0xA5, dtype=tt.uint8, device="cuda")
+        if pos:
+            tqa.q8_0_append(rows(200, pos), cache, 0, CAPACITY, kind=kind)
+        tqa.q8_0_append(rows(0, n_new), cache, pos, CAPACITY, kind=kind)
+        want = np_(tqa.q8_0_store(tt.cat([x[:, 200:200 + pos], x[:, :n_new]], dim=1), kind=kind)[0]).reshape(N_SEQS, -1, row)
+        got = np_(cache).reshape(N_SEQS, -1, row)
+        assert np.array_equal(got[:, :want.shape[1]], want), (pos, n_new)
+        assert (got[:, want.shape[1]:] == 0xA5).all(), (pos, n_new)

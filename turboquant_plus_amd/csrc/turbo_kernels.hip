@@ -1729,20 +1729,44 @@ __device__ __forceinline__ bool resolve_append(AppendArgs &a, int64_t wg) {
 
 __device__ inline float block_norm(const uint8_t *block, int bits, int token);
 
-// one workgroup rebuilds block `wg` (sequence wg / n_touched, touched block wg % n_touched)
+// One workgroup rebuilds block `wg` (sequence wg / n_touched, touched block wg % n_touched).
+// What bounds it is the chain of one workgroup (a chunk of 512 tokens for 32 sequences is one workgroup per CU): the
+// rows' load latency, the quantiser, the packing.  So eight wavefronts share a block, each 16-lane row requests its four
+// tokens at once before the constants' barrier, and a partly filled V tile takes its tokens on four threads per row (one
+// per 16-token group, whose dwords are its own) instead of one.
+constexpr int APPEND_THREADS = 512, APPEND_ROWS = TQ_ROWS_PER_BLOCK * 16 / APPEND_THREADS;  // tokens per 16-lane row
 template <int BITS, typename TI>
 __device__ __forceinline__ void append_block(const TI *x, uint8_t *packed, const AppendArgs &a, const int64_t wg) {
-    constexpr int NB = (1 << BITS) - 1;
+    constexpr int NB = (1 << BITS) - 1, NT = APPEND_THREADS, GROUPS = NT / 16;
     __shared__ __attribute__((aligned(16))) uint8_t codes[TQ_ROWS_PER_BLOCK * CODE_STRIDE];
     __shared__ float norms_s[TQ_ROWS_PER_BLOCK];
     __shared__ float csq_s[1 << BITS];
+    __shared__ __attribute__((aligned(16))) uint8_t old_s[block_bytes(BITS)];
 
     const int tid = threadIdx.x, lane = tid & 63;
     const int li = lane & 15, grp = tid >> 4;
     const int64_t seq = wg / a.n_touched, bis = a.first_block + wg % a.n_touched;
     const int64_t tok0 = bis * TQ_ROWS_PER_BLOCK;
     uint8_t *block = packed + (seq * a.blocks_per_seq + bis) * block_bytes(BITS);
+    const int n_old = (int)(a.pos - tok0 < 0 ? 0 : a.pos - tok0);  // rows already in the block (< 128: the block is touched)
+    const int n_end = (int)(a.pos + a.n_new - tok0 > TQ_ROWS_PER_BLOCK ? TQ_ROWS_PER_BLOCK : a.pos + a.n_new - tok0);  // first empty row
+    // K rows are tokens: the rows already there stay untouched in memory and need not be unpacked.  V rows of a block
+    // that already holds tokens: the block comes into LDS and the new tokens' codes are put into the packed rows in
+    // place (every row of the tile has one pair position per token), so nothing is unpacked or re-packed.
+    const bool keep_rows = a.kind == TQ_KIND_K, merge = n_old > 0 && !keep_rows;
+    constexpr int PIECES = block_bytes(BITS) / 16, NP = (PIECES + NT - 1) / NT;
 
+    float xv[APPEND_ROWS][8];
+#pragma unroll
+    for (int it = 0; it < APPEND_ROWS; ++it) {
+        const int t = min(max(it * GROUPS + grp, n_old), n_end - 1);  // rows outside the new ones request a new one and drop it
+        load8(x + ((seq * a.n_new + (tok0 + t - a.pos)) * 128 + 8 * li), xv[it]);
+    }
+    uint4 pre[NP];
+    if (merge) {
+#pragma unroll
+        for (int i = 0; i < NP; ++i) pre[i] = reinterpret_cast<const uint4 *>(block)[min(tid + NT * i, PIECES - 1)];
+    }
     float bnd[NB];
 #pragma unroll
     for (int k = 0; k < NB; ++k) bnd[k] = a.bounds[k];
@@ -1756,48 +1780,57 @@ __device__ __forceinline__ void append_block(const TI *x, uint8_t *packed, const
         s1v[m] = a.s1[8 * li + m];
         s2v[m] = a.s2[8 * li + m] * RSQRT128;
     }
-    // rows already in the block: the block is copied into LDS with coalesced loads and unpacked from there
-    const int n_old = (int)(a.pos - tok0 < 0 ? 0 : (a.pos - tok0 > TQ_ROWS_PER_BLOCK ? TQ_ROWS_PER_BLOCK : a.pos - tok0));
-    const int n_end = (int)(a.pos + a.n_new - tok0 > TQ_ROWS_PER_BLOCK ? TQ_ROWS_PER_BLOCK : a.pos + a.n_new - tok0);  // first empty row
-    __shared__ __attribute__((aligned(16))) uint8_t old_s[block_bytes(BITS)];
-    // K rows are tokens: the rows already there stay untouched in memory and need not be unpacked
-    const bool keep_rows = a.kind == TQ_KIND_K;
-    if (n_old > 0 && !keep_rows) {
-        // V rows of a block that already holds tokens: the new tokens' codes are put into the packed rows in
-        // place (every row of the tile has one pair position per token), so nothing is unpacked or re-packed.
-        // Rows past the new tokens keep the code of 0.0 that the block's first append gave them.
-        constexpr int PIECES = block_bytes(BITS) / 16, NP = (PIECES + 255) / 256;
-        constexpr uint32_t CM = (1u << BITS) - 1u;
-        uint4 pre[NP];
-#pragma unroll
-        for (int i = 0; i < NP; ++i) pre[i] = reinterpret_cast<const uint4 *>(block)[min(tid + 256 * i, PIECES - 1)];
-        __syncthreads();  // csq_s is ready
-#pragma unroll 1
-        for (int it = 0; it < 8; ++it) {
-            const int t = it * 16 + grp;
-            if (t < n_old || t >= n_end) continue;
-            float xv[8];
-            load8(x + ((seq * a.n_new + (tok0 + t - a.pos)) * 128 + 8 * li), xv);
-            uint2 c8;
-            const float g = quantize_vec16<BITS>(xv, lane, bnd, s1v, s2v, csq_s, a.norm_correction, c8);
-            *reinterpret_cast<uint2 *>(&codes[t * CODE_STRIDE + 8 * li]) = c8;
-            if (li == 0) norms_s[t] = g;
+    if (!merge) {
+        // rows past the new tokens hold the code of 0.0 and norm 0 (what quantising a zero vector gives)
+        for (int e = tid; e < (TQ_ROWS_PER_BLOCK - n_end) * 32; e += NT) {
+            const int t = n_end + (e >> 5), q = e & 31;
+            *reinterpret_cast<uint32_t *>(&codes[t * CODE_STRIDE + 4 * q]) = 0x01010101u * (uint32_t)a.zero_code;
         }
+    }
+    for (int t = n_end + tid; t < TQ_ROWS_PER_BLOCK; t += NT) norms_s[t] = 0.0f;
+    __syncthreads();
+
 #pragma unroll
-        for (int i = 0; i < NP; ++i)
-            if (tid + 256 * i < PIECES) reinterpret_cast<uint4 *>(old_s)[tid + 256 * i] = pre[i];
+    for (int it = 0; it < APPEND_ROWS; ++it) {
+        const int t = it * GROUPS + grp;
+        if (t < n_old || t >= n_end) continue;  // whole 16-lane rows skip together
+        uint2 c8;
+        const float g = quantize_vec16<BITS>(xv[it], lane, bnd, s1v, s2v, csq_s, a.norm_correction, c8);
+        *reinterpret_cast<uint2 *>(&codes[t * CODE_STRIDE + 8 * li]) = c8;
+        if (li == 0) norms_s[t] = g;
+    }
+    if (!merge) {
         __syncthreads();
-        if (tid < TQ_ROWS_PER_BLOCK) {
-            // new tokens take their codes; tokens from n_end to the end of their 16-token group take the code of 0.0
-            // (as do the whole groups after it, below): what tq_store writes past the end of a sequence
-            const int r = tid, rr = r & 63, t_lo = max(n_old, r & 64), t_end = (r & 64) + 64;
-            const int t_hi = min(max((n_end + 15) & ~15, t_lo), t_end);
-            for (int t = t_lo; t < t_hi; ++t) {
-                const int tl = t & 63, g = tl >> 4, k0 = (tl & 12) | ((tl >> 1) & 1), hs = (tl & 1) * BITS;
+        pack_block<BITS, NT>(codes, norms_s, block, a.kind, n_old);  // n_old > 0 only with K rows
+        return;
+    }
+#pragma unroll
+    for (int i = 0; i < NP; ++i)
+        if (tid + NT * i < PIECES) reinterpret_cast<uint4 *>(old_s)[tid + NT * i] = pre[i];
+    __syncthreads();
+    {
+        // Thread: row r (64 rows per 64-token half of the block) and a 16-token group of that half.  New tokens take their
+        // codes; tokens from n_end to the end of their group, and whole groups past it, the code of 0.0: what tq_store
+        // writes past the end of a sequence.
+        constexpr uint32_t CM = (1u << BITS) - 1u;
+        const int r = tid & 127, g = tid >> 7, rr = r & 63, base = (r & 64) + 16 * g;
+        uint8_t *rowp = old_s + r * 16 + g * 4;
+        if (base >= n_end) {
+            uint32_t fill = 0;
+#pragma unroll
+            for (int f = 0; f < 32 / BITS; ++f) fill |= (uint32_t)a.zero_code << (f * BITS);
+#pragma unroll
+            for (int j = 0; j < BITS; ++j) {
+                uint32_t w = fill;
+                if constexpr (BITS == 3) w = (fill & 0x00FFFFFFu) | (((fill & 0x00FFFFFFu) >> (8 * j)) << 24);
+                *reinterpret_cast<uint32_t *>(rowp + j * 2048) = w;
+            }
+        } else {
+            for (int tl = max(n_old - base, 0); tl < 16; ++tl) {
+                const int t = base + tl, k0 = (tl & 12) | ((tl >> 1) & 1), hs = (tl & 1) * BITS;
                 const bool fresh = t < n_end;
                 const uint32_t c0 = fresh ? codes[t * CODE_STRIDE + rr] : (uint32_t)a.zero_code;
                 const uint32_t c1 = fresh ? codes[t * CODE_STRIDE + 64 + rr] : (uint32_t)a.zero_code;
-                uint8_t *rowp = old_s + r * 16 + g * 4;
                 if (BITS == 3 && k0 >= 12) {
                     uint32_t *d0 = reinterpret_cast<uint32_t *>(rowp), *d1 = reinterpret_cast<uint32_t *>(rowp + 2048),
                              *d2 = reinterpret_cast<uint32_t *>(rowp + 4096);
@@ -1813,61 +1846,25 @@ __device__ __forceinline__ void append_block(const TI *x, uint8_t *packed, const
                     *d = (*d & ~((CM << s0) | (CM << s1))) | (c0 << s0) | (c1 << s1);
                 }
             }
-            // whole 16-token groups past the new tokens: every field the code of 0.0
-            uint32_t fill = 0;
-#pragma unroll
-            for (int f = 0; f < 32 / BITS; ++f) fill |= (uint32_t)a.zero_code << (f * BITS);
-            for (int t = max(t_hi, t_lo); t < t_end; t += 16) {
-                uint8_t *rowp = old_s + r * 16 + ((t & 63) >> 4) * 4;
-#pragma unroll
-                for (int j = 0; j < BITS; ++j) {
-                    uint32_t w = fill;
-                    if constexpr (BITS == 3) w = (fill & 0x00FFFFFFu) | (((fill & 0x00FFFFFFu) >> (8 * j)) << 24);
-                    *reinterpret_cast<uint32_t *>(rowp + j * 2048) = w;
-                }
-            }
         }
-        for (int t = n_old + tid; t < TQ_ROWS_PER_BLOCK; t += 256)
-            reinterpret_cast<__half *>(old_s + block_code_bytes(BITS))[t] = __float2half_rn(t < n_end ? norms_s[t] : 0.0f);
-        __syncthreads();
+    }
+    for (int t = n_old + tid; t < TQ_ROWS_PER_BLOCK; t += NT)
+        reinterpret_cast<__half *>(old_s + block_code_bytes(BITS))[t] = __float2half_rn(norms_s[t]);
+    __syncthreads();
 #pragma unroll
-        for (int i = 0; i < NP; ++i)
-            if (tid + 256 * i < PIECES) reinterpret_cast<uint4 *>(block)[tid + 256 * i] = reinterpret_cast<const uint4 *>(old_s)[tid + 256 * i];
-        return;
-    }
-    // rows past the new tokens hold the code of 0.0 and norm 0 (what quantising a zero vector gives)
-    for (int e = tid; e < (TQ_ROWS_PER_BLOCK - n_end) * 32; e += 256) {
-        const int t = n_end + (e >> 5), q = e & 31;
-        *reinterpret_cast<uint32_t *>(&codes[t * CODE_STRIDE + 4 * q]) = 0x01010101u * (uint32_t)a.zero_code;
-    }
-    for (int t = n_end + tid; t < TQ_ROWS_PER_BLOCK; t += 256) norms_s[t] = 0.0f;
-    __syncthreads();
-
-#pragma unroll 1
-    for (int it = 0; it < 8; ++it) {
-        const int t = it * 16 + grp;
-        if (t < n_old || t >= n_end) continue;  // whole 16-lane rows skip together
-        const int64_t rel = tok0 + t - a.pos;
-        float xv[8];
-        load8(x + ((seq * a.n_new + rel) * 128 + 8 * li), xv);
-        uint2 c8;
-        const float g = quantize_vec16<BITS>(xv, lane, bnd, s1v, s2v, csq_s, a.norm_correction, c8);
-        *reinterpret_cast<uint2 *>(&codes[t * CODE_STRIDE + 8 * li]) = c8;
-        if (li == 0) norms_s[t] = g;
-    }
-    __syncthreads();
-    pack_block<BITS, 256>(codes, norms_s, block, a.kind, keep_rows ? n_old : 0);
+    for (int i = 0; i < NP; ++i)
+        if (tid + NT * i < PIECES) reinterpret_cast<uint4 *>(block)[tid + NT * i] = reinterpret_cast<const uint4 *>(old_s)[tid + NT * i];
 }
 
 template <int BITS, typename TI>
-__global__ __launch_bounds__(256) void k_append(const TI *x, uint8_t *packed, AppendArgs a) {
+__global__ __launch_bounds__(APPEND_THREADS) void k_append(const TI *x, uint8_t *packed, AppendArgs a) {
     if (!resolve_append(a, blockIdx.x)) return;
     append_block<BITS, TI>(x, packed, a, blockIdx.x);
 }
 
 // K and V of a decode step in one launch: the first half of the grid rebuilds K blocks, the second half V blocks
 template <int KB, int VB, typename TI>
-__global__ __launch_bounds__(256) void k_append_kv(const TI *xk, uint8_t *pk, AppendArgs ka, const TI *xv, uint8_t *pv, AppendArgs va) {
+__global__ __launch_bounds__(APPEND_THREADS) void k_append_kv(const TI *xk, uint8_t *pk, AppendArgs ka, const TI *xv, uint8_t *pv, AppendArgs va) {
     const unsigned half = gridDim.x >> 1;
     if (blockIdx.x < half) {
         if (resolve_append(ka, blockIdx.x)) append_block<KB, TI>(xk, pk, ka, blockIdx.x);
@@ -3963,7 +3960,7 @@ int tqk_append_kv(const tq_handle *hk, const tq_handle *hv, const void *k, const
     const unsigned grid = 2u * (unsigned)(n_seqs * ka.n_touched);
     const int kb = hk->bits, vb = hv->bits;
 #define TQ_APPEND_KV(KB, VB)                                                                                                   \
-    DISPATCH_T(in_dtype, TI, (k_append_kv<KB, VB, TI><<<grid, 256, 0, s>>>((const TI *)k, (uint8_t *)packed_k, ka, (const TI *)v, \
+    DISPATCH_T(in_dtype, TI, (k_append_kv<KB, VB, TI><<<grid, APPEND_THREADS, 0, s>>>((const TI *)k, (uint8_t *)packed_k, ka, (const TI *)v, \
                                                                             (uint8_t *)packed_v, va)))
     if (kb == 3 && vb == 3) { TQ_APPEND_KV(3, 3); }
     else if (kb == 4 && vb == 4) { TQ_APPEND_KV(4, 4); }
@@ -3985,7 +3982,7 @@ int tqk_append(const tq_handle *h, const void *x, int64_t n_seqs, int64_t pos, i
     const AppendArgs a = make_append_args(h, pos, pos_dev, n_new, capacity, kind, overrun);
     const unsigned grid = (unsigned)(n_seqs * a.n_touched);
 #define TQ_APPEND_BITS(B) \
-    DISPATCH_T(in_dtype, TI, (k_append<B, TI><<<grid, 256, 0, s>>>((const TI *)x, (uint8_t *)packed, a)))
+    DISPATCH_T(in_dtype, TI, (k_append<B, TI><<<grid, APPEND_THREADS, 0, s>>>((const TI *)x, (uint8_t *)packed, a)))
     switch (h->bits) {
     case 2: TQ_APPEND_BITS(2); break;
     case 3: TQ_APPEND_BITS(3); break;
