@@ -2743,54 +2743,107 @@ __global__ __launch_bounds__(256) void k_q8_0_store_v_f16(const __half *x, uint8
 
 // Streaming append for both layouts: one workgroup per (sequence, touched block).  Tokens before `pos` stay, the
 // n_new tokens from `pos` on are quantised from x [n_seqs, n_new, 128], and the rest of the last touched block
-// becomes zeros (what the store kernels write past a sequence's end).  Bytes of neighbouring tokens share words in
-// the V layout; byte stores keep them apart.
+// becomes zeros (what the store kernels write past a sequence's end).  Same arithmetic as the store kernels.
+// Bound by how the rows are read and written: sixteen lanes take a token in 8-value pieces that are contiguous across
+// the lanes, all four of a lane's pieces are requested at once, and the quantised bytes pass through LDS so that a
+// wavefront stores 1 KB of a chunk in one piece (V rows: a thread gathers a dim's 16 tokens; bytes of neighbouring
+// tokens share those 16 bytes, and only the 16-token group that `pos` falls into is stored byte by byte).
+// x need not be 16-byte aligned: `wide` says whether it is.
+constexpr int Q8A_THREADS = 512, Q8A_ROW = 136;  // LDS bytes per token (an odd multiple of 8)
+struct Q8AppendArgs {
+    int64_t pos, n_new, blocks_per_seq, first_block, n_touched, capacity;
+    const int64_t *pos_dev;
+    uint32_t *overrun;
+    int wide;
+};
 template <typename TI, int KIND>
-__global__ __launch_bounds__(256) void k_q8_0_append(const TI *x, uint8_t *packed, int64_t pos, int64_t n_new,
-                                                     int64_t blocks_per_seq, int64_t first_block, int64_t n_touched,
-                                                     const int64_t *pos_dev, int64_t capacity, uint32_t *overrun) {
-    if (pos_dev) {  // the position is read when the launch runs (see resolve_append)
-        pos = *pos_dev;
-        if (!append_position_ok(pos, n_new, capacity, overrun, blockIdx.x == 0)) return;
+__device__ __forceinline__ void q8_0_append_block(const TI *x, uint8_t *packed, const Q8AppendArgs &a, const unsigned wg) {
+    __shared__ __attribute__((aligned(16))) uint8_t rows_s[TQ_ROWS_PER_BLOCK * Q8A_ROW];
+    __shared__ __attribute__((aligned(16))) __half scales_s[TQ_ROWS_PER_BLOCK * 4];  // K: [token][group], V: as stored
+    int64_t pos = a.pos, first_block = a.first_block;
+    if (a.pos_dev) {  // the position is read when the launch runs (see resolve_append)
+        pos = *a.pos_dev;
+        if (!append_position_ok(pos, a.n_new, a.capacity, a.overrun, wg == 0)) return;
         first_block = pos / TQ_ROWS_PER_BLOCK;
-        if ((int64_t)(blockIdx.x % n_touched) >= (pos + n_new - 1) / TQ_ROWS_PER_BLOCK - first_block + 1) return;
+        if ((int64_t)(wg % a.n_touched) >= (pos + a.n_new - 1) / TQ_ROWS_PER_BLOCK - first_block + 1) return;
     }
-    const int64_t seq = blockIdx.x / n_touched, bis = first_block + blockIdx.x % n_touched;
+    const int tid = threadIdx.x;
+    const int64_t seq = wg / a.n_touched, bis = first_block + wg % a.n_touched;
     const int64_t tok0 = bis * TQ_ROWS_PER_BLOCK;
-    uint8_t *block = packed + (seq * blocks_per_seq + bis) * (int64_t)(TQ_ROWS_PER_BLOCK * 136);
-    __half *scales = reinterpret_cast<__half *>(block + 8 * 2048);
-    for (int u = threadIdx.x; u < TQ_ROWS_PER_BLOCK * 4; u += 256) {
-        const int t = KIND == TQ_KIND_V ? u & 127 : u >> 2, gq = KIND == TQ_KIND_V ? u >> 7 : u & 3;
-        const int64_t tok = tok0 + t;
-        if (tok < pos) continue;
-        const bool valid = tok < pos + n_new;
-        float v[32];
+    uint8_t *block = packed + (seq * a.blocks_per_seq + bis) * (int64_t)(TQ_ROWS_PER_BLOCK * 136);
+    const int n_old = (int)(pos - tok0 < 0 ? 0 : pos - tok0);
+    const int n_end = (int)(pos + a.n_new - tok0 > TQ_ROWS_PER_BLOCK ? TQ_ROWS_PER_BLOCK : pos + a.n_new - tok0);
+    constexpr int NP = TQ_ROWS_PER_BLOCK * 16 / Q8A_THREADS;
+    const int c8 = tid & 15;  // the lane's dims: 8 c8 .. 8 c8 + 7
+    float v[NP][8];
+#pragma unroll
+    for (int i = 0; i < NP; ++i) {
+        const int t = min(max(i * (Q8A_THREADS / 16) + (tid >> 4), n_old), n_end - 1);  // others request a new row and drop it
+        const TI *p = x + (seq * a.n_new + (tok0 + t - pos)) * 128 + 8 * c8;
+        if (a.wide) {
+            load8(p, v[i]);
+        } else {
+#pragma unroll
+            for (int j = 0; j < 8; ++j) v[i][j] = ld1(p + j);
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < NP; ++i) {
+        const int t = i * (Q8A_THREADS / 16) + (tid >> 4);
         float amax = 0.0f;
 #pragma unroll
-        for (int j = 0; j < 32; ++j) {
-            v[j] = valid ? ld1(x + (seq * n_new + (tok - pos)) * 128 + gq * 32 + j) : 0.0f;
-            amax = fmaxf(amax, fabsf(v[j]));
+        for (int j = 0; j < 8; ++j) {
+            if (t >= n_end) v[i][j] = 0.0f;
+            amax = fmaxf(amax, fabsf(v[i][j]));
         }
+        amax = fmaxf(amax, xor_lane<1>(amax));
+        amax = fmaxf(amax, xor_lane<2>(amax));
         const float d = amax / 127.0f;
         const float id = d > 0.0f ? 1.0f / d : 0.0f;
-        uint32_t w[8];
+        uint32_t w[2] = {0u, 0u};
 #pragma unroll
-        for (int j = 0; j < 8; ++j) w[j] = 0;
-#pragma unroll
-        for (int j = 0; j < 32; ++j) {
-            const float tq = v[j] * id;
+        for (int j = 0; j < 8; ++j) {
+            const float tq = v[i][j] * id;
             const int qv = (int)roundf(tq);
-            if constexpr (KIND == TQ_KIND_V) block[q8v_byte(t, gq * 32 + j)] = (uint8_t)(qv & 0xFF);
-            else w[j >> 2] |= ((uint32_t)(qv & 0xFF)) << (8 * (j & 3));
+            w[j >> 2] |= ((uint32_t)(qv & 0xFF)) << (8 * (j & 3));
         }
+        *reinterpret_cast<uint2 *>(rows_s + t * Q8A_ROW + 8 * c8) = make_uint2(w[0], w[1]);
+        if ((c8 & 3) == 0) scales_s[KIND == TQ_KIND_V ? q8v_scale(t, c8 >> 2) : t * 4 + (c8 >> 2)] = __float2half_rn(d);
+    }
+    __syncthreads();
+    __half *scales = reinterpret_cast<__half *>(block + 8 * 2048);
+#pragma unroll
+    for (int i = 0; i < 1024 / Q8A_THREADS; ++i) {
+        const int u = tid + Q8A_THREADS * i;
         if constexpr (KIND == TQ_KIND_V) {
-            scales[q8v_scale(t, gq)] = __float2half_rn(d);
+            // unit = (16-token group c16 of the block, dim 64 hf + l): one 16-byte chunk of the row of dim l
+            const int l = u & 63, hf = (u >> 6) & 1, c16 = u >> 7;
+            if (16 * c16 + 16 <= n_old) continue;
+            const uint8_t *src = rows_s + 16 * c16 * Q8A_ROW + 64 * hf + l;
+            uint8_t *dst = block + (4 * hf + (c16 & 3)) * 2048 + (64 * (c16 >> 2) + l) * 16;
+            if (16 * c16 >= n_old) {
+                uint32_t w[4] = {0u, 0u, 0u, 0u};
+#pragma unroll
+                for (int e = 0; e < 16; ++e) w[e >> 2] |= (uint32_t)src[e * Q8A_ROW] << (8 * (e & 3));
+                *reinterpret_cast<uint4 *>(dst) = make_uint4(w[0], w[1], w[2], w[3]);
+            } else {
+                for (int e = n_old & 15; e < 16; ++e) dst[e] = src[e * Q8A_ROW];
+            }
         } else {
-            *reinterpret_cast<uint4 *>(block + (2 * gq) * 2048 + t * 16) = make_uint4(w[0], w[1], w[2], w[3]);
-            *reinterpret_cast<uint4 *>(block + (2 * gq + 1) * 2048 + t * 16) = make_uint4(w[4], w[5], w[6], w[7]);
-            scales[t * 4 + gq] = __float2half_rn(d);
+            const int c = u >> 7, t = u & 127;
+            if (t < n_old) continue;
+            const uint2 lo = *reinterpret_cast<const uint2 *>(rows_s + t * Q8A_ROW + 16 * c);
+            const uint2 hi = *reinterpret_cast<const uint2 *>(rows_s + t * Q8A_ROW + 16 * c + 8);
+            *reinterpret_cast<uint4 *>(block + c * 2048 + t * 16) = make_uint4(lo.x, lo.y, hi.x, hi.y);
         }
     }
+    const int ts = KIND == TQ_KIND_V ? (tid >> 8) * 64 + (tid & 63) : tid >> 2;  // the token of scale `tid`
+    if (ts >= n_old) scales[tid] = scales_s[tid];
+}
+
+template <typename TI, int KIND>
+__global__ __launch_bounds__(Q8A_THREADS) void k_q8_0_append(const TI *x, uint8_t *packed, Q8AppendArgs a) {
+    q8_0_append_block<TI, KIND>(x, packed, a, blockIdx.x);
 }
 
 __global__ __launch_bounds__(256) void k_q8_0_unpack(const uint8_t *packed, int8_t *q, float *scales, int64_t tokens,
@@ -4182,20 +4235,27 @@ int tqk_q8_0_store_v(const void *x, int64_t n_seqs, int64_t tokens, int in_dtype
     return tq_check_launch("q8_0_store_v");
 }
 
+static Q8AppendArgs make_q8_append_args(const void *x, int64_t pos, const int64_t *pos_dev, int64_t n_new, int64_t capacity,
+                                        uint32_t *overrun) {
+    Q8AppendArgs a;
+    a.pos = pos; a.pos_dev = pos_dev; a.n_new = n_new; a.capacity = capacity; a.blocks_per_seq = blocks_for(capacity);
+    a.first_block = pos / TQ_ROWS_PER_BLOCK;
+    a.n_touched = pos_dev ? (n_new + TQ_ROWS_PER_BLOCK - 2) / TQ_ROWS_PER_BLOCK + 1  // at the worst alignment
+                          : (pos + n_new - 1) / TQ_ROWS_PER_BLOCK - a.first_block + 1;
+    a.overrun = overrun;
+    a.wide = (reinterpret_cast<uintptr_t>(x) & 15u) == 0;
+    return a;
+}
+
 int tqk_q8_0_append(const void *x, int64_t n_seqs, int64_t pos, int64_t n_new, int64_t capacity, int in_dtype, int kind,
                     void *packed, hipStream_t s, const int64_t *pos_dev, uint32_t *overrun) {
     if (n_seqs == 0 || n_new == 0) return TQ_OK;
-    const int64_t bps = blocks_for(capacity);
-    const int64_t first = pos / TQ_ROWS_PER_BLOCK;
-    const int64_t n_touched = pos_dev ? (n_new + TQ_ROWS_PER_BLOCK - 2) / TQ_ROWS_PER_BLOCK + 1  // at the worst alignment
-                                      : (pos + n_new - 1) / TQ_ROWS_PER_BLOCK - first + 1;
-    const unsigned grid = (unsigned)(n_seqs * n_touched);
+    const Q8AppendArgs a = make_q8_append_args(x, pos, pos_dev, n_new, capacity, overrun);
+    const unsigned grid = (unsigned)(n_seqs * a.n_touched);
     if (kind == TQ_KIND_V) {
-        DISPATCH_T(in_dtype, TI, (k_q8_0_append<TI, TQ_KIND_V><<<grid, 256, 0, s>>>((const TI *)x, (uint8_t *)packed, pos, n_new,
-                                                                                   bps, first, n_touched, pos_dev, capacity, overrun)));
+        DISPATCH_T(in_dtype, TI, (k_q8_0_append<TI, TQ_KIND_V><<<grid, Q8A_THREADS, 0, s>>>((const TI *)x, (uint8_t *)packed, a)));
     } else {
-        DISPATCH_T(in_dtype, TI, (k_q8_0_append<TI, TQ_KIND_K><<<grid, 256, 0, s>>>((const TI *)x, (uint8_t *)packed, pos, n_new,
-                                                                                   bps, first, n_touched, pos_dev, capacity, overrun)));
+        DISPATCH_T(in_dtype, TI, (k_q8_0_append<TI, TQ_KIND_K><<<grid, Q8A_THREADS, 0, s>>>((const TI *)x, (uint8_t *)packed, a)));
     }
     return tq_check_launch("q8_0_append");
 }
