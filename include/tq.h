@@ -163,6 +163,14 @@ int tq_append(const tq_handle *h, const void *x, int64_t n_seqs, int64_t pos, in
 int tq_append_kv(const tq_handle *hk, const tq_handle *hv, const void *k, const void *v, int64_t n_seqs, int64_t pos,
                  int64_t n_new, int64_t capacity, int in_dtype, void *packed_k, void *packed_v, void *stream);
 
+/* The K and the V tokens of one step in one launch for a layer of any two formats: hk / hv NULL stands for q8_0-style
+ * rows on that side (tq_q8_0_append), whose input then needs no alignment.  pos_dev NULL: positions from `pos` on; not
+ * NULL: `pos` is ignored and *pos_dev counts, with overrun_dev as in tq_append_kv_at.  Same results as the two calls it
+ * stands for. */
+int tq_append_layer(const tq_handle *hk, const tq_handle *hv, const void *k, const void *v, int64_t n_seqs, int64_t pos,
+                    const int64_t *pos_dev, int64_t n_new, int64_t capacity, int in_dtype, void *packed_k, void *packed_v,
+                    uint32_t *overrun_dev, void *stream);
+
 /* tq_append_kv with the position read from device memory when the launch runs (*pos_dev, an int64): a decode
  * step captured once (HIP graph) can be replayed while the cache grows; the caller advances the counter
  * between replays (any kernel on the same stream).  A position that is negative or does not leave room for

@@ -59,3 +59,38 @@ def test_q8_0_rows(kind, dtype, shift):
         got = np_(cache).reshape(N_SEQS, -1, row)
         assert np.array_equal(got[:, :want.shape[1]], want), (pos, n_new)
         assert (got[:, want.shape[1]:] == 0xA5).all(), (pos, n_new)
+
+
+@pytest.mark.parametrize("fmt", [("q8_0", "q8_0"), ("q8_0", "turbo2"), ("q8_0", "turbo3"), ("q8_0", "turbo4"), ("turbo2", "q8_0"),
+                                 ("turbo3", "q8_0"), ("turbo4", "q8_0")])
+@pytest.mark.parametrize("dtypes", [("float16", "float16"), ("float32", "float32"), ("float64", "float64"), ("float16", "float32")])
+def test_layer_with_8_bit_rows(fmt, dtypes):
+    """K and V of a step in one launch write the bytes of an append per side, with the position on the host and on the
+    device; rows of different types keep taking two calls, and a position that does not fit writes nothing."""
+    tt = L.torch()
+    layer = tqa.LayerKV(tqa.LayerFormat(*fmt))
+    gen = tt.Generator("cuda").manual_seed(1)
+    k = tt.randn((N_SEQS, 400, D), generator=gen, device="cuda").to(getattr(tt, dtypes[0]))
+    v = tt.randn((N_SEQS, 400, D), generator=gen, device="cuda").to(getattr(tt, dtypes[1]))
+    one, two, dev = (layer.new_cache(N_SEQS, CAPACITY) for _ in range(3))
+    over = tt.zeros(1, dtype=tt.int32, device="cuda")
+    pos = 0
+    for n_new in (1, 14, 2, 47, 63, 2, 258):
+        kn, vn = k[:, pos:pos + n_new], v[:, pos:pos + n_new]
+        layer.append(kn, vn, *one, pos, CAPACITY)
+        layer.append(kn, vn, *dev, tt.tensor([pos], device="cuda"), CAPACITY, overrun=over)
+        for codec, x, buf, kind in ((layer.k_codec, kn, two[0], "k"), (layer.v_codec, vn, two[1], "v")):
+            if codec is None:
+                tqa.q8_0_append(x, buf, pos, CAPACITY, kind=kind)
+            else:
+                codec.append(x, buf, pos, CAPACITY, kind=kind)
+        pos += n_new
+        for a, b, c in zip(one, two, dev):
+            assert tt.equal(a, b) and tt.equal(c, b), (pos, n_new)
+    assert int(over) == 0
+    layer.append(k[:, :9], v[:, :9], *dev, tt.tensor([CAPACITY - 8], device="cuda"), CAPACITY, overrun=over)
+    assert int(over) != 0 and all(tt.equal(c, b) for b, c in zip(two, dev))
+    with pytest.raises(ValueError):
+        layer.append(k[:, :9], v[:, :9], *one, CAPACITY - 8, CAPACITY)
+    with pytest.raises(ValueError):
+        layer.append(k[:, :1], v[:, :1], one[0], one[1][:-16], 0, CAPACITY)

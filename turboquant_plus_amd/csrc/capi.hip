@@ -558,6 +558,26 @@ int tq_append_kv(const tq_handle *hk, const tq_handle *hv, const void *k, const 
     return tqk_append_kv(hk, hv, k, v, n_seqs, pos, n_new, capacity, in_dtype, packed_k, packed_v, (hipStream_t)stream);
 }
 
+int tq_append_layer(const tq_handle *hk, const tq_handle *hv, const void *k, const void *v, int64_t n_seqs, int64_t pos,
+                    const int64_t *pos_dev, int64_t n_new, int64_t capacity, int in_dtype, void *packed_k, void *packed_v,
+                    uint32_t *overrun_dev, void *stream) {
+    int rc = hk ? check_fast(hk, "tq_append_layer") : TQ_OK;
+    rc = rc ? rc : hv ? check_fast(hv, "tq_append_layer") : TQ_OK;
+    if (rc) return rc;
+    REQUIRE(n_seqs >= 0 && n_new >= 0 && capacity >= 0 && (pos_dev || pos >= 0), TQ_ERR_ARG, "tq_append_layer: bad argument");
+    if (pos_dev) pos = 0;
+    REQUIRE(n_new <= capacity && pos <= capacity - n_new, TQ_ERR_ARG, "tq_append_layer: %lld tokens from %lld on do not fit a capacity of %lld",
+            (long long)n_new, (long long)pos, (long long)capacity);
+    if (n_seqs == 0 || n_new == 0) return TQ_OK;
+    REQUIRE(k && v && packed_k && packed_v, TQ_ERR_ARG, "tq_append_layer: null pointer");
+    REQUIRE((!hk || aligned16(k)) && (!hv || aligned16(v)) && aligned16(packed_k) && aligned16(packed_v), TQ_ERR_ALIGN,
+            "tq_append_layer: packed buffers and the inputs of turbo formats must be 16-byte aligned");
+    REQUIRE((reinterpret_cast<uintptr_t>(pos_dev) & 7u) == 0, TQ_ERR_ALIGN, "tq_append_layer: pos_dev must be 8-byte aligned");
+    REQUIRE((reinterpret_cast<uintptr_t>(overrun_dev) & 3u) == 0, TQ_ERR_ALIGN, "tq_append_layer: overrun_dev must be 4-byte aligned");
+    return tqk_append_kv(hk, hv, k, v, n_seqs, pos, n_new, capacity, in_dtype, packed_k, packed_v, (hipStream_t)stream, pos_dev,
+                         overrun_dev);
+}
+
 int tq_append_at(const tq_handle *h, const void *x, int64_t n_seqs, const int64_t *pos_dev, int64_t n_new, int64_t capacity,
                  int in_dtype, int kind, void *packed, uint32_t *overrun_dev, void *stream) {
     int rc = check_fast(h, "tq_append_at");

@@ -1862,17 +1862,6 @@ __global__ __launch_bounds__(APPEND_THREADS) void k_append(const TI *x, uint8_t 
     append_block<BITS, TI>(x, packed, a, blockIdx.x);
 }
 
-// K and V of a decode step in one launch: the first half of the grid rebuilds K blocks, the second half V blocks
-template <int KB, int VB, typename TI>
-__global__ __launch_bounds__(APPEND_THREADS) void k_append_kv(const TI *xk, uint8_t *pk, AppendArgs ka, const TI *xv, uint8_t *pv, AppendArgs va) {
-    const unsigned half = gridDim.x >> 1;
-    if (blockIdx.x < half) {
-        if (resolve_append(ka, blockIdx.x)) append_block<KB, TI>(xk, pk, ka, blockIdx.x);
-    } else {
-        if (resolve_append(va, blockIdx.x - half)) append_block<VB, TI>(xv, pv, va, blockIdx.x - half);
-    }
-}
-
 // ---- K2 + K4 in float64: codes, corrected norm, residual sign sketch ---------------
 struct StoreQjlArgs {
     const double *s1, *s2, *bounds, *cent;
@@ -2844,6 +2833,24 @@ __device__ __forceinline__ void q8_0_append_block(const TI *x, uint8_t *packed, 
 template <typename TI, int KIND>
 __global__ __launch_bounds__(Q8A_THREADS) void k_q8_0_append(const TI *x, uint8_t *packed, Q8AppendArgs a) {
     q8_0_append_block<TI, KIND>(x, packed, a, blockIdx.x);
+}
+
+// K and V of a decode step in one launch: the first half of the grid rebuilds K blocks, the second half V blocks.  A
+// width of 0 stands for q8_0-style rows: 8-bit K with turbo V took two launches and two calls into the library.
+template <int BITS> struct AppendSide { using Args = AppendArgs; };
+template <> struct AppendSide<0> { using Args = Q8AppendArgs; };
+template <int BITS, int KIND, typename TI>
+__device__ __forceinline__ void append_side(const TI *x, uint8_t *packed, typename AppendSide<BITS>::Args &a, const unsigned wg) {
+    if constexpr (BITS == 0) q8_0_append_block<TI, KIND>(x, packed, a, wg);
+    else if (resolve_append(a, wg)) append_block<BITS, TI>(x, packed, a, wg);
+}
+static_assert(APPEND_THREADS == Q8A_THREADS, "both kinds of rows run in one launch");
+template <int KB, int VB, typename TI>
+__global__ __launch_bounds__(APPEND_THREADS) void k_append_kv(const TI *xk, uint8_t *pk, typename AppendSide<KB>::Args ka, const TI *xv,
+                                                              uint8_t *pv, typename AppendSide<VB>::Args va) {
+    const unsigned half = gridDim.x >> 1;
+    if (blockIdx.x < half) append_side<KB, TQ_KIND_K, TI>(xk, pk, ka, blockIdx.x);
+    else append_side<VB, TQ_KIND_V, TI>(xv, pv, va, blockIdx.x - half);
 }
 
 __global__ __launch_bounds__(256) void k_q8_0_unpack(const uint8_t *packed, int8_t *q, float *scales, int64_t tokens,
@@ -4004,26 +4011,52 @@ static AppendArgs make_append_args(const tq_handle *h, int64_t pos, const int64_
     return a;
 }
 
+static Q8AppendArgs make_q8_append_args(const void *x, int64_t pos, const int64_t *pos_dev, int64_t n_new, int64_t capacity,
+                                        uint32_t *overrun) {
+    Q8AppendArgs a;
+    a.pos = pos; a.pos_dev = pos_dev; a.n_new = n_new; a.capacity = capacity; a.blocks_per_seq = blocks_for(capacity);
+    a.first_block = pos / TQ_ROWS_PER_BLOCK;
+    a.n_touched = pos_dev ? (n_new + TQ_ROWS_PER_BLOCK - 2) / TQ_ROWS_PER_BLOCK + 1  // at the worst alignment
+                          : (pos + n_new - 1) / TQ_ROWS_PER_BLOCK - a.first_block + 1;
+    a.overrun = overrun;
+    a.wide = (reinterpret_cast<uintptr_t>(x) & 15u) == 0;
+    return a;
+}
+
+// hk / hv NULL: q8_0-style rows on that side
 int tqk_append_kv(const tq_handle *hk, const tq_handle *hv, const void *k, const void *v, int64_t n_seqs, int64_t pos,
                   int64_t n_new, int64_t capacity, int in_dtype, void *packed_k, void *packed_v, hipStream_t s,
                   const int64_t *pos_dev, uint32_t *overrun) {
     if (n_seqs == 0 || n_new == 0) return TQ_OK;
-    const AppendArgs ka = make_append_args(hk, pos, pos_dev, n_new, capacity, TQ_KIND_K, overrun);
-    const AppendArgs va = make_append_args(hv, pos, pos_dev, n_new, capacity, TQ_KIND_V);  // the K half reports
-    const unsigned grid = 2u * (unsigned)(n_seqs * ka.n_touched);
-    const int kb = hk->bits, vb = hv->bits;
-#define TQ_APPEND_KV(KB, VB)                                                                                                   \
-    DISPATCH_T(in_dtype, TI, (k_append_kv<KB, VB, TI><<<grid, APPEND_THREADS, 0, s>>>((const TI *)k, (uint8_t *)packed_k, ka, (const TI *)v, \
-                                                                            (uint8_t *)packed_v, va)))
-    if (kb == 3 && vb == 3) { TQ_APPEND_KV(3, 3); }
-    else if (kb == 4 && vb == 4) { TQ_APPEND_KV(4, 4); }
-    else if (kb == 2 && vb == 2) { TQ_APPEND_KV(2, 2); }
-    else if (kb == 4 && vb == 2) { TQ_APPEND_KV(4, 2); }
-    else if (kb == 3 && vb == 2) { TQ_APPEND_KV(3, 2); }
-    else if (kb == 4 && vb == 3) { TQ_APPEND_KV(4, 3); }
-    else {  // other pairs: two launches
+    const Q8AppendArgs qk = make_q8_append_args(k, pos, pos_dev, n_new, capacity, pos_dev ? overrun : nullptr);
+    const Q8AppendArgs qv = make_q8_append_args(v, pos, pos_dev, n_new, capacity, nullptr);  // the K half reports
+    AppendArgs ka{}, va{};
+    if (hk) ka = make_append_args(hk, pos, pos_dev, n_new, capacity, TQ_KIND_K, overrun);
+    if (hv) va = make_append_args(hv, pos, pos_dev, n_new, capacity, TQ_KIND_V);
+    const unsigned grid = 2u * (unsigned)(n_seqs * qk.n_touched);
+    const int kb = hk ? hk->bits : 0, vb = hv ? hv->bits : 0;
+#define TQ_APPEND_KV(KB, VB, KA, VA)                                                                                           \
+    DISPATCH_T(in_dtype, TI, (k_append_kv<KB, VB, TI><<<grid, APPEND_THREADS, 0, s>>>((const TI *)k, (uint8_t *)packed_k, KA,  \
+                                                                                      (const TI *)v, (uint8_t *)packed_v, VA)));
+    switch (8 * kb + vb) {
+    case 8 * 3 + 3: TQ_APPEND_KV(3, 3, ka, va) break;
+    case 8 * 4 + 4: TQ_APPEND_KV(4, 4, ka, va) break;
+    case 8 * 2 + 2: TQ_APPEND_KV(2, 2, ka, va) break;
+    case 8 * 4 + 2: TQ_APPEND_KV(4, 2, ka, va) break;
+    case 8 * 3 + 2: TQ_APPEND_KV(3, 2, ka, va) break;
+    case 8 * 4 + 3: TQ_APPEND_KV(4, 3, ka, va) break;
+    case 2: TQ_APPEND_KV(0, 2, qk, va) break;
+    case 3: TQ_APPEND_KV(0, 3, qk, va) break;
+    case 4: TQ_APPEND_KV(0, 4, qk, va) break;
+    case 8 * 2: TQ_APPEND_KV(2, 0, ka, qv) break;
+    case 8 * 3: TQ_APPEND_KV(3, 0, ka, qv) break;
+    case 8 * 4: TQ_APPEND_KV(4, 0, ka, qv) break;
+    case 0: TQ_APPEND_KV(0, 0, qk, qv) break;
+    default: {  // turbo V wider than turbo K: two launches
+        if (!hk || !hv) { tq_set_error("tq_append_layer: bits must be 2, 3 or 4 (got %d and %d)", kb, vb); return TQ_ERR_UNSUPPORTED; }
         const int rc = tqk_append(hk, k, n_seqs, pos, n_new, capacity, in_dtype, TQ_KIND_K, packed_k, s, pos_dev, overrun);
         return rc ? rc : tqk_append(hv, v, n_seqs, pos, n_new, capacity, in_dtype, TQ_KIND_V, packed_v, s, pos_dev, overrun);
+    }
     }
 #undef TQ_APPEND_KV
     return tq_check_launch("append_kv");
@@ -4233,18 +4266,6 @@ int tqk_q8_0_store_v(const void *x, int64_t n_seqs, int64_t tokens, int in_dtype
     }
     DISPATCH_T(in_dtype, TI, (k_q8_0_store_v<TI><<<grid, 256, 0, s>>>((const TI *)x, (uint8_t *)packed, tokens, bps)));
     return tq_check_launch("q8_0_store_v");
-}
-
-static Q8AppendArgs make_q8_append_args(const void *x, int64_t pos, const int64_t *pos_dev, int64_t n_new, int64_t capacity,
-                                        uint32_t *overrun) {
-    Q8AppendArgs a;
-    a.pos = pos; a.pos_dev = pos_dev; a.n_new = n_new; a.capacity = capacity; a.blocks_per_seq = blocks_for(capacity);
-    a.first_block = pos / TQ_ROWS_PER_BLOCK;
-    a.n_touched = pos_dev ? (n_new + TQ_ROWS_PER_BLOCK - 2) / TQ_ROWS_PER_BLOCK + 1  // at the worst alignment
-                          : (pos + n_new - 1) / TQ_ROWS_PER_BLOCK - a.first_block + 1;
-    a.overrun = overrun;
-    a.wide = (reinterpret_cast<uintptr_t>(x) & 15u) == 0;
-    return a;
 }
 
 int tqk_q8_0_append(const void *x, int64_t n_seqs, int64_t pos, int64_t n_new, int64_t capacity, int in_dtype, int kind,

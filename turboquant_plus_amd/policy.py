@@ -20,7 +20,7 @@ from __future__ import annotations
 from dataclasses import dataclass
 
 from . import _lib as L
-from .turbo import DecodeAttention, TurboCodec, packed_bytes, q8_0_append, q8_0_store
+from .turbo import DecodeAttention, TurboCodec, append_layer, packed_bytes, q8_0_append, q8_0_store
 
 FORMATS = ("q8_0", "turbo4", "turbo3", "turbo2")
 
@@ -122,14 +122,19 @@ class LayerKV:
         if self.k_codec is not None and self.v_codec is not None:
             self.k_codec.append_kv(self.v_codec, k, v, k_cache, v_cache, pos, capacity, overrun=overrun)
             return k_cache, v_cache
+        kd, n_seqs, n_new = TurboCodec._as_seqs(k)
+        vd, vs, vn = TurboCodec._as_seqs(v)
+        if (vs, vn) == (n_seqs, n_new) and vd.dtype == kd.dtype:   # q8_0-style rows on either side: one launch too
+            append_layer(self.k_codec, self.v_codec, kd, vd, n_seqs, n_new, k_cache, v_cache, pos, capacity, overrun)
+            return k_cache, v_cache
         if self.k_codec is None:
-            q8_0_append(k, k_cache, pos, capacity, kind="k", overrun=overrun)
+            q8_0_append(kd, k_cache, pos, capacity, kind="k", overrun=overrun)
         else:
-            self.k_codec.append(k, k_cache, pos, capacity, kind="k", overrun=overrun)
+            self.k_codec.append(kd, k_cache, pos, capacity, kind="k", overrun=overrun)
         if self.v_codec is None:
-            q8_0_append(v, v_cache, pos, capacity, kind="v", overrun=overrun)
+            q8_0_append(vd, v_cache, pos, capacity, kind="v", overrun=overrun)
         else:
-            self.v_codec.append(v, v_cache, pos, capacity, kind="v", overrun=overrun)
+            self.v_codec.append(vd, v_cache, pos, capacity, kind="v", overrun=overrun)
         return k_cache, v_cache
 
     def prefill(self, k, v, k_cache, v_cache, capacity: int):

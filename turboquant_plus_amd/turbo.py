@@ -398,6 +398,21 @@ def q8_0_append(x, packed, pos, capacity: int, kind: str = "k", overrun=None):
     return packed
 
 
+def append_layer(k_codec, v_codec, kd, vd, n_seqs: int, n_new: int, k_cache, v_cache, pos, capacity: int, overrun=None):
+    """The K and V tokens of one step in one launch, a codec of None standing for q8_0-style rows (tq_append_layer);
+    kd, vd: device tensors [n_seqs, n_new, 128] of one dtype.  LayerKV.append's way for layers with 8-bit rows."""
+    lib = L.lib()
+    for codec, buf in ((k_codec, k_cache), (v_codec, v_cache)):
+        need = int(lib.tq_q8_0_bytes(n_seqs, capacity)) if codec is None else packed_bytes(codec.bits, n_seqs, capacity)
+        if buf.numel() < need:
+            raise ValueError(f"packed holds {buf.numel()} bytes, need {need}")
+    on_device = _position_on_device(pos)
+    L.check(lib.tq_append_layer(None if k_codec is None else k_codec.handle.h, None if v_codec is None else v_codec.handle.h,
+                                L.ptr(kd), L.ptr(vd), n_seqs, 0 if on_device else pos, L.ptr(pos) if on_device else None, n_new,
+                                capacity, L.dtype_code(kd), L.ptr(k_cache), L.ptr(v_cache),
+                                _overrun_ptr(overrun) if on_device else None, L.stream_ptr()))
+
+
 def q8_0_unpack(packed, n_seqs: int, tokens: int, kind: str = "k"):
     """int8 values [n_seqs, tokens, 128] and fp32 scales [n_seqs, tokens, 4] of a q8_0_store buffer."""
     tt = L.torch()
