@@ -462,6 +462,9 @@ class DecodeAttention:
                                       eight_heads=head_dim == HEAD_DIM and n_q_heads // max(n_kv_heads, 1) > 4,
                                       turbo_rows=k_codec is not None and v_codec is not None,
                                       one_workgroup_per_cu=v_codec is None or (head_dim != HEAD_DIM and k_codec is None))
+            if head_dim == HEAD_DIM:
+                n_splits = balanced_splits(batch * n_kv_heads, tokens, n_splits, eight_heads=n_q_heads // max(n_kv_heads, 1) > 4,
+                                           turbo_k=k_codec is not None, turbo_v=v_codec is not None)
         self.params = L.TQAttnParams(batch=batch, n_q_heads=n_q_heads, n_kv_heads=n_kv_heads, tokens=tokens,
                                      capacity=capacity, n_splits=n_splits, k_format=L.KFMT_TURBO if k_codec is not None else L.KFMT_Q8_0,
                                      v_format=L.KFMT_TURBO if v_codec is not None else L.KFMT_Q8_0,
@@ -590,3 +593,61 @@ def default_splits(n_groups: int, tokens: int, eight_heads: bool = False, turbo_
     if n >= 16:
         return n // 16 * 16
     return 1 << (n.bit_length() - 1)
+
+
+def _workgroups(n: int, n_groups: int, eight_heads: bool, turbo_k: bool, turbo_v: bool) -> tuple[int, int, int]:
+    """(wavefronts per workgroup, partials per group, workgroups) that the library runs `n` splits with (attn_plan)."""
+    most = 8 if not turbo_v or eight_heads else 16
+    if n < most and most % n == 0:     # several groups in a workgroup
+        share = most // n
+        while share > 1 and (n_groups % share or n_groups // share < 256):
+            share >>= 1
+        if share > 1:
+            return share * n, 1, n_groups // share
+    waves = 12 if eight_heads and turbo_k and turbo_v and n % 12 == 0 else most
+    while n % waves:
+        waves >>= 1
+    while waves > 4 and waves % 2 == 0 and n_groups * (n // waves) < 256:
+        waves >>= 1
+    return waves, n // waves, n_groups * n // waves
+
+
+# What a step takes, in microseconds: a constant, per tile that the fullest CU works through, per tile on the longest
+# wavefront of each round of workgroups, per partial of a group to merge, per round; and the wavefronts that a CU holds.
+# Fitted to 1300 timings (4 to 192 groups, 21 to 938 tiles of 64 tokens, 8 to 16 split counts each) to 6 - 8 %.
+_SPLIT_COST = {  # by (more than four heads per KV head, turbo V rows); 8-bit V rows: one line for both
+    (False, True): (2.85, 0.22, 0.41, 0.08, 7.42, 16),
+    (False, False): (5.2, 0.36, 0.0, 0.11, 5.2, 8),
+    (True, True): (6.09, 0.34, 0.72, 0.21, 7.2, 8),
+}
+_SPLIT_COUNTS = (8, 12, 16, 20, 24, 28, 32, 36, 40, 48, 56, 64, 72, 80, 96, 112, 128, 160, 192, 256)
+
+
+def balanced_splits(n_groups: int, tokens: int, default: int, *, eight_heads: bool, turbo_k: bool, turbo_v: bool) -> int:
+    """The split count for 128-dim heads: `default` (default_splits) unless another count spreads the tiles over the CUs
+    clearly better.  default_splits aims at a number of wavefronts and rounds down to multiples of 16, which suits group
+    counts and lengths that are powers of two.  With others it makes little more than a round of the 256 workgroups that fit
+    (20 groups: 320 workgroups of six), gives short contexts half the wavefronts they could use (63 tiles: 16 splits for 31),
+    or hundreds of partials to merge (two groups: 528 splits).  The estimate counts what the fullest CU has to do; another
+    count is taken where it is put 12 % below the default (18 % for eight heads on 8-bit V rows, whose fit is the poorest; its
+    error is 6 - 8 %).  Of 178 shapes measured that it would order differently 73 pass that line: all faster, 19 % on
+    average; at 5 % 21 of 110 were slower, by up to 12 %.  Default and this rule: 20 groups at 115 800 tokens, eight heads:
+    1.36 times as fast with 72 splits for 96; 40 groups at 25 000 tokens: 72.0 and 48.2 us (36 for 48); 8 groups at 4000, four
+    heads: 14.6 and 13.6 us (32 for 16); 144 groups at 13 000, four heads: 1.37 times (28 for 8)."""
+    cost = _SPLIT_COST.get((eight_heads, turbo_v), _SPLIT_COST[(False, False)])
+    tiles = max(1, (tokens + 63) // 64)
+
+    def estimate(n):
+        waves, parts, wgs = _workgroups(n, n_groups, eight_heads, turbo_k, turbo_v)
+        per_cu, deep = -(-wgs // 256), -(-tiles // n)
+        rounds = -(-per_cu // max(1, cost[5] // waves))
+        return cost[0] + cost[1] * per_cu * waves * deep + cost[2] * rounds * deep + cost[3] * parts + cost[4] * rounds
+
+    # two tiles per wavefront at least; 256 to 8192 wavefronts, the range of the fit; eight heads: at most three rounds (with
+    # four the estimate was wrong by 30 %)
+    counts = [n for n in _SPLIT_COUNTS if n <= tiles // 2 + 1 and 256 <= n * n_groups <= 8192
+              and (not eight_heads or _workgroups(n, n_groups, eight_heads, turbo_k, turbo_v)[2] <= 768)]
+    if not counts:
+        return default
+    best = min(counts, key=estimate)
+    return best if estimate(best) < (0.88 if turbo_v or not eight_heads else 0.82) * estimate(default) else default
