@@ -98,6 +98,9 @@ int main() {
     EXPECT(tq_q8_0_append_at(ok, 1, (const int64_t *)ok, 129, 128, TQ_F16, TQ_KIND_K, ok, nullptr, nullptr) == TQ_ERR_ARG);
     EXPECT(tq_append_at(nullptr, ok, 1, (const int64_t *)ok, 1, 128, TQ_F16, TQ_KIND_K, ok, nullptr, nullptr) == TQ_ERR_ARG);
     EXPECT(tq_append_kv_at(nullptr, nullptr, ok, ok, 1, (const int64_t *)ok, 1, 128, TQ_F16, ok, ok, nullptr, nullptr) == TQ_ERR_ARG);
+    EXPECT(tq_store_layer(nullptr, nullptr, ok, ok, 1, 129, 128, TQ_F16, ok, ok, nullptr) == TQ_ERR_ARG);
+    EXPECT(tq_store_layer(nullptr, nullptr, ok, nullptr, 1, 1, 128, TQ_F16, ok, ok, nullptr) == TQ_ERR_ARG);
+    EXPECT(tq_store_layer(nullptr, nullptr, ok, ok, 0, 1, 128, TQ_F16, ok, ok, nullptr) == TQ_OK);
     EXPECT(tq_append_layer(nullptr, nullptr, ok, ok, 1, 0, nullptr, 129, 128, TQ_F16, ok, ok, nullptr, nullptr) == TQ_ERR_ARG);
     EXPECT(tq_append_layer(nullptr, nullptr, ok, ok, 1, -1, nullptr, 1, 128, TQ_F16, ok, ok, nullptr, nullptr) == TQ_ERR_ARG);
     EXPECT(tq_append_layer(nullptr, nullptr, nullptr, ok, 1, 0, nullptr, 1, 128, TQ_F16, ok, ok, nullptr, nullptr) == TQ_ERR_ARG);

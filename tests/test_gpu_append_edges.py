@@ -94,3 +94,24 @@ def test_layer_with_8_bit_rows(fmt, dtypes):
         layer.append(k[:, :9], v[:, :9], *one, CAPACITY - 8, CAPACITY)
     with pytest.raises(ValueError):
         layer.append(k[:, :1], v[:, :1], one[0], one[1][:-16], 0, CAPACITY)
+
+
+@pytest.mark.parametrize("fmt", [("q8_0", "turbo3"), ("q8_0", "turbo4"), ("turbo2", "q8_0"), ("turbo4", "q8_0")])
+@pytest.mark.parametrize("dtype", ["float16", "float32", "float64"])
+@pytest.mark.parametrize("tokens", [1023, 1025, 1152])
+def test_prompt_of_a_layer_with_8_bit_rows(fmt, dtype, tokens):
+    """64 sequences of 8 (one launch of the append kernel for K and V at float64 only) and 9 blocks: the 8-bit side as
+    appended, the turbo side as stored, sequence by sequence, and nothing past a sequence's last block."""
+    tt = L.torch()
+    n, capacity = 64, 2048
+    layer = tqa.LayerKV(tqa.LayerFormat(*fmt))
+    gen = tt.Generator("cuda").manual_seed(tokens)
+    k, v = (tt.randn((n, tokens, D), generator=gen, device="cuda").to(getattr(tt, dtype)) for _ in range(2))
+    caches = [b.fill_(0xA5) for b in layer.new_cache(n, capacity)]
+    layer.prefill(k, v, *caches, capacity)
+    for codec, x, cache, kind in ((layer.k_codec, k, caches[0], "k"), (layer.v_codec, v, caches[1], "v")):
+        want = tqa.q8_0_store(x, kind=kind)[0] if codec is None else codec.store(x, kind=kind)
+        blocks = -(-tokens // 128)
+        got = cache.view(n, capacity // 128, -1)
+        assert tt.equal(got[:, :blocks], want.view(n, blocks, -1)), kind
+        assert bool((got[:, blocks:] == 0xA5).all()), kind

@@ -67,6 +67,7 @@ PROTOTYPES = {
     "tq_store_kv_cache": (_I, [_P, _P, _P, _P, _L, _L, _L, _I, _P, _P, _P]),
     "tq_append": (_I, [_P, _P, _L, _L, _L, _L, _I, _I, _P, _P]),
     "tq_append_kv": (_I, [_P, _P, _P, _P, _L, _L, _L, _L, _I, _P, _P, _P]),
+    "tq_store_layer": (_I, [_P, _P, _P, _P, _L, _L, _L, _I, _P, _P, _P]),
     "tq_append_layer": (_I, [_P, _P, _P, _P, _L, _L, _P, _L, _L, _I, _P, _P, _P, _P]),
     "tq_append_kv_at": (_I, [_P, _P, _P, _P, _L, _P, _L, _L, _I, _P, _P, _P, _P]),
     "tq_append_at": (_I, [_P, _P, _L, _P, _L, _L, _I, _I, _P, _P, _P]),

@@ -704,6 +704,21 @@ int tq_store_kv(const tq_handle *hk, const tq_handle *hv, const void *k, const v
     return tqk_store_kv(hk, hv, k, v, n_seqs, tokens, 0, in_dtype, packed_k, packed_v, (hipStream_t)stream);
 }
 
+int tq_store_layer(const tq_handle *hk, const tq_handle *hv, const void *k, const void *v, int64_t n_seqs, int64_t tokens,
+                   int64_t capacity, int in_dtype, void *packed_k, void *packed_v, void *stream) {
+    int rc = hk ? check_fast(hk, "tq_store_layer") : TQ_OK;
+    rc = rc ? rc : hv ? check_fast(hv, "tq_store_layer") : TQ_OK;
+    if (rc) return rc;
+    REQUIRE(n_seqs >= 0 && tokens >= 0 && capacity >= 0, TQ_ERR_ARG, "tq_store_layer: bad argument");
+    REQUIRE(tokens <= capacity, TQ_ERR_ARG, "tq_store_layer: %lld tokens do not fit a capacity of %lld", (long long)tokens,
+            (long long)capacity);
+    if (n_seqs == 0 || tokens == 0) return TQ_OK;
+    REQUIRE(k && v && packed_k && packed_v, TQ_ERR_ARG, "tq_store_layer: null pointer");
+    REQUIRE((!hk || aligned16(k)) && (!hv || aligned16(v)) && aligned16(packed_k) && aligned16(packed_v), TQ_ERR_ALIGN,
+            "tq_store_layer: packed buffers and the inputs of turbo formats must be 16-byte aligned");
+    return tqk_store_layer(hk, hv, k, v, n_seqs, tokens, capacity, in_dtype, packed_k, packed_v, (hipStream_t)stream);
+}
+
 int tq_store_kv_cache(const tq_handle *hk, const tq_handle *hv, const void *k, const void *v, int64_t n_seqs, int64_t tokens,
                       int64_t capacity, int in_dtype, void *packed_k, void *packed_v, void *stream) {
     int rc = check_fast(hk, "tq_store_kv_cache");

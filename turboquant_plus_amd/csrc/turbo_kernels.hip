@@ -2993,6 +2993,38 @@ static int launch_store_v(const tq_handle *h, const void *x, int in_dtype, void 
 }
 
 constexpr int64_t SINGLE_VIA_FUSED_BLOCKS = 512;  // 65 536 vectors
+// One tensor through the matrix-core store (store_fast_ok), sequences `out_bps` blocks apart in `packed`
+static int store_one(const tq_handle *h, const void *x, int64_t n_seqs, int64_t tokens, int64_t out_bps, int in_dtype, int kind,
+                     void *packed, hipStream_t s) {
+    const int64_t bps = blocks_for(tokens), n_blocks = n_seqs * bps;
+    const bool ragged = tokens != bps * TQ_ROWS_PER_BLOCK || out_bps != bps;
+    StoreKArgs ka = make_k_args(h, tokens, bps, n_blocks);
+    StoreVArgs va = make_v_args(h, tokens, bps, n_blocks);
+    ka.out_blocks_per_seq = va.out_blocks_per_seq = (uint32_t)out_bps;
+    if (kind == TQ_KIND_V && n_blocks >= SINGLE_VIA_FUSED_BLOCKS && in_dtype == TQ_F16) {
+        // A large V tensor: the K+V kernel with an empty K share (one workgroup of twelve wavefronts per CU drawing
+        // tiles from a queue) is faster than k_store_v - 262 144 vectors: 20.9 against 21.9 us (3-bit), 22.4
+        // against 23.3 us (4-bit), 18.2 against 19.1 us (2-bit).  K tensors are slower that way (17.7 against
+        // 16.6 us, 20.8 against 17.8 us with the 64 KB table) and keep k_store_k.  Every CU gets a workgroup (there
+        // are more tiles than CUs here); a grid of a twelfth of the tiles left half of them idle at 96 000 vectors.
+        va.share_k_lut = 1;
+        ka.n_units = 0;
+        const unsigned grid = va.n_units < 256u ? va.n_units : 256u;
+#define TQ_ONE(B)                                                                                                                  \
+    if (ragged) k_store_kv<B, B, true><<<grid, 768, 0, s>>>((const __half *)x, (const __half *)x, va.n_units, ka.n_units, (uint8_t *)packed, (uint8_t *)packed, ka, va); \
+    else k_store_kv<B, B, false><<<grid, 768, 0, s>>>((const __half *)x, (const __half *)x, va.n_units, ka.n_units, (uint8_t *)packed, (uint8_t *)packed, ka, va)
+        switch (h->bits) {
+        case 2: TQ_ONE(2); break;
+        case 3: TQ_ONE(3); break;
+        default: TQ_ONE(4); break;
+        }
+#undef TQ_ONE
+        return tq_check_launch("store_v (through the K+V kernel)");
+    }
+    if (kind == TQ_KIND_K) return launch_store_k(h, x, in_dtype, packed, ka, ragged, s);
+    return launch_store_v(h, x, in_dtype, packed, va, ragged, s);
+}
+
 int tqk_store(const tq_handle *h, const void *x, int64_t n_seqs, int64_t tokens, int in_dtype, int kind, void *packed,
               uint8_t *sign_bits, void *rnorms, hipStream_t s) {
     const int64_t bps = blocks_for(tokens);
@@ -3028,34 +3060,7 @@ int tqk_store(const tq_handle *h, const void *x, int64_t n_seqs, int64_t tokens,
 #undef TQ_STOREQ_BITS
         return tq_check_launch("store_qjl");
     }
-    if (store_fast_ok(h, in_dtype, n_seqs * bps)) {
-        const int64_t n_blocks = n_seqs * bps;
-        const bool ragged = tokens != bps * TQ_ROWS_PER_BLOCK;
-        if (kind == TQ_KIND_V && n_blocks >= SINGLE_VIA_FUSED_BLOCKS && in_dtype == TQ_F16) {
-            // A large V tensor: the K+V kernel with an empty K share (one workgroup of twelve wavefronts per CU drawing
-            // tiles from a queue) is faster than k_store_v - 262 144 vectors: 20.9 against 21.9 us (3-bit), 22.4
-            // against 23.3 us (4-bit), 18.2 against 19.1 us (2-bit).  K tensors are slower that way (17.7 against
-            // 16.6 us, 20.8 against 17.8 us with the 64 KB table) and keep k_store_k.
-            StoreKArgs ka = make_k_args(h, tokens, bps, n_blocks);
-            StoreVArgs va = make_v_args(h, tokens, bps, n_blocks);
-            va.share_k_lut = 1;
-            const uint32_t units12 = (va.n_units + 11) / 12;
-            ka.n_units = 0;
-            const unsigned grid = units12 < 256u ? units12 : 256u;
-#define TQ_ONE(B)                                                                                                                  \
-    if (ragged) k_store_kv<B, B, true><<<grid, 768, 0, s>>>((const __half *)x, (const __half *)x, va.n_units, ka.n_units, (uint8_t *)packed, (uint8_t *)packed, ka, va); \
-    else k_store_kv<B, B, false><<<grid, 768, 0, s>>>((const __half *)x, (const __half *)x, va.n_units, ka.n_units, (uint8_t *)packed, (uint8_t *)packed, ka, va)
-            switch (h->bits) {
-            case 2: TQ_ONE(2); break;
-            case 3: TQ_ONE(3); break;
-            default: TQ_ONE(4); break;
-            }
-#undef TQ_ONE
-            return tq_check_launch("store_v (through the K+V kernel)");
-        }
-        if (kind == TQ_KIND_K) return launch_store_k(h, x, in_dtype, packed, make_k_args(h, tokens, bps, n_blocks), ragged, s);
-        return launch_store_v(h, x, in_dtype, packed, make_v_args(h, tokens, bps, n_blocks), ragged, s);
-    }
+    if (store_fast_ok(h, in_dtype, n_seqs * bps)) return store_one(h, x, n_seqs, tokens, bps, in_dtype, kind, packed, s);
     StoreArgs a;
     a.s1 = h->s1_32; a.s2 = h->s2_32; a.bounds = h->bounds32; a.cent = h->centroids32;
     a.kind = kind; a.norm_correction = h->norm_correction;
@@ -4140,6 +4145,26 @@ int tqk_store_kv(const tq_handle *hk, const tq_handle *hv, const void *k, const 
 #undef TQ_KV_V
 #undef TQ_KV
     return tq_check_launch("store_kv");
+}
+
+// Prompt of a layer of any two formats (hk / hv NULL: q8_0-style rows) into caches laid out for `capacity` tokens.
+// One 8-bit side: a long prompt's turbo side goes through the matrix-core store (the append's butterfly is bound by its
+// vector instructions) and the 8-bit side through its own launch; a short one is one launch of the append kernel.
+// From 512 blocks on two launches are the faster (one / two, us; 8-bit K with turbo3 V, fp16: 512 blocks 19.9 / 17.4, 752 28.6 /
+// 22.8, 2048 62.3 / 47.3; turbo4 V 70.7 / 48.9; turbo3 K with 8-bit V 56.9 / 41.7); below, calls take the host 15 us either way.
+constexpr int64_t PREFILL_SPLIT_BLOCKS = 512;
+int tqk_store_layer(const tq_handle *hk, const tq_handle *hv, const void *k, const void *v, int64_t n_seqs, int64_t tokens,
+                    int64_t capacity, int in_dtype, void *packed_k, void *packed_v, hipStream_t s) {
+    if (hk && hv) return tqk_store_kv(hk, hv, k, v, n_seqs, tokens, capacity, in_dtype, packed_k, packed_v, s);
+    const tq_handle *h = hk ? hk : hv;
+    const int64_t n_blocks = n_seqs * blocks_for(tokens), out_bps = blocks_for(capacity);
+    if (!h || n_blocks < PREFILL_SPLIT_BLOCKS || !store_fast_ok(h, in_dtype, n_blocks) || out_bps * n_seqs >= (1ll << 28))
+        return tqk_append_kv(hk, hv, k, v, n_seqs, 0, tokens, capacity, in_dtype, packed_k, packed_v, s);
+    const int rc = hk ? tqk_q8_0_append(v, n_seqs, 0, tokens, capacity, in_dtype, TQ_KIND_V, packed_v, s, nullptr, nullptr)
+                      : tqk_q8_0_append(k, n_seqs, 0, tokens, capacity, in_dtype, TQ_KIND_K, packed_k, s, nullptr, nullptr);
+    if (rc) return rc;
+    return hk ? store_one(hk, k, n_seqs, tokens, out_bps, in_dtype, TQ_KIND_K, packed_k, s)
+              : store_one(hv, v, n_seqs, tokens, out_bps, in_dtype, TQ_KIND_V, packed_v, s);
 }
 
 // K and V of a layer to fp16 in the original domain.  One launch when both handles hold the fragments of the

@@ -20,7 +20,7 @@ from __future__ import annotations
 from dataclasses import dataclass
 
 from . import _lib as L
-from .turbo import DecodeAttention, TurboCodec, append_layer, packed_bytes, q8_0_append, q8_0_store
+from .turbo import DecodeAttention, TurboCodec, append_layer, packed_bytes, q8_0_append, q8_0_store, store_layer
 
 FORMATS = ("q8_0", "turbo4", "turbo3", "turbo2")
 
@@ -140,9 +140,15 @@ class LayerKV:
     def prefill(self, k, v, k_cache, v_cache, capacity: int):
         """The prompt's K and V [n_seqs, tokens, 128] into caches laid out for `capacity` tokens, from position 0:
         turbo K with turbo V through the fused store (TurboCodec.store_kv(capacity=...), the matrix-core kernels for
-        fp16 rows), any other pair through append() at position 0."""
+        fp16 rows), layers with 8-bit rows through the same kernels for a long prompt's turbo side, else through append()
+        at position 0."""
         if self.k_codec is not None and self.v_codec is not None:
             self.k_codec.store_kv(self.v_codec, k, v, out_k=k_cache, out_v=v_cache, capacity=capacity)
+            return k_cache, v_cache
+        kd, n_seqs, tokens = TurboCodec._as_seqs(k)
+        vd, vs, vt = TurboCodec._as_seqs(v)
+        if (vs, vt) == (n_seqs, tokens) and vd.dtype == kd.dtype:
+            store_layer(self.k_codec, self.v_codec, kd, vd, n_seqs, tokens, k_cache, v_cache, capacity)
             return k_cache, v_cache
         return self.append(k, v, k_cache, v_cache, 0, capacity)
 

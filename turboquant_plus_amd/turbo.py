@@ -398,19 +398,31 @@ def q8_0_append(x, packed, pos, capacity: int, kind: str = "k", overrun=None):
     return packed
 
 
-def append_layer(k_codec, v_codec, kd, vd, n_seqs: int, n_new: int, k_cache, v_cache, pos, capacity: int, overrun=None):
-    """The K and V tokens of one step in one launch, a codec of None standing for q8_0-style rows (tq_append_layer);
-    kd, vd: device tensors [n_seqs, n_new, 128] of one dtype.  LayerKV.append's way for layers with 8-bit rows."""
+def _layer_buffers(k_codec, v_codec, n_seqs: int, capacity: int, k_cache, v_cache):
+    """The two handles of a layer (None: q8_0-style rows), after a check that its caches hold `capacity` tokens."""
     lib = L.lib()
     for codec, buf in ((k_codec, k_cache), (v_codec, v_cache)):
         need = int(lib.tq_q8_0_bytes(n_seqs, capacity)) if codec is None else packed_bytes(codec.bits, n_seqs, capacity)
         if buf.numel() < need:
             raise ValueError(f"packed holds {buf.numel()} bytes, need {need}")
+    return (None if c is None else c.handle.h for c in (k_codec, v_codec))
+
+
+def append_layer(k_codec, v_codec, kd, vd, n_seqs: int, n_new: int, k_cache, v_cache, pos, capacity: int, overrun=None):
+    """The K and V tokens of one step in one launch, a codec of None standing for q8_0-style rows (tq_append_layer);
+    kd, vd: device tensors [n_seqs, n_new, 128] of one dtype.  LayerKV.append's way for layers with 8-bit rows."""
+    hk, hv = _layer_buffers(k_codec, v_codec, n_seqs, capacity, k_cache, v_cache)
     on_device = _position_on_device(pos)
-    L.check(lib.tq_append_layer(None if k_codec is None else k_codec.handle.h, None if v_codec is None else v_codec.handle.h,
-                                L.ptr(kd), L.ptr(vd), n_seqs, 0 if on_device else pos, L.ptr(pos) if on_device else None, n_new,
-                                capacity, L.dtype_code(kd), L.ptr(k_cache), L.ptr(v_cache),
-                                _overrun_ptr(overrun) if on_device else None, L.stream_ptr()))
+    L.check(L.lib().tq_append_layer(hk, hv, L.ptr(kd), L.ptr(vd), n_seqs, 0 if on_device else pos, L.ptr(pos) if on_device else None,
+                                    n_new, capacity, L.dtype_code(kd), L.ptr(k_cache), L.ptr(v_cache),
+                                    _overrun_ptr(overrun) if on_device else None, L.stream_ptr()))
+
+
+def store_layer(k_codec, v_codec, kd, vd, n_seqs: int, tokens: int, k_cache, v_cache, capacity: int):
+    """A prompt's K and V into the caches of a layer with q8_0-style rows (codec None) on either side (tq_store_layer)."""
+    hk, hv = _layer_buffers(k_codec, v_codec, n_seqs, capacity, k_cache, v_cache)
+    L.check(L.lib().tq_store_layer(hk, hv, L.ptr(kd), L.ptr(vd), n_seqs, tokens, capacity, L.dtype_code(kd), L.ptr(k_cache),
+                                   L.ptr(v_cache), L.stream_ptr()))
 
 
 def q8_0_unpack(packed, n_seqs: int, tokens: int, kind: str = "k"):
