@@ -115,3 +115,28 @@ def test_prompt_of_a_layer_with_8_bit_rows(fmt, dtype, tokens):
         got = cache.view(n, capacity // 128, -1)
         assert tt.equal(got[:, :blocks], want.view(n, blocks, -1)), kind
         assert bool((got[:, blocks:] == 0xA5).all()), kind
+
+
+@pytest.mark.parametrize("bits", [2, 3, 4])
+@pytest.mark.parametrize("order", ["ascending", "shuffled", "with gaps"])
+def test_codes_are_the_number_of_boundaries_below(bits, order):
+    """Codebooks in any order, values on, next to and far beyond their boundaries: the code is the count of midpoints of
+    neighbouring entries below the value, whatever their order (rows of one non-zero value rotate to +-1/sqrt(128) times it, so
+    every rotated value of the row has that size)."""
+    rng = np.random.default_rng(bits)
+    cent = np.sort(rng.uniform(-0.3, 0.3, 1 << bits))
+    if order == "shuffled":
+        cent = rng.permutation(cent)
+    if order == "with gaps":   # entries of equal value and far outside the rows' range
+        cent[: 1 << (bits - 1)] = cent[0] * 100
+    codec = tqa.TurboCodec(bits, seed=5, centroids=cent)
+    x = rng.standard_normal((1, 384, D))
+    x[0, 0], x[0, 1], x[0, 2] = 0, np.eye(D)[7], -3 * np.eye(D)[100]
+    cache = L.torch().zeros(tqa.packed_bytes(bits, 1, 384), dtype=L.torch().uint8, device="cuda")
+    codec.append(x, cache, 0, 384, kind="k")
+    idx = np_(codec.unpack_codes(cache, 1, 384, kind="k")[0])[0].astype(int)
+    mid = (cent[1:] + cent[:-1]) / 2
+    y = O.rotate_fast(x[0] / np.maximum(np.linalg.norm(x[0], axis=1, keepdims=True), 1e-300), codec.signs1, codec.signs2, D)
+    lo, hi = ((mid[None, None] < (y + e)[..., None]).sum(-1) for e in (-2e-6, 2e-6))   # 32-bit rotation of values up to 1
+    assert ((idx >= lo) & (idx <= hi)).all()
+    assert (lo == hi).mean() > 0.999

@@ -4,6 +4,8 @@
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
+#include <algorithm>
+#include <limits>
 #include <vector>
 
 #include "tq_internal.h"
@@ -180,9 +182,15 @@ int tq_create(tq_handle **out, const tq_config *cfg) {
     }
     if (d == 128 && cfg->rotation == TQ_ROT_WHT && cfg->bits <= 4) {
         std::vector<float> c32(cent.begin(), cent.end()), b32(bounds.begin(), bounds.end());
+        // the quantiser counts the boundaries below a value, so their order is free: ascending, as its search wants them
+        // (a codebook may come in any order), and one that compares with nothing is one that nothing exceeds
+        std::vector<float> ascending = b32;
+        for (float &b : ascending)
+            if (b != b) b = std::numeric_limits<float>::infinity();
+        std::sort(ascending.begin(), ascending.end());
         std::vector<float> s1f(s1.begin(), s1.end()), s2f(s2.begin(), s2.end());
         rc = rc ? rc : upload(&h->centroids32, c32);
-        rc = rc ? rc : upload(&h->bounds32, b32);
+        rc = rc ? rc : upload(&h->bounds32, ascending);
         rc = rc ? rc : upload(&h->s1_32, s1f);
         rc = rc ? rc : upload(&h->s2_32, s2f);
         // pair LUT: entry (hi << bits | lo) = half2(c[lo], c[hi])

@@ -1603,13 +1603,40 @@ __global__ __launch_bounds__(768) void k_store_kv(const TI *xv, const TI *xk, ui
 }
 
 // ---- K2: fused quantise + pack ---------------------------------------------------
+// Number of boundaries below y, which come ascending: BITS compares with the next boundary picked by the results so far.
+// Instructions per value (compares, selects, the code's bits) against a compare and an add per boundary: 2-bit 6 and 6,
+// 3-bit 10 and 14, 4-bit 19 and 30; the kernels that quantise this way are bound by them.
+template <int BITS> __device__ __forceinline__ uint32_t count_below(const float (&b)[(1 << BITS) - 1], float y) {
+    if constexpr (BITS == 2) {
+        uint32_t c = 0;
+#pragma unroll
+        for (int k = 0; k < 3; ++k) c += (b[k] < y) ? 1u : 0u;
+        return c;
+    } else if constexpr (BITS == 3) {
+        const bool p2 = b[3] < y;
+        const float t1 = p2 ? b[5] : b[1], lo = p2 ? b[4] : b[0], hi = p2 ? b[6] : b[2];
+        const bool p1 = t1 < y;
+        const bool p0 = (p1 ? hi : lo) < y;
+        uint32_t c = p2 ? 1u : 0u;
+        c = c + c + (p1 ? 1u : 0u);
+        return c + c + (p0 ? 1u : 0u);
+    } else {
+        static_assert(BITS == 4, "2, 3 or 4 bits");
+        const bool p3 = b[7] < y;
+        float h[7];  // the seven boundaries of the half
+#pragma unroll
+        for (int k = 0; k < 7; ++k) h[k] = p3 ? b[8 + k] : b[k];
+        const uint32_t c = count_below<3>(h, y);
+        return c + (p3 ? 8u : 0u);
+    }
+}
+
 // One vector on the 16 lanes of a DPP row, 8 values per lane: norm, s1, 128-point butterfly,
 // s2/sqrt(128), normalise, compare-count against the boundaries, sum c^2.  Returns the
 // lane's 8 codes as bytes and (valid on every lane of the row) the norm to store.
 template <int BITS>
 __device__ __forceinline__ float quantize_vec16(float (&xv)[8], int lane, const float (&bnd)[(1 << BITS) - 1], const float (&s1v)[8],
                                                 const float (&s2v)[8], const float *csq_s, int norm_correction, uint2 &codes8) {
-    constexpr int NB = (1 << BITS) - 1;
     float ss = 0.0f;
 #pragma unroll
     for (int m = 0; m < 8; ++m) ss = fmaf(xv[m], xv[m], ss);
@@ -1624,9 +1651,7 @@ __device__ __forceinline__ float quantize_vec16(float (&xv)[8], int lane, const 
 #pragma unroll
     for (int m = 0; m < 8; ++m) {
         const float yv = (xv[m] * s2v[m]) * inv;
-        uint32_t c = 0;
-#pragma unroll
-        for (int k = 0; k < NB; ++k) c += (bnd[k] < yv) ? 1u : 0u;
+        const uint32_t c = count_below<BITS>(bnd, yv);
         cs += csq_s[c];
         if (m < 4) w0 |= c << (8 * m);
         else w1 |= c << (8 * (m - 4));
