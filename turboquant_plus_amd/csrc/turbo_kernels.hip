@@ -1605,7 +1605,8 @@ __global__ __launch_bounds__(768) void k_store_kv(const TI *xv, const TI *xk, ui
 // ---- K2: fused quantise + pack ---------------------------------------------------
 // Number of boundaries below y, which come ascending: BITS compares with the next boundary picked by the results so far.
 // Instructions per value (compares, selects, the code's bits) against a compare and an add per boundary: 2-bit 6 and 6,
-// 3-bit 10 and 14, 4-bit 19 and 30; the kernels that quantise this way are bound by them.
+// 3-bit 10 and 14, 4-bit 19 and 30; the kernels that quantise this way are bound by them (64 x 2048 tokens appended, K and V:
+// turbo4 fp32 63.5 -> 55.1 us, turbo3 fp16 50.8 -> 48.4 us).
 template <int BITS> __device__ __forceinline__ uint32_t count_below(const float (&b)[(1 << BITS) - 1], float y) {
     if constexpr (BITS == 2) {
         uint32_t c = 0;
@@ -1758,7 +1759,7 @@ __device__ inline float block_norm(const uint8_t *block, int bits, int token);
 // What bounds it is the chain of one workgroup (a chunk of 512 tokens for 32 sequences is one workgroup per CU): the
 // rows' load latency, the quantiser, the packing.  So eight wavefronts share a block, each 16-lane row requests its four
 // tokens at once before the constants' barrier, and a partly filled V tile takes its tokens on four threads per row (one
-// per 16-token group, whose dwords are its own) instead of one.
+// per 16-token group, whose dwords are its own) instead of one.  512 tokens x 32 sequences, turbo4: call 15.7 -> 14.4 us.
 constexpr int APPEND_THREADS = 512, APPEND_ROWS = TQ_ROWS_PER_BLOCK * 16 / APPEND_THREADS;  // tokens per 16-lane row
 template <int BITS, typename TI>
 __device__ __forceinline__ void append_block(const TI *x, uint8_t *packed, const AppendArgs &a, const int64_t wg) {
@@ -2762,6 +2763,7 @@ __global__ __launch_bounds__(256) void k_q8_0_store_v_f16(const __half *x, uint8
 // the lanes, all four of a lane's pieces are requested at once, and the quantised bytes pass through LDS so that a
 // wavefront stores 1 KB of a chunk in one piece (V rows: a thread gathers a dim's 16 tokens; bytes of neighbouring
 // tokens share those 16 bytes, and only the 16-token group that `pos` falls into is stored byte by byte).
+// 16 x 6001 tokens: 20 us for K and V (33 us for K alone when a thread read 32 values one by one and V left in bytes).
 // x need not be 16-byte aligned: `wide` says whether it is.
 constexpr int Q8A_THREADS = 512, Q8A_ROW = 136;  // LDS bytes per token (an odd multiple of 8)
 struct Q8AppendArgs {
