@@ -31,7 +31,9 @@ class CompressedKVCache:
 
 def _joined(pieces):
     """The (layer, head) arrays one after another.  compress() hands out views that follow each other in one array: pieces
-    of one base whose memory is adjacent are taken as the stretch they are, others are copied together."""
+    of one base whose memory is adjacent are taken as the stretch they are, others are copied together.  The stretch gets
+    the strides of its shape: a piece is contiguous whatever stride its axes of one entry have, and those strides (of a
+    token-major container, say) lead elsewhere."""
     pieces = [np.asarray(p) for p in pieces]
     first = pieces[0]
     at = first.__array_interface__["data"][0]
@@ -40,7 +42,11 @@ def _joined(pieces):
                 or not p.flags.c_contiguous or p.__array_interface__["data"][0] != at):
             return np.concatenate(pieces, axis=0)
         at += p.nbytes
-    return np.lib.stride_tricks.as_strided(first, (len(pieces) * first.shape[0],) + first.shape[1:], first.strides)
+    shape = (len(pieces) * first.shape[0],) + first.shape[1:]
+    strides = [first.itemsize]
+    for n in shape[:0:-1]:
+        strides.insert(0, n * strides[0])
+    return np.lib.stride_tricks.as_strided(first, shape, strides)
 
 
 class KVCacheCompressor:
