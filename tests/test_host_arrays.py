@@ -25,3 +25,11 @@ def test_joined_equals_concatenate():
         for pieces in ([a[i, j] for i in range(a.shape[0]) for j in range(a.shape[1])], [a[i, 0] for i in range(a.shape[0])],
                        [a[0, 0], a[0, 0]], [a[0, 0]], [a[0, 0], a[0, 1].astype(np.float32)]):
             assert np.array_equal(_joined(pieces), np.concatenate(pieces, axis=0))
+
+
+def test_scalar_norms_join():
+    """Containers of one token may hold a plain number per (layer, head)."""
+    for scalars in ([np.float64(2.5), 3, np.array(4.0)], list(np.arange(3.0)[:, None].T.reshape(3))):
+        assert np.array_equal(_joined(scalars), np.asarray(scalars, dtype=np.float64))
+    z = np.arange(3.0)
+    assert np.array_equal(_joined([z[i:i + 1].reshape(()) for i in range(3)]), z)

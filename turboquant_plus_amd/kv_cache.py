@@ -34,7 +34,7 @@ def _joined(pieces):
     of one base whose memory is adjacent are taken as the stretch they are, others are copied together.  The stretch gets
     the strides of its shape: a piece is contiguous whatever stride its axes of one entry have, and those strides (of a
     token-major container, say) lead elsewhere."""
-    pieces = [np.asarray(p) for p in pieces]
+    pieces = [np.atleast_1d(np.asarray(p)) for p in pieces]     # the norm of one token may be a plain number
     first = pieces[0]
     at = first.__array_interface__["data"][0]
     for p in pieces:
