@@ -1,8 +1,14 @@
 """Host-array handling of the NumPy classes that needs no GPU."""
+import os
+import subprocess
+import sys
+
 import numpy as np
 import pytest
 
 from turboquant_plus_amd.kv_cache import _joined
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 
 
 @pytest.mark.parametrize("t", [0, 1, 4])
@@ -33,3 +39,29 @@ def test_scalar_norms_join():
         assert np.array_equal(_joined(scalars), np.asarray(scalars, dtype=np.float64))
     z = np.arange(3.0)
     assert np.array_equal(_joined([z[i:i + 1].reshape(()) for i in range(3)]), z)
+
+
+@pytest.mark.parametrize("when", ["after a fork", "at exit", "in a thread that outlives the main one"])
+def test_copy_threads_that_are_not_there(when):
+    """Large host arrays are handled where the copy threads are gone: in a forked child, and once the interpreter ends."""
+    code = """
+import atexit, os, sys, threading, time
+import numpy as np
+from turboquant_plus_amd import _lib as L
+i = np.random.default_rng(0).integers(0, 8, 700_000)
+def narrow():
+    assert np.array_equal(L.narrow_indices(i, 8), i)
+    print("done", flush=True)
+narrow()
+together = threading.Barrier(L.COPY_THREADS)
+for w in [L._copy_pool().submit(together.wait) for _ in range(L.COPY_THREADS)]:   # every thread has started
+    w.result()
+"""
+    code += {"after a fork": "pid = os.fork()\nif pid == 0:\n    narrow()\n    os._exit(0)\n"
+                             "end = time.time() + 30\nwhile time.time() < end and os.waitpid(pid, os.WNOHANG)[0] == 0:\n    time.sleep(0.05)\n"
+                             "if time.time() >= end:\n    os.kill(pid, 9)\n    os.waitpid(pid, 0)\n",
+             "at exit": "atexit.register(narrow)\n",
+             "in a thread that outlives the main one": "def late():\n    threading.main_thread().join()\n    time.sleep(0.3)\n    narrow()\n"
+                                                       "threading.Thread(target=late).start()\n"}[when]
+    out = subprocess.run([sys.executable, "-c", code], cwd=ROOT, capture_output=True, text=True, timeout=120)
+    assert out.returncode == 0 and out.stdout.count("done") == 2, out.stdout + out.stderr

@@ -9,7 +9,7 @@ import ctypes as C
 import math
 import os
 import threading
-from concurrent.futures import ThreadPoolExecutor
+from concurrent.futures import Future, ThreadPoolExecutor
 
 import numpy as np
 
@@ -210,6 +210,33 @@ def _copy_pool():
         return _copiers
 
 
+def _forget_copiers():
+    """A forked child has none of the threads, and the lock as it happened to be held."""
+    global _copiers, _copiers_lock
+    _copiers, _copiers_lock = None, threading.Lock()
+
+
+os.register_at_fork(after_in_child=_forget_copiers)
+
+
+def _hand_over(fn, *args):
+    """A future of fn(*args), run on the copy threads or, where those take no more work (the interpreter is ending, no
+    thread can be started), here.  A submit that fails may have queued the work all the same: who comes first runs it."""
+    done, claim = Future(), threading.Lock()
+
+    def run():
+        if claim.acquire(blocking=False):
+            try:
+                done.set_result(fn(*args))
+            except BaseException as e:
+                done.set_exception(e)
+    try:
+        _copy_pool().submit(run)
+    except RuntimeError:
+        run()
+    return done
+
+
 def _shares(n, item_bytes):
     """(start, stop) shares of n elements for the copy threads: one per MiB, at most COPY_THREADS.  Up to 4 MiB one
     thread does it all: handing the work over costs more (256 vectors of 1536 both ways: 0.8 against 1.4 ms)."""
@@ -228,7 +255,7 @@ def _fetch_staged(t, out):
     host = [s.numpy() for s in slots]
     done = [tt.cuda.Event() for _ in slots]
     work = [[], []]
-    pool, n = _copy_pool(), src.numel()
+    n = src.numel()
 
     def empty_slot(i, at, count):
         done[i].synchronize()
@@ -236,7 +263,7 @@ def _fetch_staged(t, out):
         if len(shares) == 1:
             np.copyto(dst[at:at + count], host[i][:count])
         else:
-            work[i] = [pool.submit(np.copyto, dst[at + a:at + b], host[i][a:b]) for a, b in shares]
+            work[i] = [_hand_over(np.copyto, dst[at + a:at + b], host[i][a:b]) for a, b in shares]
 
     last = None
     for k, at in enumerate(range(0, n, step)):
@@ -275,7 +302,7 @@ def narrow_indices(indices, n_centroids):
         seen = share(*shares[0])
     else:
         seen = 0
-        for w in [_copy_pool().submit(share, a, b) for a, b in shares]:
+        for w in [_hand_over(share, a, b) for a, b in shares]:
             seen |= w.result()
     if seen & ~(n_centroids - 1):
         refuse()
