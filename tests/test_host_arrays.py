@@ -6,6 +6,7 @@ import sys
 import numpy as np
 import pytest
 
+from turboquant_plus_amd import _lib as L
 from turboquant_plus_amd.kv_cache import _joined
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
@@ -65,3 +66,12 @@ for w in [L._copy_pool().submit(together.wait) for _ in range(L.COPY_THREADS)]: 
                                                        "threading.Thread(target=late).start()\n"}[when]
     out = subprocess.run([sys.executable, "-c", code], cwd=ROOT, capture_output=True, text=True, timeout=120)
     assert out.returncode == 0 and out.stdout.count("done") == 2, out.stdout + out.stderr
+
+
+def test_more_norms_than_vectors():
+    """Norms past the last vector are not used; too few are refused."""
+    assert L.host_norms(np.arange(5.0), 3).tolist() == [0.0, 1.0, 2.0]
+    assert L.host_norms([[1, 2], [3, 4]], 4).tolist() == [1.0, 2.0, 3.0, 4.0]
+    assert L.host_norms(np.arange(12.0).reshape(3, 4)[:, ::2], 5).flags.c_contiguous
+    with pytest.raises(ValueError, match="norms"):
+        L.host_norms(np.ones(2), 3)

@@ -345,8 +345,8 @@ _NP_DTYPES = {"torch.uint8": np.dtype(np.uint8), "torch.int8": np.dtype(np.int8)
 
 
 def host_norms(norms, n):
-    """Norms of n vectors as a contiguous float64 array."""
-    a = np.ascontiguousarray(np.asarray(norms, dtype=np.float64).reshape(-1))
+    """The first n norms, those of n vectors, as a contiguous float64 array."""
+    a = np.ascontiguousarray(np.asarray(norms, dtype=np.float64).reshape(-1)[:n])
     if a.size != n:
         raise ValueError(f"{a.size} norms for {n} vectors")
     return a
