@@ -8,6 +8,7 @@ import pytest
 
 from turboquant_plus_amd import _lib as L
 from turboquant_plus_amd.kv_cache import _joined
+from turboquant_plus_amd.turboquant import CompressedVector, TurboQuant
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 
@@ -75,3 +76,25 @@ def test_more_norms_than_vectors():
     assert L.host_norms(np.arange(12.0).reshape(3, 4)[:, ::2], 5).flags.c_contiguous
     with pytest.raises(ValueError, match="norms"):
         L.host_norms(np.ones(2), 3)
+
+
+class _Part:
+    """A quantiser stage with the public methods only."""
+
+    def __init__(self, d):
+        self.d = d
+
+    def dequantize(self, codes, norms, shrinkage=1.0):
+        return np.asarray(codes) * (np.asarray(norms)[..., None] * shrinkage)
+
+
+@pytest.mark.parametrize("idx,signs", [((5, 8), (1, 8)), ((5, 8), (8,)), ((1, 8), (5, 8)), ((8,), (5, 8))])
+def test_signs_that_broadcast_against_indices(idx, signs):
+    """TurboQuant.dequantize is the sum of its two stages' results, also where their shapes broadcast."""
+    tq = TurboQuant(8, 3)
+    tq.polar_quant, tq.qjl = _Part(8), _Part(8)
+    rng = np.random.default_rng(1)
+    i, s = rng.integers(0, 4, idx), rng.choice([-1, 1], signs).astype(np.int8)
+    n, rn = rng.random(idx[:-1]), rng.random(signs[:-1])
+    got = tq.dequantize(CompressedVector(i, n, s, rn, 3), shrinkage=0.5)
+    assert np.array_equal(got, i * n[..., None] + s * rn[..., None] * 0.5)

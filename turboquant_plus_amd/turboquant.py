@@ -66,12 +66,12 @@ class TurboQuant:
     def dequantize(self, compressed: CompressedVector, shrinkage: float = 1.0):
         idx, signs = np.asarray(compressed.mse_indices), np.asarray(compressed.qjl_signs)
         norms, rnorms = compressed.vector_norms, compressed.residual_norms
+        if signs.shape != idx.shape:    # shapes that broadcast against each other: the sum of two results
+            return self.polar_quant.dequantize(idx, norms) + self.qjl.dequantize(signs, rnorms, shrinkage=shrinkage)
         single = idx.ndim == 1
         if single:
             idx, signs, norms, rnorms = idx[None, :], signs[None, :], np.array([norms]), np.array([rnorms])
         self.polar_quant._check(idx, "dequantize")
-        if signs.shape != idx.shape:
-            raise ValueError(f"dequantize: indices are {idx.shape} and signs {signs.shape}")
         n = idx.shape[0]
         tt = L.torch()
         idx_d, norms_d, signs_d, rnorms_d = L.upload(L.narrow_indices(idx, self.polar_quant.n_centroids), L.host_norms(norms, n),
