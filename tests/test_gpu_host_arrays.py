@@ -62,3 +62,16 @@ def test_views_of_one_cache_are_taken_together():
     c.v_indices[1][2] = c.v_indices[1][2].astype(np.int32)
     k2, v2 = kv.decompress(c)
     assert np.array_equal(k, k2) and np.array_equal(v, v2)
+
+
+def test_a_subclass_that_overrides_quantize():
+    """The residual is that of the indices and norms which the subclass's quantize gives."""
+    class Coarse(tqa.PolarQuant):
+        def quantize(self, x):
+            idx, norms = super().quantize(x)
+            return idx | 1, norms
+    own, other = tqa.PolarQuant(24, 3, seed=4), Coarse(24, 3, seed=4)
+    for x in (np.random.default_rng(0).standard_normal((6, 24)), np.random.default_rng(1).standard_normal(24)):
+        idx, norms, res = other.quantize_and_residual(x)
+        assert np.array_equal(idx, own.quantize(x)[0] | 1) and np.array_equal(norms, own.quantize(x)[1])
+        np.testing.assert_allclose(res, x - own.dequantize(idx, norms), atol=1e-13)

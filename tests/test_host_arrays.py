@@ -7,7 +7,9 @@ import numpy as np
 import pytest
 
 from turboquant_plus_amd import _lib as L
-from turboquant_plus_amd.kv_cache import _joined
+from turboquant_plus_amd.kv_cache import KVCacheCompressor, _joined
+from turboquant_plus_amd.polar_quant import PolarQuant
+from turboquant_plus_amd.qjl import QJL
 from turboquant_plus_amd.turboquant import CompressedVector, TurboQuant
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
@@ -98,3 +100,59 @@ def test_signs_that_broadcast_against_indices(idx, signs):
     n, rn = rng.random(idx[:-1]), rng.random(signs[:-1])
     got = tq.dequantize(CompressedVector(i, n, s, rn, 3), shrinkage=0.5)
     assert np.array_equal(got, i * n[..., None] + s * rn[..., None] * 0.5)
+
+
+class _Recorder:
+    """The public methods of every stage, without a GPU."""
+
+    def __init__(self, d):
+        self.d = d
+
+    def quantize(self, x):
+        return np.sign(x).astype(np.int64), np.abs(x).sum(axis=-1)
+
+    def quantize_and_residual(self, x):
+        return (*self.quantize(x), x * 0.25)
+
+
+def test_replaced_stages_are_asked_through_their_public_methods():
+    tq = TurboQuant(8, 3)
+    tq.polar_quant, tq.qjl = _Recorder(8), _Recorder(8)
+    x = np.random.default_rng(2).standard_normal((5, 8))
+    for rows in (x, x[0]):
+        c = tq.quantize(rows)
+        assert np.array_equal(c.mse_indices, np.sign(rows)) and np.array_equal(c.residual_norms, np.abs(rows * 0.25).sum(axis=-1))
+        assert c.bit_width == 3
+    kv = KVCacheCompressor(8)
+    kv.k_quantizer, kv.v_quantizer.polar_quant = tq, _Recorder(8)
+    k = np.random.default_rng(3).standard_normal((2, 3, 5, 8))
+    c = kv.compress(k, -k)
+    assert np.array_equal(c.k_compressed[1][2].mse_indices, np.sign(k[1, 2]))
+    assert np.array_equal(c.v_indices[0][1], np.sign(-k[0, 1])) and np.array_equal(c.v_norms[1][0], np.abs(k[1, 0]).sum(axis=-1))
+
+
+def test_overridden_methods_are_called(monkeypatch):
+    """In a subclass, on an object, on the class."""
+    class Polar(PolarQuant):
+        def quantize(self, x):
+            return np.full(np.shape(x), 7), np.zeros(np.shape(x)[:-1])
+
+        def _residual_of(self, x, idx, norms):      # what follows on the device
+            return idx * 2.0
+    idx, _, res = Polar(8, 3).quantize_and_residual(np.ones((2, 8)))
+    assert (idx == 7).all() and (res == 14).all()
+    tq = TurboQuant(8, 3)
+    tq.polar_quant.quantize_and_residual = lambda x: (1, 2, 3)
+    monkeypatch.setattr(QJL, "quantize", lambda self, r: (r, r))
+    c = tq.quantize(np.ones((2, 8)))
+    assert (c.mse_indices, c.vector_norms, c.qjl_signs) == (1, 2, 3)
+    tq = TurboQuant(8, 3)
+    tq.polar_quant.dequantize = tq.qjl.dequantize = lambda *a, **k: 1.0
+    z = np.zeros((2, 8), np.int64)
+    assert tq.dequantize(CompressedVector(z, z[:, 0], z, z[:, 0], 3)) == 2.0
+    kv = KVCacheCompressor(8)
+    kv.k_quantizer.quantize = lambda x: CompressedVector(x, x[:, 0], x, x[:, 1], 3)
+    kv.v_quantizer.quantize = lambda x: (x, x[:, 2])
+    k = np.random.default_rng(3).standard_normal((2, 3, 5, 8))
+    c = kv.compress(k, k)
+    assert np.array_equal(c.k_compressed[1][1].residual_norms, k[1, 1, :, 1]) and np.array_equal(c.v_norms[0][2], k[0, 2, :, 2])

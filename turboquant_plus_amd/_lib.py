@@ -181,6 +181,13 @@ def to_device(x, float_ok=(np.float16, np.float32, np.float64)):
 
 # ---- results of the NumPy classes: device buffers and their way into host arrays -----------------------------------
 
+def unchanged(obj, *methods):
+    """Whether these functions are what `obj` answers to by their names: not where it is of another class or where a
+    subclass, the object or a patch of its class has them replaced.  The classes take each other's device-side steps only
+    then, else the public methods."""
+    return all(getattr(getattr(obj, f.__name__, None), "__func__", None) is f for f in methods)
+
+
 def device_block(*specs):
     """(buffer, tensors): one uint8 device buffer and views of it for the (shape, torch dtype) specs, so that small
     results travel to or from the host in one copy."""

@@ -12,6 +12,7 @@ from dataclasses import dataclass, field
 import numpy as np
 
 from . import _lib as lib
+from . import polar_quant, turboquant
 from .turboquant import CompressedVector, TurboQuant, TurboQuantMSE
 
 
@@ -59,18 +60,28 @@ class KVCacheCompressor:
         self.v_quantizer = TurboQuantMSE(head_dim, bit_width=v_bits, seed=seed + 500,
                                          norm_correction=norm_correction)
 
+    def _on_device(self):
+        k, v = self.k_quantizer, self.v_quantizer
+        return (lib.unchanged(k, *turboquant.METHODS) and k._on_device() and lib.unchanged(v, *turboquant.MSE_METHODS)
+                and lib.unchanged(v.polar_quant, *polar_quant.METHODS))
+
     def compress(self, k_cache: np.ndarray, v_cache: np.ndarray) -> CompressedKVCache:
         L, H, S, D = k_cache.shape
         assert D == self.head_dim
         assert v_cache.shape == k_cache.shape
         out = CompressedKVCache(num_layers=L, num_heads=H, seq_len=S, head_dim=D,
                                 k_bit_width=self.k_bits, v_bit_width=self.v_bits)
-        # both tensors are on their way before the first results are waited for
-        kq, vq = self.k_quantizer, self.v_quantizer.polar_quant
-        k_block = kq._launch_quantize(lib.to_device(np.asarray(k_cache).reshape(L * H * S, D)))
-        v_block = vq._start_quantize(np.asarray(v_cache).reshape(L * H * S, D))
-        k_idx, k_nrm, k_sgn, k_rn = kq._fetch(k_block)
-        vi, vn = vq._fetch(v_block)
+        k_rows, v_rows = np.asarray(k_cache).reshape(L * H * S, D), np.asarray(v_cache).reshape(L * H * S, D)
+        if self._on_device():   # both tensors are on their way before the first results are waited for
+            kq, vq = self.k_quantizer, self.v_quantizer.polar_quant
+            k_block = kq._launch_quantize(lib.to_device(k_rows))
+            v_block = vq._start_quantize(v_rows)
+            k_idx, k_nrm, k_sgn, k_rn = kq._fetch(k_block)
+            vi, vn = vq._fetch(v_block)
+        else:
+            kc = self.k_quantizer.quantize(k_rows)
+            k_idx, k_nrm, k_sgn, k_rn = kc.mse_indices, kc.vector_norms, kc.qjl_signs, kc.residual_norms
+            vi, vn = self.v_quantizer.quantize(v_rows)
         k_idx, k_sgn, vi = (a.reshape(L, H, S, D) for a in (k_idx, k_sgn, vi))
         k_nrm, k_rn, vn = (a.reshape(L, H, S) for a in (k_nrm, k_rn, vn))
         for l in range(L):

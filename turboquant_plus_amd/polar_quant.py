@@ -105,11 +105,29 @@ class PolarQuant:
         out_h = L.fetch(buf, (out, np.float64))[0]
         return out_h[0] if single else out_h
 
+    def _residual_of(self, x, indices, norms):
+        """x - dequantize(indices, norms) for host arrays."""
+        tt = L.torch()
+        single = x.ndim == 1
+        i2 = np.asarray(indices)[None, :] if single else np.asarray(indices)
+        x2 = x[None, :] if single else x
+        self._check(i2, "dequantize")
+        self._check(x2, "quantize")
+        xd = L.to_device(x2)
+        idx, nrm = L.upload(L.narrow_indices(i2, self.n_centroids), L.host_norms(norms, i2.shape[0]))
+        buf, (res,) = L.device_block((tuple(i2.shape), tt.float64))
+        self._launch_residual(xd, idx, nrm, res)
+        res_h = L.fetch(buf, (res, np.float64))[0]
+        return res_h[0] if single else res_h
+
     def quantize_and_residual(self, x):
         """(indices, norms, x - dequantize(indices, norms)) (turboquant/polar_quant.py:121-132)."""
         x = np.asarray(x)
         single = x.ndim == 1
         x2 = x[None, :] if single else x
+        if not L.unchanged(self, *METHODS[:1]):
+            idx, norms = self.quantize(x)
+            return idx, norms, self._residual_of(x, idx, norms)
         self._check(x2, "quantize")
         tt = L.torch()
         xd = L.to_device(x2)
@@ -119,3 +137,6 @@ class PolarQuant:
         self._launch_residual(xd, idx, norms, res)
         idx_h, norms_h, res_h = L.fetch(buf, (idx, np.int64), (norms, np.float64), (res, np.float64))
         return (idx_h[0], norms_h[0], res_h[0]) if single else (idx_h, norms_h, res_h)
+
+
+METHODS = (PolarQuant.quantize, PolarQuant.quantize_and_residual, PolarQuant.dequantize)    # for _lib.unchanged

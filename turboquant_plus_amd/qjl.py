@@ -84,3 +84,6 @@ class QJL:
         self._launch_dequantize(sd, nd, shrinkage, out)
         res = L.fetch(buf, (out, np.float64))[0]
         return res[0] if single else res
+
+
+METHODS = (QJL.quantize, QJL.dequantize)    # for _lib.unchanged

@@ -7,6 +7,7 @@ from dataclasses import dataclass
 import numpy as np
 
 from . import _lib as L
+from . import polar_quant, qjl
 from .polar_quant import PolarQuant
 from .qjl import QJL
 
@@ -35,6 +36,9 @@ class TurboQuant:
 
     # Both directions stay on the device between the stages: indices, norms and the residual are handed over there, and
     # only what the caller gets crosses to the host.
+    def _on_device(self):
+        return L.unchanged(self.polar_quant, *polar_quant.METHODS) and L.unchanged(self.qjl, *qjl.METHODS)
+
     def _launch_quantize(self, xd):
         """Device vectors [n, d] -> (block, indices uint8, norms, signs, residual norms) on the device."""
         tt = L.torch()
@@ -56,17 +60,21 @@ class TurboQuant:
         x = np.asarray(x)
         single = x.ndim == 1
         x2 = x[None, :] if single else x
-        self.polar_quant._check(x2, "quantize")
-        idx, norms, signs, rnorms = self._fetch(self._launch_quantize(L.to_device(x2)))
-        if single:
-            idx, norms, signs, rnorms = idx[0], norms[0], signs[0], rnorms[0]
+        if not self._on_device():
+            idx, norms, residual = self.polar_quant.quantize_and_residual(x)
+            signs, rnorms = self.qjl.quantize(residual)
+        else:
+            self.polar_quant._check(x2, "quantize")
+            idx, norms, signs, rnorms = self._fetch(self._launch_quantize(L.to_device(x2)))
+            if single:
+                idx, norms, signs, rnorms = idx[0], norms[0], signs[0], rnorms[0]
         return CompressedVector(mse_indices=idx, vector_norms=norms, qjl_signs=signs, residual_norms=rnorms,
                                 bit_width=self.bit_width)
 
     def dequantize(self, compressed: CompressedVector, shrinkage: float = 1.0):
         idx, signs = np.asarray(compressed.mse_indices), np.asarray(compressed.qjl_signs)
         norms, rnorms = compressed.vector_norms, compressed.residual_norms
-        if signs.shape != idx.shape:    # shapes that broadcast against each other: the sum of two results
+        if signs.shape != idx.shape or not self._on_device():    # shapes may broadcast: the sum of two results
             return self.polar_quant.dequantize(idx, norms) + self.qjl.dequantize(signs, rnorms, shrinkage=shrinkage)
         single = idx.ndim == 1
         if single:
@@ -105,3 +113,7 @@ class TurboQuantMSE:
 
     def dequantize(self, indices, norms):
         return self.polar_quant.dequantize(indices, norms)
+
+
+METHODS = (TurboQuant.quantize, TurboQuant.dequantize)    # for _lib.unchanged
+MSE_METHODS = (TurboQuantMSE.quantize, TurboQuantMSE.dequantize)
