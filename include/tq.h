@@ -45,7 +45,7 @@ typedef struct tq_config {
     int32_t bits;             /* codebook bits, 1..8                                  */
     int32_t rotation;         /* TQ_ROT_DENSE | TQ_ROT_WHT                            */
     int32_t norm_correction;  /* polar_quant.py:109-112                               */
-    const double *centroids;  /* [1<<bits], sorted (codebook.py:29-49)                */
+    const double *centroids;  /* [1<<bits], in any order (codebook.py:29-49)          */
     const double *signs1;     /* [padded_d], WHT mode (rotation.py:94)                */
     const double *signs2;     /* [padded_d], WHT mode (rotation.py:95)                */
     const double *rotation_matrix; /* [d*d] row-major, dense mode (rotation.py:25-50) */

@@ -7,6 +7,7 @@ import pytest
 
 import tq_oracle as O
 import turboquant_plus_amd as tqa
+from turboquant_plus_amd import _lib as L
 
 pytestmark = pytest.mark.gpu
 
@@ -60,3 +61,32 @@ def test_level_search_at_every_width(bits):
     assert np.array_equal(idx[~near], np.searchsorted(mid, y.ravel(), side="left").reshape(y.shape)[~near])
     w = tqa.PolarQuant(64, bits, seed=3, rotation="wht")
     assert np.array_equal(w.quantize(x)[0], O.PolarRef(64, bits, seed=3, rotation="wht").quantize(x)[0])
+
+
+def quantize_indices(handle, x, rotated=None):
+    """tq_quantize_indices on a device tensor: indices and norms as NumPy arrays (rotated: a device tensor or None)."""
+    tt = L.torch()
+    n, d = x.shape
+    idx, norms = tt.empty((n, d), dtype=tt.uint8, device="cuda"), tt.empty(n, dtype=tt.float64, device="cuda")
+    L.check(L.lib().tq_quantize_indices(handle.h, L.ptr(x), n, L.dtype_code(x), L.ptr(idx), L.ptr(norms), L.ptr(rotated), L.stream_ptr()))
+    return idx.cpu().numpy(), norms.cpu().numpy()
+
+
+@pytest.mark.parametrize("bits", [1, 2, 3, 4, 6])
+@pytest.mark.parametrize("rotation", ["dense", "wht"])
+@pytest.mark.parametrize("order", ["shuffled", "with gaps"])
+def test_codebooks_in_any_order(bits, rotation, order):
+    """The code is the number of midpoints of neighbouring entries below the value, whatever their order."""
+    d, rng = 96, np.random.default_rng(bits)
+    cent = rng.uniform(-0.3, 0.3, 1 << bits)
+    if order == "with gaps":
+        cent[: 1 << (bits - 1)] = cent[0] * 100
+    q = O.PolarRef(d, 3, seed=7, rotation=rotation)
+    tables = dict(rotation=q.rotation) if rotation == "dense" else dict(signs1=q.s1, signs2=q.s2)
+    x = rng.standard_normal((300, d))
+    xd = L.torch().from_numpy(x).cuda()
+    idx, _ = quantize_indices(L.Handle(d, bits, cent, **tables), xd)
+    y, _ = q.rotated(x)
+    mid = (cent[1:] + cent[:-1]) / 2
+    clear = np.abs(y[..., None] - mid).min(axis=-1) > bound(2 * d)
+    assert clear.mean() > 0.99 and np.array_equal(idx[clear], (mid < y[..., None]).sum(axis=-1)[clear])

@@ -157,7 +157,15 @@ int tq_create(tq_handle **out, const tq_config *cfg) {
     for (int k = 0; k < nc && k < 16; ++k) h->centroids_host[k] = cent[k];
     for (int k = 0; k + 1 < nc && k < 15; ++k) h->bounds_host[k] = bounds[k];
     rc = rc ? rc : upload(&h->centroids64, cent);
-    rc = rc ? rc : upload(&h->bounds64, bounds);
+    // The quantisers count the boundaries below a value, so their order is free: ascending, as their search wants them (a
+    // codebook may come in any order), and one that compares with nothing is one that nothing exceeds.
+    auto ascending = [](auto b) {
+        for (auto &v : b)
+            if (v != v) v = std::numeric_limits<double>::infinity();
+        std::sort(b.begin(), b.end());
+        return b;
+    };
+    rc = rc ? rc : upload(&h->bounds64, ascending(bounds));
     std::vector<double> s1, s2;
     if (cfg->rotation == TQ_ROT_WHT) {
         s1.assign(cfg->signs1, cfg->signs1 + pd);
@@ -182,15 +190,9 @@ int tq_create(tq_handle **out, const tq_config *cfg) {
     }
     if (d == 128 && cfg->rotation == TQ_ROT_WHT && cfg->bits <= 4) {
         std::vector<float> c32(cent.begin(), cent.end()), b32(bounds.begin(), bounds.end());
-        // the quantiser counts the boundaries below a value, so their order is free: ascending, as its search wants them
-        // (a codebook may come in any order), and one that compares with nothing is one that nothing exceeds
-        std::vector<float> ascending = b32;
-        for (float &b : ascending)
-            if (b != b) b = std::numeric_limits<float>::infinity();
-        std::sort(ascending.begin(), ascending.end());
         std::vector<float> s1f(s1.begin(), s1.end()), s2f(s2.begin(), s2.end());
         rc = rc ? rc : upload(&h->centroids32, c32);
-        rc = rc ? rc : upload(&h->bounds32, ascending);
+        rc = rc ? rc : upload(&h->bounds32, ascending(b32));
         rc = rc ? rc : upload(&h->s1_32, s1f);
         rc = rc ? rc : upload(&h->s2_32, s2f);
         // pair LUT: entry (hi << bits | lo) = half2(c[lo], c[hi])

@@ -15,7 +15,7 @@ struct tq_handle {
     int device;
     // float64 tables (reference-API kernels)
     double *centroids64;   // [n_centroids]
-    double *bounds64;      // [n_centroids-1] midpoints
+    double *bounds64;      // [n_centroids-1] midpoints, ascending
     double *s1_64, *s2_64; // [pd] (WHT)
     double *rot64;         // [d*d]  Pi,   row-major          (dense)
     double *rot64_t;       // [d*d]  Pi^T, row-major          (dense)
@@ -25,7 +25,7 @@ struct tq_handle {
     int has_proj;
     // float32 tables (production kernels, d == 128, WHT)
     float *centroids32;    // [n_centroids]
-    float *bounds32;       // [n_centroids-1]
+    float *bounds32;       // [n_centroids-1], ascending
     float *s1_32, *s2_32;  // [128]
     double *projrot64_t;   // [128*128] entry [k*128+j] = (S R^T)[j][k]   (d == 128, WHT, projection)
     void *pair_lut;        // [4^bits] half2: (c[lo], c[hi]) for a pair code (bits <= 3), or [256] for 4
