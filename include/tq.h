@@ -147,7 +147,7 @@ int tq_store_kv_cache(const tq_handle *hk, const tq_handle *hv, const void *k, c
 /* The prompt of a layer of any two formats into caches laid out for `capacity` tokens, from position 0: hk / hv NULL
  * stands for q8_0-style rows on that side, whose input then needs no alignment.  Turbo K with turbo V: tq_store_kv_cache.
  * Otherwise the 8-bit side holds the bytes of tq_q8_0_append at position 0 and the turbo side tq_append's or, for long
- * fp16 and fp32 prompts, tq_store's (equal but for values on a code boundary to within 32-bit rounding). */
+ * fp16 prompts, tq_store's (equal but for values on a code boundary to within 32-bit rounding). */
 int tq_store_layer(const tq_handle *hk, const tq_handle *hv, const void *k, const void *v, int64_t n_seqs, int64_t tokens,
                    int64_t capacity, int in_dtype, void *packed_k, void *packed_v, void *stream);
 

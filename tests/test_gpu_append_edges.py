@@ -100,8 +100,9 @@ def test_layer_with_8_bit_rows(fmt, dtypes):
 @pytest.mark.parametrize("dtype", ["float16", "float32", "float64"])
 @pytest.mark.parametrize("tokens", [1023, 1025, 1152])
 def test_prompt_of_a_layer_with_8_bit_rows(fmt, dtype, tokens):
-    """64 sequences of 8 (one launch of the append kernel for K and V at float64 only) and 9 blocks: the 8-bit side as
-    appended, the turbo side as stored, sequence by sequence, and nothing past a sequence's last block."""
+    """64 sequences of 8 (one launch of the append kernel for K and V but for float16) and 9 blocks: the 8-bit side as
+    appended, the turbo side as stored (float16) or appended, sequence by sequence, and nothing past a sequence's last
+    block.  (tq_store takes float32 rows as two fp16 terms: no oracle for rows that are computed in 32 bits.)"""
     tt = L.torch()
     n, capacity = 64, 2048
     layer = tqa.LayerKV(tqa.LayerFormat(*fmt))
@@ -110,8 +111,13 @@ def test_prompt_of_a_layer_with_8_bit_rows(fmt, dtype, tokens):
     caches = [b.fill_(0xA5) for b in layer.new_cache(n, capacity)]
     layer.prefill(k, v, *caches, capacity)
     for codec, x, cache, kind in ((layer.k_codec, k, caches[0], "k"), (layer.v_codec, v, caches[1], "v")):
-        want = tqa.q8_0_store(x, kind=kind)[0] if codec is None else codec.store(x, kind=kind)
         blocks = -(-tokens // 128)
+        if codec is None:
+            want = tqa.q8_0_store(x, kind=kind)[0]
+        elif dtype == "float32":
+            want = codec.append(x, tt.zeros(n * blocks * O.block_bytes(codec.bits), dtype=tt.uint8, device="cuda"), 0, 128 * blocks, kind=kind)
+        else:
+            want = codec.store(x, kind=kind)
         got = cache.view(n, capacity // 128, -1)
         assert tt.equal(got[:, :blocks], want.view(n, blocks, -1)), kind
         assert bool((got[:, blocks:] == 0xA5).all()), kind
@@ -140,3 +146,26 @@ def test_codes_are_the_number_of_boundaries_below(bits, order):
     lo, hi = ((mid[None, None] < (y + e)[..., None]).sum(-1) for e in (-2e-6, 2e-6))   # 32-bit rotation of values up to 1
     assert ((idx >= lo) & (idx <= hi)).all()
     assert (lo == hi).mean() > 0.999
+
+
+@pytest.mark.parametrize("fmt", [("q8_0", "turbo3"), ("turbo4", "q8_0"), ("turbo2", "q8_0")])
+@pytest.mark.parametrize("tokens", [128 * 127, 128 * 128])
+def test_float32_prompts_keep_their_low_bits(fmt, tokens):
+    """Rows of two entries that differ in the last of their 24 bits: half of the rotated values are that difference, on one
+    side of the boundary at zero or the other.  Exact in 32-bit sums, whatever the length of the prompt."""
+    tt = L.torch()
+    layer = tqa.LayerKV(tqa.LayerFormat(*fmt))
+    codec, kind = (layer.v_codec, "v") if layer.k_codec is None else (layer.k_codec, "k")
+    x = np.zeros((4, tokens, D), np.float32)
+    rng = np.random.default_rng(tokens)
+    t = np.arange(tokens)
+    for s in range(4):
+        pair = rng.permuted(np.tile(np.arange(D), (tokens, 1)), axis=1)[:, :2]
+        x[s, t, pair[:, 0]], x[s, t, pair[:, 1]] = 1 + 2.0 ** -12 + 2.0 ** -23, 1 + 2.0 ** -12
+    xd = tt.from_numpy(x).cuda()
+    caches = layer.new_cache(4, tokens)
+    layer.prefill(xd, xd, *caches, tokens)
+    idx = np_(codec.unpack_codes(caches[kind == "v"], 4, tokens, kind=kind)[0]).astype(int)
+    y = O.rotate_fast(x.reshape(-1, D).astype(np.float64), codec.signs1, codec.signs2, D).reshape(x.shape)
+    small = np.abs(y) < 1e-6
+    assert small.mean() == 0.5 and np.array_equal(idx[small], np.where(y > 0, 1 << (codec.bits - 1), (1 << (codec.bits - 1)) - 1)[small])

@@ -4175,8 +4175,10 @@ int tqk_store_kv(const tq_handle *hk, const tq_handle *hv, const void *k, const 
 }
 
 // Prompt of a layer of any two formats (hk / hv NULL: q8_0-style rows) into caches laid out for `capacity` tokens.
-// One 8-bit side: a long prompt's turbo side goes through the matrix-core store (the append's butterfly is bound by its
-// vector instructions) and the 8-bit side through its own launch; a short one is one launch of the append kernel.
+// One 8-bit side and fp16 rows: a long prompt's turbo side goes through the matrix-core store (the append's butterfly is bound
+// by its vector instructions; fp16 products with +-1 are exact there, so both sum the same 32-bit values) and the 8-bit side
+// through its own launch; a short one is one launch of the append kernel.  fp32 rows stay with the append kernel: the
+// matrix cores would take them as two fp16 terms, which drop what lies below 2^-22 of a value (split8).
 // From 512 blocks on two launches are the faster (one / two, us; 8-bit K with turbo3 V, fp16: 512 blocks 19.9 / 17.4, 752 28.6 /
 // 22.8, 2048 62.3 / 47.3; turbo4 V 70.7 / 48.9; turbo3 K with 8-bit V 56.9 / 41.7); below, calls take the host 15 us either way.
 constexpr int64_t PREFILL_SPLIT_BLOCKS = 512;
@@ -4185,7 +4187,8 @@ int tqk_store_layer(const tq_handle *hk, const tq_handle *hv, const void *k, con
     if (hk && hv) return tqk_store_kv(hk, hv, k, v, n_seqs, tokens, capacity, in_dtype, packed_k, packed_v, s);
     const tq_handle *h = hk ? hk : hv;
     const int64_t n_blocks = n_seqs * blocks_for(tokens), out_bps = blocks_for(capacity);
-    if (!h || n_blocks < PREFILL_SPLIT_BLOCKS || !store_fast_ok(h, in_dtype, n_blocks) || out_bps * n_seqs >= (1ll << 28))
+    if (!h || in_dtype != TQ_F16 || n_blocks < PREFILL_SPLIT_BLOCKS || !store_fast_ok(h, in_dtype, n_blocks) ||
+        out_bps * n_seqs >= (1ll << 28))
         return tqk_append_kv(hk, hv, k, v, n_seqs, 0, tokens, capacity, in_dtype, packed_k, packed_v, s);
     const int rc = hk ? tqk_q8_0_append(v, n_seqs, 0, tokens, capacity, in_dtype, TQ_KIND_V, packed_v, s, nullptr, nullptr)
                       : tqk_q8_0_append(k, n_seqs, 0, tokens, capacity, in_dtype, TQ_KIND_K, packed_k, s, nullptr, nullptr);
