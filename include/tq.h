@@ -69,7 +69,8 @@ int tq_fwht(const void *x, void *y, int64_t n, int32_t len, int in_dtype, int ou
 /* The handle's rotation applied to n rows of length d: dense Pi x (polar_quant.py:78)
  * or D2 H D1 x with zero padding (rotation.py:124-185); transpose != 0 applies the
  * transpose (polar_quant.py:114, rotation.py:148-160).  With d == 128, WHT mode and
- * no float64 on either side the one-wavefront-per-vector fp32 butterfly runs. */
+ * no float64 on either side the one-wavefront-per-vector fp32 butterfly runs.
+ * y may be x where both are of one type. */
 int tq_rotate(const tq_handle *h, const void *x, void *y, int64_t n, int in_dtype, int out_dtype,
               int transpose, void *stream);
 
@@ -79,7 +80,7 @@ int tq_nearest_centroid(const double *values, int64_t n, const double *centroids
                         int32_t *idx, void *stream);
 
 /* polar_quant.py:56-85 PolarQuant.quantize: idx [n,d] uint8, norms [n] float64.
- * rotated (optional, may be NULL) receives the rotated unit vectors [n,d] float64. */
+ * rotated (optional, may be NULL) receives the rotated unit vectors [n,d] float64; it may be a float64 x. */
 int tq_quantize_indices(const tq_handle *h, const void *x, int64_t n, int in_dtype, uint8_t *idx, double *norms,
                         double *rotated, void *stream);
 

@@ -90,3 +90,42 @@ def test_codebooks_in_any_order(bits, rotation, order):
     mid = (cent[1:] + cent[:-1]) / 2
     clear = np.abs(y[..., None] - mid).min(axis=-1) > bound(2 * d)
     assert clear.mean() > 0.99 and np.array_equal(idx[clear], (mid < y[..., None]).sum(axis=-1)[clear])
+
+
+def rotate(handle, x, out, transpose=0):
+    """tq_rotate on device tensors."""
+    L.check(L.lib().tq_rotate(handle.h, L.ptr(x), L.ptr(out), x.shape[0], L.dtype_code(x), L.dtype_code(out), transpose, L.stream_ptr()))
+    return out
+
+
+def rounding(dtype):
+    """Half a unit in the last place, relative, and half of the smallest step of a type."""
+    return {"float16": (2.0 ** -11, 2.0 ** -25), "float32": (2.0 ** -24, 2.0 ** -150), "float64": (2.0 ** -53, 0.0)}[dtype]
+
+
+@pytest.mark.parametrize("n,d", [(1, 1), (1, 33), (16, 17), (17, 300), (65, 64), (1001, 130), (9, 1030), (5, 2100)])
+@pytest.mark.parametrize("dtype", ["float16", "float32", "float64"])
+def test_dense_results_in_the_memory_of_the_input(n, d, dtype):
+    """Every column of a row needs the whole row: more than one column block reads what another one stores."""
+    tt = L.torch()
+    rng = np.random.default_rng(n + d)
+    m = np.linalg.qr(rng.standard_normal((d, d)))[0]
+    h = L.Handle(d, 3, np.sort(rng.uniform(-0.3, 0.3, 8)), rotation=m)
+    x = tt.from_numpy(rng.standard_normal((n, d)).astype(dtype)).cuda()
+    x64 = x.cpu().numpy().astype(np.float64)
+    size = np.linalg.norm(x64, axis=1, keepdims=True)
+    rel, step = rounding(dtype)
+    for transpose, want in ((0, x64 @ m.T), (1, x64 @ m)):
+        y = x.clone()
+        rotate(h, y, y, transpose)
+        assert np.all(np.abs(y.cpu().numpy().astype(np.float64) - want) <= (1 + 2.0 ** -20) * (rel * np.abs(want) + bound(d) * size) + step)
+    if dtype == "float64":
+        y = x.clone()
+        idx, norms = quantize_indices(h, y, rotated=y)
+        rotated = x64 @ m.T / size
+        assert np.all(np.abs(y.cpu().numpy() - rotated) <= bound(d))
+        np.testing.assert_allclose(norms, size[:, 0], rtol=bound(d))
+        apart, idx_apart = tt.empty_like(x), quantize_indices(h, x, rotated=None)[0]
+        quantize_indices(h, x, rotated=apart)
+        assert np.all(np.abs(apart.cpu().numpy() - rotated) <= bound(d))
+        assert (idx != idx_apart).mean() < 1e-3

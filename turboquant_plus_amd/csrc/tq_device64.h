@@ -1,6 +1,7 @@
 // float64 block helpers shared by the reference-API kernels and the QJL store
 // kernel: VB vectors staged in LDS, rotated by the sign-diagonal Walsh-Hadamard
-// butterfly in the reference's stage order.
+// butterfly in the reference's stage order, or by a dense matrix where a product
+// has to end in the memory that its rows come from.
 #pragma once
 #include "tq_internal.h"
 
@@ -18,6 +19,7 @@ template <> __device__ inline void std_<__half>(__half *p, int64_t i, double v) 
 
 struct RotArgs {
     int d, pd;
+    const double *mat;      // dense matrix M, row-major, out[j] = sum_k M[k][j] in[k] (pd = d); NULL: the butterfly
     const double *sa, *sb;  // signs applied before / after the butterfly (NULL = ones)
 };
 
@@ -26,6 +28,20 @@ template <int VB>
 __device__ void rotate_block(const RotArgs &r, double *xs, double *ys) {
     const int tid = threadIdx.x;
     const int pd = r.pd;
+    if (r.mat) {
+        for (int j = tid; j < r.d; j += NT) {
+            double acc[VB] = {};
+            for (int k = 0; k < r.d; ++k) {
+                const double m = r.mat[(int64_t)k * r.d + j];
+#pragma unroll
+                for (int v = 0; v < VB; ++v) acc[v] = fma(m, xs[v * pd + k], acc[v]);
+            }
+#pragma unroll
+            for (int v = 0; v < VB; ++v) ys[v * pd + j] = acc[v];
+        }
+        __syncthreads();
+        return;
+    }
     if (r.sa) {
         for (int i = tid; i < VB * pd; i += NT) xs[i] *= r.sa[i % pd];
         __syncthreads();
