@@ -129,3 +129,22 @@ def test_dense_results_in_the_memory_of_the_input(n, d, dtype):
         quantize_indices(h, x, rotated=apart)
         assert np.all(np.abs(apart.cpu().numpy() - rotated) <= bound(d))
         assert (idx != idx_apart).mean() < 1e-3
+
+
+@pytest.mark.parametrize("d", [5, 17, 40, 64, 100, 128, 200, 272, 384, 515])
+def test_results_do_not_depend_on_the_batch(d):
+    """A vector alone, in a batch of a tile row, of some and of many: the same bits, whatever launch each takes."""
+    n = 70_003 if d < 300 else 9_001          # unsplit products
+    x = np.random.default_rng(d).standard_normal((n, d))
+    tq = tqa.TurboQuant(d, 3)
+    g = tq.polar_quant
+    whole = tq.quantize(x)
+    residual = g.quantize_and_residual(x[:3000])[2]
+    back = tq.dequantize(whole)
+    for size in (1, 16, 17, 40, 600, 3000):
+        for at in (0, n - size):
+            part = tq.quantize(x[at:at + size])
+            for name in ("mse_indices", "vector_norms", "qjl_signs", "residual_norms"):
+                assert np.array_equal(getattr(part, name), getattr(whole, name)[at:at + size]), (name, size)
+            assert np.array_equal(tq.dequantize(part), back[at:at + size])
+        assert np.array_equal(g.quantize_and_residual(x[:size])[2], residual[:size])

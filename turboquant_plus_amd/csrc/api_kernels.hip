@@ -30,13 +30,15 @@ __device__ __forceinline__ int level_of(double v, const double *bounds, int bits
 // ---- dense products: out[row][j] = sum_k f(in[row][k]) M[k][j], float64 matrix cores -----------------------------
 // One thread per (output, vector) read the whole matrix from L2 once per VB vectors and an LDS operand per multiply:
 // 1.56 ms per product for 256 vectors of 1536 (0.8 of 75 TFLOP/s), 92 us for 32 768 of 128.  Here a wavefront owns RT x
-// CT tiles of 16 x 16 outputs of v_mfma_f64_16x16x4_f64 and a share of the contraction: 31 and 33 us for the same.  What
+// CT tiles of 16 x 16 outputs of v_mfma_f64_16x16x4_f64 and a slice of the contraction or all of it: 39 and 42 us.  What
 // bounds it is the matrix instruction (64 clocks; 22 and 20 us of them at the 1.7 GHz the part holds here), then the
 // uneven last round of workgroups.  The order of the contraction is free, so in a chunk of 16 values lane quarter q takes
 // values 4q .. 4q+3 for the chunk's four steps: the A operand of four steps is one vector load, the B operand of a step
 // four runs of 128 bytes.  Nothing is staged in LDS during the product.
-// `ks` wavefronts of a workgroup split the contraction (the chunks in turn) and add their tiles in LDS in a fixed
-// order at the end; the other wavefronts work on further rows.  Column blocks are dealt to the XCDs in turn, so that
+// The contraction is summed in `slices` slices (the chunks in turn), as many as the dimension alone says, and the slices are
+// added in their order, so that a vector's results do not depend on the batch it comes in.  SPLIT: a wavefront per slice, the
+// tiles added in LDS at the end, wavefronts past the slices on further rows.  Else a wavefront goes through the slices of its
+// tiles one after the other and keeps their sum beside the running one.  Column blocks are dealt to the XCDs in turn, so that
 // each XCD's L2 holds only its eighth of the matrix (an 18.9 MB matrix at d = 1536 against 4 MB of L2).
 // The vectors' norms are row properties that the contraction's own operands give (one multiply-add per operand
 // beside the tiles' matrix instructions) and divide the finished sums, so nothing passes over the input twice.
@@ -47,7 +49,7 @@ struct DenseArgs {
     int64_t n;
     const double *mat;        // M, row-major [d][d]
     const void *in;           // [n][d]: vectors, indices or signs
-    int ks;                   // wavefronts that share a tile's contraction
+    int slices;               // of the contraction; SPLIT: wavefronts that share a tile's
     unsigned n_row, n_col;    // row and column blocks of the launch
     // quantize: bounds, bits; dequantize: centroids, norm_correction
     const double *bounds, *centroids;
@@ -65,16 +67,17 @@ struct DenseArgs {
 typedef double double4_t __attribute__((ext_vector_type(4)));
 
 // OP, element type of the input, and of the output (of x: DEQUANTIZE)
-template <DenseOp OP, typename TI, typename TO, int RT, int CT, int NW>
+template <DenseOp OP, typename TI, typename TO, int RT, int CT, int NW, bool SPLIT>
 __global__ __launch_bounds__(64 * NW) void k_dense64(DenseArgs a) {
     constexpr bool NORMS = OP == DENSE_QUANTIZE || OP == DENSE_QJL_QUANTIZE || OP == DENSE_DEQUANTIZE;
     constexpr int NT_ = RT * CT;
-    extern __shared__ double sm[];   // [NW][NT_][4][64] partial tiles when ks > 1
+    extern __shared__ double sm[];   // SPLIT: [NW][NT_][4][64] tiles of one slice
     __shared__ double table[OP == DENSE_DEQUANTIZE || OP == DENSE_QUANTIZE ? 256 : 1];
     __shared__ double sq_s[NW][RT * 16];
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int c16 = lane & 15, q = lane >> 4;
-    const int kslice = wave % a.ks, rgroup = wave / a.ks, rgs = NW / a.ks;
+    const int ks = SPLIT ? a.slices : 1;   // wavefronts per tile
+    const int kslice = wave % ks, rgroup = wave / ks, rgs = NW / ks;
     unsigned row_b, col_b;
     if (a.n_col >= 8) {   // column block % 8 = blockIdx % 8 = the XCD
         const unsigned i = blockIdx.x >> 3;
@@ -143,27 +146,8 @@ __global__ __launch_bounds__(64 * NW) void k_dense64(DenseArgs a) {
             }
         }
     };
-    // whole chunks; the request past this wavefront's last one repeats it, so that what has to be waited for is the same on
-    // every path (a branch around the request made the compiler wait for the newest one everywhere: 59 against 32 us for
-    // 256 vectors of 1536; holding the request in front of the products with scheduling barriers changed nothing)
     const int full = d >> 4;
-    int left = (full - kslice + a.ks - 1) / a.ks;
-    if (left > 0) {
-        Operands o0, o1;
-        int c = kslice;
-        load(c, o0);
-        while (true) {
-            c = left > 1 ? c + a.ks : c;
-            load(c, o1);
-            multiply(o0);
-            if (--left == 0) break;
-            c = left > 1 ? c + a.ks : c;
-            load(c, o0);
-            multiply(o1);
-            if (--left == 0) break;
-        }
-    }
-    if ((d & 15) && kslice == full % a.ks) {   // the rest of the contraction, value by value
+    if ((d & 15) && kslice == 0) {   // what is past the whole chunks opens the first slice, value by value
         const int k0 = 16 * full + 4 * q;
 #pragma unroll
         for (int s = 0; s < 4; ++s) {
@@ -180,17 +164,75 @@ __global__ __launch_bounds__(64 * NW) void k_dense64(DenseArgs a) {
             }
         }
     }
-    // norms: this wavefront's share of a row's squares, summed over the lane quarters, then over the wavefronts
+    // squares of a slice of a row, summed over the lane quarters
+    auto slice_sq = [&](int rt) {
+        double s = sq[rt][0] + sq[rt][1];
+        s += __shfl_xor(s, 16);
+        return s + __shfl_xor(s, 32);
+    };
+    // whole chunks; the request past this wavefront's last one repeats it, so that what has to be waited for is the same on
+    // every path (a branch around the request made the compiler wait for the newest one everywhere: 59 against 32 us for
+    // 256 vectors of 1536; holding the request in front of the products with scheduling barriers changed nothing)
+    int left = SPLIT ? (full - kslice + ks - 1) / ks : full;
+    double4_t sum[SPLIT ? 1 : RT][SPLIT ? 1 : CT];   // the finished slices
+    double sq_sum[RT];
+    if constexpr (!SPLIT) {
+#pragma unroll
+        for (int rt = 0; rt < RT; ++rt) {
+            sq_sum[rt] = 0.0;
+#pragma unroll
+            for (int ct = 0; ct < CT; ++ct) sum[rt][ct] = double4_t{0.0, 0.0, 0.0, 0.0};
+        }
+    }
+    auto after = [&](int c) {   // the chunk after c
+        c += a.slices;
+        return SPLIT || c < full ? c : c % a.slices + 1;
+    };
+    auto finish = [&](int c) {   // c: the chunk just multiplied; the last one of its slice?
+        if constexpr (!SPLIT) {
+            if (c + a.slices < full) return;
+#pragma unroll
+            for (int rt = 0; rt < RT; ++rt) {
+                if constexpr (NORMS) {
+                    sq_sum[rt] += slice_sq(rt);
+                    sq[rt][0] = sq[rt][1] = 0.0;
+                }
+#pragma unroll
+                for (int ct = 0; ct < CT; ++ct) {
+                    sum[rt][ct] += acc[rt][ct];
+                    acc[rt][ct] = double4_t{0.0, 0.0, 0.0, 0.0};
+                }
+            }
+        }
+    };
+    if (left > 0) {
+        Operands o0, o1;
+        int c = kslice, next;
+        load(c, o0);
+        while (true) {
+            next = left > 1 ? after(c) : c;
+            load(next, o1);
+            multiply(o0);
+            finish(c);
+            c = next;
+            if (--left == 0) break;
+            next = left > 1 ? after(c) : c;
+            load(next, o0);
+            multiply(o1);
+            finish(c);
+            c = next;
+            if (--left == 0) break;
+        }
+    }
+    // norms: this wavefront's share of a row's squares
     if constexpr (NORMS) {
 #pragma unroll
         for (int rt = 0; rt < RT; ++rt) {
-            double s = sq[rt][0] + sq[rt][1];
-            s += __shfl_xor(s, 16);
-            s += __shfl_xor(s, 32);
+            const double s = SPLIT ? slice_sq(rt) : sq_sum[rt];
             if (q == 0) sq_s[wave][16 * rt + c16] = s;
         }
     }
-    if (a.ks > 1) {
+    if (SPLIT && ks > 1) {
         double *mine = sm + (size_t)wave * NT_ * 256 + lane;
 #pragma unroll
         for (int t = 0; t < NT_; ++t)
@@ -200,7 +242,7 @@ __global__ __launch_bounds__(64 * NW) void k_dense64(DenseArgs a) {
     __syncthreads();
     auto norm_of = [&](int r) {   // row r of this wavefront's rows
         double s = 0.0;
-        for (int w = 0; w < a.ks; ++w) s += sq_s[rgroup * a.ks + w][r];
+        for (int w = 0; w < ks; ++w) s += sq_s[rgroup * ks + w][r];
         return sqrt(s);
     };
     if constexpr (OP == DENSE_QUANTIZE || OP == DENSE_QJL_QUANTIZE) {
@@ -210,17 +252,19 @@ __global__ __launch_bounds__(64 * NW) void k_dense64(DenseArgs a) {
     }
 #pragma unroll
     for (int t = 0; t < NT_; ++t) {
-        if (t % a.ks != kslice) continue;   // the tile's wavefronts share out its tiles
+        if (t % ks != kslice) continue;   // the tile's wavefronts share out its tiles
         const int rt = t / CT, ct = t % CT, col = col0 + 16 * ct + c16;
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
             const int r = 16 * rt + 4 * i + q;
             const int64_t row = row0 + r;
             double y;
-            if (a.ks > 1) {
+            if constexpr (!SPLIT) {
+                y = sum[rt][ct][i];
+            } else if (ks > 1) {
                 y = 0.0;
-                const double *part = sm + (size_t)(rgroup * a.ks) * NT_ * 256 + (t * 4 + i) * 64 + lane;
-                for (int w = 0; w < a.ks; ++w) y += part[(size_t)w * NT_ * 256];
+                const double *part = sm + (size_t)(rgroup * ks) * NT_ * 256 + (t * 4 + i) * 64 + lane;
+                for (int w = 0; w < ks; ++w) y += part[(size_t)w * NT_ * 256];
             } else {
                 y = acc[rt][ct][i];
             }
@@ -252,36 +296,39 @@ __global__ __launch_bounds__(64 * NW) void k_dense64(DenseArgs a) {
     }
 }
 
-template <DenseOp OP, typename TI, typename TO, int RT, int CT, int NW>
-void launch_dense_tiles(DenseArgs a, int ks, hipStream_t s) {
-    a.ks = ks;
+template <DenseOp OP, typename TI, typename TO, int RT, int CT, bool SPLIT>
+void launch_dense_tiles(DenseArgs a, int slices, hipStream_t s) {
+    constexpr int NW = 8;
+    a.slices = slices;
+    const int ks = SPLIT ? slices : 1;
     const int rows = NW / ks * RT * 16;
     a.n_row = (unsigned)((a.n + rows - 1) / rows);
     a.n_col = (unsigned)((a.d + CT * 16 - 1) / (CT * 16));
     const unsigned grid = a.n_col >= 8 ? a.n_row * ((a.n_col + 7) / 8 * 8) : a.n_row * a.n_col;
     const size_t lds = ks > 1 ? (size_t)NW * RT * CT * 256 * sizeof(double) : 0;
     if (lds > 48 * 1024)
-        (void)hipFuncSetAttribute((const void *)k_dense64<OP, TI, TO, RT, CT, NW>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-    k_dense64<OP, TI, TO, RT, CT, NW><<<grid, 64 * NW, lds, s>>>(a);
+        (void)hipFuncSetAttribute((const void *)k_dense64<OP, TI, TO, RT, CT, NW, SPLIT>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+    k_dense64<OP, TI, TO, RT, CT, NW, SPLIT><<<grid, 64 * NW, lds, s>>>(a);
 }
 
-// Tiles and split of the contraction (us per product, splits of 8 / 4 / 2 / 1):
-//   4096 and more 2 x 2 tiles: no split (32 768 vectors of 128: 54 / 40 / 35 / 33); twice the split for half the tiles, so
-//   that a launch has about 4096 wavefronts (4096 of 128: 8.5 / 8.6 / 12.5 / 20; 1000 of 384: 12.6 / 13.0 / 22 / 38);
-//   fewer than 256 of them: 1 x 2 tiles, so that more CUs get a workgroup (100 of 768: 9.1 against 12.2);
-//   up to 16 vectors: single tiles over sixteen wavefronts - what counts is how many wavefronts stream the matrix (one
-//   vector of 1536: 7.9 against 11.0, sixteen: 10.4 against 12.9).
+// Slices: eight, or as many as there are chunks of 16 values; by the dimension alone (see k_dense64).
+// Tiles and wavefronts per tile, by the amount of work (us per product; SPLIT / not):
+//   not SPLIT where whole tiles fill the chip - from 1536 tiles of 2 x 2 below 512 dimensions, where a slice is short beside
+//   the exchange of its tiles (32 768 vectors of 128: 55 / 42; 4096 of 384: 50 / 43; 8192 of 128, 1024 tiles: 17 / 22), from
+//   4096 above (4096 of 768, 3072 tiles: 117 / 141; 4096 of 1536, 6144 tiles: equal);
+//   fewer than 256 tiles of 2 x 2: tiles of 1 x 2, so that more CUs get a workgroup (100 of 768: 10.5 against 13.5);
+//   up to 16 vectors: single tiles (one vector of 1536: 8.0 against 11.5; sixteen: 12.7 against 15.3).
+// A count of slices that follows the work as well (16 / 8 / 4 / 2 / none) has 36.5 us for 32 768 of 128 and 105 for 121 at 32 768
+// of 256, and differs in the last place between a batch and its vectors one by one.
 template <DenseOp OP, typename TI, typename TO>
 int launch_dense(const DenseArgs &a, const char *what, hipStream_t s) {
     const int64_t tiles = ((a.n + 31) / 32) * ((a.d + 31) / 32);
-    const int chunks = (a.d + 15) / 16;
-    auto split = [&](int most) {   // at least one chunk for every wavefront
-        while (most > 1 && most > chunks) most >>= 1;
-        return most;
-    };
-    if (a.n <= 16) launch_dense_tiles<OP, TI, TO, 1, 1, 16>(a, split(16), s);
-    else if (tiles < 256) launch_dense_tiles<OP, TI, TO, 1, 2, 8>(a, split(8), s);
-    else launch_dense_tiles<OP, TI, TO, 2, 2, 8>(a, split(tiles < 1024 ? 8 : tiles < 2048 ? 4 : tiles < 4096 ? 2 : 1), s);
+    int slices = 8;
+    while (slices > 1 && 16 * slices > a.d) slices >>= 1;
+    if (a.n <= 16) launch_dense_tiles<OP, TI, TO, 1, 1, true>(a, slices, s);
+    else if (tiles < 256) launch_dense_tiles<OP, TI, TO, 1, 2, true>(a, slices, s);
+    else if (slices == 1 || tiles < (a.d < 512 ? 1536 : 4096)) launch_dense_tiles<OP, TI, TO, 2, 2, true>(a, slices, s);
+    else launch_dense_tiles<OP, TI, TO, 2, 2, false>(a, slices, s);
     return tq_check_launch(what);
 }
 
