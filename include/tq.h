@@ -85,7 +85,8 @@ int tq_quantize_indices(const tq_handle *h, const void *x, int64_t n, int in_dty
                         double *rotated, void *stream);
 
 /* polar_quant.py:87-119 PolarQuant.dequantize -> out [n,d] float64.  When residual is not
- * NULL also writes residual = x - out (polar_quant.py:121-132); out may then be NULL. */
+ * NULL also writes residual = x - out (polar_quant.py:121-132); out may then be NULL.
+ * An index past the codebook stands for its last entry. */
 int tq_dequantize_indices(const tq_handle *h, const uint8_t *idx, const double *norms, int64_t n, double *out,
                           const void *x, int x_dtype, double *residual, void *stream);
 

@@ -148,3 +148,18 @@ def test_results_do_not_depend_on_the_batch(d):
                 assert np.array_equal(getattr(part, name), getattr(whole, name)[at:at + size]), (name, size)
             assert np.array_equal(tq.dequantize(part), back[at:at + size])
         assert np.array_equal(g.quantize_and_residual(x[:size])[2], residual[:size])
+
+
+@pytest.mark.parametrize("n", [3, 40])
+@pytest.mark.parametrize("rotation", ["dense", "wht"])
+def test_indices_past_the_codebook(rotation, n):
+    """They stand for its last entry, in both modes."""
+    tt = L.torch()
+    d, q = 48, O.PolarRef(48, 3, seed=7, rotation=rotation)
+    tables = dict(rotation=q.rotation) if rotation == "dense" else dict(signs1=q.s1, signs2=q.s2)
+    h = L.Handle(d, 3, q.centroids, **tables)
+    idx = np.random.default_rng(n).integers(0, 256, (n, d)).astype(np.uint8)
+    norms, out = np.linspace(0.5, 2, n), tt.empty((n, d), dtype=tt.float64, device="cuda")
+    idx_d, norms_d = tt.from_numpy(idx).cuda(), tt.from_numpy(norms).cuda()
+    L.check(L.lib().tq_dequantize_indices(h.h, L.ptr(idx_d), L.ptr(norms_d), n, L.ptr(out), None, L.TQ_F64, None, L.stream_ptr()))
+    np.testing.assert_allclose(out.cpu().numpy(), q.dequantize(np.minimum(idx, 7), norms), atol=4 * bound(d) * 2)

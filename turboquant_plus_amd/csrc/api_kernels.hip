@@ -11,8 +11,6 @@
 #include "tq_internal.h"
 #include "tq_device64.h"
 
-#include <type_traits>
-
 namespace {
 
 using namespace tq64;
@@ -92,7 +90,7 @@ __global__ __launch_bounds__(64 * NW) void k_dense64(DenseArgs a) {
     const int64_t row0 = ((int64_t)row_b * rgs + rgroup) * (RT * 16);
     const int col0 = (int)col_b * (CT * 16);
     if constexpr (OP == DENSE_DEQUANTIZE) {
-        for (int e = tid; e < 256; e += 64 * NW) table[e] = e < (1 << a.bits) ? a.centroids[e] : 0.0;
+        for (int e = tid; e < 256; e += 64 * NW) table[e] = a.centroids[min(e, (1 << a.bits) - 1)];
         __syncthreads();
     }
     if constexpr (OP == DENSE_QUANTIZE)
@@ -131,7 +129,7 @@ __global__ __launch_bounds__(64 * NW) void k_dense64(DenseArgs a) {
         for (int ct = 0; ct < CT; ++ct) acc[rt][ct] = double4_t{0.0, 0.0, 0.0, 0.0};
     }
     auto value = [&](TI e) {
-        if constexpr (OP == DENSE_DEQUANTIZE) return table[e];   // 256 entries, those past the codebook 0
+        if constexpr (OP == DENSE_DEQUANTIZE) return table[e];   // 256 entries, those past the codebook its last
         else return ldd(&e, 0);
     };
     auto multiply = [&](const Operands &o) {
