@@ -891,3 +891,33 @@ def test_decode_attention_eight_heads_per_kv_head(kfmt, vfmt):
         if tau:
             assert abs(attn.skip_rate() - skip_o) <= 0.02 * max(skip_o, 1e-3) + 1e-4
             assert int(attn.skip.cpu()[1]) == B * Hq * N
+
+
+def test_split_counts_with_and_without_a_bias_list():
+    """A DecodeAttention picks its split count for either kind of call (the eight-head variant runs other workgroups with a
+    bias list) and has room for both: the two kinds in turn, against the same counts asked for."""
+    B, Hq, Hkv, N = 5, 32, 4, 13000
+    rng = np.random.default_rng(8)
+    kc, vc = tqa.TurboCodec(4, seed=42), tqa.TurboCodec(3, seed=542)
+    kp = kc.store(rng.standard_normal((B * Hkv, N, D)).astype(np.float16), kind="k")
+    vp = vc.store(rng.standard_normal((B * Hkv, N, D)).astype(np.float16), kind="v")
+    q = rng.standard_normal((B, Hq, D)).astype(np.float16)
+    tt = L.torch()
+    pos = tt.arange(0, N, N // 7, dtype=tt.int32, device="cuda")[:7].expand(B, Hq, 7).contiguous()
+    bias = (pos, tt.full((B, Hq, 7), 4.0, device="cuda"))
+    attn = tqa.DecodeAttention(kc, vc, B, Hq, Hkv, N)
+    counts = {}
+    for sb in (None, bias, None, bias):
+        got = np_(attn(q, kp, vp, sparse_bias=sb)).copy()
+        n = counts.setdefault(sb is None, attn.params.n_splits)
+        assert attn.params.n_splits == n
+        want = np_(tqa.DecodeAttention(kc, vc, B, Hq, Hkv, N, n_splits=n)(q, kp, vp, sparse_bias=sb))
+        assert np.array_equal(got, want)
+    assert counts[True] != counts[False]
+    attn.params.n_splits = 16      # the caller's own
+    attn(q, kp, vp)
+    assert attn.params.n_splits == 16
+    p = L.TQAttnParams.from_buffer_copy(attn.params)
+    for n in counts.values():
+        p.n_splits = n
+        assert L.lib().tq_attn_workspace_bytes(L.C.byref(p)) <= attn.workspace.numel()

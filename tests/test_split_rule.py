@@ -41,3 +41,17 @@ def test_rule():
         d = T.default_splits(groups, tokens, eight_heads=kw["eight_heads"])
         n = T.balanced_splits(groups, tokens, d, **kw)
         assert n == d or (n in T._SPLIT_COUNTS and 2 * n <= (tokens + 63) // 64 + 2)
+
+
+def test_room_for_the_table_and_plan_of_a_bias_list():
+    four, eight = dict(eight_heads=False, turbo_k=True, turbo_v=True), dict(eight_heads=True, turbo_k=True, turbo_v=True)
+    # 1000 workgroups of four: four fit a CU, three beside a 32 KB table (8 splits: 25.7 us, 20: 31.3)
+    assert T.balanced_splits(200, 3175, 8, **four) == 20
+    assert T.balanced_splits(200, 3175, 8, three_bit=True, **four) == 8
+    # without workgroups of twelve 36 splits are 360 workgroups of four (48: 49.8 us, 36: 58.0)
+    assert T.balanced_splits(40, 27579, 48, **eight) == 36
+    assert T.balanced_splits(40, 27579, 48, bias_list=True, **eight) == 48
+    # a workgroup of four per CU with Sparse V (32: 38.8 us, 20: 44.7) or a list; without, at 29 700 tokens, 55.3 and 48.0
+    q8v = dict(eight_heads=False, turbo_k=True, turbo_v=False, three_bit=True)
+    assert T.balanced_splits(48, 18060, 32, **q8v) == 20
+    assert T.balanced_splits(48, 18060, 32, sparse_v=True, **q8v) == T.balanced_splits(48, 18060, 32, bias_list=True, **q8v) == 32

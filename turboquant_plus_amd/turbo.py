@@ -474,9 +474,16 @@ class DecodeAttention:
                                       eight_heads=head_dim == HEAD_DIM and n_q_heads // max(n_kv_heads, 1) > 4,
                                       turbo_rows=k_codec is not None and v_codec is not None,
                                       one_workgroup_per_cu=v_codec is None or (head_dim != HEAD_DIM and k_codec is None))
+            self._own_splits = (n_splits, n_splits)
             if head_dim == HEAD_DIM:
-                n_splits = balanced_splits(batch * n_kv_heads, tokens, n_splits, eight_heads=n_q_heads // max(n_kv_heads, 1) > 4,
-                                           turbo_k=k_codec is not None, turbo_v=v_codec is not None)
+                eight, bits = n_q_heads // max(n_kv_heads, 1) > 4, [c.bits for c in (k_codec, v_codec) if c is not None]
+                own = lambda bias_list: balanced_splits(batch * n_kv_heads, tokens, n_splits, eight_heads=eight, turbo_k=k_codec is not None,
+                                                        turbo_v=v_codec is not None, three_bit=3 in bits, bias_list=bias_list,
+                                                        sparse_v=sparse_v_tau > 0)
+                self._own_splits = (own(False), own(True))
+            n_splits = self._own_splits[0]
+        else:
+            self._own_splits = (n_splits, n_splits)
         self.params = L.TQAttnParams(batch=batch, n_q_heads=n_q_heads, n_kv_heads=n_kv_heads, tokens=tokens,
                                      capacity=capacity, n_splits=n_splits, k_format=L.KFMT_TURBO if k_codec is not None else L.KFMT_Q8_0,
                                      v_format=L.KFMT_TURBO if v_codec is not None else L.KFMT_Q8_0,
@@ -489,9 +496,12 @@ class DecodeAttention:
             if sparse_v_tau > 0:
                 raise ValueError("Sparse V keeps no count for a context length read from device memory")
             self.params.tokens_dev = tokens_on_device.data_ptr()
-        nbytes = L.lib().tq_attn_workspace_bytes(C.byref(self.params))
-        if nbytes < 0:
-            L.check(L.ERR_ARG)
+        nbytes = 0
+        for self.params.n_splits in self._own_splits[::-1]:     # room for either kind of call; without a list comes last
+            need = L.lib().tq_attn_workspace_bytes(C.byref(self.params))
+            if need < 0:
+                L.check(L.ERR_ARG)
+            nbytes = max(nbytes, need)
         self.workspace = tt.empty(int(nbytes), dtype=tt.uint8, device=dev)
         self.skip = tt.zeros(2, dtype=tt.int64, device=dev)
         self.out = tt.empty((batch, n_q_heads, head_dim), dtype=tt.float32, device=dev)
@@ -519,6 +529,8 @@ class DecodeAttention:
         else:
             self.params.bias_entries = 0
             self.params.bias_pos = self.params.bias_val = None
+        if self.params.n_splits in self._own_splits:    # not where the caller has set another one
+            self.params.n_splits = self._own_splits[self.params.bias_entries > 0]
         hk = self.k_codec.handle.h if self.k_codec is not None else None
         hv = self.v_codec.handle.h if self.v_codec is not None else None
         L.check(L.lib().tq_decode_attention(hk, hv, C.byref(self.params), L.ptr(qd),
@@ -626,39 +638,59 @@ def _workgroups(n: int, n_groups: int, eight_heads: bool, turbo_k: bool, turbo_v
 
 # What a step takes, in microseconds: a constant, per tile that the fullest CU works through, per tile on the longest
 # wavefront of each round of workgroups, per partial of a group to merge, per round; and the wavefronts that a CU holds.
-# Fitted to 1300 timings (4 to 192 groups, 21 to 938 tiles of 64 tokens, 8 to 16 split counts each) to 6 - 8 %.
+# Fitted to 1300 timings (4 to 192 groups, 21 to 938 tiles of 64 tokens, 8 to 16 split counts each) to 6 - 8 %; over 9400
+# shapes drawn since, its ratios between counts of one shape scatter by 13 - 16 %.
 _SPLIT_COST = {  # by (more than four heads per KV head, turbo V rows); 8-bit V rows: one line for both
     (False, True): (2.85, 0.22, 0.41, 0.08, 7.42, 16),
     (False, False): (5.2, 0.36, 0.0, 0.11, 5.2, 8),
     (True, True): (6.09, 0.34, 0.72, 0.21, 7.2, 8),
 }
 _SPLIT_COUNTS = (8, 12, 16, 20, 24, 28, 32, 36, 40, 48, 56, 64, 72, 80, 96, 112, 128, 160, 192, 256)
+_LDS_PER_CU, _WAVE_MERGE_BYTES, _QUERY_BYTES = 160 * 1024, 2080, 1024    # the latter two per set of four heads
 
 
-def balanced_splits(n_groups: int, tokens: int, default: int, *, eight_heads: bool, turbo_k: bool, turbo_v: bool) -> int:
+def balanced_splits(n_groups: int, tokens: int, default: int, *, eight_heads: bool, turbo_k: bool, turbo_v: bool,
+                    three_bit: bool = False, bias_list: bool = False, sparse_v: bool = False) -> int:
     """The split count for 128-dim heads: `default` (default_splits) unless another count spreads the tiles over the CUs
     clearly better.  default_splits aims at a number of wavefronts and rounds down to multiples of 16, which suits group
     counts and lengths that are powers of two.  With others it makes little more than a round of the 256 workgroups that fit
     (20 groups: 320 workgroups of six), gives short contexts half the wavefronts they could use (63 tiles: 16 splits for 31),
     or hundreds of partials to merge (two groups: 528 splits).  The estimate counts what the fullest CU has to do; another
-    count is taken where it is put 12 % below the default (18 % for eight heads on 8-bit V rows, whose fit is the poorest; its
-    error is 6 - 8 %).  Of 178 shapes measured that it would order differently 73 pass that line: all faster, 19 % on
-    average; at 5 % 21 of 110 were slower, by up to 12 %.  Default and this rule: 20 groups at 115 800 tokens, eight heads:
-    1.36 times as fast with 72 splits for 96; 40 groups at 25 000 tokens: 72.0 and 48.2 us (36 for 48); 8 groups at 4000, four
-    heads: 14.6 and 13.6 us (32 for 16); 144 groups at 13 000, four heads: 1.37 times (28 for 8)."""
+    count is taken where it is put 12 % below the default (18 % for eight heads on 8-bit V rows, whose fit is the poorest; at
+    5 % a fifth of the shapes were slower, by up to 12 %).
+    three_bit: 3-bit codes on either side, whose 32 KB table leaves a CU room for three workgroups of four wavefronts where
+    the registers hold four (200 groups at 3175 tokens: 25.7 us with 8 splits, 31.3 with 20).
+    bias_list: the call carries a sparse bias, which runs without the eight-head variant's workgroups of twelve (40 groups at
+    27 600 tokens: 49.8 us with 48 splits, 58.0 with 36, which without a list are the better ones).
+    sparse_v: the call skips V rows.  With it or a bias list, turbo K with 8-bit V rows is worse off with a workgroup of four
+    wavefronts per CU than the estimate says (48 groups at 18 000 tokens: 38.8 us with 32 splits, 44.7 with 20), which counts
+    only where it saves the merge of many partials.
+    Of 9400 shapes timed with every count, 2240 calls without a bias list get another count than the default (21 % faster on
+    average; 21 of them more than 3 % slower, one 10 %), and 2075 of those with one (18 %; 24, one 15 %)."""
     cost = _SPLIT_COST.get((eight_heads, turbo_v), _SPLIT_COST[(False, False)])
     tiles = max(1, (tokens + 63) // 64)
+    sets = 2 if eight_heads else 1
+    table = 32768 if three_bit else 2048
+
+    def plan(n):
+        waves, parts, wgs = _workgroups(n, n_groups, eight_heads, turbo_k and not bias_list, turbo_v)
+        return waves, parts, -(-wgs // 256)
 
     def estimate(n):
-        waves, parts, wgs = _workgroups(n, n_groups, eight_heads, turbo_k, turbo_v)
-        per_cu, deep = -(-wgs // 256), -(-tiles // n)
-        rounds = -(-per_cu // max(1, cost[5] // waves))
+        waves, parts, per_cu = plan(n)
+        room = _LDS_PER_CU // (table + sets * (waves * _WAVE_MERGE_BYTES + _QUERY_BYTES))
+        deep, rounds = -(-tiles // n), -(-per_cu // max(1, min(cost[5] // waves, room)))
         return cost[0] + cost[1] * per_cu * waves * deep + cost[2] * rounds * deep + cost[3] * parts + cost[4] * rounds
+
+    def wavefronts(n):      # on the fullest CU
+        waves, _, per_cu = plan(n)
+        return waves * per_cu
 
     # two tiles per wavefront at least; 256 to 8192 wavefronts, the range of the fit; eight heads: at most three rounds (with
     # four the estimate was wrong by 30 %)
-    counts = [n for n in _SPLIT_COUNTS if n <= tiles // 2 + 1 and 256 <= n * n_groups <= 8192
-              and (not eight_heads or _workgroups(n, n_groups, eight_heads, turbo_k, turbo_v)[2] <= 768)]
+    counts = [n for n in _SPLIT_COUNTS if n <= tiles // 2 + 1 and 256 <= n * n_groups <= 8192 and (not eight_heads or plan(n)[2] <= 3)]
+    if turbo_k and not turbo_v and (bias_list or sparse_v) and plan(default)[1] <= 8:
+        counts = [n for n in counts if wavefronts(n) >= min(8, wavefronts(default))]
     if not counts:
         return default
     best = min(counts, key=estimate)
