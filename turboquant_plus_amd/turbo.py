@@ -480,7 +480,8 @@ class DecodeAttention:
                 own = lambda bias_list: balanced_splits(batch * n_kv_heads, tokens, n_splits, eight_heads=eight, turbo_k=k_codec is not None,
                                                         turbo_v=v_codec is not None, three_bit=3 in bits, bias_list=bias_list,
                                                         sparse_v=sparse_v_tau > 0)
-                self._own_splits = (own(False), own(True))
+                plain = own(False)      # a bias list changes the plan of eight heads on turbo K, and the rule for 8-bit V rows
+                self._own_splits = (plain, own(True) if k_codec is not None and (eight or v_codec is None) else plain)
             n_splits = self._own_splits[0]
         else:
             self._own_splits = (n_splits, n_splits)
