@@ -17,9 +17,11 @@ def bound(d):
 
 
 # one vector and up to 16 (single tiles), one tile row more, several rows and a remainder; dimensions below, at and past a
-# chunk of 16 values, a tile of 16 columns and the eight column blocks that are dealt to the XCDs
+# chunk of 16 values, a tile of 16 columns and the eight column blocks that are dealt to the XCDs; the last four go through
+# the slices of their contraction in one wavefront: eight row groups a workgroup, the last ones past the end
 @pytest.mark.parametrize("n,d", [(1, 1), (3, 2), (16, 16), (17, 15), (2, 17), (33, 31), (16, 130), (31, 33), (65, 64), (5, 250),
-                                 (40, 257), (700, 129), (2100, 200), (4500, 272)])
+                                 (40, 257), (700, 129), (2100, 200), (4500, 272), (9001, 272),
+                                 (40003, 100), (52001, 31), (6700, 600)])
 @pytest.mark.parametrize("dtype", [np.float32, np.float64])
 def test_dense_products_at_tile_edges(n, d, dtype):
     x = (np.random.default_rng(n * 1000 + d).standard_normal((n, d)) * np.logspace(-3, 3, n)[:, None]).astype(dtype)
@@ -51,7 +53,7 @@ def test_dense_products_at_tile_edges(n, d, dtype):
 
 @pytest.mark.parametrize("bits", [1, 5, 8])
 def test_level_search_at_every_width(bits):
-    """The level of a value is the number of midpoints below it; midpoints themselves and NaN included."""
+    """The level of a value is the number of midpoints below it."""
     g = tqa.PolarQuant(64, bits, seed=3)
     x = np.random.default_rng(bits).standard_normal((300, 64))
     idx, norms = g.quantize(x)
@@ -163,3 +165,51 @@ def test_indices_past_the_codebook(rotation, n):
     idx_d, norms_d = tt.from_numpy(idx).cuda(), tt.from_numpy(norms).cuda()
     L.check(L.lib().tq_dequantize_indices(h.h, L.ptr(idx_d), L.ptr(norms_d), n, L.ptr(out), None, L.TQ_F64, None, L.stream_ptr()))
     np.testing.assert_allclose(out.cpu().numpy(), q.dequantize(np.minimum(idx, 7), norms), atol=4 * bound(d) * 2)
+
+
+@pytest.mark.parametrize("bits", [1, 2, 3, 4, 5, 8])
+@pytest.mark.parametrize("rotation", ["dense", "wht"])
+def test_values_on_a_midpoint_and_nan(bits, rotation):
+    """A value equal to a midpoint takes the level below it, NaN level 0.  Every step is exact: midpoints are multiples of
+    1/8 (or of a finer power of two), rows have norm 1 and entries 0, +-1/2, +-1/4 or +-1/8, the rotation is the identity or a
+    butterfly that gives them back."""
+    d, rng = 64, np.random.default_rng(bits)
+    rows = np.zeros((96, d))
+    for r in range(96):
+        count = (4, 16, 64)[r % 3]
+        rows[r, rng.permutation(d)[:count]] = rng.choice([-1.0, 1.0], count) / np.sqrt(count)
+    cent = (np.arange(1 << bits) + 0.5) / (1 << (bits - 1)) - 1.0
+    mid = (cent[:-1] + cent[1:]) / 2
+    assert bits == 1 or np.isin(rows, mid).any()
+    if rotation == "dense":
+        h, x = L.Handle(d, bits, cent, rotation=np.eye(d)), rows.copy()
+    else:
+        h, x = L.Handle(d, bits, cent, signs1=np.ones(d), signs2=np.ones(d)), O.rotate_fast(rows, np.ones(d), np.ones(d), d)
+    x[5, 7] = np.nan
+    tt = L.torch()
+    for n in (1, 40, 96):
+        idx, norms = quantize_indices(h, tt.from_numpy(x[:n]).cuda())
+        want = np.searchsorted(mid, rows[:n].ravel(), side="left").reshape(n, d)
+        if n > 5:
+            want[5] = 0
+            assert np.isnan(norms[5])
+        assert np.array_equal(idx, want) and np.array_equal(np.delete(norms, 5) if n > 5 else norms, np.ones(n - (n > 5)))
+
+
+@pytest.mark.parametrize("n,d", [(3, 40), (100, 130), (60_000, 33)])
+@pytest.mark.parametrize("dtype", ["float16", "float32", "float64"])
+@pytest.mark.parametrize("out_dtype", ["float16", "float32", "float64"])
+def test_dense_rotation(n, d, dtype, out_dtype):
+    """tq_rotate on a dense handle, forward and transposed, every pair of types in each of the launches."""
+    tt = L.torch()
+    rng = np.random.default_rng(n + d)
+    m = np.linalg.qr(rng.standard_normal((d, d)))[0]
+    h = L.Handle(d, 2, np.linspace(-0.3, 0.3, 4), rotation=m)
+    x = tt.from_numpy(rng.standard_normal((n, d)).astype(dtype)).cuda()
+    x64 = x.cpu().numpy().astype(np.float64)
+    size = np.linalg.norm(x64, axis=1, keepdims=True)
+    rel, step = rounding(out_dtype)
+    for transpose, want in ((0, x64 @ m.T), (1, x64 @ m)):
+        y = rotate(h, x, tt.empty((n, d), dtype=getattr(tt, out_dtype), device="cuda"), transpose)
+        # fp16 results are rounded to fp32 on the way
+        assert np.all(np.abs(y.cpu().numpy().astype(np.float64) - want) <= (1 + 2.0 ** -10) * (rel * np.abs(want) + bound(d) * size) + step)

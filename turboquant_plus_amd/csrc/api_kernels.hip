@@ -28,7 +28,7 @@ __device__ __forceinline__ int level_of(double v, const double *bounds, int bits
 // ---- dense products: out[row][j] = sum_k f(in[row][k]) M[k][j], float64 matrix cores -----------------------------
 // One thread per (output, vector) read the whole matrix from L2 once per VB vectors and an LDS operand per multiply:
 // 1.56 ms per product for 256 vectors of 1536 (0.8 of 75 TFLOP/s), 92 us for 32 768 of 128.  Here a wavefront owns RT x
-// CT tiles of 16 x 16 outputs of v_mfma_f64_16x16x4_f64 and a slice of the contraction or all of it: 39 and 42 us.  What
+// CT tiles of 16 x 16 outputs of v_mfma_f64_16x16x4_f64 and a slice of the contraction or all of it: 39 and 39 us.  What
 // bounds it is the matrix instruction (64 clocks; 22 and 20 us of them at the 1.7 GHz the part holds here), then the
 // uneven last round of workgroups.  The order of the contraction is free, so in a chunk of 16 values lane quarter q takes
 // values 4q .. 4q+3 for the chunk's four steps: the A operand of four steps is one vector load, the B operand of a step
@@ -38,7 +38,8 @@ __device__ __forceinline__ int level_of(double v, const double *bounds, int bits
 // tiles added in LDS at the end, wavefronts past the slices on further rows.  Else a wavefront goes through the slices of its
 // tiles one after the other and keeps their sum beside the running one.  Column blocks are dealt to the XCDs in turn, so that
 // each XCD's L2 holds only its eighth of the matrix (an 18.9 MB matrix at d = 1536 against 4 MB of L2).
-// The vectors' norms are row properties that the contraction's own operands give (one multiply-add per operand
+// The vectors' norms are row properties that the contraction's own operands give, a lane quarter's squares summed over the
+// slices and then over the quarters (one multiply-add per operand
 // beside the tiles' matrix instructions) and divide the finished sums, so nothing passes over the input twice.
 enum DenseOp { DENSE_ROTATE, DENSE_QUANTIZE, DENSE_DEQUANTIZE, DENSE_QJL_QUANTIZE, DENSE_QJL_DEQUANTIZE };
 
@@ -71,7 +72,8 @@ __global__ __launch_bounds__(64 * NW) void k_dense64(DenseArgs a) {
     constexpr int NT_ = RT * CT;
     extern __shared__ double sm[];   // SPLIT: [NW][NT_][4][64] tiles of one slice
     __shared__ double table[OP == DENSE_DEQUANTIZE || OP == DENSE_QUANTIZE ? 256 : 1];
-    __shared__ double sq_s[NW][RT * 16];
+    __shared__ double sq_s[NORMS && SPLIT ? NW : 1][4][RT * 16];   // squares of a slice's rows by lane quarter
+    __shared__ double norm_s[NORMS ? NW : 1][RT * 16];
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int c16 = lane & 15, q = lane >> 4;
     const int ks = SPLIT ? a.slices : 1;   // wavefronts per tile
@@ -162,12 +164,6 @@ __global__ __launch_bounds__(64 * NW) void k_dense64(DenseArgs a) {
             }
         }
     }
-    // squares of a slice of a row, summed over the lane quarters
-    auto slice_sq = [&](int rt) {
-        double s = sq[rt][0] + sq[rt][1];
-        s += __shfl_xor(s, 16);
-        return s + __shfl_xor(s, 32);
-    };
     // whole chunks; the request past this wavefront's last one repeats it, so that what has to be waited for is the same on
     // every path (a branch around the request made the compiler wait for the newest one everywhere: 59 against 32 us for
     // 256 vectors of 1536; holding the request in front of the products with scheduling barriers changed nothing)
@@ -192,7 +188,7 @@ __global__ __launch_bounds__(64 * NW) void k_dense64(DenseArgs a) {
 #pragma unroll
             for (int rt = 0; rt < RT; ++rt) {
                 if constexpr (NORMS) {
-                    sq_sum[rt] += slice_sq(rt);
+                    sq_sum[rt] += sq[rt][0] + sq[rt][1];
                     sq[rt][0] = sq[rt][1] = 0.0;
                 }
 #pragma unroll
@@ -222,12 +218,18 @@ __global__ __launch_bounds__(64 * NW) void k_dense64(DenseArgs a) {
             if (--left == 0) break;
         }
     }
-    // norms: this wavefront's share of a row's squares
+    // norms: a lane quarter's squares, summed over the slices, then over the quarters
     if constexpr (NORMS) {
 #pragma unroll
         for (int rt = 0; rt < RT; ++rt) {
-            const double s = SPLIT ? slice_sq(rt) : sq_sum[rt];
-            if (q == 0) sq_s[wave][16 * rt + c16] = s;
+            double s = SPLIT ? sq[rt][0] + sq[rt][1] : sq_sum[rt];
+            if (SPLIT && ks > 1) {
+                sq_s[wave][q][16 * rt + c16] = s;
+            } else {
+                s += __shfl_xor(s, 16);
+                s += __shfl_xor(s, 32);
+                if (q == 0) norm_s[rgroup][16 * rt + c16] = sqrt(s);
+            }
         }
     }
     if (SPLIT && ks > 1) {
@@ -238,15 +240,23 @@ __global__ __launch_bounds__(64 * NW) void k_dense64(DenseArgs a) {
             for (int i = 0; i < 4; ++i) mine[(t * 4 + i) * 64] = acc[t / CT][t % CT][i];
     }
     __syncthreads();
-    auto norm_of = [&](int r) {   // row r of this wavefront's rows
-        double s = 0.0;
-        for (int w = 0; w < ks; ++w) s += sq_s[rgroup * ks + w][r];
-        return sqrt(s);
-    };
+    if constexpr (NORMS && SPLIT) {
+        if (ks > 1) {
+            for (int e = tid; e < rgs * RT * 16; e += 64 * NW) {
+                const int g = e / (RT * 16), r = e % (RT * 16);
+                double t[4] = {0.0, 0.0, 0.0, 0.0};
+                for (int w = 0; w < ks; ++w)
+#pragma unroll
+                    for (int k = 0; k < 4; ++k) t[k] += sq_s[g * ks + w][k][r];
+                norm_s[g][r] = sqrt((t[0] + t[1]) + (t[2] + t[3]));
+            }
+            __syncthreads();
+        }
+    }
     if constexpr (OP == DENSE_QUANTIZE || OP == DENSE_QJL_QUANTIZE) {
         if (col_b == 0 && kslice == 0)
             for (int r = lane; r < RT * 16; r += 64)
-                if (row0 + r < a.n) a.norms_out[row0 + r] = norm_of(r);
+                if (row0 + r < a.n) a.norms_out[row0 + r] = norm_s[rgroup][r];
     }
 #pragma unroll
     for (int t = 0; t < NT_; ++t) {
@@ -271,13 +281,13 @@ __global__ __launch_bounds__(64 * NW) void k_dense64(DenseArgs a) {
             if constexpr (OP == DENSE_ROTATE) {
                 std_(reinterpret_cast<TO *>(a.out), at, y);
             } else if constexpr (OP == DENSE_QUANTIZE) {
-                const double nv = norm_of(r);
+                const double nv = norm_s[rgroup][r];
                 y /= nv > 0.0 ? nv : 1.0;
                 reinterpret_cast<uint8_t *>(a.out)[at] = (uint8_t)level_of(y, table, a.bits);
                 if (a.rotated) a.rotated[at] = y;
             } else if constexpr (OP == DENSE_DEQUANTIZE) {
                 if (a.norm_correction) {
-                    const double cn = norm_of(r);
+                    const double cn = norm_s[rgroup][r];
                     y /= cn > 1e-10 ? cn : 1.0;
                 }
                 const double v = y * a.norms_in[row];
@@ -312,12 +322,13 @@ void launch_dense_tiles(DenseArgs a, int slices, hipStream_t s) {
 // Slices: eight, or as many as there are chunks of 16 values; by the dimension alone (see k_dense64).
 // Tiles and wavefronts per tile, by the amount of work (us per product; SPLIT / not):
 //   not SPLIT where whole tiles fill the chip - from 1536 tiles of 2 x 2 below 512 dimensions, where a slice is short beside
-//   the exchange of its tiles (32 768 vectors of 128: 55 / 42; 4096 of 384: 50 / 43; 8192 of 128, 1024 tiles: 17 / 22), from
+//   the exchange of its tiles (32 768 vectors of 128: 55 / 39; 4096 of 384: 50 / 43; 8192 of 128, 1024 tiles: 17 / 22), from
 //   4096 above (4096 of 768, 3072 tiles: 117 / 141; 4096 of 1536, 6144 tiles: equal);
 //   fewer than 256 tiles of 2 x 2: tiles of 1 x 2, so that more CUs get a workgroup (100 of 768: 10.5 against 13.5);
 //   up to 16 vectors: single tiles (one vector of 1536: 8.0 against 11.5; sixteen: 12.7 against 15.3).
-// A count of slices that follows the work as well (16 / 8 / 4 / 2 / none) has 36.5 us for 32 768 of 128 and 105 for 121 at 32 768
-// of 256, and differs in the last place between a batch and its vectors one by one.
+// A count of slices that follows the work as well (16 / 8 / 4 / 2 / none) is up to a tenth faster for many vectors (32 768 of
+// 128: 37.9 us, of 256: 106 for 116, 1000 of 1536: 102 for 114) and differs in the last place between a batch and its vectors
+// one by one.
 template <DenseOp OP, typename TI, typename TO>
 int launch_dense(const DenseArgs &a, const char *what, hipStream_t s) {
     const int64_t tiles = ((a.n + 31) / 32) * ((a.d + 31) / 32);
