@@ -914,9 +914,11 @@ def test_split_counts_with_and_without_a_bias_list():
         want = np_(tqa.DecodeAttention(kc, vc, B, Hq, Hkv, N, n_splits=n)(q, kp, vp, sparse_bias=sb))
         assert np.array_equal(got, want)
     assert counts[True] != counts[False]
-    attn.params.n_splits = 16      # the caller's own
-    attn(q, kp, vp)
-    assert attn.params.n_splits == 16
+    for n in (16, counts[True]):      # the caller's own, also where it is the other kind's
+        attn.params.n_splits = n
+        attn(q, kp, vp)
+        attn(q, kp, vp, sparse_bias=bias)
+        assert attn.params.n_splits == n
     p = L.TQAttnParams.from_buffer_copy(attn.params)
     for n in counts.values():
         p.n_splits = n

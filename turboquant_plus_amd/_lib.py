@@ -200,9 +200,14 @@ def device_block(*specs):
     return buf, [buf[o:o + math.prod(shape) * dtype.itemsize].view(dtype).view(shape) for o, (shape, dtype) in zip(offs, specs)]
 
 
-ONE_COPY = 1 << 19      # a block up to this size travels as one pageable copy (a copy costs 14 us before its first byte)
-# Bytes of the result that one pinned staging slot holds, and threads that empty it (2 x 4 x 4096 vectors of 128 compressed
-# and decompressed: 8.8 ms; 1 MiB slots 16.2, 4 MiB 11.4, 16 MiB 9.7, four threads 9.6, eight 9.2).
+# A block up to this size travels as one pageable copy (a copy costs 14 us before its first byte).  64 rows of 384: 0.23 ms, 0.25
+# with 128 KiB; a cache of 2 x 4 x 512 x 128: 1.44 and 1.55.
+ONE_COPY = 1 << 19
+# Bytes of the result that one pinned staging slot holds, and threads that empty it.  Both ways through the classes, ms, with
+# slots of 1 / 4 / 8 / 16 MiB and with three / eight threads: a cache of 2 x 4 x 4096 x 128 in float32 15.3 / 14.2 / 9.3 / 9.4 and
+# 10.0 / 10.5, in float64 16.7 / 15.5 / 10.8 / 10.8 and 11.3 / 11.6; 20 000 rows of 384 in float32 14.3 / 13.2 / 9.2 / 8.1 and 10.0 /
+# 10.0, 4096 of 1536 in float64 18.8 / 21.3 / 9.9 / 9.5 and 11.3 / 10.5; 256 rows of 1536 and a cache of 2 x 4 x 512 x 128 alike with
+# all of them.  On one host with 16 CPUs; with fewer the threads are the limit.
 STAGE = 8 << 20
 COPY_THREADS = 6
 _copiers = None

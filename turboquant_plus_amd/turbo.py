@@ -503,6 +503,7 @@ class DecodeAttention:
             if need < 0:
                 L.check(L.ERR_ARG)
             nbytes = max(nbytes, need)
+        self._splits_set = self.params.n_splits
         self.workspace = tt.empty(int(nbytes), dtype=tt.uint8, device=dev)
         self.skip = tt.zeros(2, dtype=tt.int64, device=dev)
         self.out = tt.empty((batch, n_q_heads, head_dim), dtype=tt.float32, device=dev)
@@ -530,8 +531,8 @@ class DecodeAttention:
         else:
             self.params.bias_entries = 0
             self.params.bias_pos = self.params.bias_val = None
-        if self.params.n_splits in self._own_splits:    # not where the caller has set another one
-            self.params.n_splits = self._own_splits[self.params.bias_entries > 0]
+        if self.params.n_splits == self._splits_set:    # not where the caller has set another one
+            self.params.n_splits = self._splits_set = self._own_splits[self.params.bias_entries > 0]
         hk = self.k_codec.handle.h if self.k_codec is not None else None
         hv = self.v_codec.handle.h if self.v_codec is not None else None
         L.check(L.lib().tq_decode_attention(hk, hv, C.byref(self.params), L.ptr(qd),
