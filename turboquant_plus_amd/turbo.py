@@ -674,25 +674,27 @@ def balanced_splits(n_groups: int, tokens: int, default: int, *, eight_heads: bo
     sets = 2 if eight_heads else 1
     table = 32768 if three_bit else 2048
 
-    def plan(n):
+    # two tiles per wavefront at least; 256 to 8192 wavefronts, the range of the fit
+    counts = [n for n in _SPLIT_COUNTS if n <= tiles // 2 + 1 and 256 <= n * n_groups <= 8192]
+    if not counts:
+        return default
+    # wavefronts per workgroup, partials per group, workgroups on the fullest CU
+    plans = {}
+    for n in {default, *counts}:
         waves, parts, wgs = _workgroups(n, n_groups, eight_heads, turbo_k and not bias_list, turbo_v)
-        return waves, parts, -(-wgs // 256)
+        plans[n] = waves, parts, -(-wgs // 256)
 
     def estimate(n):
-        waves, parts, per_cu = plan(n)
+        waves, parts, per_cu = plans[n]
         room = _LDS_PER_CU // (table + sets * (waves * _WAVE_MERGE_BYTES + _QUERY_BYTES))
         deep, rounds = -(-tiles // n), -(-per_cu // max(1, min(cost[5] // waves, room)))
         return cost[0] + cost[1] * per_cu * waves * deep + cost[2] * rounds * deep + cost[3] * parts + cost[4] * rounds
 
-    def wavefronts(n):      # on the fullest CU
-        waves, _, per_cu = plan(n)
-        return waves * per_cu
-
-    # two tiles per wavefront at least; 256 to 8192 wavefronts, the range of the fit; eight heads: at most three rounds (with
-    # four the estimate was wrong by 30 %)
-    counts = [n for n in _SPLIT_COUNTS if n <= tiles // 2 + 1 and 256 <= n * n_groups <= 8192 and (not eight_heads or plan(n)[2] <= 3)]
-    if turbo_k and not turbo_v and (bias_list or sparse_v) and plan(default)[1] <= 8:
-        counts = [n for n in counts if wavefronts(n) >= min(8, wavefronts(default))]
+    if eight_heads:     # at most three rounds: with four the estimate was wrong by 30 %
+        counts = [n for n in counts if plans[n][2] <= 3]
+    waves, parts, per_cu = plans[default]
+    if turbo_k and not turbo_v and (bias_list or sparse_v) and parts <= 8:
+        counts = [n for n in counts if plans[n][0] * plans[n][2] >= min(8, waves * per_cu)]
     if not counts:
         return default
     best = min(counts, key=estimate)
