@@ -213,3 +213,27 @@ def test_dense_rotation(n, d, dtype, out_dtype):
         y = rotate(h, x, tt.empty((n, d), dtype=getattr(tt, out_dtype), device="cuda"), transpose)
         # fp16 results are rounded to fp32 on the way
         assert np.all(np.abs(y.cpu().numpy().astype(np.float64) - want) <= (1 + 2.0 ** -10) * (rel * np.abs(want) + bound(d) * size) + step)
+
+
+@pytest.mark.parametrize("n", [8, 40, 300])
+@pytest.mark.parametrize("rotation", ["dense", "wht"])
+def test_rows_whose_norm_is_past_the_range(rotation, n):
+    """Finite entries over an infinite norm are zeros (their sums may overflow first); an infinite entry makes NaN."""
+    d, rng = 100, np.random.default_rng(n)
+    q = O.PolarRef(d, 3, seed=7, rotation=rotation)
+    tables = dict(rotation=q.rotation) if rotation == "dense" else dict(signs1=q.s1, signs2=q.s2)
+    h = L.Handle(d, 3, q.centroids, **tables)
+    x = rng.standard_normal((n, d))
+    x[0] = rng.choice([-1.0, 1.0], d) * 1.7e308
+    x[1] = 1.7e308
+    x[2] *= 1e200
+    x[3, 5] = -np.inf
+    tt = L.torch()
+    rotated = tt.empty((n, d), dtype=tt.float64, device="cuda")
+    idx, norms = quantize_indices(h, tt.from_numpy(x).cuda(), rotated=rotated)
+    zero = int((((q.centroids[1:] + q.centroids[:-1]) / 2) < 0.0).sum())
+    y = rotated.cpu().numpy()
+    assert (idx[:3] == zero).all() and (y[:3] == 0.0).all() and np.isinf(norms[:4]).all()
+    assert (idx[3] == 0).all() and np.isnan(y[3]).all()
+    want, wn = q.quantize(x[4:])
+    assert (idx[4:] != want).mean() < 1e-3 and np.allclose(norms[4:], wn, rtol=1e-13)

@@ -283,6 +283,11 @@ __global__ __launch_bounds__(64 * NW) void k_dense64(DenseArgs a) {
             } else if constexpr (OP == DENSE_QUANTIZE) {
                 const double nv = norm_s[rgroup][r];
                 y /= nv > 0.0 ? nv : 1.0;
+                // a norm past the type's range: finite entries over it are zeros, whatever their sums came to
+                if (sizeof(TI) == 8 && nv == INFINITY) {
+                    y = 0.0;
+                    for (int k = 0; k < d; ++k) y += value(reinterpret_cast<const TI *>(a.in)[row * d + k]) * 0.0;
+                }
                 reinterpret_cast<uint8_t *>(a.out)[at] = (uint8_t)level_of(y, table, a.bits);
                 if (a.rotated) a.rotated[at] = y;
             } else if constexpr (OP == DENSE_DEQUANTIZE) {
