@@ -7,7 +7,7 @@ import pytest
 import tq_oracle as O
 import turboquant_plus_amd as tqa
 from turboquant_plus_amd import _lib as L
-from test_gpu_turbo import np_
+from test_gpu_turbo import check_codes, np_
 
 pytestmark = pytest.mark.gpu
 SPANS = [(0, 1), (0, 16), (0, 127), (1, 15), (15, 1), (15, 2), (16, 16), (17, 30), (31, 33), (47, 81), (63, 1), (63, 66), (64, 63),
@@ -30,6 +30,31 @@ def test_turbo_rows(bits, kind):
         got = np_(cache).reshape(N_SEQS, -1, O.block_bytes(bits))
         assert np.array_equal(got[:, :want.shape[1]], want), (pos, n_new)
         assert (got[:, want.shape[1]:] == 0xA5).all(), (pos, n_new)
+
+
+@pytest.mark.parametrize("bits", [2, 3, 4])
+@pytest.mark.parametrize("kind", ["k", "v"])
+@pytest.mark.parametrize("on_device", [False, True])
+def test_turbo_rows_on_the_matrix_cores(bits, kind, on_device):
+    """float16 rows go through the matrix cores in units of 16 tokens.  Whatever tokens stay before a span (all-zero rows among
+    both), the bytes are those of one append of all of them, whose codes and norms agree with the oracle, and nothing
+    outside the touched blocks is written."""
+    tt = L.torch()
+    codec = tqa.TurboCodec(bits, seed=3)
+    x = tt.randn((N_SEQS, 400, D), generator=tt.Generator("cuda").manual_seed(bits), device="cuda").half()
+    x[0, 20] = x[1, 203] = 0
+    for pos, n_new in SPANS:
+        rows = tt.cat([x[:, 200:200 + pos], x[:, :n_new]], dim=1)
+        want, got = (tt.full((tqa.packed_bytes(bits, N_SEQS, CAPACITY),), 0xA5, dtype=tt.uint8, device="cuda") for _ in range(2))
+        codec.append(rows, want, 0, CAPACITY, kind=kind)
+        if pos:
+            codec.append(x[:, 200:200 + pos], got, 0, CAPACITY, kind=kind)
+        codec.append(x[:, :n_new], got, tt.tensor([pos], device="cuda") if on_device else pos, CAPACITY, kind=kind)
+        assert tt.equal(got, want), (pos, n_new)
+        blocks = -(-(pos + n_new) // 128)
+        assert bool((got.view(N_SEQS, -1, O.block_bytes(bits))[:, blocks:] == 0xA5).all()), (pos, n_new)
+        idx, g = (np_(a)[:, :pos + n_new] for a in codec.unpack_codes(got, N_SEQS, CAPACITY, kind=kind))
+        check_codes(codec, np_(rows).reshape(-1, D), idx.reshape(-1, D), g.reshape(-1))
 
 
 @pytest.mark.parametrize("kind", ["k", "v"])

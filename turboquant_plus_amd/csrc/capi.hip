@@ -272,7 +272,10 @@ int tq_create(tq_handle **out, const tq_config *cfg) {
         st[0] = b32[mid];
         for (int j = 1; j <= mid; ++j) st[j] = b32[mid + j];
         rc = rc ? rc : upload(&h->symthr32, st);
-        for (int j = 0; j < 8; ++j) h->symthr_host[j] = j <= mid ? st[j] : 0.0f;
+        for (int j = 0; j < 8; ++j) {
+            h->symthr_host[j] = j <= mid ? st[j] : 0.0f;
+            h->symthr_lo_host[j] = j <= mid ? (float)(bounds[mid + j] - (double)st[j]) : 0.0f;
+        }
         // magnitude level by table: a bin of the value's top 12 bits holds at most one boundary, so
         // level = (boundaries below the bin) + (|value| > the bin's boundary)
         {

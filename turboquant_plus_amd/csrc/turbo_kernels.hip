@@ -14,6 +14,7 @@
 //   k_q8_0_store   32-value int8 blocks with fp16 scale, 128-token block layout.
 #include <cstdlib>
 #include <cstring>
+#include <type_traits>
 
 #include "tq_device.h"
 #include "tq_device64.h"
@@ -542,10 +543,10 @@ __device__ __forceinline__ half8_t signs_to_half8(uint32_t bits) {
 }
 // K rows (tq_handle::rfrag16k): fragment f0*4+ks, lane l, element e = s1[k] H[m][k], m = 32(l%16/4) + 4 f0 + l%4,
 // k = 32(l/16) + 8 ks + e.  m and k share the bits of e with 4 f0 + l%4 and the bits of l/16 with l%16/4.
-__device__ __forceinline__ void build_k_fragments(half8_t (&af)[8], const uint32_t (&s1neg)[4], int lane) {
-    const uint32_t r = lane & 15, kb = lane >> 4;
+// s1neg: the sign mask's word l/16.
+__device__ __forceinline__ void build_k_fragments(half8_t (&af)[8], uint32_t s1neg, int lane) {
+    const uint32_t r = lane & 15, kb = lane >> 4, w = s1neg;
     const uint32_t hi = (uint32_t)__builtin_popcount((r >> 2) & kb) & 1u ? 0xFFu : 0u;
-    const uint32_t w = kb == 0 ? s1neg[0] : kb == 1 ? s1neg[1] : kb == 2 ? s1neg[2] : s1neg[3];
 #pragma unroll
     for (int f0 = 0; f0 < 2; ++f0) {
         const uint32_t pat = h8_row(4u * f0 + (r & 3u)) ^ hi;
@@ -616,6 +617,153 @@ __device__ __forceinline__ uint32_t take_ticket(uint32_t *counter, int lane) {
     uint32_t t = 0;
     if (lane == 0) t = atomicAdd(counter, 1u);
     return __builtin_amdgcn_readfirstlane(t);
+}
+
+// A unit's matrix results -> its codes (BITS dwords of the lane's pair group) and the norm to store, returned on every lane.
+// q: slices' partial sums, ss: the squared norm, rowscale: the power of two an fp32 row was multiplied by.  LUT: how 4-bit
+// levels are found, by a table of the normalised values (once or twice per entry in LDS) or, LUT_NONE, by compares with
+// scaled boundaries as for the other widths; the latter also takes the boundaries in 48 bits (thr0 + thr_lo) and roots and
+// quotients rounded to the last place.
+enum LevelLut { LUT_NONE, LUT_ONCE, LUT_TWICE };
+template <int BITS, LevelLut LUT>
+__device__ __forceinline__ float k_unit_codes(const float4_t (&q)[2][4], float ss, float rowscale, const float (&thr0)[1 << (BITS - 1)],
+                                              const float (&thr_lo)[1 << (BITS - 1)], const float (&coef)[1 << (BITS - 1)], const uint32_t (&flip)[4], uint32_t zero_word,
+                                              int norm_correction, const uint2 *qlut, uint32_t (&g)[BITS]) {
+    constexpr int NT = 1 << (BITS - 1);
+    constexpr bool EXACT = LUT == LUT_NONE, NORMALISED = BITS == 4 && !EXACT;
+    // root of 1 ulp: scales boundaries (1e-7 relative) and the stored fp16 norm
+    const float norm = EXACT ? sqrtf(ss) : __builtin_amdgcn_sqrtf(ss);
+    const float scale = norm > 0.0f ? (EXACT ? sqrtf(128.0f * ss) * rowscale : norm * rowscale * 11.313708498984761f) : 1.0f;  // y' = sqrt(128) ||x|| y
+    float thr[NT];
+#pragma unroll
+    for (int k = 0; k < NT; ++k) thr[k] = EXACT ? fmaf(thr0[k], scale, thr_lo[k] * scale) : thr0[k] * scale;
+    // table path (4 bits): values are normalised instead of the boundaries being scaled
+    const float inv = norm > 0.0f ? __builtin_amdgcn_rsqf(ss) * (0.08838834764831845f * pow2_reciprocal(rowscale)) : 1.0f;
+
+    // butterfly over the input slices: fragment 2*fh + f0 holds dims 32kc + 8fh + 4f0 + i
+    float4_t y[8];
+#pragma unroll
+    for (int f0 = 0; f0 < 2; ++f0) {
+#if TQ_KNOCKOUT & 2
+        const float ko_s = NORMALISED ? inv : 1.0f;  // the table path expects normalised values
+        y[0 + f0] = q[f0][0] * ko_s; y[2 + f0] = q[f0][1] * ko_s; y[4 + f0] = q[f0][2] * ko_s; y[6 + f0] = q[f0][3] * ko_s;
+#else
+        const float4_t s01 = q[f0][0] + q[f0][1], d01 = q[f0][0] - q[f0][1];
+        const float4_t s23 = q[f0][2] + q[f0][3], d23 = q[f0][2] - q[f0][3];
+        if constexpr (NORMALISED) {  // the table is indexed by the normalised value
+            const float4_t iv = {inv, inv, inv, inv};
+            const float4_t s23i = s23 * iv, d23i = d23 * iv;
+            y[0 + f0] = fma4(s01, iv, s23i);
+            y[2 + f0] = fma4(d01, iv, d23i);
+            y[4 + f0] = fma4(s01, iv, -s23i);
+            y[6 + f0] = fma4(d01, iv, -d23i);
+        } else {
+            y[0 + f0] = s01 + s23;
+            y[2 + f0] = d01 + d23;
+            y[4 + f0] = s01 - s23;
+            y[6 + f0] = d01 - d23;
+        }
+#endif
+    }
+    // value v = 0..31 of this lane (dim 32*kc + v) up to the sign s2
+    auto val = [&](int v) -> float { return y[v >> 2][v & 3]; };
+    const bool nonzero = norm > 0.0f;  // all-zero rows get the code of an exact 0 everywhere
+    // EXACT: and so do single values (one in ten million of fp16 rows), whose sign bit says nothing: their sign fields
+    uint32_t zero[4] = {0, 0, 0, 0};
+    if constexpr (EXACT) {
+        float least = fabsf(val(0));
+#pragma unroll
+        for (int v = 1; v < 32; ++v) least = fminf(least, fabsf(val(v)));
+        if (__builtin_amdgcn_ballot_w64(least == 0.0f) != 0) {
+            constexpr int PER = BITS == 2 ? 16 : 8;
+#pragma unroll
+            for (int v = 0; v < 32; ++v) zero[v / PER] |= val(v) == 0.0f ? 1u << (BITS * (v % PER) + BITS - 1) : 0u;
+        }
+    }
+    // the appended sign bits of dword j -> "positive"
+    auto positive = [&](uint32_t w, int j) {
+        w ^= flip[j];
+        return EXACT ? (w & ~zero[j]) | (zero_word & zero[j]) : w;
+    };
+    uint32_t n[NT];
+#pragma unroll
+    for (int k = 0; k < NT; ++k) n[k] = 0;
+    if constexpr (BITS == 3) {
+        // four words of eight values: dwords 0..2 and the tail, whose byte j rides on top of dword j
+        uint32_t w4[4];
+#pragma unroll
+        for (int j = 3; j >= 0; --j) {
+            const int v = 8 * j;
+#if TQ_KNOCKOUT & 1
+            uint32_t w = ko_append4(thr[1] > 0.f ? 0u : 1u, val(v + 7), val(v + 6), val(v + 5), val(v + 4));
+            w = ko_append4(w, val(v + 3), val(v + 2), val(v + 1), val(v));
+#else
+            uint32_t w = append4_b3(0u, val(v + 7), val(v + 6), val(v + 5), val(v + 4), thr);
+            w = append4_b3(w, val(v + 3), val(v + 2), val(v + 1), val(v), thr);
+#endif
+#if !(TQ_KNOCKOUT & 4)
+            count_levels<3>(w, n);
+#endif
+            w4[j] = fold_codes<3>(nonzero ? positive(w, j) : (zero_word & 0x00924924u));
+        }
+        g[0] = __builtin_amdgcn_perm(w4[3], w4[0], 0x04020100u);
+        g[1] = __builtin_amdgcn_perm(w4[3], w4[1], 0x05020100u);
+        g[2] = __builtin_amdgcn_perm(w4[3], w4[2], 0x06020100u);
+    } else if constexpr (BITS == 4) {
+        uint32_t unfolded[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            // eight values into one unfolded dword, highest value first
+            const int v = 8 * j;
+            uint32_t w;
+            if constexpr (LUT == LUT_NONE) {
+                w = append4_b4(0u, val(v + 7), val(v + 6), val(v + 5), val(v + 4), thr);
+                w = append4_b4(w, val(v + 3), val(v + 2), val(v + 1), val(v), thr);
+            } else {
+                float yn[8];
+                uint2 e[8];
+#pragma unroll
+                for (int m = 0; m < 8; ++m) {
+                    yn[m] = val(v + m);  // normalised in the butterfly
+#if TQ_KNOCKOUT & 1
+                    if (m == 0)
+#endif
+                    e[m] = *reinterpret_cast<const uint2 *>(reinterpret_cast<const char *>(qlut) + quant_lut_offset<LUT == LUT_TWICE>(yn[m]));
+                }
+#if TQ_KNOCKOUT & 1
+                w = ko_append4(e[0].x & 1u, yn[7], yn[6], yn[5], yn[4]);
+                w = ko_append4(w, yn[3], yn[2], yn[1], yn[0]);
+#else
+                w = append4_lut(0u, yn[7], yn[6], yn[5], yn[4], e[7], e[6], e[5], e[4]);
+                w = append4_lut(w, yn[3], yn[2], yn[1], yn[0], e[3], e[2], e[1], e[0]);
+#endif
+            }
+            unfolded[j] = w;
+            g[j] = fold_codes<4>(nonzero ? positive(w, j) : (zero_word & 0x88888888u));
+        }
+#if !(TQ_KNOCKOUT & 4)
+        count_levels4_merged(unfolded, n);
+#endif
+    } else {
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+            uint32_t w = 0;
+#pragma unroll
+            for (int v = 16 * j + 12; v >= 16 * j; v -= 4) w = append4_b2(w, val(v + 3), val(v + 2), val(v + 1), val(v), thr);
+            count_levels<2>(w, n);
+            g[j] = fold_codes<2>(nonzero ? positive(w, j) : (zero_word & 0xAAAAAAAAu));
+        }
+    }
+    float gn = norm;
+    if (norm_correction) {
+        float cs = 32.0f * coef[0];
+#pragma unroll
+        for (int k = 1; k < NT; ++k) cs = fmaf(coef[k], (float)n[k], cs);
+        cs += xor_lane<16>(cs);
+        cs += xor_lane<32>(cs);
+        gn = EXACT ? norm / sqrtf(cs) : norm * __builtin_amdgcn_rsqf(cs);  // cs >= 128 min c^2 > 0
+    }
+    return gn;
 }
 
 constexpr uint32_t DRAW_TICKET = 0xFFFFFFFFu;
@@ -689,7 +837,7 @@ __device__ __forceinline__ void store_k_units(const TI *x, uint8_t *packed, cons
     half8_t af[8];
     uint32_t flip[4];
     if constexpr (REG) {
-        build_k_fragments(af, a.s1neg, lane);
+        build_k_fragments(af, kc == 0 ? a.s1neg[0] : kc == 1 ? a.s1neg[1] : kc == 2 ? a.s1neg[2] : a.s1neg[3], lane);
 #pragma unroll
         for (int j = 0; j < 4; ++j) flip[j] = kc == 0 ? a.flipw[j] : kc == 1 ? a.flipw[4 + j] : kc == 2 ? a.flipw[8 + j] : a.flipw[12 + j];
     } else {
@@ -800,115 +948,8 @@ __device__ __forceinline__ void store_k_units(const TI *x, uint8_t *packed, cons
                 ss += xor_lane<16>(ss);
                 ss += xor_lane<32>(ss);
             }
-            const float norm = __builtin_amdgcn_sqrtf(ss);  // 1 ulp: scales boundaries (1e-7 relative) and the stored fp16 norm
-            const float scale = norm > 0.0f ? norm * rowscale * 11.313708498984761f : 1.0f;  // y' = sqrt(128) ||x|| y
-            float thr[NT];
-#pragma unroll
-            for (int k = 0; k < NT; ++k) thr[k] = thr0[k] * scale;
-            // table path (4 bits): values are normalised instead of the boundaries being scaled
-            const float inv = norm > 0.0f ? __builtin_amdgcn_rsqf(ss) * (0.08838834764831845f * pow2_reciprocal(rowscale)) : 1.0f;
-
-            // butterfly over the input slices: fragment 2*fh + f0 holds dims 32kc + 8fh + 4f0 + i
-            float4_t y[8];
-#pragma unroll
-            for (int f0 = 0; f0 < 2; ++f0) {
-#if TQ_KNOCKOUT & 2
-                const float ko_s = BITS == 4 ? inv : 1.0f;  // the table path expects normalised values
-                y[0 + f0] = q[f0][0] * ko_s; y[2 + f0] = q[f0][1] * ko_s; y[4 + f0] = q[f0][2] * ko_s; y[6 + f0] = q[f0][3] * ko_s;
-#else
-                const float4_t s01 = q[f0][0] + q[f0][1], d01 = q[f0][0] - q[f0][1];
-                const float4_t s23 = q[f0][2] + q[f0][3], d23 = q[f0][2] - q[f0][3];
-                if constexpr (BITS == 4) {  // the table is indexed by the normalised value
-                    const float4_t iv = {inv, inv, inv, inv};
-                    const float4_t s23i = s23 * iv, d23i = d23 * iv;
-                    y[0 + f0] = fma4(s01, iv, s23i);
-                    y[2 + f0] = fma4(d01, iv, d23i);
-                    y[4 + f0] = fma4(s01, iv, -s23i);
-                    y[6 + f0] = fma4(d01, iv, -d23i);
-                } else {
-                    y[0 + f0] = s01 + s23;
-                    y[2 + f0] = d01 + d23;
-                    y[4 + f0] = s01 - s23;
-                    y[6 + f0] = d01 - d23;
-                }
-#endif
-            }
-            // value v = 0..31 of this lane (dim 32*kc + v) up to the sign s2
-            auto val = [&](int v) -> float { return y[v >> 2][v & 3]; };
-            const bool nonzero = norm > 0.0f;  // all-zero rows get the code of an exact 0 everywhere
             uint32_t g[BITS];
-            uint32_t n[NT];
-#pragma unroll
-            for (int k = 0; k < NT; ++k) n[k] = 0;
-            if constexpr (BITS == 3) {
-                // four words of eight values: dwords 0..2 and the tail, whose byte j rides on top of dword j
-                uint32_t w4[4];
-#pragma unroll
-                for (int j = 3; j >= 0; --j) {
-                    const int v = 8 * j;
-#if TQ_KNOCKOUT & 1
-                    uint32_t w = ko_append4(thr[1] > 0.f ? 0u : 1u, val(v + 7), val(v + 6), val(v + 5), val(v + 4));
-                    w = ko_append4(w, val(v + 3), val(v + 2), val(v + 1), val(v));
-#else
-                    uint32_t w = append4_b3(0u, val(v + 7), val(v + 6), val(v + 5), val(v + 4), thr);
-                    w = append4_b3(w, val(v + 3), val(v + 2), val(v + 1), val(v), thr);
-#endif
-#if !(TQ_KNOCKOUT & 4)
-                    count_levels<3>(w, n);
-#endif
-                    w4[j] = fold_codes<3>(nonzero ? w ^ flip[j] : (zero_word & 0x00924924u));
-                }
-                g[0] = __builtin_amdgcn_perm(w4[3], w4[0], 0x04020100u);
-                g[1] = __builtin_amdgcn_perm(w4[3], w4[1], 0x05020100u);
-                g[2] = __builtin_amdgcn_perm(w4[3], w4[2], 0x06020100u);
-            } else if constexpr (BITS == 4) {
-                uint32_t unfolded[4];
-#pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    // eight values into one unfolded dword through the table, highest value first
-                    const int v = 8 * j;
-                    float yn[8];
-                    uint2 e[8];
-#pragma unroll
-                    for (int m = 0; m < 8; ++m) {
-                        yn[m] = val(v + m);  // normalised in the butterfly
-#if TQ_KNOCKOUT & 1
-                        if (m == 0)
-#endif
-                        e[m] = *reinterpret_cast<const uint2 *>(reinterpret_cast<const char *>(qlut) + quant_lut_offset<DUP_LUT>(yn[m]));
-                    }
-#if TQ_KNOCKOUT & 1
-                    uint32_t w = ko_append4(e[0].x & 1u, yn[7], yn[6], yn[5], yn[4]);
-                    w = ko_append4(w, yn[3], yn[2], yn[1], yn[0]);
-#else
-                    uint32_t w = append4_lut(0u, yn[7], yn[6], yn[5], yn[4], e[7], e[6], e[5], e[4]);
-                    w = append4_lut(w, yn[3], yn[2], yn[1], yn[0], e[3], e[2], e[1], e[0]);
-#endif
-                    unfolded[j] = w;
-                    g[j] = fold_codes<4>(nonzero ? w ^ flip[j] : (zero_word & 0x88888888u));
-                }
-#if !(TQ_KNOCKOUT & 4)
-                count_levels4_merged(unfolded, n);
-#endif
-            } else {
-#pragma unroll
-                for (int j = 0; j < 2; ++j) {
-                    uint32_t w = 0;
-#pragma unroll
-                    for (int v = 16 * j + 12; v >= 16 * j; v -= 4) w = append4_b2(w, val(v + 3), val(v + 2), val(v + 1), val(v), thr);
-                    count_levels<2>(w, n);
-                    g[j] = fold_codes<2>(nonzero ? w ^ flip[j] : (zero_word & 0xAAAAAAAAu));
-                }
-            }
-            float gn = norm;
-            if (a.norm_correction) {
-                float cs = 32.0f * coef[0];
-#pragma unroll
-                for (int k = 1; k < NT; ++k) cs = fmaf(coef[k], (float)n[k], cs);
-                cs += xor_lane<16>(cs);
-                cs += xor_lane<32>(cs);
-                gn = norm * __builtin_amdgcn_rsqf(cs);  // cs >= 128 min c^2 > 0
-            }
+            const float gn = k_unit_codes<BITS, DUP_LUT ? LUT_TWICE : LUT_ONCE>(q, ss, rowscale, thr0, thr0, coef, flip, zero_word, a.norm_correction, qlut, g);
 #pragma unroll
             for (int j = 0; j < BITS; ++j) pend_g[j] = g[j];
             pend_gn = gn;
@@ -1056,6 +1097,158 @@ __host__ __device__ constexpr uint32_t v_sign_mask(int bits, int j, int hf, uint
             if ((tokmask >> (4 * (k >> 2) + 2 * (k & 1) + h)) & 1) m |= 1u << (grp_shift(bits, k) + bits * h + bits - 1);
     }
     return m;
+}
+
+// A sub-tile's matrix results (token 4 kq + i of its 16, dims 16 dd + 64 hf + n16) -> the eight codes per row dd appended to
+// w[dd] and the norm to store of token n16 % 4 of the lane quarter, returned.  gram: the tokens' squared norms, element i of
+// column 4 kq + i.  zero_tokens: bit i = token i is all zero.  zero_values (LUT_NONE only): the sign fields of the values of
+// w[dd] that are 0, whose sign bit says nothing.
+template <int BITS, bool F32, LevelLut LUT>
+__device__ __forceinline__ float v_subtile_codes(const float4_t (&qq)[2][4], const float4_t &gram, int n16, int kq,
+                                                 const float (&thr0)[1 << (BITS - 1)], const float (&thr_lo)[1 << (BITS - 1)],
+                                                 const float (&coef)[1 << (BITS - 1)], int norm_correction, const uint2 *qlut,
+                                                 uint32_t (&w)[4], uint32_t &zero_tokens, uint32_t (&zero_values)[4]) {
+    constexpr int NT = 1 << (BITS - 1);
+    constexpr bool EXACT = LUT == LUT_NONE, NORMALISED = BITS == 4 && !EXACT;  // as in k_unit_codes
+    float nrm[4];  // EXACT: their squares
+    float4_t inv;
+    float thr_tok[4][NT];  // unless values are normalised: this token's boundaries scaled by sqrt(128) ||x|| (as the K rows do)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const float ss = row16_sum(n16 == 4 * kq + i ? gram[i] : 0.0f);
+        nrm[i] = EXACT ? ss : __builtin_amdgcn_sqrtf(ss);
+        const bool nz = ss > 0.0f;
+        const float rowscale = F32 ? row_pow2_scale(nrm[i]) : 1.0f;  // the power of two the token's fp32 row was multiplied by
+        if constexpr (NORMALISED) {
+            inv[i] = nz ? __builtin_amdgcn_rsqf(ss) * (0.08838834764831845f * pow2_reciprocal(rowscale)) : 1.0f;  // 1 / (||x|| sqrt(128))
+        } else {
+            inv[i] = 1.0f;
+            const float scale = nz ? (EXACT ? sqrtf(128.0f * ss) : nrm[i] * rowscale * 11.313708498984761f) : 1.0f;
+#pragma unroll
+            for (int k = 0; k < NT; ++k) thr_tok[i][k] = EXACT ? fmaf(thr0[k], scale, thr_lo[k] * scale) : thr0[k] * scale;
+        }
+        zero_tokens |= nz ? 0u : 1u << i;
+    }
+    // butterfly over the input slices, then normalise: y[fh][d0] is row dd = 2(fh % 2) + d0, dim half fh / 2
+    float4_t y[4][2];
+#pragma unroll
+    for (int d0 = 0; d0 < 2; ++d0) {
+#if TQ_KNOCKOUT & 2
+        y[0][d0] = qq[d0][0] * inv; y[1][d0] = qq[d0][1] * inv; y[2][d0] = qq[d0][2] * inv; y[3][d0] = qq[d0][3] * inv;
+#else
+        const float4_t s01 = qq[d0][0] + qq[d0][1], d01 = qq[d0][0] - qq[d0][1];
+        const float4_t s23 = qq[d0][2] + qq[d0][3], d23 = qq[d0][2] - qq[d0][3];
+        if constexpr (NORMALISED) {  // the table is indexed by the normalised value
+            const float4_t s23i = s23 * inv, d23i = d23 * inv;
+            y[0][d0] = fma4(s01, inv, s23i);
+            y[1][d0] = fma4(d01, inv, d23i);
+            y[2][d0] = fma4(s01, inv, -s23i);
+            y[3][d0] = fma4(d01, inv, -d23i);
+        } else {
+            y[0][d0] = s01 + s23;
+            y[1][d0] = d01 + d23;
+            y[2][d0] = s01 - s23;
+            y[3][d0] = d01 - d23;
+        }
+#endif
+    }
+    if constexpr (EXACT) {
+        float least = INFINITY;
+#pragma unroll
+        for (int e = 0; e < 32; ++e) least = fminf(least, fabsf(y[e >> 3][(e >> 2) & 1][e & 3]));
+        if (__builtin_amdgcn_ballot_w64(least == 0.0f) != 0) {
+#pragma unroll
+            for (int dd = 0; dd < 4; ++dd)
+#pragma unroll
+                for (int e = 0; e < 8; ++e)  // field 4 hf + i
+                    zero_values[dd] |= y[(dd >> 1) | ((e >> 2) << 1)][dd & 1][e & 3] == 0.0f ? 1u << (BITS * e + BITS - 1) : 0u;
+        }
+    }
+    uint32_t n1[4] = {0, 0, 0, 0};  // 2-bit: per-token count of the level bit
+    // groups in descending pair order: pair 2hf + i/2 of the sub-tile's four, high code (odd i) first
+#pragma unroll
+    for (int g = 0; g < 8; ++g) {
+        const int i = 3 - (g & 3), hf = g & 4 ? 0 : 1;
+        const float y0 = y[0 | (hf << 1)][0][i], y1 = y[0 | (hf << 1)][1][i];
+        const float y2 = y[1 | (hf << 1)][0][i], y3 = y[1 | (hf << 1)][1][i];
+#if TQ_KNOCKOUT & 1
+        w[0] = (w[0] << 1) ^ __float_as_uint(y0); w[1] = (w[1] << 1) ^ __float_as_uint(y1);
+        w[2] = (w[2] << 1) ^ __float_as_uint(y2); w[3] = (w[3] << 1) ^ __float_as_uint(y3);
+        if constexpr (BITS == 99)
+#endif
+        if constexpr (BITS == 3) append_rows_b3(w[0], w[1], w[2], w[3], y0, y1, y2, y3, thr_tok[i]);
+        else if constexpr (BITS == 2) append_rows_b2(w[0], w[1], w[2], w[3], n1[i], y0, y1, y2, y3, thr_tok[i]);
+        else if constexpr (LUT == LUT_NONE) append_rows_b4(w[0], w[1], w[2], w[3], y0, y1, y2, y3, thr_tok[i]);
+        else {
+            const char *ql = reinterpret_cast<const char *>(qlut);
+            append_rows_lut(w[0], w[1], w[2], w[3], y0, y1, y2, y3,
+                            *reinterpret_cast<const uint2 *>(ql + quant_lut_offset<LUT == LUT_TWICE>(y0)),
+                            *reinterpret_cast<const uint2 *>(ql + quant_lut_offset<LUT == LUT_TWICE>(y1)),
+                            *reinterpret_cast<const uint2 *>(ql + quant_lut_offset<LUT == LUT_TWICE>(y2)),
+                            *reinterpret_cast<const uint2 *>(ql + quant_lut_offset<LUT == LUT_TWICE>(y3)));
+        }
+    }
+    // level counts of the four tokens, one byte per token, summed over the 16 columns
+    uint32_t cnt[NT];
+#if TQ_KNOCKOUT & 4
+#pragma unroll
+    for (int p = 0; p < NT; ++p) cnt[p] = 0x01010101u;
+    if constexpr (BITS == 99)
+#endif
+    if constexpr (BITS == 4) {
+        // the dword of every row is complete: vertical sums of the level-bit products over the rows
+        constexpr uint32_t K0 = 0x11111111u;
+        uint32_t sum[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+#pragma unroll
+        for (int dd = 0; dd < 4; ++dd) {
+            const uint32_t ww = w[dd];
+            const uint32_t b0 = ww & K0, b1 = (ww >> 1) & K0, b2 = (ww >> 2) & K0, b01 = b0 & b1;
+            sum[1] += b0; sum[2] += b1; sum[3] += b01; sum[4] += b2;
+            sum[5] += b0 & b2; sum[6] += b1 & b2; sum[7] += b01 & b2;
+        }
+#pragma unroll
+        for (int p = 1; p < 8; ++p) {
+            // token i sits at nibble i (hf 0) and nibble 4 + i (hf 1); bytes of cnt: tokens 0, 2, 1, 3
+            const uint32_t t = sum[p] + (sum[p] >> 16);
+            cnt[p] = (t & 0x0F0Fu) | ((t & 0xF0F0u) << 12);
+        }
+    } else if constexpr (BITS == 3) {
+        // the word of every row (the tail word for the last four tokens of a group) is complete: 3-bit fields 4hf + i hold token i's
+        // code; field-wise sums of the level-bit products over the four rows stay below 8
+        constexpr uint32_t K0 = 0x00249249u;
+        uint32_t sum[4] = {0, 0, 0, 0};
+#pragma unroll
+        for (int dd = 0; dd < 4; ++dd) {
+            const uint32_t ww = w[dd];
+            const uint32_t b0 = ww & K0, b1 = (ww >> 1) & K0;
+            sum[1] += b0; sum[2] += b1; sum[3] += b0 & b1;
+        }
+#pragma unroll
+        for (int p = 1; p < 4; ++p) {
+            // dim halves added in 6-bit lanes: e = tokens 0 and 2, o = tokens 1 and 3; then one byte per token
+            const uint32_t lo = sum[p] & 0xFFFu, hi = sum[p] >> 12;
+            const uint32_t e = (lo & 0x1C7u) + (hi & 0x1C7u), o = ((lo >> 3) & 0x1C7u) + ((hi >> 3) & 0x1C7u);
+            cnt[p] = (e & 0x3Fu) | ((o & 0x3Fu) << 8) | ((e & 0xFC0u) << 10) | ((o & 0xFC0u) << 18);
+        }
+    } else {
+        cnt[1] = n1[0] | (n1[1] << 8) | (n1[2] << 16) | (n1[3] << 24);
+    }
+    float cs = 128.0f * coef[0];
+    const int sh = BITS == 4 ? 8 * (((n16 & 1) << 1) | ((n16 >> 1) & 1)) : 8 * (n16 & 3);
+#if TQ_KNOCKOUT & 4
+    cs += (float)(cnt[NT - 1] >> sh);
+#else
+#pragma unroll
+    for (int p = 1; p < NT; ++p) cs = fmaf(coef[p], (float)((row16_sum(cnt[p]) >> sh) & 0xFFu), cs);
+#endif
+    const int isel = n16 & 3;
+    float nsel = isel == 0 ? nrm[0] : isel == 1 ? nrm[1] : isel == 2 ? nrm[2] : nrm[3];
+    if constexpr (EXACT) {
+        nsel = sqrtf(nsel);
+        return norm_correction ? nsel / sqrtf(cs) : nsel;
+    }
+    const float gn = norm_correction ? nsel * __builtin_amdgcn_rsqf(cs) : nsel;
+    return gn;
 }
 
 struct StoreVArgs {
@@ -1309,128 +1502,13 @@ __device__ __forceinline__ void store_v_units(const TI *x, uint8_t *packed, cons
             if (q == 1 && tl_n == 1 && gram[0] != 12345.678f) TQ_TL(12);
 #endif
 
-            float nrm[4];
-            float4_t inv;
-            float thr_tok[4][NT];  // 2- and 3-bit codes: this token's boundaries scaled by sqrt(128) ||x|| (as the K rows do)
+            const int jw = grp_word(BITS, 4 * u);
+            uint32_t wu[4] = {w[0][jw], w[1][jw], w[2][jw], w[3][jw]}, zero_tokens = 0, zero_values[4];
+            const float gn = v_subtile_codes<BITS, F32, DUP_LUT ? LUT_TWICE : LUT_ONCE>(qq, gram, n16, kq, thr0, thr0, coef, a.norm_correction, qlut, wu,
+                                                                                        zero_tokens, zero_values);
 #pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const float ss = row16_sum(n16 == 4 * kq + i ? gram[i] : 0.0f);
-                nrm[i] = __builtin_amdgcn_sqrtf(ss);
-                const bool nz = ss > 0.0f;
-                const float rowscale = F32 ? row_pow2_scale(nrm[i]) : 1.0f;  // the power of two the token's fp32 row was multiplied by
-                if constexpr (BITS == 4) {
-                    inv[i] = nz ? __builtin_amdgcn_rsqf(ss) * (0.08838834764831845f * pow2_reciprocal(rowscale)) : 1.0f;  // 1 / (||x|| sqrt(128))
-                } else {
-                    inv[i] = 1.0f;
-                    const float scale = nz ? nrm[i] * rowscale * 11.313708498984761f : 1.0f;
-#pragma unroll
-                    for (int k = 0; k < NT; ++k) thr_tok[i][k] = thr0[k] * scale;
-                }
-                zbits |= nz ? 0u : 1u << (4 * u + i);
-            }
-            // butterfly over the input slices, then normalise: y[fh][d0] is row dd = 2(fh % 2) + d0, dim half fh / 2
-            float4_t y[4][2];
-#pragma unroll
-            for (int d0 = 0; d0 < 2; ++d0) {
-#if TQ_KNOCKOUT & 2
-                y[0][d0] = qq[d0][0] * inv; y[1][d0] = qq[d0][1] * inv; y[2][d0] = qq[d0][2] * inv; y[3][d0] = qq[d0][3] * inv;
-#else
-                const float4_t s01 = qq[d0][0] + qq[d0][1], d01 = qq[d0][0] - qq[d0][1];
-                const float4_t s23 = qq[d0][2] + qq[d0][3], d23 = qq[d0][2] - qq[d0][3];
-                if constexpr (BITS == 4) {  // the table is indexed by the normalised value
-                    const float4_t s23i = s23 * inv, d23i = d23 * inv;
-                    y[0][d0] = fma4(s01, inv, s23i);
-                    y[1][d0] = fma4(d01, inv, d23i);
-                    y[2][d0] = fma4(s01, inv, -s23i);
-                    y[3][d0] = fma4(d01, inv, -d23i);
-                } else {
-                    y[0][d0] = s01 + s23;
-                    y[1][d0] = d01 + d23;
-                    y[2][d0] = s01 - s23;
-                    y[3][d0] = d01 - d23;
-                }
-#endif
-            }
-            uint32_t n1[4] = {0, 0, 0, 0};  // 2-bit: per-token count of the level bit
-            // groups in descending pair order: pair 4u + 2hf + i/2, high code (odd i) first
-#pragma unroll
-            for (int g = 0; g < 8; ++g) {
-                const int i = 3 - (g & 3), hf = g & 4 ? 0 : 1;
-                const int j = grp_word(BITS, 4 * u);
-                const float y0 = y[0 | (hf << 1)][0][i], y1 = y[0 | (hf << 1)][1][i];
-                const float y2 = y[1 | (hf << 1)][0][i], y3 = y[1 | (hf << 1)][1][i];
-#if TQ_KNOCKOUT & 1
-                w[0][j] = (w[0][j] << 1) ^ __float_as_uint(y0); w[1][j] = (w[1][j] << 1) ^ __float_as_uint(y1);
-                w[2][j] = (w[2][j] << 1) ^ __float_as_uint(y2); w[3][j] = (w[3][j] << 1) ^ __float_as_uint(y3);
-                if constexpr (BITS == 99)
-#endif
-                if constexpr (BITS == 3) append_rows_b3(w[0][j], w[1][j], w[2][j], w[3][j], y0, y1, y2, y3, thr_tok[i]);
-                else if constexpr (BITS == 2) append_rows_b2(w[0][j], w[1][j], w[2][j], w[3][j], n1[i], y0, y1, y2, y3, thr_tok[i]);
-                else {
-                    const char *ql = reinterpret_cast<const char *>(qlut);
-                    append_rows_lut(w[0][j], w[1][j], w[2][j], w[3][j], y0, y1, y2, y3,
-                                    *reinterpret_cast<const uint2 *>(ql + quant_lut_offset<DUP_LUT>(y0)),
-                                    *reinterpret_cast<const uint2 *>(ql + quant_lut_offset<DUP_LUT>(y1)),
-                                    *reinterpret_cast<const uint2 *>(ql + quant_lut_offset<DUP_LUT>(y2)),
-                                    *reinterpret_cast<const uint2 *>(ql + quant_lut_offset<DUP_LUT>(y3)));
-                }
-            }
-            // level counts of the four tokens, one byte per token, summed over the 16 columns
-            uint32_t cnt[NT];
-#if TQ_KNOCKOUT & 4
-#pragma unroll
-            for (int p = 0; p < NT; ++p) cnt[p] = 0x01010101u;
-            if constexpr (BITS == 99)
-#endif
-            if constexpr (BITS == 4) {
-                // dword u of every row is complete: vertical sums of the level-bit products over the rows
-                constexpr uint32_t K0 = 0x11111111u;
-                uint32_t sum[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-#pragma unroll
-                for (int dd = 0; dd < 4; ++dd) {
-                    const uint32_t ww = w[dd][u];
-                    const uint32_t b0 = ww & K0, b1 = (ww >> 1) & K0, b2 = (ww >> 2) & K0, b01 = b0 & b1;
-                    sum[1] += b0; sum[2] += b1; sum[3] += b01; sum[4] += b2;
-                    sum[5] += b0 & b2; sum[6] += b1 & b2; sum[7] += b01 & b2;
-                }
-#pragma unroll
-                for (int p = 1; p < 8; ++p) {
-                    // token i sits at nibble i (hf 0) and nibble 4 + i (hf 1); bytes of cnt: tokens 0, 2, 1, 3
-                    const uint32_t t = sum[p] + (sum[p] >> 16);
-                    cnt[p] = (t & 0x0F0Fu) | ((t & 0xF0F0u) << 12);
-                }
-            } else if constexpr (BITS == 3) {
-                // word u of every row (the tail word for u = 3) is complete: 3-bit fields 4hf + i hold token i's
-                // code; field-wise sums of the level-bit products over the four rows stay below 8
-                constexpr uint32_t K0 = 0x00249249u;
-                uint32_t sum[4] = {0, 0, 0, 0};
-#pragma unroll
-                for (int dd = 0; dd < 4; ++dd) {
-                    const uint32_t ww = w[dd][u];
-                    const uint32_t b0 = ww & K0, b1 = (ww >> 1) & K0;
-                    sum[1] += b0; sum[2] += b1; sum[3] += b0 & b1;
-                }
-#pragma unroll
-                for (int p = 1; p < 4; ++p) {
-                    // dim halves added in 6-bit lanes: e = tokens 0 and 2, o = tokens 1 and 3; then one byte per token
-                    const uint32_t lo = sum[p] & 0xFFFu, hi = sum[p] >> 12;
-                    const uint32_t e = (lo & 0x1C7u) + (hi & 0x1C7u), o = ((lo >> 3) & 0x1C7u) + ((hi >> 3) & 0x1C7u);
-                    cnt[p] = (e & 0x3Fu) | ((o & 0x3Fu) << 8) | ((e & 0xFC0u) << 10) | ((o & 0xFC0u) << 18);
-                }
-            } else {
-                cnt[1] = n1[0] | (n1[1] << 8) | (n1[2] << 16) | (n1[3] << 24);
-            }
-            float cs = 128.0f * coef[0];
-            const int sh = BITS == 4 ? 8 * (((n16 & 1) << 1) | ((n16 >> 1) & 1)) : 8 * (n16 & 3);
-#if TQ_KNOCKOUT & 4
-            cs += (float)(cnt[NT - 1] >> sh);
-#else
-#pragma unroll
-            for (int p = 1; p < NT; ++p) cs = fmaf(coef[p], (float)((row16_sum(cnt[p]) >> sh) & 0xFFu), cs);
-#endif
-            const int isel = n16 & 3;
-            const float nsel = isel == 0 ? nrm[0] : isel == 1 ? nrm[1] : isel == 2 ? nrm[2] : nrm[3];
-            const float gn = a.norm_correction ? nsel * __builtin_amdgcn_rsqf(cs) : nsel;
+            for (int dd = 0; dd < 4; ++dd) w[dd][jw] = wu[dd];
+            zbits |= zero_tokens << (4 * u);
             if constexpr (DEFER) {
                 park_norm = gn;
                 if (completes(u)) {
@@ -1886,6 +1964,162 @@ template <int BITS, typename TI>
 __global__ __launch_bounds__(APPEND_THREADS) void k_append(const TI *x, uint8_t *packed, AppendArgs a) {
     if (!resolve_append(a, blockIdx.x)) return;
     append_block<BITS, TI>(x, packed, a, blockIdx.x);
+}
+
+// ---- the same on the matrix cores: fp16 rows of symmetric codebooks --------------------------------------
+// A wavefront takes 16 consecutive tokens of a block, as a K unit or as a fourth of a V tile, through the store kernels'
+// steps (k_unit_codes, v_subtile_codes; without their 1-ulp roots and their table).  No LDS and no barrier: a K unit's
+// dwords are its own rows', a V unit's are one dword per (row, chunk) of its token group, which no other wavefront writes;
+// where `pos` falls inside the group, the codes of the tokens before it are taken over from memory.
+// A value that is exactly 0 gets the code below or above the middle boundary like any other (the sign bit of a 0 is not its
+// side), so codes and norms are as close to 64-bit arithmetic as the butterfly's or closer: shares off, 1e9 fp16 values and
+// 8e6 norms per width, 2 / 3 / 4 bits: codes 1.0 / 7.1 / 9.8e-8 (butterfly 3.7 / 7.8 / 14.3e-8), norms 4.9 / 4.9 / 5.4e-5
+// (5.4 / 5.4 / 6.2e-5).
+// Bound: vector instructions (650 to 1230 for 16 tokens; the butterfly needs about 300 for each four, and its codes go
+// through LDS).  64 x 2048 tokens, K and V: turbo2 35.0 -> 21.0 us, turbo3 45.6 -> 25.8, turbo4 47.3 -> 29.4, 8-bit K with
+// turbo3 V 39.0 -> 26.8 (copies of these bytes: 15 to 18 us).
+struct AppendUnitArgs {
+    int64_t pos, n_new, capacity, blocks_per_seq, first_block;
+    const int64_t *pos_dev;  // as in AppendArgs
+    uint32_t *overrun;
+    uint32_t n_touched;
+    FastDiv touched_div;     // division by n_touched
+    int norm_correction;
+    uint32_t s1neg[4], s2neg[4], flipw[16];  // the constants by value, as in StoreKArgs and StoreVArgs
+    float thr[8], thr_lo[8], coef[8];       // boundaries: thr + thr_lo
+};
+template <int BITS, int KIND>
+__device__ __forceinline__ void append_units(const __half *x, uint8_t *packed, const AppendUnitArgs &a, const unsigned wg) {
+    constexpr int NT = 1 << (BITS - 1);
+    const int lane = threadIdx.x & 63, n16 = lane & 15, kq = lane >> 4;
+    const int unit = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), t0 = 16 * unit;
+    const uint32_t seq = a.touched_div.div(wg), nth = wg - seq * a.n_touched;
+    int64_t pos = a.pos, first_block = a.first_block;
+    if (a.pos_dev) {  // the position is read when the launch runs (see resolve_append)
+        pos = *a.pos_dev;
+        if (!append_position_ok(pos, a.n_new, a.capacity, a.overrun, wg == 0)) return;
+        first_block = pos / TQ_ROWS_PER_BLOCK;
+        if ((int64_t)nth >= (pos + a.n_new - 1) / TQ_ROWS_PER_BLOCK - first_block + 1) return;
+    }
+    const int64_t bis = first_block + nth, tok0 = bis * TQ_ROWS_PER_BLOCK;
+    const int n_old = (int)(pos - tok0 < 0 ? 0 : pos - tok0);
+    const int n_end = (int)(pos + a.n_new - tok0 > TQ_ROWS_PER_BLOCK ? TQ_ROWS_PER_BLOCK : pos + a.n_new - tok0);
+    if (t0 + 16 <= n_old) return;  // nothing but tokens that stay
+    uint8_t *block = packed + ((int64_t)seq * a.blocks_per_seq + bis) * block_bytes(BITS);
+
+    const int t = t0 + n16;  // the token of this lane's inputs; tokens outside the new ones request a new one's and drop them
+    const __half *row = x + ((int64_t)seq * a.n_new + (tok0 + min(max(t, n_old), n_end - 1) - pos)) * 128;
+    const uint4 *p = reinterpret_cast<const uint4 *>(row + (KIND == TQ_KIND_K ? 32 : 8) * kq);
+    uint4 xb[4];
+#pragma unroll
+    for (int ks = 0; ks < 4; ++ks) xb[ks] = p[KIND == TQ_KIND_K ? ks : 4 * ks];
+    // V: dword `jd` of the lane's rows 16 dd + n16 of the tile is what the lane stores
+    const int jd = BITS == 2 ? kq >> 1 : kq;
+    const bool stores = BITS == 4 || (BITS == 3 ? kq < 3 : (kq & 1) == 0);
+    uint32_t *dst = reinterpret_cast<uint32_t *>(block + (stores ? jd : 0) * 2048 + ((unit >> 2) * 64 + n16) * 16 + (unit & 3) * 4);
+    uint32_t old[4] = {0, 0, 0, 0};
+    const bool merge = KIND == TQ_KIND_V && n_old > t0;  // wave-uniform
+    if (merge) {
+#pragma unroll
+        for (int dd = 0; dd < 4; ++dd) old[dd] = dst[64 * dd];
+    }
+    float thr0[NT], thr_lo[NT], coef[NT];
+#pragma unroll
+    for (int k = 0; k < NT; ++k) {
+        thr0[k] = a.thr[k];
+        thr_lo[k] = a.thr_lo[k];
+        coef[k] = a.coef[k];
+    }
+    const uint32_t zero_word = thr0[0] < 0.0f ? 0xFFFFFFFFu : 0u;  // an exact zero counts as positive only then
+    // entry kq of four: by masks (a chain of selects over kernel arguments becomes branches around loads)
+    const uint32_t quarter[4] = {kq == 0 ? ~0u : 0u, kq == 1 ? ~0u : 0u, kq == 2 ? ~0u : 0u, kq == 3 ? ~0u : 0u};
+    auto of_quarter = [&](uint32_t e0, uint32_t e1, uint32_t e2, uint32_t e3) {
+        return (e0 & quarter[0]) | (e1 & quarter[1]) | (e2 & quarter[2]) | (e3 & quarter[3]);
+    };
+    half8_t fr[8];
+    if constexpr (KIND == TQ_KIND_K) build_k_fragments(fr, of_quarter(a.s1neg[0], a.s1neg[1], a.s1neg[2], a.s1neg[3]), lane);
+    else build_v_fragments(fr, a.s1neg, lane);
+    const bool fresh = t >= n_old && t < n_end;
+    half8_t xh[4];
+#pragma unroll
+    for (int ks = 0; ks < 4; ++ks) xh[ks] = __builtin_bit_cast(half8_t, fresh ? xb[ks] : make_uint4(0, 0, 0, 0));
+
+    // token n16's squared norm over the four lanes that share it, in four short sums: closer than the matrix cores' X X^T
+    float part[4];
+#pragma unroll
+    for (int ks = 0; ks < 4; ++ks) {
+        part[ks] = 0.0f;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) part[ks] = fmaf((float)xh[ks][e], (float)xh[ks][e], part[ks]);
+    }
+    float ss = (part[0] + part[1]) + (part[2] + part[3]);
+    ss += xor_lane<16>(ss);
+    ss += xor_lane<32>(ss);
+    float4_t q[2][4];
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+#pragma unroll
+        for (int ks = 0; ks < 4; ++ks)
+            q[h][ks] = KIND == TQ_KIND_K ? __builtin_amdgcn_mfma_f32_16x16x32_f16(fr[h * 4 + ks], xh[ks], float4_t{0.f, 0.f, 0.f, 0.f}, 0, 0, 0)
+                                         : __builtin_amdgcn_mfma_f32_16x16x32_f16(xh[ks], fr[h * 4 + ks], float4_t{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+
+    __half *norms = reinterpret_cast<__half *>(block + block_code_bytes(BITS));
+    settle_matrix_results();  // what follows may be compiled to branches
+    if constexpr (KIND == TQ_KIND_K) {
+        uint32_t flip[4], g[BITS];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) flip[j] = of_quarter(a.flipw[j], a.flipw[4 + j], a.flipw[8 + j], a.flipw[12 + j]);
+        const float gn = k_unit_codes<BITS, LUT_NONE>(q, ss, 1.0f, thr0, thr_lo, coef, flip, zero_word, a.norm_correction, nullptr, g);
+        if (t >= n_old) {
+#pragma unroll
+            for (int j = 0; j < BITS; ++j) *reinterpret_cast<uint32_t *>(block + j * 2048 + t * 16 + kq * 4) = g[j];
+            if (kq == 0) norms[t] = __float2half_rn(gn);
+        }
+    } else {
+        uint32_t w[4] = {0, 0, 0, 0}, zero_tokens = 0, zm[4] = {0, 0, 0, 0};
+        const float gn = v_subtile_codes<BITS, false, LUT_NONE>(q, float4_t{ss, ss, ss, ss}, n16, kq, thr0, thr_lo, coef, a.norm_correction, nullptr, w, zero_tokens,
+                                                                 zm);  // a token of zeros has nothing but zero values
+        // field 4 hf + i of a word is token i's code of dim half hf
+        constexpr uint32_t CM = (1u << BITS) - 1u, SB = 1u << (BITS - 1);
+        // the codes of tokens before `pos` in the words of token quarter k
+        auto before = [&](int k) {
+            uint32_t m = 0;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) m |= t0 + 4 * k + i < n_old ? (CM << (BITS * i)) | (CM << (BITS * (4 + i))) : 0u;
+            return m;
+        };
+        uint32_t keep = before(kq);
+        if constexpr (BITS == 2) keep |= before(kq + 1) << 16;
+        if constexpr (BITS == 3) keep |= ((before(3) >> (8 * kq)) & 0xFFu) << 24;
+#pragma unroll
+        for (int dd = 0; dd < 4; ++dd) {
+            uint32_t fm = 0;  // sign fields of the dims with s2 = +1
+#pragma unroll
+            for (int hf = 0; hf < 2; ++hf) {
+                constexpr uint32_t four = SB | (SB << BITS) | (SB << (2 * BITS)) | (SB << (3 * BITS));
+                fm |= (a.s2neg[2 * hf + (dd >> 1)] >> (16 * (dd & 1) + n16)) & 1u ? 0u : four << (4 * BITS * hf);
+            }
+            uint32_t ww = w[dd] ^ fm;
+            ww = fold_codes<BITS>((ww & ~zm[dd]) | (zero_word & zm[dd]));
+            if constexpr (BITS == 2) {  // a dword is two quarters' words
+                ww &= 0xFFFFu;
+                ww |= xor_lane<16>(ww) << 16;
+            }
+            if constexpr (BITS == 3) {  // the last quarter's word rides on the others' top bytes
+                const uint32_t tail = (uint32_t)__shfl((int)ww, 48 + n16);
+                ww = __builtin_amdgcn_perm(tail, ww, 0x04020100u + ((uint32_t)kq << 24));
+            }
+            if (merge) ww = (old[dd] & keep) | (ww & ~keep);
+            if (stores) dst[64 * dd] = ww;
+        }
+        const int tn = t0 + 4 * kq + n16;
+        if (n16 < 4 && tn >= n_old) norms[tn] = __float2half_rn(gn);
+    }
+}
+
+template <int BITS, int KIND>
+__global__ __launch_bounds__(APPEND_THREADS, 4) void k_append_units(const __half *x, uint8_t *packed, AppendUnitArgs a) {
+    append_units<BITS, KIND>(x, packed, a, blockIdx.x);
 }
 
 // ---- K2 + K4 in float64: codes, corrected norm, residual sign sketch ---------------
@@ -2864,16 +3098,17 @@ __global__ __launch_bounds__(Q8A_THREADS) void k_q8_0_append(const TI *x, uint8_
 
 // K and V of a decode step in one launch: the first half of the grid rebuilds K blocks, the second half V blocks.  A
 // width of 0 stands for q8_0-style rows: 8-bit K with turbo V took two launches and two calls into the library.
-template <int BITS> struct AppendSide { using Args = AppendArgs; };
-template <> struct AppendSide<0> { using Args = Q8AppendArgs; };
-template <int BITS, int KIND, typename TI>
-__device__ __forceinline__ void append_side(const TI *x, uint8_t *packed, typename AppendSide<BITS>::Args &a, const unsigned wg) {
-    if constexpr (BITS == 0) q8_0_append_block<TI, KIND>(x, packed, a, wg);
-    else if (resolve_append(a, wg)) append_block<BITS, TI>(x, packed, a, wg);
+constexpr int UNITS = 16;  // added to a turbo side's width: the side runs on the matrix cores (append_units)
+template <int SIDE> struct AppendSide { using Args = std::conditional_t<SIDE == 0, Q8AppendArgs, std::conditional_t<(SIDE > UNITS), AppendUnitArgs, AppendArgs>>; };
+template <int SIDE, int KIND, typename TI>
+__device__ __forceinline__ void append_side(const TI *x, uint8_t *packed, typename AppendSide<SIDE>::Args &a, const unsigned wg) {
+    if constexpr (SIDE == 0) q8_0_append_block<TI, KIND>(x, packed, a, wg);
+    else if constexpr (SIDE > UNITS) append_units<SIDE - UNITS, KIND>(x, packed, a, wg);
+    else if (resolve_append(a, wg)) append_block<SIDE, TI>(x, packed, a, wg);
 }
 static_assert(APPEND_THREADS == Q8A_THREADS, "both kinds of rows run in one launch");
 template <int KB, int VB, typename TI>
-__global__ __launch_bounds__(APPEND_THREADS) void k_append_kv(const TI *xk, uint8_t *pk, typename AppendSide<KB>::Args ka, const TI *xv,
+__global__ __launch_bounds__(APPEND_THREADS, (KB > UNITS || VB > UNITS) ? 4 : 1) void k_append_kv(const TI *xk, uint8_t *pk, typename AppendSide<KB>::Args ka, const TI *xv,
                                                               uint8_t *pv, typename AppendSide<VB>::Args va) {
     const unsigned half = gridDim.x >> 1;
     if (blockIdx.x < half) append_side<KB, TQ_KIND_K, TI>(xk, pk, ka, blockIdx.x);
@@ -4055,6 +4290,24 @@ static Q8AppendArgs make_q8_append_args(const void *x, int64_t pos, const int64_
     return a;
 }
 
+// Rows that append_units takes: fp16, whose products with the +-1 factor are exact on the matrix cores, of the codebooks that
+// the matrix-core store takes.  (fp32 rows stay with the butterfly: the store's two fp16 terms per value are 22 bits.)
+static bool append_units_ok(const tq_handle *h, int in_dtype) { return in_dtype == TQ_F16 && store_fast_ok(h, in_dtype, 0); }
+
+static AppendUnitArgs make_append_unit_args(const tq_handle *h, int64_t pos, const int64_t *pos_dev, int64_t n_new, int64_t capacity,
+                                            uint32_t *overrun) {
+    AppendUnitArgs u{};
+    const AppendArgs a = make_append_args(h, pos, pos_dev, n_new, capacity, TQ_KIND_K, overrun);
+    u.pos = a.pos; u.n_new = a.n_new; u.capacity = a.capacity; u.blocks_per_seq = a.blocks_per_seq; u.first_block = a.first_block;
+    u.pos_dev = a.pos_dev; u.overrun = a.overrun;
+    u.n_touched = (uint32_t)a.n_touched; u.touched_div = make_fast_div(u.n_touched);
+    u.norm_correction = h->norm_correction;
+    for (int i = 0; i < 4; ++i) { u.s1neg[i] = h->s1neg_host[i]; u.s2neg[i] = h->s2neg_host[i]; }
+    for (int i = 0; i < 16; ++i) u.flipw[i] = h->s2flip_host[i];
+    for (int i = 0; i < 8; ++i) { u.thr[i] = h->symthr_host[i]; u.thr_lo[i] = h->symthr_lo_host[i]; u.coef[i] = h->sqcoef_host[i]; }
+    return u;
+}
+
 // hk / hv NULL: q8_0-style rows on that side
 int tqk_append_kv(const tq_handle *hk, const tq_handle *hv, const void *k, const void *v, int64_t n_seqs, int64_t pos,
                   int64_t n_new, int64_t capacity, int in_dtype, void *packed_k, void *packed_v, hipStream_t s,
@@ -4062,34 +4315,52 @@ int tqk_append_kv(const tq_handle *hk, const tq_handle *hv, const void *k, const
     if (n_seqs == 0 || n_new == 0) return TQ_OK;
     const Q8AppendArgs qk = make_q8_append_args(k, pos, pos_dev, n_new, capacity, pos_dev ? overrun : nullptr);
     const Q8AppendArgs qv = make_q8_append_args(v, pos, pos_dev, n_new, capacity, nullptr);  // the K half reports
-    AppendArgs ka{}, va{};
-    if (hk) ka = make_append_args(hk, pos, pos_dev, n_new, capacity, TQ_KIND_K, overrun);
-    if (hv) va = make_append_args(hv, pos, pos_dev, n_new, capacity, TQ_KIND_V);
     const unsigned grid = 2u * (unsigned)(n_seqs * qk.n_touched);
     const int kb = hk ? hk->bits : 0, vb = hv ? hv->bits : 0;
-#define TQ_APPEND_KV(KB, VB, KA, VA)                                                                                           \
-    DISPATCH_T(in_dtype, TI, (k_append_kv<KB, VB, TI><<<grid, APPEND_THREADS, 0, s>>>((const TI *)k, (uint8_t *)packed_k, KA,  \
-                                                                                      (const TI *)v, (uint8_t *)packed_v, VA)));
-    switch (8 * kb + vb) {
-    case 8 * 3 + 3: TQ_APPEND_KV(3, 3, ka, va) break;
-    case 8 * 4 + 4: TQ_APPEND_KV(4, 4, ka, va) break;
-    case 8 * 2 + 2: TQ_APPEND_KV(2, 2, ka, va) break;
-    case 8 * 4 + 2: TQ_APPEND_KV(4, 2, ka, va) break;
-    case 8 * 3 + 2: TQ_APPEND_KV(3, 2, ka, va) break;
-    case 8 * 4 + 3: TQ_APPEND_KV(4, 3, ka, va) break;
-    case 2: TQ_APPEND_KV(0, 2, qk, va) break;
-    case 3: TQ_APPEND_KV(0, 3, qk, va) break;
-    case 4: TQ_APPEND_KV(0, 4, qk, va) break;
-    case 8 * 2: TQ_APPEND_KV(2, 0, ka, qv) break;
-    case 8 * 3: TQ_APPEND_KV(3, 0, ka, qv) break;
-    case 8 * 4: TQ_APPEND_KV(4, 0, ka, qv) break;
-    case 0: TQ_APPEND_KV(0, 0, qk, qv) break;
-    default: {  // turbo V wider than turbo K: two launches
+#define TQ_APPEND_KV(KB, VB, TI, KA, VA)                                                                                     \
+    k_append_kv<KB, VB, TI><<<grid, APPEND_THREADS, 0, s>>>((const TI *)k, (uint8_t *)packed_k, KA, (const TI *)v, (uint8_t *)packed_v, VA)
+    // U: 0, or UNITS for turbo sides on the matrix cores
+#define TQ_APPEND_PAIRS(U, TI)                                              \
+    switch (8 * kb + vb) {                                                  \
+    case 8 * 3 + 3: TQ_APPEND_KV(U + 3, U + 3, TI, ka, va); break;          \
+    case 8 * 4 + 4: TQ_APPEND_KV(U + 4, U + 4, TI, ka, va); break;          \
+    case 8 * 2 + 2: TQ_APPEND_KV(U + 2, U + 2, TI, ka, va); break;          \
+    case 8 * 4 + 2: TQ_APPEND_KV(U + 4, U + 2, TI, ka, va); break;          \
+    case 8 * 3 + 2: TQ_APPEND_KV(U + 3, U + 2, TI, ka, va); break;          \
+    case 8 * 4 + 3: TQ_APPEND_KV(U + 4, U + 3, TI, ka, va); break;          \
+    case 2: TQ_APPEND_KV(0, U + 2, TI, qk, va); break;                      \
+    case 3: TQ_APPEND_KV(0, U + 3, TI, qk, va); break;                      \
+    case 4: TQ_APPEND_KV(0, U + 4, TI, qk, va); break;                      \
+    case 8 * 2: TQ_APPEND_KV(U + 2, 0, TI, ka, qv); break;                  \
+    case 8 * 3: TQ_APPEND_KV(U + 3, 0, TI, ka, qv); break;                  \
+    case 8 * 4: TQ_APPEND_KV(U + 4, 0, TI, ka, qv); break;                  \
+    default: one_launch = false;                                            \
+    }
+    bool one_launch = true;
+    if (!hk && !hv) {
+        DISPATCH_T(in_dtype, TI, (TQ_APPEND_KV(0, 0, TI, qk, qv)));
+    } else {
+        const bool ku = hk && append_units_ok(hk, in_dtype), vu = hv && append_units_ok(hv, in_dtype);
+        if ((ku || !hk) && (vu || !hv)) {
+            AppendUnitArgs ka{}, va{};
+            if (hk) ka = make_append_unit_args(hk, pos, pos_dev, n_new, capacity, overrun);
+            if (hv) va = make_append_unit_args(hv, pos, pos_dev, n_new, capacity, nullptr);
+            TQ_APPEND_PAIRS(UNITS, __half)
+        } else if (ku || vu) {
+            one_launch = false;  // a codebook of either kind
+        } else {
+            AppendArgs ka{}, va{};
+            if (hk) ka = make_append_args(hk, pos, pos_dev, n_new, capacity, TQ_KIND_K, overrun);
+            if (hv) va = make_append_args(hv, pos, pos_dev, n_new, capacity, TQ_KIND_V);
+            DISPATCH_T(in_dtype, TI, TQ_APPEND_PAIRS(0, TI));
+        }
+    }
+    if (!one_launch) {  // turbo V wider than turbo K, or one side's codebook not for the matrix cores
         if (!hk || !hv) { tq_set_error("tq_append_layer: bits must be 2, 3 or 4 (got %d and %d)", kb, vb); return TQ_ERR_UNSUPPORTED; }
         const int rc = tqk_append(hk, k, n_seqs, pos, n_new, capacity, in_dtype, TQ_KIND_K, packed_k, s, pos_dev, overrun);
         return rc ? rc : tqk_append(hv, v, n_seqs, pos, n_new, capacity, in_dtype, TQ_KIND_V, packed_v, s, pos_dev, overrun);
     }
-    }
+#undef TQ_APPEND_PAIRS
 #undef TQ_APPEND_KV
     return tq_check_launch("append_kv");
 }
@@ -4099,6 +4370,19 @@ int tqk_append(const tq_handle *h, const void *x, int64_t n_seqs, int64_t pos, i
     if (n_seqs == 0 || n_new == 0) return TQ_OK;
     const AppendArgs a = make_append_args(h, pos, pos_dev, n_new, capacity, kind, overrun);
     const unsigned grid = (unsigned)(n_seqs * a.n_touched);
+    if (append_units_ok(h, in_dtype)) {
+        const AppendUnitArgs u = make_append_unit_args(h, pos, pos_dev, n_new, capacity, overrun);
+#define TQ_UNITS(B)                                                                                                          \
+    if (kind == TQ_KIND_K) k_append_units<B, TQ_KIND_K><<<grid, APPEND_THREADS, 0, s>>>((const __half *)x, (uint8_t *)packed, u); \
+    else k_append_units<B, TQ_KIND_V><<<grid, APPEND_THREADS, 0, s>>>((const __half *)x, (uint8_t *)packed, u)
+        switch (h->bits) {
+        case 2: TQ_UNITS(2); break;
+        case 3: TQ_UNITS(3); break;
+        default: TQ_UNITS(4); break;
+        }
+#undef TQ_UNITS
+        return tq_check_launch("append_units");
+    }
 #define TQ_APPEND_BITS(B) \
     DISPATCH_T(in_dtype, TI, (k_append<B, TI><<<grid, APPEND_THREADS, 0, s>>>((const TI *)x, (uint8_t *)packed, a)))
     switch (h->bits) {
