@@ -194,3 +194,23 @@ def test_float32_prompts_keep_their_low_bits(fmt, tokens):
     y = O.rotate_fast(x.reshape(-1, D).astype(np.float64), codec.signs1, codec.signs2, D).reshape(x.shape)
     small = np.abs(y) < 1e-6
     assert small.mean() == 0.5 and np.array_equal(idx[small], np.where(y > 0, 1 << (codec.bits - 1), (1 << (codec.bits - 1)) - 1)[small])
+
+
+@pytest.mark.parametrize("pair", [(2, 2), (3, 3), (4, 4), (4, 2), (4, 3), (3, 2), (2, 4)])
+@pytest.mark.parametrize("shape", [(1, 1), (3, 333), (2, 16 * 128), (64, 4 * 128), (64, 4 * 128 + 1)])
+def test_short_prompts_have_the_bytes_of_the_store(pair, shape):
+    """Prompts of up to 256 blocks in float16 (and one of 320): K and V in one launch have the bytes of a store per side, into
+    buffers of their length and into caches laid out for more tokens."""
+    tt = L.torch()
+    n, tokens = shape
+    kc, vc = (tqa.TurboCodec(b, seed=s) for b, s in zip(pair, (3, 503)))
+    k, v = (tt.randn((n, tokens, D), generator=tt.Generator("cuda").manual_seed(s), device="cuda").half() for s in (1, 2))
+    k[0, tokens // 2] = 0
+    blocks, capacity = -(-tokens // 128), 128 * (-(-tokens // 128) + 3)
+    want = kc.store(k, kind="k"), vc.store(v, kind="v")
+    assert all(tt.equal(a, b) for a, b in zip(kc.store_kv(vc, k, v), want))
+    caches = [tt.full((tqa.packed_bytes(b, n, capacity),), 0xA5, dtype=tt.uint8, device="cuda") for b in pair]
+    kc.store_kv(vc, k, v, *caches, capacity=capacity)
+    for cache, w in zip(caches, want):
+        assert tt.equal(cache.view(n, blocks + 3, -1)[:, :blocks], w.view(n, blocks, -1))
+        assert bool((cache.view(n, blocks + 3, -1)[:, blocks:] == 0xA5).all())

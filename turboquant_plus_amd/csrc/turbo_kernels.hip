@@ -621,10 +621,10 @@ __device__ __forceinline__ uint32_t take_ticket(uint32_t *counter, int lane) {
 
 // A unit's matrix results -> its codes (BITS dwords of the lane's pair group) and the norm to store, returned on every lane.
 // q: slices' partial sums, ss: the squared norm, rowscale: the power of two an fp32 row was multiplied by.  LUT: how 4-bit
-// levels are found, by a table of the normalised values (once or twice per entry in LDS) or, LUT_NONE, by compares with
-// scaled boundaries as for the other widths; the latter also takes the boundaries in 48 bits (thr0 + thr_lo) and roots and
-// quotients rounded to the last place.
-enum LevelLut { LUT_NONE, LUT_ONCE, LUT_TWICE };
+// levels are found, by a table of the normalised values (once or twice per entry in LDS), LUT_SEARCH: by the table's
+// comparisons without the table, or LUT_NONE: by comparisons with scaled boundaries as for the other widths; the last also
+// takes the boundaries in 48 bits (thr0 + thr_lo) and roots and quotients rounded to the last place.
+enum LevelLut { LUT_NONE, LUT_SEARCH, LUT_ONCE, LUT_TWICE };
 template <int BITS, LevelLut LUT>
 __device__ __forceinline__ float k_unit_codes(const float4_t (&q)[2][4], float ss, float rowscale, const float (&thr0)[1 << (BITS - 1)],
                                               const float (&thr_lo)[1 << (BITS - 1)], const float (&coef)[1 << (BITS - 1)], const uint32_t (&flip)[4], uint32_t zero_word,
@@ -716,9 +716,9 @@ __device__ __forceinline__ float k_unit_codes(const float4_t (&q)[2][4], float s
             // eight values into one unfolded dword, highest value first
             const int v = 8 * j;
             uint32_t w;
-            if constexpr (LUT == LUT_NONE) {
-                w = append4_b4(0u, val(v + 7), val(v + 6), val(v + 5), val(v + 4), thr);
-                w = append4_b4(w, val(v + 3), val(v + 2), val(v + 1), val(v), thr);
+            if constexpr (LUT <= LUT_SEARCH) {
+                w = append4_b4(0u, val(v + 7), val(v + 6), val(v + 5), val(v + 4), EXACT ? thr : thr0);
+                w = append4_b4(w, val(v + 3), val(v + 2), val(v + 1), val(v), EXACT ? thr : thr0);
             } else {
                 float yn[8];
                 uint2 e[8];
@@ -1178,7 +1178,7 @@ __device__ __forceinline__ float v_subtile_codes(const float4_t (&qq)[2][4], con
 #endif
         if constexpr (BITS == 3) append_rows_b3(w[0], w[1], w[2], w[3], y0, y1, y2, y3, thr_tok[i]);
         else if constexpr (BITS == 2) append_rows_b2(w[0], w[1], w[2], w[3], n1[i], y0, y1, y2, y3, thr_tok[i]);
-        else if constexpr (LUT == LUT_NONE) append_rows_b4(w[0], w[1], w[2], w[3], y0, y1, y2, y3, thr_tok[i]);
+        else if constexpr (LUT <= LUT_SEARCH) append_rows_b4(w[0], w[1], w[2], w[3], y0, y1, y2, y3, EXACT ? thr_tok[i] : thr0);
         else {
             const char *ql = reinterpret_cast<const char *>(qlut);
             append_rows_lut(w[0], w[1], w[2], w[3], y0, y1, y2, y3,
@@ -1988,9 +1988,11 @@ struct AppendUnitArgs {
     uint32_t s1neg[4], s2neg[4], flipw[16];  // the constants by value, as in StoreKArgs and StoreVArgs
     float thr[8], thr_lo[8], coef[8];       // boundaries: thr + thr_lo
 };
-template <int BITS, int KIND>
+// AS_STORE: a prompt's rows, whose bytes are those of tq_store (the store kernels' roots, table decisions and zeros).
+template <int BITS, int KIND, bool AS_STORE>
 __device__ __forceinline__ void append_units(const __half *x, uint8_t *packed, const AppendUnitArgs &a, const unsigned wg) {
     constexpr int NT = 1 << (BITS - 1);
+    constexpr LevelLut LUT = AS_STORE ? LUT_SEARCH : LUT_NONE;
     const int lane = threadIdx.x & 63, n16 = lane & 15, kq = lane >> 4;
     const int unit = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), t0 = 16 * unit;
     const uint32_t seq = a.touched_div.div(wg), nth = wg - seq * a.n_touched;
@@ -2044,17 +2046,25 @@ __device__ __forceinline__ void append_units(const __half *x, uint8_t *packed, c
 #pragma unroll
     for (int ks = 0; ks < 4; ++ks) xh[ks] = __builtin_bit_cast(half8_t, fresh ? xb[ks] : make_uint4(0, 0, 0, 0));
 
-    // token n16's squared norm over the four lanes that share it, in four short sums: closer than the matrix cores' X X^T
-    float part[4];
+    float4_t gram = {0.f, 0.f, 0.f, 0.f};  // of token 4 kq + i: element i of column 4 kq + i
+    float ss = 0.0f;                       // of token n16
+    if constexpr (AS_STORE) {
 #pragma unroll
-    for (int ks = 0; ks < 4; ++ks) {
-        part[ks] = 0.0f;
+        for (int ks = 0; ks < 4; ++ks) gram = __builtin_amdgcn_mfma_f32_16x16x32_f16(xh[ks], xh[ks], gram, 0, 0, 0);
+    } else {
+        // over the four lanes that share the token, in four short sums: closer than the matrix cores' X X^T
+        float part[4];
 #pragma unroll
-        for (int e = 0; e < 8; ++e) part[ks] = fmaf((float)xh[ks][e], (float)xh[ks][e], part[ks]);
+        for (int ks = 0; ks < 4; ++ks) {
+            part[ks] = 0.0f;
+#pragma unroll
+            for (int e = 0; e < 8; ++e) part[ks] = fmaf((float)xh[ks][e], (float)xh[ks][e], part[ks]);
+        }
+        ss = (part[0] + part[1]) + (part[2] + part[3]);
+        ss += xor_lane<16>(ss);
+        ss += xor_lane<32>(ss);
+        gram = float4_t{ss, ss, ss, ss};
     }
-    float ss = (part[0] + part[1]) + (part[2] + part[3]);
-    ss += xor_lane<16>(ss);
-    ss += xor_lane<32>(ss);
     float4_t q[2][4];
 #pragma unroll
     for (int h = 0; h < 2; ++h)
@@ -2066,10 +2076,16 @@ __device__ __forceinline__ void append_units(const __half *x, uint8_t *packed, c
     __half *norms = reinterpret_cast<__half *>(block + block_code_bytes(BITS));
     settle_matrix_results();  // what follows may be compiled to branches
     if constexpr (KIND == TQ_KIND_K) {
+        if constexpr (AS_STORE) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) ss += n16 == 4 * kq + i ? gram[i] : 0.0f;
+            ss += xor_lane<16>(ss);
+            ss += xor_lane<32>(ss);
+        }
         uint32_t flip[4], g[BITS];
 #pragma unroll
         for (int j = 0; j < 4; ++j) flip[j] = of_quarter(a.flipw[j], a.flipw[4 + j], a.flipw[8 + j], a.flipw[12 + j]);
-        const float gn = k_unit_codes<BITS, LUT_NONE>(q, ss, 1.0f, thr0, thr_lo, coef, flip, zero_word, a.norm_correction, nullptr, g);
+        const float gn = k_unit_codes<BITS, LUT>(q, ss, 1.0f, thr0, thr_lo, coef, flip, zero_word, a.norm_correction, nullptr, g);
         if (t >= n_old) {
 #pragma unroll
             for (int j = 0; j < BITS; ++j) *reinterpret_cast<uint32_t *>(block + j * 2048 + t * 16 + kq * 4) = g[j];
@@ -2077,10 +2093,14 @@ __device__ __forceinline__ void append_units(const __half *x, uint8_t *packed, c
         }
     } else {
         uint32_t w[4] = {0, 0, 0, 0}, zero_tokens = 0, zm[4] = {0, 0, 0, 0};
-        const float gn = v_subtile_codes<BITS, false, LUT_NONE>(q, float4_t{ss, ss, ss, ss}, n16, kq, thr0, thr_lo, coef, a.norm_correction, nullptr, w, zero_tokens,
-                                                                 zm);  // a token of zeros has nothing but zero values
+        const float gn = v_subtile_codes<BITS, false, LUT>(q, gram, n16, kq, thr0, thr_lo, coef, a.norm_correction, nullptr, w, zero_tokens, zm);
         // field 4 hf + i of a word is token i's code of dim half hf
         constexpr uint32_t CM = (1u << BITS) - 1u, SB = 1u << (BITS - 1);
+        if constexpr (AS_STORE) {  // (else a token of zeros has nothing but zero values)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) zm[0] |= (zero_tokens >> i) & 1u ? (SB << (BITS * i)) | (SB << (BITS * (4 + i))) : 0u;
+            zm[1] = zm[2] = zm[3] = zm[0];
+        }
         // the codes of tokens before `pos` in the words of token quarter k
         auto before = [&](int k) {
             uint32_t m = 0;
@@ -2119,7 +2139,7 @@ __device__ __forceinline__ void append_units(const __half *x, uint8_t *packed, c
 
 template <int BITS, int KIND>
 __global__ __launch_bounds__(APPEND_THREADS, 4) void k_append_units(const __half *x, uint8_t *packed, AppendUnitArgs a) {
-    append_units<BITS, KIND>(x, packed, a, blockIdx.x);
+    append_units<BITS, KIND, false>(x, packed, a, blockIdx.x);
 }
 
 // ---- K2 + K4 in float64: codes, corrected norm, residual sign sketch ---------------
@@ -2998,27 +3018,39 @@ __global__ __launch_bounds__(256) void k_q8_0_store_v_f16(const __half *x, uint8
 // wavefront stores 1 KB of a chunk in one piece (V rows: a thread gathers a dim's 16 tokens; bytes of neighbouring
 // tokens share those 16 bytes, and only the 16-token group that `pos` falls into is stored byte by byte).
 // 16 x 6001 tokens: 20 us for K and V (33 us for K alone when a thread read 32 values one by one and V left in bytes).
+// Next come its vector instructions: a rounding of three instead of six and no 64-bit divisions took the K kernel's listing from
+// 672 to 495 and 64 x 2048 tokens of 8-bit K with turbo3 V from 26.8 to 25.2 us.
 // x need not be 16-byte aligned: `wide` says whether it is.
 constexpr int Q8A_THREADS = 512, Q8A_ROW = 136;  // LDS bytes per token (an odd multiple of 8)
 struct Q8AppendArgs {
-    int64_t pos, n_new, blocks_per_seq, first_block, n_touched, capacity;
+    int64_t pos, n_new, blocks_per_seq, first_block, capacity;
     const int64_t *pos_dev;
     uint32_t *overrun;
+    uint32_t n_touched;
+    FastDiv touched_div;  // division by n_touched
     int wide;
 };
+// roundf(t) as an integer: the truncation of t plus the largest float below one half, of t's sign (one half itself would
+// carry that largest float to 1; what is added here rounds back below the next integer for every t that is not at the half).
+// t is a rounded product: it must not become the product of a fused multiply-add.
+__device__ __forceinline__ int round_half_away(float t) {
+#pragma clang fp contract(off)
+    return (int)(t + copysignf(0.49999997f, t));
+}
 template <typename TI, int KIND>
 __device__ __forceinline__ void q8_0_append_block(const TI *x, uint8_t *packed, const Q8AppendArgs &a, const unsigned wg) {
     __shared__ __attribute__((aligned(16))) uint8_t rows_s[TQ_ROWS_PER_BLOCK * Q8A_ROW];
     __shared__ __attribute__((aligned(16))) __half scales_s[TQ_ROWS_PER_BLOCK * 4];  // K: [token][group], V: as stored
     int64_t pos = a.pos, first_block = a.first_block;
+    const uint32_t seq_n = a.touched_div.div(wg), nth = wg - seq_n * a.n_touched;
     if (a.pos_dev) {  // the position is read when the launch runs (see resolve_append)
         pos = *a.pos_dev;
         if (!append_position_ok(pos, a.n_new, a.capacity, a.overrun, wg == 0)) return;
         first_block = pos / TQ_ROWS_PER_BLOCK;
-        if ((int64_t)(wg % a.n_touched) >= (pos + a.n_new - 1) / TQ_ROWS_PER_BLOCK - first_block + 1) return;
+        if ((int64_t)nth >= (pos + a.n_new - 1) / TQ_ROWS_PER_BLOCK - first_block + 1) return;
     }
     const int tid = threadIdx.x;
-    const int64_t seq = wg / a.n_touched, bis = first_block + wg % a.n_touched;
+    const int64_t seq = seq_n, bis = first_block + nth;
     const int64_t tok0 = bis * TQ_ROWS_PER_BLOCK;
     uint8_t *block = packed + (seq * a.blocks_per_seq + bis) * (int64_t)(TQ_ROWS_PER_BLOCK * 136);
     const int n_old = (int)(pos - tok0 < 0 ? 0 : pos - tok0);
@@ -3054,7 +3086,7 @@ __device__ __forceinline__ void q8_0_append_block(const TI *x, uint8_t *packed, 
 #pragma unroll
         for (int j = 0; j < 8; ++j) {
             const float tq = v[i][j] * id;
-            const int qv = (int)roundf(tq);
+            const int qv = round_half_away(tq);
             w[j >> 2] |= ((uint32_t)(qv & 0xFF)) << (8 * (j & 3));
         }
         *reinterpret_cast<uint2 *>(rows_s + t * Q8A_ROW + 8 * c8) = make_uint2(w[0], w[1]);
@@ -3098,12 +3130,13 @@ __global__ __launch_bounds__(Q8A_THREADS) void k_q8_0_append(const TI *x, uint8_
 
 // K and V of a decode step in one launch: the first half of the grid rebuilds K blocks, the second half V blocks.  A
 // width of 0 stands for q8_0-style rows: 8-bit K with turbo V took two launches and two calls into the library.
-constexpr int UNITS = 16;  // added to a turbo side's width: the side runs on the matrix cores (append_units)
+// added to a turbo side's width: the side runs on the matrix cores (append_units; UNITS_AS_STORE: with the store's bytes)
+constexpr int UNITS = 16, UNITS_AS_STORE = 32;
 template <int SIDE> struct AppendSide { using Args = std::conditional_t<SIDE == 0, Q8AppendArgs, std::conditional_t<(SIDE > UNITS), AppendUnitArgs, AppendArgs>>; };
 template <int SIDE, int KIND, typename TI>
 __device__ __forceinline__ void append_side(const TI *x, uint8_t *packed, typename AppendSide<SIDE>::Args &a, const unsigned wg) {
     if constexpr (SIDE == 0) q8_0_append_block<TI, KIND>(x, packed, a, wg);
-    else if constexpr (SIDE > UNITS) append_units<SIDE - UNITS, KIND>(x, packed, a, wg);
+    else if constexpr (SIDE > UNITS) append_units<SIDE % UNITS, KIND, (SIDE > UNITS_AS_STORE)>(x, packed, a, wg);
     else if (resolve_append(a, wg)) append_block<SIDE, TI>(x, packed, a, wg);
 }
 static_assert(APPEND_THREADS == Q8A_THREADS, "both kinds of rows run in one launch");
@@ -4283,8 +4316,9 @@ static Q8AppendArgs make_q8_append_args(const void *x, int64_t pos, const int64_
     Q8AppendArgs a;
     a.pos = pos; a.pos_dev = pos_dev; a.n_new = n_new; a.capacity = capacity; a.blocks_per_seq = blocks_for(capacity);
     a.first_block = pos / TQ_ROWS_PER_BLOCK;
-    a.n_touched = pos_dev ? (n_new + TQ_ROWS_PER_BLOCK - 2) / TQ_ROWS_PER_BLOCK + 1  // at the worst alignment
-                          : (pos + n_new - 1) / TQ_ROWS_PER_BLOCK - a.first_block + 1;
+    a.n_touched = (uint32_t)(pos_dev ? (n_new + TQ_ROWS_PER_BLOCK - 2) / TQ_ROWS_PER_BLOCK + 1  // at the worst alignment
+                                     : (pos + n_new - 1) / TQ_ROWS_PER_BLOCK - a.first_block + 1);
+    a.touched_div = make_fast_div(a.n_touched);
     a.overrun = overrun;
     a.wide = (reinterpret_cast<uintptr_t>(x) & 15u) == 0;
     return a;
@@ -4308,18 +4342,10 @@ static AppendUnitArgs make_append_unit_args(const tq_handle *h, int64_t pos, con
     return u;
 }
 
-// hk / hv NULL: q8_0-style rows on that side
-int tqk_append_kv(const tq_handle *hk, const tq_handle *hv, const void *k, const void *v, int64_t n_seqs, int64_t pos,
-                  int64_t n_new, int64_t capacity, int in_dtype, void *packed_k, void *packed_v, hipStream_t s,
-                  const int64_t *pos_dev, uint32_t *overrun) {
-    if (n_seqs == 0 || n_new == 0) return TQ_OK;
-    const Q8AppendArgs qk = make_q8_append_args(k, pos, pos_dev, n_new, capacity, pos_dev ? overrun : nullptr);
-    const Q8AppendArgs qv = make_q8_append_args(v, pos, pos_dev, n_new, capacity, nullptr);  // the K half reports
-    const unsigned grid = 2u * (unsigned)(n_seqs * qk.n_touched);
-    const int kb = hk ? hk->bits : 0, vb = hv ? hv->bits : 0;
+// The widths that have a kernel for K and V in one launch (0: q8_0-style rows); U: 0, or what append_side says is added to a
+// turbo side.  `one_launch` becomes false where there is none (turbo V wider than turbo K).
 #define TQ_APPEND_KV(KB, VB, TI, KA, VA)                                                                                     \
     k_append_kv<KB, VB, TI><<<grid, APPEND_THREADS, 0, s>>>((const TI *)k, (uint8_t *)packed_k, KA, (const TI *)v, (uint8_t *)packed_v, VA)
-    // U: 0, or UNITS for turbo sides on the matrix cores
 #define TQ_APPEND_PAIRS(U, TI)                                              \
     switch (8 * kb + vb) {                                                  \
     case 8 * 3 + 3: TQ_APPEND_KV(U + 3, U + 3, TI, ka, va); break;          \
@@ -4336,34 +4362,58 @@ int tqk_append_kv(const tq_handle *hk, const tq_handle *hv, const void *k, const
     case 8 * 4: TQ_APPEND_KV(U + 4, 0, TI, ka, qv); break;                  \
     default: one_launch = false;                                            \
     }
+
+// K and V through append_units (both turbo sides fit for it, one at least); false: no kernel for this pair
+static bool launch_units_kv(const tq_handle *hk, const tq_handle *hv, const void *k, const void *v, int64_t n_seqs, int64_t pos,
+                            int64_t n_new, int64_t capacity, bool as_store, void *packed_k, void *packed_v, hipStream_t s,
+                            const int64_t *pos_dev, uint32_t *overrun) {
+    const Q8AppendArgs qk = make_q8_append_args(k, pos, pos_dev, n_new, capacity, pos_dev ? overrun : nullptr);
+    const Q8AppendArgs qv = make_q8_append_args(v, pos, pos_dev, n_new, capacity, nullptr);  // the K half reports
+    AppendUnitArgs ka{}, va{};
+    if (hk) ka = make_append_unit_args(hk, pos, pos_dev, n_new, capacity, overrun);
+    if (hv) va = make_append_unit_args(hv, pos, pos_dev, n_new, capacity, nullptr);
+    const unsigned grid = 2u * (unsigned)(n_seqs * qk.n_touched);
+    const int kb = hk ? hk->bits : 0, vb = hv ? hv->bits : 0;
     bool one_launch = true;
-    if (!hk && !hv) {
-        DISPATCH_T(in_dtype, TI, (TQ_APPEND_KV(0, 0, TI, qk, qv)));
+    if (as_store) TQ_APPEND_PAIRS(UNITS_AS_STORE, __half)
+    else TQ_APPEND_PAIRS(UNITS, __half)
+    return one_launch;
+}
+
+// hk / hv NULL: q8_0-style rows on that side
+int tqk_append_kv(const tq_handle *hk, const tq_handle *hv, const void *k, const void *v, int64_t n_seqs, int64_t pos,
+                  int64_t n_new, int64_t capacity, int in_dtype, void *packed_k, void *packed_v, hipStream_t s,
+                  const int64_t *pos_dev, uint32_t *overrun) {
+    if (n_seqs == 0 || n_new == 0) return TQ_OK;
+    const int kb = hk ? hk->bits : 0, vb = hv ? hv->bits : 0;
+    const bool ku = hk && append_units_ok(hk, in_dtype), vu = hv && append_units_ok(hv, in_dtype);
+    bool one_launch = true;
+    if ((ku || vu) && (ku || !hk) && (vu || !hv)) {
+        one_launch = launch_units_kv(hk, hv, k, v, n_seqs, pos, n_new, capacity, false, packed_k, packed_v, s, pos_dev, overrun);
+    } else if (ku || vu) {
+        one_launch = false;  // one side's codebook is for the butterfly
     } else {
-        const bool ku = hk && append_units_ok(hk, in_dtype), vu = hv && append_units_ok(hv, in_dtype);
-        if ((ku || !hk) && (vu || !hv)) {
-            AppendUnitArgs ka{}, va{};
-            if (hk) ka = make_append_unit_args(hk, pos, pos_dev, n_new, capacity, overrun);
-            if (hv) va = make_append_unit_args(hv, pos, pos_dev, n_new, capacity, nullptr);
-            TQ_APPEND_PAIRS(UNITS, __half)
-        } else if (ku || vu) {
-            one_launch = false;  // a codebook of either kind
+        const Q8AppendArgs qk = make_q8_append_args(k, pos, pos_dev, n_new, capacity, pos_dev ? overrun : nullptr);
+        const Q8AppendArgs qv = make_q8_append_args(v, pos, pos_dev, n_new, capacity, nullptr);
+        AppendArgs ka{}, va{};
+        if (hk) ka = make_append_args(hk, pos, pos_dev, n_new, capacity, TQ_KIND_K, overrun);
+        if (hv) va = make_append_args(hv, pos, pos_dev, n_new, capacity, TQ_KIND_V);
+        const unsigned grid = 2u * (unsigned)(n_seqs * qk.n_touched);
+        if (!hk && !hv) {
+            DISPATCH_T(in_dtype, TI, (TQ_APPEND_KV(0, 0, TI, qk, qv)));
         } else {
-            AppendArgs ka{}, va{};
-            if (hk) ka = make_append_args(hk, pos, pos_dev, n_new, capacity, TQ_KIND_K, overrun);
-            if (hv) va = make_append_args(hv, pos, pos_dev, n_new, capacity, TQ_KIND_V);
             DISPATCH_T(in_dtype, TI, TQ_APPEND_PAIRS(0, TI));
         }
     }
-    if (!one_launch) {  // turbo V wider than turbo K, or one side's codebook not for the matrix cores
+    if (!one_launch) {
         if (!hk || !hv) { tq_set_error("tq_append_layer: bits must be 2, 3 or 4 (got %d and %d)", kb, vb); return TQ_ERR_UNSUPPORTED; }
         const int rc = tqk_append(hk, k, n_seqs, pos, n_new, capacity, in_dtype, TQ_KIND_K, packed_k, s, pos_dev, overrun);
         return rc ? rc : tqk_append(hv, v, n_seqs, pos, n_new, capacity, in_dtype, TQ_KIND_V, packed_v, s, pos_dev, overrun);
     }
-#undef TQ_APPEND_PAIRS
-#undef TQ_APPEND_KV
     return tq_check_launch("append_kv");
 }
+#undef TQ_APPEND_PAIRS
+#undef TQ_APPEND_KV
 
 int tqk_append(const tq_handle *h, const void *x, int64_t n_seqs, int64_t pos, int64_t n_new, int64_t capacity, int in_dtype,
                int kind, void *packed, hipStream_t s, const int64_t *pos_dev, uint32_t *overrun) {
@@ -4395,6 +4445,12 @@ int tqk_append(const tq_handle *h, const void *x, int64_t n_seqs, int64_t pos, i
     return tq_check_launch("append");
 }
 
+// fp16 prompts up to this many blocks take a wavefront per 16 tokens (append_units) instead of the persistent store, where a
+// V tile of 64 is one wavefront's chain of 4 to 8 us however few there are.  Two workgroups per CU: beyond, the store's queue
+// and prefetch are the better ones for the wide formats (kernel, us, store / units: turbo3 8 x 777 tokens 7.8 / 4.6, 256
+// blocks 8.9 / 7.4, 384 10.5 / 9.9, 448 11.6 / 12.6; turbo4 8.7 / 5.2, 10.0 / 8.4, 11.0 / 11.5, 12.5 / 14.3; turbo2 6.5 / 4.1,
+// 7.3 / 6.3, 8.8 / 8.7, 9.7 / 9.6).  The bytes are the same.
+constexpr int64_t SHORT_PROMPT_BLOCKS = 256;
 // capacity > 0: the packed buffers are caches laid out for `capacity` tokens per sequence (tq_append's layout) and the
 // `tokens` tokens of every sequence go to its first blocks; 0: sequences follow each other at blocks_for(tokens)
 int tqk_store_kv(const tq_handle *hk, const tq_handle *hv, const void *k, const void *v, int64_t n_seqs, int64_t tokens,
@@ -4408,6 +4464,9 @@ int tqk_store_kv(const tq_handle *hk, const tq_handle *hv, const void *k, const 
         const int rc = tqk_store(hk, k, n_seqs, tokens, in_dtype, TQ_KIND_K, packed_k, nullptr, nullptr, s);
         return rc ? rc : tqk_store(hv, v, n_seqs, tokens, in_dtype, TQ_KIND_V, packed_v, nullptr, nullptr, s);
     }
+    if (in_dtype == TQ_F16 && n_blocks <= SHORT_PROMPT_BLOCKS &&
+        launch_units_kv(hk, hv, k, v, n_seqs, 0, tokens, out_bps * TQ_ROWS_PER_BLOCK, true, packed_k, packed_v, s, nullptr, nullptr))
+        return tq_check_launch("store_kv (short)");
     StoreKArgs ka = make_k_args(hk, tokens, bps, n_blocks);
     StoreVArgs va = make_v_args(hv, tokens, bps, n_blocks);
     ka.out_blocks_per_seq = va.out_blocks_per_seq = (uint32_t)out_bps;
@@ -4458,27 +4517,23 @@ int tqk_store_kv(const tq_handle *hk, const tq_handle *hv, const void *k, const 
     return tq_check_launch("store_kv");
 }
 
-// Prompt of a layer of any two formats (hk / hv NULL: q8_0-style rows) into caches laid out for `capacity` tokens.
-// One 8-bit side and fp16 rows: a long prompt's turbo side goes through the matrix-core store (the append's butterfly is bound
-// by its vector instructions; fp16 products with +-1 are exact there, so both sum the same 32-bit values) and the 8-bit side
-// through its own launch; a short one is one launch of the append kernel.  fp32 rows stay with the append kernel: the
-// matrix cores would take them as two fp16 terms, which drop what lies below 2^-22 of a value (split8).
-// From 512 blocks on two launches are the faster (one / two, us; 8-bit K with turbo3 V, fp16: 512 blocks 19.9 / 17.4, 752 28.6 /
-// 22.8, 2048 62.3 / 47.3; turbo4 V 70.7 / 48.9; turbo3 K with 8-bit V 56.9 / 41.7); below, calls take the host 15 us either way.
-constexpr int64_t PREFILL_SPLIT_BLOCKS = 512;
+// Prompt of a layer of any two formats (hk / hv NULL: q8_0-style rows) into caches laid out for `capacity` tokens, one launch.
+// fp16 rows of a long prompt (512 blocks) have the turbo side's bytes from tq_store's arithmetic, all others from the
+// append's.  fp32 rows stay with the butterfly: the matrix cores would take them as two fp16 terms, which drop what lies
+// below 2^-22 of a value (split8).
+// (Two launches, the 8-bit side's append and the persistent store, took (kernels, us; 8-bit K with turbo3 V, fp16) 21.0 for 528
+// blocks, 23.2 for 752 and 44.5 for 2048; in one launch 13.9, 16.4 and 40.7; turbo4 V 22.4, 24.8 and 46.4 against 15.5, 18.0 and
+// 44.8; turbo3 K with 8-bit V 16.7, 19.4 and 42.2 against 12.5, 15.7 and 38.2.)
+constexpr int64_t AS_STORE_BLOCKS = 512;
 int tqk_store_layer(const tq_handle *hk, const tq_handle *hv, const void *k, const void *v, int64_t n_seqs, int64_t tokens,
                     int64_t capacity, int in_dtype, void *packed_k, void *packed_v, hipStream_t s) {
     if (hk && hv) return tqk_store_kv(hk, hv, k, v, n_seqs, tokens, capacity, in_dtype, packed_k, packed_v, s);
     const tq_handle *h = hk ? hk : hv;
     const int64_t n_blocks = n_seqs * blocks_for(tokens), out_bps = blocks_for(capacity);
-    if (!h || in_dtype != TQ_F16 || n_blocks < PREFILL_SPLIT_BLOCKS || !store_fast_ok(h, in_dtype, n_blocks) ||
-        out_bps * n_seqs >= (1ll << 28))
+    if (!h || in_dtype != TQ_F16 || n_blocks < AS_STORE_BLOCKS || !store_fast_ok(h, in_dtype, n_blocks) || out_bps * n_seqs >= (1ll << 28))
         return tqk_append_kv(hk, hv, k, v, n_seqs, 0, tokens, capacity, in_dtype, packed_k, packed_v, s);
-    const int rc = hk ? tqk_q8_0_append(v, n_seqs, 0, tokens, capacity, in_dtype, TQ_KIND_V, packed_v, s, nullptr, nullptr)
-                      : tqk_q8_0_append(k, n_seqs, 0, tokens, capacity, in_dtype, TQ_KIND_K, packed_k, s, nullptr, nullptr);
-    if (rc) return rc;
-    return hk ? store_one(hk, k, n_seqs, tokens, out_bps, in_dtype, TQ_KIND_K, packed_k, s)
-              : store_one(hv, v, n_seqs, tokens, out_bps, in_dtype, TQ_KIND_V, packed_v, s);
+    launch_units_kv(hk, hv, k, v, n_seqs, 0, tokens, capacity, true, packed_k, packed_v, s, nullptr, nullptr);
+    return tq_check_launch("store_layer");
 }
 
 // K and V of a layer to fp16 in the original domain.  One launch when both handles hold the fragments of the
