@@ -2009,6 +2009,18 @@ __device__ __forceinline__ void append_units(const __half *x, uint8_t *packed, c
     if (t0 + 16 <= n_old) return;  // nothing but tokens that stay
     uint8_t *block = packed + ((int64_t)seq * a.blocks_per_seq + bis) * block_bytes(BITS);
 
+    __half *norms = reinterpret_cast<__half *>(block + block_code_bytes(BITS));
+    if (t0 >= n_end) {  // nothing but rows past the new ones: norm 0 and the code of 0.0, which is as many dwords in K rows as in V's
+        const uint32_t code = a.thr[0] < 0.0f ? 1u << (BITS - 1) : (1u << (BITS - 1)) - 1u;
+        const uint32_t fill = code * (BITS == 4 ? 0x11111111u : BITS == 3 ? 0x00249249u : 0x55555555u);
+        uint32_t *out = reinterpret_cast<uint32_t *>(KIND == TQ_KIND_K ? block + t0 * 16 + lane * 4
+                                                                       : block + ((unit >> 2) * 64 + lane) * 16 + (unit & 3) * 4);
+#pragma unroll
+        for (int j = 0; j < BITS; ++j) out[512 * j] = BITS == 3 ? fill | (((fill >> (8 * j)) & 0xFFu) << 24) : fill;
+        if (lane < 16) norms[t0 + lane] = __float2half_rn(0.0f);
+        return;
+    }
+
     const int t = t0 + n16;  // the token of this lane's inputs; tokens outside the new ones request a new one's and drop them
     const __half *row = x + ((int64_t)seq * a.n_new + (tok0 + min(max(t, n_old), n_end - 1) - pos)) * 128;
     const uint4 *p = reinterpret_cast<const uint4 *>(row + (KIND == TQ_KIND_K ? 32 : 8) * kq);
@@ -2073,7 +2085,6 @@ __device__ __forceinline__ void append_units(const __half *x, uint8_t *packed, c
             q[h][ks] = KIND == TQ_KIND_K ? __builtin_amdgcn_mfma_f32_16x16x32_f16(fr[h * 4 + ks], xh[ks], float4_t{0.f, 0.f, 0.f, 0.f}, 0, 0, 0)
                                          : __builtin_amdgcn_mfma_f32_16x16x32_f16(xh[ks], fr[h * 4 + ks], float4_t{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
 
-    __half *norms = reinterpret_cast<__half *>(block + block_code_bytes(BITS));
     settle_matrix_results();  // what follows may be compiled to branches
     if constexpr (KIND == TQ_KIND_K) {
         if constexpr (AS_STORE) {
