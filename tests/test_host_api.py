@@ -196,3 +196,17 @@ def test_probe_library_is_separate_from_the_codec_abi():
     assert not any(n.startswith("tq_probe") for n in header_symbols())
     assert not hasattr(L.lib(), "tq_probe_stream")
     assert all(hasattr(probes.lib(), n) for n in ("tq_probe_stream", "tq_probe_flat", "tq_probe_mfma_f16"))
+
+
+@pytest.mark.parametrize("n_seqs,tokens", [(0, 5), (1, 0), (1, 1), (3, 128), (7, 129), (40, 100003)])
+def test_buffer_sizes_equal_the_library_s(n_seqs, tokens):
+    from turboquant_plus_amd.turbo import _q8_0_bytes
+    lib = L.lib()
+    for bits in (2, 3, 4):
+        assert tqa.packed_bytes(bits, n_seqs, tokens) == lib.tq_packed_bytes(bits, n_seqs, tokens)
+    assert _q8_0_bytes(n_seqs, tokens) == lib.tq_q8_0_bytes(n_seqs, tokens)
+    for bad in ((5, 1, 1), (3, -1, 1), (3, 1, -1)):
+        with pytest.raises(ValueError):
+            tqa.packed_bytes(*bad)
+    with pytest.raises(C.ArgumentError):
+        tqa.packed_bytes(3, 1.0, 128)

@@ -131,12 +131,19 @@ def check(rc: int) -> None:
 
 
 _torch = None
+_FLOATS = {}            # torch dtype -> code, for the three that the kernels take
+_current_device = _raw_stream = None
 
 
 def torch():
-    global _torch
+    global _torch, _current_device, _raw_stream
     if _torch is None:
         import torch as _t
+        _FLOATS.update({_t.float16: TQ_F16, _t.float32: TQ_F32, _t.float64: TQ_F64})
+        # torch's own short ways to the current device and to a stream's handle, where it has them: the public ones cost 0.3 and
+        # 2.7 us of a call that launches in 3.5
+        _current_device = getattr(_t._C, "_cuda_getDevice", None) or _t.cuda.current_device
+        _raw_stream = getattr(_t._C, "_cuda_getCurrentRawStream", None) or (lambda d: _t.cuda.current_stream(d).cuda_stream)
         _torch = _t
     return _torch
 
@@ -148,14 +155,11 @@ def require_gpu():
 
 
 def dtype_code(t) -> int:
-    tt = torch()
-    if t.dtype == tt.float16:
-        return TQ_F16
-    if t.dtype == tt.float32:
-        return TQ_F32
-    if t.dtype == tt.float64:
-        return TQ_F64
-    raise TypeError(f"unsupported dtype {t.dtype}")
+    torch()
+    code = _FLOATS.get(t.dtype)
+    if code is None:
+        raise TypeError(f"unsupported dtype {t.dtype}")
+    return code
 
 
 def torch_dtype(code: int):
@@ -167,16 +171,17 @@ def to_device(x, float_ok=(np.float16, np.float32, np.float64)):
     """NumPy array or torch tensor -> contiguous CUDA tensor (floats keep their
     width, everything else becomes float64 as NumPy promotion would)."""
     tt = torch()
-    dev = require_gpu()
     if isinstance(x, tt.Tensor):
-        t = x.to(dev)
+        if x.is_cuda and x.dtype in _FLOATS and x.is_contiguous() and x.get_device() == _current_device():
+            return x        # in place already
+        t = x.to(require_gpu())
         if t.dtype not in (tt.float16, tt.float32, tt.float64):
             t = t.to(tt.float64)
         return t.contiguous()
     a = np.asarray(x)
     if a.dtype not in [np.dtype(f) for f in float_ok]:
         a = a.astype(np.float64)
-    return tt.from_numpy(np.ascontiguousarray(a)).to(dev)
+    return tt.from_numpy(np.ascontiguousarray(a)).to(require_gpu())
 
 
 # ---- results of the NumPy classes: device buffers and their way into host arrays -----------------------------------
@@ -382,11 +387,14 @@ def upload(*arrays):
 
 
 def stream_ptr():
-    return C.c_void_p(torch().cuda.current_stream().cuda_stream)
+    """The handle of the current device's current stream, for a void * argument."""
+    if not torch().cuda.is_initialized():
+        torch().cuda.init()
+    return _raw_stream(_current_device())
 
 
 def ptr(t):
-    return C.c_void_p(t.data_ptr()) if t is not None else C.c_void_p(0)
+    return t.data_ptr() if t is not None else None
 
 
 def dbl_ptr(a):

@@ -29,7 +29,17 @@ HEAD_DIM = 128
 BLOCK_TOKENS = 128
 
 
+def _q8_0_bytes(n_seqs: int, tokens: int) -> int:
+    """tq_q8_0_bytes (a negative size is answered with -1)."""
+    if type(n_seqs) is type(tokens) is int and n_seqs >= 0 and tokens >= 0:
+        return n_seqs * -(-tokens // BLOCK_TOKENS) * BLOCK_TOKENS * 136     # as in packed_bytes
+    return int(L.lib().tq_q8_0_bytes(n_seqs, tokens))
+
+
 def packed_bytes(bits: int, n_seqs: int, tokens: int) -> int:
+    if type(bits) is type(n_seqs) is type(tokens) is int and 2 <= bits <= 4 and n_seqs >= 0 and tokens >= 0:
+        # without a call into the library: two to four of these come before every launch
+        return n_seqs * -(-tokens // BLOCK_TOKENS) * BLOCK_TOKENS * (16 * bits + 2)
     n = L.lib().tq_packed_bytes(bits, n_seqs, tokens)
     if n < 0:
         raise ValueError("bits must be 2, 3 or 4 and sizes non-negative")
@@ -93,8 +103,11 @@ class TurboCodec:
     @staticmethod
     def _as_seqs(x):
         xd = L.to_device(x)
-        if xd.shape[-1] != HEAD_DIM:
-            raise ValueError(f"last dimension must be {HEAD_DIM}, got {xd.shape[-1]}")
+        shape = xd.shape
+        if shape[-1] != HEAD_DIM:
+            raise ValueError(f"last dimension must be {HEAD_DIM}, got {shape[-1]}")
+        if len(shape) == 3 and shape[1]:
+            return xd, shape[0], shape[1]
         if xd.dim() == 2:
             xd = xd[None]
         tokens = xd.shape[-2]
@@ -385,7 +398,7 @@ def q8_0_append(x, packed, pos, capacity: int, kind: str = "k", overrun=None):
     out for `capacity` tokens per sequence (zero-initialised; tq_q8_0_append).  pos: an int, or an int64 device
     tensor with one element read when the launch runs (tq_q8_0_append_at; `overrun` as in TurboCodec.append)."""
     xd, n_seqs, n_new = TurboCodec._as_seqs(x)
-    need = int(L.lib().tq_q8_0_bytes(n_seqs, capacity))
+    need = _q8_0_bytes(n_seqs, capacity)
     if packed.numel() < need:
         raise ValueError(f"packed holds {packed.numel()} bytes, need {need}")
     if _position_on_device(pos):
@@ -400,9 +413,8 @@ def q8_0_append(x, packed, pos, capacity: int, kind: str = "k", overrun=None):
 
 def _layer_buffers(k_codec, v_codec, n_seqs: int, capacity: int, k_cache, v_cache):
     """The two handles of a layer (None: q8_0-style rows), after a check that its caches hold `capacity` tokens."""
-    lib = L.lib()
     for codec, buf in ((k_codec, k_cache), (v_codec, v_cache)):
-        need = int(lib.tq_q8_0_bytes(n_seqs, capacity)) if codec is None else packed_bytes(codec.bits, n_seqs, capacity)
+        need = _q8_0_bytes(n_seqs, capacity) if codec is None else packed_bytes(codec.bits, n_seqs, capacity)
         if buf.numel() < need:
             raise ValueError(f"packed holds {buf.numel()} bytes, need {need}")
     return (None if c is None else c.handle.h for c in (k_codec, v_codec))
@@ -517,30 +529,31 @@ class DecodeAttention:
         qd = L.to_device(q)
         if self.poison_output:
             self.out.fill_(float("nan"))
-        tt = L.torch()
+        params = self.params
         if sparse_bias is not None:
+            tt = L.torch()
             pos, val = sparse_bias
-            want = (self.params.batch, self.params.n_q_heads)
+            want = (params.batch, params.n_q_heads)
             if (pos.dtype != tt.int32 or val.dtype != tt.float32 or not pos.is_cuda or not val.is_cuda or pos.dim() != 3
                     or tuple(pos.shape[:2]) != want or pos.shape != val.shape):
                 raise ValueError("sparse_bias must be (int32 positions, float32 values), device tensors [batch, n_q_heads, E]")
             pos, val = pos.contiguous(), val.contiguous()
-            self.params.bias_entries = int(pos.shape[2])
-            self.params.bias_pos, self.params.bias_val = pos.data_ptr(), val.data_ptr()
+            params.bias_entries = int(pos.shape[2])
+            params.bias_pos, params.bias_val = pos.data_ptr(), val.data_ptr()
             self._sparse_bias = (pos, val)   # kept alive until the next call
-        else:
-            self.params.bias_entries = 0
-            self.params.bias_pos = self.params.bias_val = None
-        if self.params.n_splits == self._splits_set:    # not where the caller has set another one
-            self.params.n_splits = self._splits_set = self._own_splits[self.params.bias_entries > 0]
+        elif params.bias_entries or params.bias_pos or params.bias_val:
+            params.bias_entries = 0
+            params.bias_pos = params.bias_val = None
+        if params.n_splits == self._splits_set:    # not where the caller has set another one
+            splits = self._own_splits[params.bias_entries > 0]
+            if splits != self._splits_set:
+                params.n_splits = self._splits_set = splits
         hk = self.k_codec.handle.h if self.k_codec is not None else None
         hv = self.v_codec.handle.h if self.v_codec is not None else None
-        L.check(L.lib().tq_decode_attention(hk, hv, C.byref(self.params), L.ptr(qd),
-                                            L.dtype_code(qd), L.ptr(k_packed), None, L.ptr(v_packed), L.ptr(bias),
-                                            L.ptr(self.out),
-                                            L.ptr(self.skip if self.params.sparse_v_tau > 0 else None),
-                                            L.ptr(self.workspace),
-                                            self.workspace.numel(), L.stream_ptr()))
+        L.check(L.lib().tq_decode_attention(hk, hv, C.byref(params), L.ptr(qd), L.dtype_code(qd), L.ptr(k_packed), None,
+                                            L.ptr(v_packed), L.ptr(bias), L.ptr(self.out),
+                                            L.ptr(self.skip if params.sparse_v_tau > 0 else None),
+                                            L.ptr(self.workspace), self.workspace.numel(), L.stream_ptr()))
         return self.out
 
     def set_tokens(self, tokens: int) -> None:
