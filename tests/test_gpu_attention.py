@@ -923,3 +923,36 @@ def test_split_counts_with_and_without_a_bias_list():
     for n in counts.values():
         p.n_splits = n
         assert L.lib().tq_attn_workspace_bytes(L.C.byref(p)) <= attn.workspace.numel()
+
+
+@pytest.mark.parametrize("hq,hkv,head_dim", [(16, 2, 256), (5, 1, 256), (36, 2, 128), (9, 1, 128)])
+@pytest.mark.parametrize("tokens,n_splits", [(70, 1), (1000, 6), (1000, 16)])
+def test_passes_of_one_launch_equal_passes_one_by_one(hq, hkv, head_dim, tokens, n_splits):
+    """More query heads than a pass takes: one launch where the workspace has room for every pass's partials, one after the
+    other in a workspace for one; the same bits, with a dense and a sparse bias and from a captured graph as well."""
+    tt = L.torch()
+    layer = tqa.LayerKV(tqa.LayerFormat("turbo3", "turbo3"))
+    gen = tt.Generator("cuda").manual_seed(tokens)
+    two = head_dim // 128
+    k, v = (tt.randn((2 * hkv, two * tokens, 128), generator=gen, device="cuda").half() for _ in range(2))
+    kp, vp = layer.store(k, v)
+    q = tt.randn((2, hq, head_dim), generator=gen, device="cuda").half()
+    together, apart = (layer.attention(2, hq, hkv, tokens, n_splits=n_splits, head_dim=head_dim) for _ in range(2))
+    p = L.TQAttnParams.from_buffer_copy(apart.params)
+    p.n_q_heads = hkv * (4 if head_dim == 256 else 8)     # as many as one pass takes
+    one = L.lib().tq_attn_workspace_bytes(L.C.byref(p))
+    assert one < together.workspace.numel()
+    apart.workspace = apart.workspace[:one]
+    bias = tt.randn((2, hq, tokens), generator=gen, device="cuda")
+    sparse = (tt.arange(3, device="cuda", dtype=tt.int32).expand(2, hq, 3).contiguous(), tt.ones((2, hq, 3), device="cuda"))
+    for kw in (dict(), dict(bias=bias), dict(sparse_bias=sparse)):
+        a, b = together(q, kp, vp, **kw), apart(q, kp, vp, **kw)
+        assert tt.equal(a, b) and bool(tt.isfinite(a).all())
+    want = together(q, kp, vp).clone()
+    graph = tt.cuda.CUDAGraph()
+    with tt.cuda.graph(graph):
+        together(q, kp, vp)
+    for _ in range(3):
+        together.out.fill_(float("nan"))
+        graph.replay()
+        assert tt.equal(together.out, want)

@@ -209,11 +209,12 @@ struct AttnArgs {
     unsigned long long *pass_totals;      // Sparse V: [pass] skipped pairs of each four-head pass of this step
     unsigned long long *skip_count;       // caller's {skipped, total} or NULL
     unsigned long long total_pairs;
-    int pass;                             // head_off / 4
+    int pass;                             // head_off / pass_heads
     int64_t tokens, blocks_per_seq;
     const int64_t *tokens_dev;  // NULL, or where the step's context length is read from (<= tokens, which then is the maximum)
     int n_groups, n_splits, tiles_per_split, n_tiles;
-    int q_group, head_off;  // query heads per KV head; first of the (up to) four heads this launch works on
+    int q_group, head_off;  // query heads per KV head; first of the heads that this launch's first pass works on
+    int pass_heads;         // heads per pass; blockIdx.y numbers the passes of a launch, whose partials and counters follow each other
     int d256;               // heads of 256 dims: a token is two 128-value rows (2 token + half) of the K and V caches
     int gpw;                // (batch, kv head) groups per workgroup: 1, or wavefronts per workgroup / n_splits when a group's
                             // splits are fewer than a workgroup's wavefronts (short contexts: the groups share the decode tables)
@@ -472,16 +473,17 @@ __device__ __forceinline__ MergedPart merge_range(const float *ml0, const float 
 // partials, and joins their results through `lds` (free LDS of 132 floats per wavefront; unused otherwise): the merge
 // runs at the very end of the launch, so its trips to memory are the launch's tail.
 template <int HG>
-__device__ __forceinline__ void merge_group(const AttnArgs &a, int group, int n_parts, int tid, int n_waves, float *lds) {
+__device__ __forceinline__ void merge_group(const AttnArgs &a, int group, int pgroup, int head_off, int n_parts, int tid, int n_waves,
+                                            float *lds) {
     constexpr int NH = 4 * HG, ML = 2 * NH, PO = 128 * NH;  // heads, (m, l) floats and output floats of one partial
     const int lane = tid & 63, wave = tid >> 6;
-    const float *ml0 = a.part_ml + (int64_t)group * n_parts * ML;
-    const float *po0 = a.part_o + (int64_t)group * n_parts * PO;
+    const float *ml0 = a.part_ml + (int64_t)pgroup * n_parts * ML;
+    const float *po0 = a.part_o + (int64_t)pgroup * n_parts * PO;
     auto finish = [&](int head, MergedPart r) {
         // heads of 256 dims (HG = 2): partial row 4 dh + i is dims 128 dh .. 128 dh + 127 of head i
         const int hq = a.d256 ? (head & 3) : head;
-        const int64_t r_out = a.d256 ? 2 * ((int64_t)group * a.q_group + a.head_off + hq) + (head >> 2)
-                                     : (int64_t)group * a.q_group + a.head_off + head;
+        const int64_t r_out = a.d256 ? 2 * ((int64_t)group * a.q_group + head_off + hq) + (head >> 2)
+                                     : (int64_t)group * a.q_group + head_off + head;
         const float invL = r.L > 0.0f ? 1.0f / r.L : 0.0f;
         float o0 = r.o0, o1 = r.o1;
         float2 res;
@@ -498,7 +500,7 @@ __device__ __forceinline__ void merge_group(const AttnArgs &a, int group, int n_
         *reinterpret_cast<float2 *>(a.out + r_out * 128 + 2 * lane) = res;
     };
     // a repeated head of a group with fewer than four left is not written
-    auto head_exists = [&](int head) { return a.head_off + (a.d256 ? (head & 3) : head) < a.q_group; };
+    auto head_exists = [&](int head) { return head_off + (a.d256 ? (head & 3) : head) < a.q_group; };
     const int n_sub = lds && n_waves >= 2 * NH && n_parts > 4 ? n_waves / NH : 1;
     if (n_sub == 1) {
         for (int head = wave; head < NH; head += n_waves)
@@ -610,6 +612,8 @@ __global__ __launch_bounds__(64 * max_waves_per_workgroup(VBITS, HG, KFMT == KFM
     const int wgs_per_group = a.wgs_per_group;
     const int group = __builtin_amdgcn_readfirstlane(a.gpw > 1 ? (int)blockIdx.x * a.gpw + gidx : (int)(blockIdx.x / wgs_per_group));
     const int part = a.gpw > 1 ? 0 : __builtin_amdgcn_readfirstlane((int)(blockIdx.x % wgs_per_group));
+    const int pass_y = HG == 2 ? (int)blockIdx.y : 0;   // one set of four heads is always one pass
+    const int head_off = a.head_off + pass_y * a.pass_heads, pgroup = pass_y * a.n_groups + group;
     const int split = part * n_waves + wave_g;  // index of this wavefront's partial
     // dynamic LDS: the wavefronts' merge space (end of the split), then 1 KB per group and set of four heads that
     // stages the rotated queries
@@ -713,8 +717,8 @@ __global__ __launch_bounds__(64 * max_waves_per_workgroup(VBITS, HG, KFMT == KFM
     if constexpr (!SHARE && VBITS == 3) vpair = a.vlut[lane];
 
     // one partial per workgroup: index (group, part), 4 HG heads each
-    float *po = a.part_o + ((int64_t)group * wgs_per_group + part) * 4 * HG * 128;
-    float *pml = a.part_ml + ((int64_t)group * wgs_per_group + part) * 4 * HG * 2;
+    float *po = a.part_o + ((int64_t)pgroup * wgs_per_group + part) * 4 * HG * 128;
+    float *pml = a.part_ml + ((int64_t)pgroup * wgs_per_group + part) * 4 * HG * 2;
 
     // A operand of QK, broadcast from one block per MFMA: lane (b, i) keeps q[head i] for the
     // dim groups g = b and g = b + 16 (4 dims each); MFMA g reads it from block g % 16.
@@ -722,8 +726,8 @@ __global__ __launch_bounds__(64 * max_waves_per_workgroup(VBITS, HG, KFMT == KFM
     // head, two values per lane), scaled and parked as fp16 in 1 KB of LDS for everybody.
     auto load_q = [&](int h, float &x0, float &x1) {
         // heads past the group's last one repeat it (their results are not written)
-        const int64_t e = D256 ? ((int64_t)group * a.q_group + min(a.head_off + (h & 3), a.q_group - 1)) * 256 + 128 * (h >> 2) + 2 * lane
-                               : ((int64_t)group * a.q_group + min(a.head_off + h, a.q_group - 1)) * 128 + 2 * lane;
+        const int64_t e = D256 ? ((int64_t)group * a.q_group + min(head_off + (h & 3), a.q_group - 1)) * 256 + 128 * (h >> 2) + 2 * lane
+                               : ((int64_t)group * a.q_group + min(head_off + h, a.q_group - 1)) * 128 + 2 * lane;
         if (a.q_dtype == TQ_F16) {
             const __half *qp = reinterpret_cast<const __half *>(a.q);
             x0 = __half2float(qp[e]);
@@ -760,7 +764,7 @@ __global__ __launch_bounds__(64 * max_waves_per_workgroup(VBITS, HG, KFMT == KFM
         sb_val[hg] = 0.0f;
     }
     // entry e of the list of this lane's head in set hg (addresses are formed where they are needed: the path is rare)
-    auto sb_entry = [&](int hg, int e) { return ((int64_t)group * a.q_group + min(a.head_off + 4 * hg + j, a.q_group - 1)) * a.sbias_n + e; };
+    auto sb_entry = [&](int hg, int e) { return ((int64_t)group * a.q_group + min(head_off + 4 * hg + j, a.q_group - 1)) * a.sbias_n + e; };
     auto sb_load = [&](int hg) {   // this lane's entry of the window
         const int e = sb_win[hg] + (lane >> 2);
         const bool in = e < a.sbias_n;
@@ -775,7 +779,7 @@ __global__ __launch_bounds__(64 * max_waves_per_workgroup(VBITS, HG, KFMT == KFM
             int below[4];
 #pragma unroll
             for (int h = 0; h < 4; ++h) {
-                const int32_t *prow = a.sbias_pos + ((int64_t)group * a.q_group + min(a.head_off + 4 * hg + h, a.q_group - 1)) * a.sbias_n;
+                const int32_t *prow = a.sbias_pos + ((int64_t)group * a.q_group + min(head_off + 4 * hg + h, a.q_group - 1)) * a.sbias_n;
                 int c = 0;
                 for (int e0 = 0; e0 < a.sbias_n; e0 += 64) {
                     const int e = e0 + lane;
@@ -845,7 +849,7 @@ __global__ __launch_bounds__(64 * max_waves_per_workgroup(VBITS, HG, KFMT == KFM
         for (int i = 0; i < 4; ++i) bv[i] = 0.0f;
         if (!a.bias) return;
         const int tk = t * TT + t4;  // the launcher checks tokens < 2^31
-        const float *row = a.bias + ((int64_t)group * a.q_group + min(a.head_off + 4 * hg + j, a.q_group - 1)) * a.tokens;
+        const float *row = a.bias + ((int64_t)group * a.q_group + min(head_off + 4 * hg + j, a.q_group - 1)) * a.tokens;
         if (bias_vec && tk + 3 < tokens_now) {
             const float4 v = *reinterpret_cast<const float4 *>(row + tk);
             bv[0] = v.x; bv[1] = v.y; bv[2] = v.z; bv[3] = v.w;
@@ -863,7 +867,7 @@ __global__ __launch_bounds__(64 * max_waves_per_workgroup(VBITS, HG, KFMT == KFM
 
     unsigned long long head_ok[HG];  // lanes whose head (lane % 4 of each set) exists in this pass
 #pragma unroll
-    for (int hg = 0; hg < HG; ++hg) head_ok[hg] = __builtin_amdgcn_ballot_w64(a.head_off + 4 * hg + j < a.q_group);
+    for (int hg = 0; hg < HG; ++hg) head_ok[hg] = __builtin_amdgcn_ballot_w64(head_off + 4 * hg + j < a.q_group);
 #pragma unroll 1
     while (tile < t_end) {
         const int64_t blk = tile >> 1;
@@ -1248,7 +1252,7 @@ __global__ __launch_bounds__(64 * max_waves_per_workgroup(VBITS, HG, KFMT == KFM
         // other partial was complete in memory before its owner's increment, hence before this one's.
         __shared__ int i_am_last;
         if (tid == 0) {
-            unsigned long long *ctr = a.flags + (int64_t)group * n_parts;
+            unsigned long long *ctr = a.flags + (int64_t)pgroup * n_parts;
             const unsigned long long tag = a.nonce & ~ARRIVAL_COUNT_MASK;
             unsigned long long seen = ld_dev(ctr), count;
             for (;;) {
@@ -1288,8 +1292,8 @@ __global__ __launch_bounds__(64 * max_waves_per_workgroup(VBITS, HG, KFMT == KFM
     }
     // the wavefronts' merge space is free again (every partial of this workgroup is in memory); with several groups
     // per workgroup every group's wavefronts finish their own group (one partial: no exchange between them)
-    merge_group<HG>(a, group, n_parts, tid_g, gw, n_waves > 1 && a.gpw <= 1 ? merge_s : nullptr);
-    if (n_parts > 1 && tid == 0) st_dev(a.flags + (int64_t)group * n_parts, 0ull);  // a replay of a captured launch (same tag) starts from zero
+    merge_group<HG>(a, group, pgroup, head_off, n_parts, tid_g, gw, n_waves > 1 && a.gpw <= 1 ? merge_s : nullptr);
+    if (n_parts > 1 && tid == 0) st_dev(a.flags + (int64_t)pgroup * n_parts, 0ull);  // a replay of a captured launch (same tag) starts from zero
     if constexpr (SPARSE) {
         if (a.poll_slots) {
             if (!__syncthreads_and(all_in)) return;
@@ -1379,8 +1383,11 @@ AttnPlan attn_plan(const tq_attn_params *p, bool bias_list) {
     pl.n_parts = p->n_splits / pl.wpw;
     return pl;
 }
-WsLayout ws_layout(const tq_attn_params *p) {
-    const int64_t groups = (int64_t)p->batch * p->n_kv_heads;
+int heads_per_pass(const tq_attn_params *p) { return p->head_dim == 256 || p->n_q_heads / p->n_kv_heads <= 4 ? 4 : 8; }
+int passes_of(const tq_attn_params *p) { return (p->n_q_heads / p->n_kv_heads + heads_per_pass(p) - 1) / heads_per_pass(p); }
+// passes: of a launch
+WsLayout ws_layout(const tq_attn_params *p, int passes) {
+    const int64_t groups = (int64_t)p->batch * p->n_kv_heads * passes;
     // a call with a bias list may run smaller workgroups (more partials per group) than one without: room for either
     const AttnPlan pl = attn_plan(p, false), pl_list = attn_plan(p, true);
     const int64_t parts = groups * (pl.n_parts > pl_list.n_parts ? pl.n_parts : pl_list.n_parts);
@@ -1396,13 +1403,20 @@ WsLayout ws_layout(const tq_attn_params *p) {
 
 }  // namespace
 
-int64_t tqk_attn_workspace_bytes(const tq_attn_params *p) { return ws_layout(p).total; }
+int64_t tqk_attn_workspace_bytes(const tq_attn_params *p) { return ws_layout(p, p->sparse_v_tau > 0.0f ? 1 : passes_of(p)).total; }
 
 int tqk_decode_attention(const tq_handle *hk, const tq_handle *hv, const tq_attn_params *p, const void *q, int q_dtype,
                          const void *k, const void *k_aux, const void *v, const float *bias, float *out,
                          unsigned long long *skip_count, void *ws, int64_t ws_bytes, hipStream_t s) {
     (void)k_aux;
-    const WsLayout w = ws_layout(p);
+    // All passes in one launch where the workspace has room: each is a chain of its own (launch, first rows, merge), one of few
+    // groups leaves most of the chip idle, and they read the same rows.  Steps of two passes over 256-dim heads (us with the
+    // append, one pass after the other / together): 2 x 8 KV heads x 259 tokens turbo4 35.0 / 19.6, 4 x 8 x 4000 turbo3 50.5 / 32.8,
+    // 1 x 1 x 100 000 turbo2 169 / 95, 8 x 4 x 16 000 8-bit K with turbo3 V 86.2 / 82.4, 16 x 8 x 12 000 turbo4 180 / 174 to 178.
+    // Sparse V counts pass by pass.
+    int n_pass = p->sparse_v_tau > 0.0f ? 1 : passes_of(p);
+    if (n_pass > 1 && ws_bytes < ws_layout(p, n_pass).total) n_pass = 1;
+    const WsLayout w = ws_layout(p, n_pass);
     if (ws_bytes < w.total) {
         tq_set_error("tq_decode_attention: workspace %lld < %lld bytes", (long long)ws_bytes, (long long)w.total);
         return TQ_ERR_ARG;
@@ -1477,7 +1491,8 @@ int tqk_decode_attention(const tq_handle *hk, const tq_handle *hv, const tq_attn
     // that divides the split count
     const AttnPlan pl = attn_plan(p, p->bias_entries > 0);
     const int wpw = pl.wpw, hg = pl.hg;
-    const unsigned grid = (unsigned)((int64_t)groups * pl.n_parts / pl.gpw);
+    const unsigned pass_wgs = (unsigned)((int64_t)groups * pl.n_parts / pl.gpw);
+    const dim3 grid(pass_wgs, n_pass);
     const unsigned wg = 64u * (unsigned)wpw;
     const int n_parts = pl.n_parts;  // partials per group: the wavefronts of a workgroup merge theirs in LDS
     // dynamic LDS: the wavefronts' merge space, then the staged queries of the workgroup's groups
@@ -1493,8 +1508,8 @@ int tqk_decode_attention(const tq_handle *hk, const tq_handle *hv, const tq_attn
     // ceil(G / 8) passes over the same K/V; a last pass with fewer heads than it has rows repeats the group's
     // last head and does not write the repeats.
     a.q_group = p->n_q_heads / p->n_kv_heads;
-    const int heads_per_pass = d256 ? 4 : 4 * hg;
-    if ((a.q_group + heads_per_pass - 1) / heads_per_pass > MAX_PASSES) {
+    a.pass_heads = heads_per_pass(p);
+    if (passes_of(p) > MAX_PASSES) {
         tq_set_error("tq_decode_attention: %d query heads per KV head (at most %d)", a.q_group, 4 * MAX_PASSES);
         return TQ_ERR_UNSUPPORTED;
     }
@@ -1502,14 +1517,14 @@ int tqk_decode_attention(const tq_handle *hk, const tq_handle *hv, const tq_attn
     a.vs1 = vs1;
     a.vs2 = vs2;
     a.flags = reinterpret_cast<unsigned long long *>((char *)ws + w.flags);
-    a.poll_slots = sparse && grid <= (unsigned)MAX_POLLED_SLOTS;
+    a.poll_slots = sparse && pass_wgs <= (unsigned)MAX_POLLED_SLOTS;
     a.pass_totals = reinterpret_cast<unsigned long long *>((char *)ws + w.pass_totals);
     a.skip_count = skip_count;
     a.total_pairs = total_pairs;
     (void)n_parts;
     (void)kb;
-    for (a.head_off = 0; a.head_off < a.q_group; a.head_off += heads_per_pass) {
-        a.pass = a.head_off / heads_per_pass;
+    for (a.head_off = 0; a.head_off < a.q_group; a.head_off += n_pass * a.pass_heads) {
+        a.pass = a.head_off / a.pass_heads;
         a.nonce = next_nonce();
         if (d256) {
 #define TQ_ATTN_256_ONE(KF, KB, VB, SH)                                                                              \
@@ -1588,7 +1603,7 @@ int tqk_decode_attention(const tq_handle *hk, const tq_handle *hv, const tq_attn
     if (rc) return rc;
     if (skip_count && !a.poll_slots) {
         // more groups than the finishing workgroups poll (or a dense step whose caller wants the counts)
-        k_skip_sum<<<1, 1024, 0, s>>>(a.skip_slots, sparse ? (int)grid : 0, skip_count, total_pairs, a.head_off > 0);
+        k_skip_sum<<<1, 1024, 0, s>>>(a.skip_slots, sparse ? (int)pass_wgs : 0, skip_count, total_pairs, a.head_off > 0);
         rc = tq_check_launch("skip_sum");
         if (rc) return rc;
     }
@@ -1634,7 +1649,7 @@ int tqk_static_scratch(void **out) {
 int tqk_decode_attention_static(const tq_handle *hk, const tq_handle *hv, const tq_attn_params *p, const void *q,
                                 int q_dtype, const void *k, const void *v, const float *bias, float *out,
                                 unsigned long long *skip_count, hipStream_t s) {
-    const int64_t need = ws_layout(p).total;
+    const int64_t need = ws_layout(p, 1).total;
     if (need > STATIC_WS_BYTES) {
         tq_set_error("tq_decode_attention_static: batch * n_kv_heads * n_splits = %lld needs %lld bytes of split "
                      "partials, the built-in workspace holds %lld; lower n_splits or use tq_decode_attention",
