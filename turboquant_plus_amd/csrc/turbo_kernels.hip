@@ -2245,6 +2245,13 @@ __global__ __launch_bounds__(512) void k_store_qjl_mfma(const TI *x, uint8_t *pa
         v += xor_lane<32>(v);
         return v;
     };
+    // v with its sign flipped where bit s of the mask is set: on the sign bit itself (a choice between v and -v per value keeps
+    // 64 lane masks, which do not fit the scalar registers: 240 moves to and from vector lanes per unit)
+    auto flip_sign = [](double v, uint32_t mask, int s) {
+        const uint64_t b = __builtin_bit_cast(uint64_t, v);
+        return __builtin_bit_cast(double, b ^ ((uint64_t)((mask << (31 - s)) & 0x80000000u) << 32));
+    };
+    const double own1 = kq & 1 ? -1.0 : 1.0, own2 = kq & 2 ? -1.0 : 1.0;  // a butterfly across lanes: own1 * own + the other's
 
 #pragma unroll 1
     for (; unit < n_units; unit += unit_step) {
@@ -2255,30 +2262,25 @@ __global__ __launch_bounds__(512) void k_store_qjl_mfma(const TI *x, uint8_t *pa
         const int64_t row0 = seq * a.tokens;
         const int t = u * 16 + n16;
         const bool valid = xvalid;
+        asm volatile("" : "+v"(neg1), "+v"(neg2));  // or the compiler keeps the 64 shifted masks of flip_sign in registers it has not got
         double e[32];
 #pragma unroll
-        for (int s = 0; s < 32; ++s) e[s] = valid ? ldd(xin, s) : 0.0;
+        for (int s = 0; s < 32; ++s) {
+            const TI v = valid ? xin[s] : (TI)0.0f;
+            e[s] = ldd(&v, 0);
+        }
         double ss = 0.0;
 #pragma unroll
         for (int s = 0; s < 32; ++s) ss = fma(e[s], e[s], ss);
         const double nrm = sqrt(quarter_sum(ss));
         const double inv = nrm > 0.0 ? 1.0 / nrm : 1.0;
 #pragma unroll
-        for (int s = 0; s < 32; ++s) {
-            e[s] = e[s] * inv;
-            if ((neg1 >> s) & 1u) e[s] = -e[s];
-        }
+        for (int s = 0; s < 32; ++s) e[s] = flip_sign(e[s] * inv, neg1, s);
         // butterfly, strides 1 and 2 across the lane quarters, then 4 .. 64 in the lane
 #pragma unroll
-        for (int s = 0; s < 32; ++s) {
-            const double p = xor_lane<16>(e[s]);
-            e[s] = (kq & 1) ? p - e[s] : e[s] + p;
-        }
+        for (int s = 0; s < 32; ++s) e[s] = fma(own1, e[s], xor_lane<16>(e[s]));
 #pragma unroll
-        for (int s = 0; s < 32; ++s) {
-            const double p = xor_lane<32>(e[s]);
-            e[s] = (kq & 2) ? p - e[s] : e[s] + p;
-        }
+        for (int s = 0; s < 32; ++s) e[s] = fma(own2, e[s], xor_lane<32>(e[s]));
 #pragma unroll
         for (int hb = 1; hb < 32; hb <<= 1)
 #pragma unroll
@@ -2291,8 +2293,7 @@ __global__ __launch_bounds__(512) void k_store_qjl_mfma(const TI *x, uint8_t *pa
         uint32_t cw[4] = {0u, 0u, 0u, 0u};  // the 32 codes, 4 bits each
 #pragma unroll
         for (int s = 0; s < 32; ++s) {
-            double yv = e[s] * inv_rn;
-            if ((neg2 >> s) & 1u) yv = -yv;
+            const double yv = flip_sign(e[s] * inv_rn, neg2, s);
             e[s] = yv;
             uint32_t c = 0;
 #pragma unroll
