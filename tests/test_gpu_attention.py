@@ -956,3 +956,18 @@ def test_passes_of_one_launch_equal_passes_one_by_one(hq, hkv, head_dim, tokens,
         together.out.fill_(float("nan"))
         graph.replay()
         assert tt.equal(together.out, want)
+
+
+@pytest.mark.parametrize("nk,nq", [(1, 129), (256, 2048), (257, 385), (700, 1000), (22_000, 400), (33_000, 300)])
+@pytest.mark.parametrize("out", ["float16", "float32"])
+def test_score_tile_shared_out_over_queries(nk, nq, out):
+    """Few keys: the query tiles go to several workgroups; the bits of one tile of queries at a time."""
+    tt = L.torch()
+    codec = tqa.TurboCodec(3, seed=42, projection="gaussian", projection_seed=2)
+    gen = tt.Generator("cuda").manual_seed(nk)
+    k, q = tt.randn((nk, 128), generator=gen, device="cuda"), tt.randn((nq, 128), generator=gen, device="cuda").half()
+    sketch = codec.store_qjl(k)
+    got = tt.full((nq, nk), float("nan"), dtype=getattr(tt, out), device="cuda")
+    codec.score_tile(q, *sketch, nk, out=got)
+    want = tt.cat([codec.score_tile(q[i:i + 128], *sketch, nk, out_dtype=got.dtype) for i in range(0, nq, 128)])
+    assert tt.equal(got, want)

@@ -34,6 +34,7 @@
 // k_score_tile: TurboQuant inner-product estimate, 32x32x16 fp16 MFMA over a
 //   K = 256 contraction ([R q | S q] against [g c[idx] | scale*rnorm*z]); key operands in registers, queries
 //   through LDS, logit rows written 64 consecutive logits per store.
+#include <algorithm>
 #include <atomic>
 #include <mutex>
 #include <cstring>
@@ -1753,13 +1754,14 @@ constexpr int SCORE_QT = 128;  // queries per LDS tile: four operand blocks of 1
 template <int BITS, typename TO, bool DRAIN>
 __global__ __launch_bounds__(512, 1) void k_score_tile(const __half *qa, const uint8_t *packed, const uint8_t *sign_bits,
                                                       const __half *rnorms, int64_t nq, int64_t nk, TO *logits,
-                                                      const uint32_t *pair_lut, float proj_scale) {
+                                                      const uint32_t *pair_lut, float proj_scale, int tiles_per) {
     extern __shared__ __attribute__((aligned(16))) _Float16 kt[];  // keys [SCORE_KEYS][KT_STRIDE], then two query tiles
     __shared__ uint32_t ptab[1 << (2 * BITS)];                     // pair code -> (c[lo], c[hi]) as two halves
     const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
     const int64_t key0 = (int64_t)blockIdx.x * SCORE_KEYS;
     const int n_blocks = (int)((nq + 31) / 32);  // operand blocks the preparation wrote
-    const int n_tiles = (int)((nq + SCORE_QT - 1) / SCORE_QT);
+    // the query tiles of this workgroup: all of them, or a share where few keys leave CUs without a workgroup
+    const int t_begin = (int)blockIdx.y * tiles_per, t_end = min(t_begin + tiles_per, (int)((nq + SCORE_QT - 1) / SCORE_QT));
     typedef uint32_t chunk_t __attribute__((ext_vector_type(4)));   // 16 bytes: what a lane feeds to one matrix instruction
     const chunk_t *qchunks = reinterpret_cast<const chunk_t *>(qa);  // [block][K step][lane]
     // chunk group g (0..7) of a tile: lanes tid + 512 g of its 4096 chunks, i.e. half g % 2 of operand block g / 2
@@ -1770,7 +1772,7 @@ __global__ __launch_bounds__(512, 1) void k_score_tile(const __half *qa, const u
     // the first tile is requested before anything else and waits in registers until the keys have left LDS
     chunk_t first_tile[8];
 #pragma unroll
-    for (int g = 0; g < 8; ++g) first_tile[g] = *tile_chunk(0, g);
+    for (int g = 0; g < 8; ++g) first_tile[g] = *tile_chunk(t_begin, g);
     if (tid < (1 << (2 * BITS))) ptab[tid] = pair_lut[tid];
     __syncthreads();
     {
@@ -1951,11 +1953,11 @@ __global__ __launch_bounds__(512, 1) void k_score_tile(const __half *qa, const u
 #pragma unroll
     for (int t = 0; t < AHEAD; ++t) pre[t] = __builtin_bit_cast(half8_t, qtile[(2 * qh) * 1024 + t * 64 + lane]);
 #pragma unroll 1
-    for (int tile = 0; tile < n_tiles; ++tile) {
-        const chunk_t *cur = qtile + (tile & 1) * 4096;
-        chunk_t *next = qtile + ((tile + 1) & 1) * 4096;
+    for (int tile = t_begin; tile < t_end; ++tile) {
+        const chunk_t *cur = qtile + ((tile - t_begin) & 1) * 4096;
+        chunk_t *next = qtile + ((tile - t_begin + 1) & 1) * 4096;
         const int row0 = tile * SCORE_QT + qh * 64;
-        const int tile_next = min(tile + 1, n_tiles - 1);  // the last tile re-reads itself
+        const int tile_next = min(tile + 1, t_end - 1);  // the last tile re-reads itself
         block(cur, next, 2 * qh, cur, 2 * qh + 1, std::integral_constant<int, 0>{}, tile_next, pre, acc_a, acc_b, pb);
         pb = pend(row0);
         block(cur, next, 2 * qh + 1, next, 2 * qh, std::integral_constant<int, 1>{}, tile_next, pre, acc_b, acc_a, pb);
@@ -1995,14 +1997,20 @@ int tqk_score_tile(const tq_handle *h, const void *q, int q_dtype, int64_t nq, c
     }
     int rc = tq_check_launch("prep_score_q");
     if (rc) return rc;
-    const unsigned grid = (unsigned)((nk + SCORE_KEYS - 1) / SCORE_KEYS);
+    // A workgroup per 256 keys, one to a CU; fewer keys than fill the chip: the query tiles are shared out too, up to one round
+    // of workgroups (each dequantises its keys again, side by side).  Scores and their preparation, us, not shared / shared: 11 835
+    // keys x 962 queries 30 / 24, x 2048 51 / 42; 2000 x 2048 48 / 13.
+    const int64_t key_wgs = (nk + SCORE_KEYS - 1) / SCORE_KEYS, tiles = (nq + SCORE_QT - 1) / SCORE_QT;
+    const int64_t shares = std::max<int64_t>(1, std::min(tiles, 256 / key_wgs));
+    const int tiles_per = (int)((tiles + shares - 1) / shares);
+    const dim3 grid((unsigned)key_wgs, (unsigned)((tiles + tiles_per - 1) / tiles_per));
     const size_t lds = (size_t)SCORE_KEYS * KT_STRIDE * sizeof(_Float16);
 #define TQ_SCORE(B, T, DR)                                                                                             \
     {                                                                                                                  \
         (void)hipFuncSetAttribute((const void *)k_score_tile<B, T, DR>, hipFuncAttributeMaxDynamicSharedMemorySize,   \
                                   (int)lds);                                                                           \
         k_score_tile<B, T, DR><<<grid, 512, lds, s>>>(qa, (const uint8_t *)packed, sign_bits, (const __half *)rnorms, \
-                                                      nq, nk, (T *)logits, (const uint32_t *)h->pair_lut, (float)h->proj_scale); \
+                                                      nq, nk, (T *)logits, (const uint32_t *)h->pair_lut, (float)h->proj_scale, tiles_per); \
     }
 #define TQ_SCORE_BITS(T, DR)                                                                              \
     if (h->bits == 2) TQ_SCORE(2, T, DR) else if (h->bits == 3) TQ_SCORE(3, T, DR) else TQ_SCORE(4, T, DR)
