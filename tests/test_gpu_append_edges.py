@@ -34,14 +34,17 @@ def test_turbo_rows(bits, kind):
 
 @pytest.mark.parametrize("bits", [2, 3, 4])
 @pytest.mark.parametrize("kind", ["k", "v"])
-@pytest.mark.parametrize("on_device", [False, True])
-def test_turbo_rows_on_the_matrix_cores(bits, kind, on_device):
-    """float16 rows go through the matrix cores in units of 16 tokens.  Whatever tokens stay before a span (all-zero rows among
+@pytest.mark.parametrize("dtype,on_device", [("float16", False), ("float16", True), ("float32", False)])
+def test_turbo_rows_on_the_matrix_cores(bits, kind, dtype, on_device):
+    """float16 and float32 rows go through the matrix cores in units of 16 tokens.  Whatever tokens stay before a span (all-zero rows among
     both), the bytes are those of one append of all of them, whose codes and norms agree with the oracle, and nothing
     outside the touched blocks is written."""
     tt = L.torch()
     codec = tqa.TurboCodec(bits, seed=3)
-    x = tt.randn((N_SEQS, 400, D), generator=tt.Generator("cuda").manual_seed(bits), device="cuda").half()
+    x = tt.randn((N_SEQS, 400, D), generator=tt.Generator("cuda").manual_seed(bits), device="cuda")
+    if dtype == "float32":      # norms over seven decades
+        x *= 10 ** (tt.rand((N_SEQS, 400, 1), generator=tt.Generator("cuda").manual_seed(5), device="cuda") * 7 - 4)
+    x = x.to(getattr(tt, dtype))
     x[0, 20] = x[1, 203] = 0
     for pos, n_new in SPANS:
         rows = tt.cat([x[:, 200:200 + pos], x[:, :n_new]], dim=1)
@@ -198,13 +201,14 @@ def test_float32_prompts_keep_their_low_bits(fmt, tokens):
 
 @pytest.mark.parametrize("pair", [(2, 2), (3, 3), (4, 4), (4, 2), (4, 3), (3, 2), (2, 4)])
 @pytest.mark.parametrize("shape", [(1, 1), (3, 333), (2, 16 * 128), (64, 4 * 128), (64, 4 * 128 + 1)])
-def test_short_prompts_have_the_bytes_of_the_store(pair, shape):
-    """Prompts of up to 256 blocks in float16 (and one of 320): K and V in one launch have the bytes of a store per side, into
+@pytest.mark.parametrize("dtype", ["float16", "float32"])
+def test_short_prompts_have_the_bytes_of_the_store(pair, shape, dtype):
+    """Prompts of up to 256 blocks (and one of 320): K and V in one launch have the bytes of a store per side, into
     buffers of their length and into caches laid out for more tokens."""
     tt = L.torch()
     n, tokens = shape
     kc, vc = (tqa.TurboCodec(b, seed=s) for b, s in zip(pair, (3, 503)))
-    k, v = (tt.randn((n, tokens, D), generator=tt.Generator("cuda").manual_seed(s), device="cuda").half() for s in (1, 2))
+    k, v = (tt.randn((n, tokens, D), generator=tt.Generator("cuda").manual_seed(s), device="cuda").to(getattr(tt, dtype)) for s in (1, 2))
     k[0, tokens // 2] = 0
     blocks, capacity = -(-tokens // 128), 128 * (-(-tokens // 128) + 3)
     want = kc.store(k, kind="k"), vc.store(v, kind="v")
@@ -214,3 +218,32 @@ def test_short_prompts_have_the_bytes_of_the_store(pair, shape):
     for cache, w in zip(caches, want):
         assert tt.equal(cache.view(n, blocks + 3, -1)[:, :blocks], w.view(n, blocks, -1))
         assert bool((cache.view(n, blocks + 3, -1)[:, blocks:] == 0xA5).all())
+
+
+@pytest.mark.parametrize("dtype", ["float16", "float32"])
+@pytest.mark.parametrize("which", ["k", "v", "both"])
+def test_codebooks_that_the_matrix_cores_do_not_take(dtype, which):
+    """An asymmetric codebook on one side or both: K and V of a step have the bytes of an append per side, and codes within
+    32-bit rounding of the boundaries, with the position on the host and on the device."""
+    tt = L.torch()
+    cent = np.sort(np.random.default_rng(2).uniform(-0.25, 0.3, 8))
+    kc, vc = (tqa.TurboCodec(3, seed=s, centroids=cent if which in (side, "both") else None) for s, side in ((3, "k"), (503, "v")))
+    k, v = (tt.randn((N_SEQS, 200, D), generator=tt.Generator("cuda").manual_seed(s), device="cuda").to(getattr(tt, dtype)) for s in (1, 2))
+    one, two, dev = ([tt.zeros(tqa.packed_bytes(3, N_SEQS, CAPACITY), dtype=tt.uint8, device="cuda") for _ in range(2)] for _ in range(3))
+    pos = 0
+    for n_new in (1, 30, 97, 2, 70):
+        kn, vn = k[:, pos:pos + n_new], v[:, pos:pos + n_new]
+        kc.append_kv(vc, kn, vn, *one, pos, CAPACITY)
+        kc.append_kv(vc, kn, vn, *dev, tt.tensor([pos], device="cuda"), CAPACITY)
+        kc.append(kn, two[0], pos, CAPACITY, kind="k")
+        vc.append(vn, two[1], pos, CAPACITY, kind="v")
+        pos += n_new
+        for a, b, c in zip(one, two, dev):
+            assert tt.equal(a, b) and tt.equal(c, b), (pos, n_new)
+    for codec, x, cache, kind in ((kc, k, one[0], "k"), (vc, v, one[1], "v")):
+        idx = np_(codec.unpack_codes(cache, N_SEQS, CAPACITY, kind=kind)[0])[:, :200].reshape(-1, D).astype(int)
+        xd = np_(x).astype(np.float64).reshape(-1, D)
+        y = O.rotate_fast(xd / np.linalg.norm(xd, axis=1, keepdims=True), codec.signs1, codec.signs2, D)
+        mid = (codec.centroids[1:] + codec.centroids[:-1]) / 2
+        lo, hi = ((mid[None, None] < (y + e)[..., None]).sum(-1) for e in (-1e-6, 1e-6))
+        assert ((idx >= lo) & (idx <= hi)).all()

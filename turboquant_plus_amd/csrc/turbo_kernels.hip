@@ -501,6 +501,22 @@ __device__ __forceinline__ void split8(uint4 a, uint4 b, float sc, half8_t &hi, 
         mid[2 * i] = m[0]; mid[2 * i + 1] = m[1];
     }
 }
+// the same in three terms: all 24 bits of a value, down to 2^-34 of the row's norm
+__device__ __forceinline__ void split8(uint4 a, uint4 b, float sc, half8_t &hi, half8_t &mid, half8_t &lo) {
+    const float v[8] = {__uint_as_float(a.x), __uint_as_float(a.y), __uint_as_float(a.z), __uint_as_float(a.w),
+                        __uint_as_float(b.x), __uint_as_float(b.y), __uint_as_float(b.z), __uint_as_float(b.w)};
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const float2_t xs = {v[2 * i] * sc, v[2 * i + 1] * sc};
+        const half2_t h = __builtin_convertvector(xs, half2_t);
+        const float2_t r = xs - __builtin_convertvector(h, float2_t);
+        const half2_t m = __builtin_convertvector(r, half2_t);
+        const half2_t l = __builtin_convertvector(r - __builtin_convertvector(m, float2_t), half2_t);
+        hi[2 * i] = h[0]; hi[2 * i + 1] = h[1];
+        mid[2 * i] = m[0]; mid[2 * i + 1] = m[1];
+        lo[2 * i] = l[0]; lo[2 * i + 1] = l[1];
+    }
+}
 __device__ __forceinline__ float sumsq8(uint4 a, uint4 b, float acc) {
     acc = fmaf(__uint_as_float(a.x), __uint_as_float(a.x), acc); acc = fmaf(__uint_as_float(a.y), __uint_as_float(a.y), acc);
     acc = fmaf(__uint_as_float(a.z), __uint_as_float(a.z), acc); acc = fmaf(__uint_as_float(a.w), __uint_as_float(a.w), acc);
@@ -633,7 +649,7 @@ __device__ __forceinline__ float k_unit_codes(const float4_t (&q)[2][4], float s
     constexpr bool EXACT = LUT == LUT_NONE, NORMALISED = BITS == 4 && !EXACT;
     // root of 1 ulp: scales boundaries (1e-7 relative) and the stored fp16 norm
     const float norm = EXACT ? sqrtf(ss) : __builtin_amdgcn_sqrtf(ss);
-    const float scale = norm > 0.0f ? (EXACT ? sqrtf(128.0f * ss) * rowscale : norm * rowscale * 11.313708498984761f) : 1.0f;  // y' = sqrt(128) ||x|| y
+    const float scale = norm > 0.0f ? (EXACT ? sqrtf(128.0f * (ss * rowscale * rowscale)) : norm * rowscale * 11.313708498984761f) : 1.0f;  // y' = sqrt(128) ||x|| y
     float thr[NT];
 #pragma unroll
     for (int k = 0; k < NT; ++k) thr[k] = EXACT ? fmaf(thr0[k], scale, thr_lo[k] * scale) : thr0[k] * scale;
@@ -1118,12 +1134,12 @@ __device__ __forceinline__ float v_subtile_codes(const float4_t (&qq)[2][4], con
         const float ss = row16_sum(n16 == 4 * kq + i ? gram[i] : 0.0f);
         nrm[i] = EXACT ? ss : __builtin_amdgcn_sqrtf(ss);
         const bool nz = ss > 0.0f;
-        const float rowscale = F32 ? row_pow2_scale(nrm[i]) : 1.0f;  // the power of two the token's fp32 row was multiplied by
+        const float rowscale = F32 ? row_pow2_scale(EXACT ? sqrtf(ss) : nrm[i]) : 1.0f;  // the power of two the token's fp32 row was multiplied by
         if constexpr (NORMALISED) {
             inv[i] = nz ? __builtin_amdgcn_rsqf(ss) * (0.08838834764831845f * pow2_reciprocal(rowscale)) : 1.0f;  // 1 / (||x|| sqrt(128))
         } else {
             inv[i] = 1.0f;
-            const float scale = nz ? (EXACT ? sqrtf(128.0f * ss) : nrm[i] * rowscale * 11.313708498984761f) : 1.0f;
+            const float scale = nz ? (EXACT ? sqrtf(128.0f * (ss * rowscale * rowscale)) : nrm[i] * rowscale * 11.313708498984761f) : 1.0f;
 #pragma unroll
             for (int k = 0; k < NT; ++k) thr_tok[i][k] = EXACT ? fmaf(thr0[k], scale, thr_lo[k] * scale) : thr0[k] * scale;
         }
@@ -1966,7 +1982,7 @@ __global__ __launch_bounds__(APPEND_THREADS) void k_append(const TI *x, uint8_t 
     append_block<BITS, TI>(x, packed, a, blockIdx.x);
 }
 
-// ---- the same on the matrix cores: fp16 rows of symmetric codebooks --------------------------------------
+// ---- the same on the matrix cores: fp16 and fp32 rows of symmetric codebooks --------------------------------------
 // A wavefront takes 16 consecutive tokens of a block, as a K unit or as a fourth of a V tile, through the store kernels'
 // steps (k_unit_codes, v_subtile_codes; without their 1-ulp roots and their table).  No LDS and no barrier: a K unit's
 // dwords are its own rows', a V unit's are one dword per (row, chunk) of its token group, which no other wavefront writes;
@@ -1977,7 +1993,9 @@ __global__ __launch_bounds__(APPEND_THREADS) void k_append(const TI *x, uint8_t 
 // (5.4 / 5.4 / 6.2e-5).
 // Bound: vector instructions (650 to 1230 for 16 tokens; the butterfly needs about 300 for each four, and its codes go
 // through LDS).  64 x 2048 tokens, K and V: turbo2 35.0 -> 21.0 us, turbo3 45.6 -> 25.8, turbo4 47.3 -> 29.4, 8-bit K with
-// turbo3 V 39.0 -> 26.8 (copies of these bytes: 15 to 18 us).
+// turbo3 V 39.0 -> 26.8 (copies of these bytes: 15 to 18 us).  fp32 rows (copies: 29 us): 41.4 -> 37.0, 47.8 -> 39.6, 54.2 ->
+// 43.4 us; shares off, norms over four decades, 2 / 3 / 4 bits: codes 3.5 / 8.0 / 16.9e-8 (butterfly 6.0 / 13.2 / 25.3e-8), norms
+// 4.9 / 5.1 / 5.6e-5 (5.2 / 5.7 / 6.1e-5).
 struct AppendUnitArgs {
     int64_t pos, n_new, capacity, blocks_per_seq, first_block;
     const int64_t *pos_dev;  // as in AppendArgs
@@ -1989,8 +2007,12 @@ struct AppendUnitArgs {
     float thr[8], thr_lo[8], coef[8];       // boundaries: thr + thr_lo
 };
 // AS_STORE: a prompt's rows, whose bytes are those of tq_store (the store kernels' roots, table decisions and zeros).
-template <int BITS, int KIND, bool AS_STORE>
-__device__ __forceinline__ void append_units(const __half *x, uint8_t *packed, const AppendUnitArgs &a, const unsigned wg) {
+// TI = float: fp32 rows as three fp16 terms per value, which hold all of its bits (a term's sums are as good as exact), or in
+// the store's two.
+template <int BITS, int KIND, bool AS_STORE, typename TI>
+__device__ __forceinline__ void append_units(const TI *x, uint8_t *packed, const AppendUnitArgs &a, const unsigned wg) {
+    constexpr bool F32 = sizeof(TI) == 4;
+    constexpr int NX = F32 ? 8 : 4;  // 16-byte pieces of a lane's 32 inputs
     constexpr int NT = 1 << (BITS - 1);
     constexpr LevelLut LUT = AS_STORE ? LUT_SEARCH : LUT_NONE;
     const int lane = threadIdx.x & 63, n16 = lane & 15, kq = lane >> 4;
@@ -2022,11 +2044,11 @@ __device__ __forceinline__ void append_units(const __half *x, uint8_t *packed, c
     }
 
     const int t = t0 + n16;  // the token of this lane's inputs; tokens outside the new ones request a new one's and drop them
-    const __half *row = x + ((int64_t)seq * a.n_new + (tok0 + min(max(t, n_old), n_end - 1) - pos)) * 128;
+    const TI *row = x + ((int64_t)seq * a.n_new + (tok0 + min(max(t, n_old), n_end - 1) - pos)) * 128;
     const uint4 *p = reinterpret_cast<const uint4 *>(row + (KIND == TQ_KIND_K ? 32 : 8) * kq);
-    uint4 xb[4];
+    uint4 xb[NX];
 #pragma unroll
-    for (int ks = 0; ks < 4; ++ks) xb[ks] = p[KIND == TQ_KIND_K ? ks : 4 * ks];
+    for (int i = 0; i < NX; ++i) xb[i] = p[KIND == TQ_KIND_K ? i : F32 ? 8 * (i >> 1) + (i & 1) : 4 * i];
     // V: dword `jd` of the lane's rows 16 dd + n16 of the tile is what the lane stores
     const int jd = BITS == 2 ? kq >> 1 : kq;
     const bool stores = BITS == 4 || (BITS == 3 ? kq < 3 : (kq & 1) == 0);
@@ -2054,40 +2076,74 @@ __device__ __forceinline__ void append_units(const __half *x, uint8_t *packed, c
     if constexpr (KIND == TQ_KIND_K) build_k_fragments(fr, of_quarter(a.s1neg[0], a.s1neg[1], a.s1neg[2], a.s1neg[3]), lane);
     else build_v_fragments(fr, a.s1neg, lane);
     const bool fresh = t >= n_old && t < n_end;
-    half8_t xh[4];
 #pragma unroll
-    for (int ks = 0; ks < 4; ++ks) xh[ks] = __builtin_bit_cast(half8_t, fresh ? xb[ks] : make_uint4(0, 0, 0, 0));
+    for (int i = 0; i < NX; ++i) xb[i] = fresh ? xb[i] : make_uint4(0, 0, 0, 0);
 
     float4_t gram = {0.f, 0.f, 0.f, 0.f};  // of token 4 kq + i: element i of column 4 kq + i
-    float ss = 0.0f;                       // of token n16
-    if constexpr (AS_STORE) {
+    float ss = 0.0f, rowscale = 1.0f;      // of token n16
+    if constexpr (AS_STORE && F32) {
+        float s0 = 0.0f, s1 = 0.0f;
 #pragma unroll
-        for (int ks = 0; ks < 4; ++ks) gram = __builtin_amdgcn_mfma_f32_16x16x32_f16(xh[ks], xh[ks], gram, 0, 0, 0);
+        for (int ks = 0; ks < 4; ks += 2) {
+            s0 = sumsq8(xb[2 * ks], xb[2 * ks + 1], s0);
+            s1 = sumsq8(xb[2 * ks + 2], xb[2 * ks + 3], s1);
+        }
+        ss = s0 + s1;
+        ss += xor_lane<16>(ss);
+        ss += xor_lane<32>(ss);
+        gram = float4_t{ss, ss, ss, ss};
+        rowscale = row_pow2_scale(__builtin_amdgcn_sqrtf(ss));
+    } else if constexpr (AS_STORE) {
+#pragma unroll
+        for (int ks = 0; ks < 4; ++ks)
+            gram = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8_t, xb[ks]), __builtin_bit_cast(half8_t, xb[ks]), gram, 0, 0, 0);
     } else {
         // over the four lanes that share the token, in four short sums: closer than the matrix cores' X X^T
         float part[4];
 #pragma unroll
         for (int ks = 0; ks < 4; ++ks) {
-            part[ks] = 0.0f;
+            if constexpr (F32) {
+                part[ks] = sumsq8(xb[2 * ks], xb[2 * ks + 1], 0.0f);
+            } else {
+                const half8_t h = __builtin_bit_cast(half8_t, xb[ks]);
+                part[ks] = 0.0f;
 #pragma unroll
-            for (int e = 0; e < 8; ++e) part[ks] = fmaf((float)xh[ks][e], (float)xh[ks][e], part[ks]);
+                for (int e = 0; e < 8; ++e) part[ks] = fmaf((float)h[e], (float)h[e], part[ks]);
+            }
         }
         ss = (part[0] + part[1]) + (part[2] + part[3]);
         ss += xor_lane<16>(ss);
         ss += xor_lane<32>(ss);
         gram = float4_t{ss, ss, ss, ss};
+        if constexpr (F32) rowscale = row_pow2_scale(sqrtf(ss));
     }
+    auto product = [&](half8_t f, half8_t v, float4_t c) {
+        return KIND == TQ_KIND_K ? __builtin_amdgcn_mfma_f32_16x16x32_f16(f, v, c, 0, 0, 0) : __builtin_amdgcn_mfma_f32_16x16x32_f16(v, f, c, 0, 0, 0);
+    };
+    const float4_t none = {0.f, 0.f, 0.f, 0.f};
     float4_t q[2][4];
 #pragma unroll
-    for (int h = 0; h < 2; ++h)
+    for (int ks = 0; ks < 4; ++ks) {
+        if constexpr (AS_STORE && F32) {
+            half8_t hi, mid;
+            split8(xb[2 * ks], xb[2 * ks + 1], rowscale, hi, mid);
 #pragma unroll
-        for (int ks = 0; ks < 4; ++ks)
-            q[h][ks] = KIND == TQ_KIND_K ? __builtin_amdgcn_mfma_f32_16x16x32_f16(fr[h * 4 + ks], xh[ks], float4_t{0.f, 0.f, 0.f, 0.f}, 0, 0, 0)
-                                         : __builtin_amdgcn_mfma_f32_16x16x32_f16(xh[ks], fr[h * 4 + ks], float4_t{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+            for (int h = 0; h < 2; ++h) q[h][ks] = product(fr[h * 4 + ks], hi, product(fr[h * 4 + ks], mid, none));
+        } else if constexpr (F32) {
+            half8_t hi, mid, lo;
+            split8(xb[2 * ks], xb[2 * ks + 1], rowscale, hi, mid, lo);
+#pragma unroll
+            for (int h = 0; h < 2; ++h)  // the small terms apart: large ones that cancel leave them whole
+                q[h][ks] = product(fr[h * 4 + ks], hi, none) + product(fr[h * 4 + ks], mid, product(fr[h * 4 + ks], lo, none));
+        } else {
+#pragma unroll
+            for (int h = 0; h < 2; ++h) q[h][ks] = product(fr[h * 4 + ks], __builtin_bit_cast(half8_t, xb[ks]), none);
+        }
+    }
 
     settle_matrix_results();  // what follows may be compiled to branches
     if constexpr (KIND == TQ_KIND_K) {
-        if constexpr (AS_STORE) {
+        if constexpr (AS_STORE && !F32) {
 #pragma unroll
             for (int i = 0; i < 4; ++i) ss += n16 == 4 * kq + i ? gram[i] : 0.0f;
             ss += xor_lane<16>(ss);
@@ -2096,7 +2152,7 @@ __device__ __forceinline__ void append_units(const __half *x, uint8_t *packed, c
         uint32_t flip[4], g[BITS];
 #pragma unroll
         for (int j = 0; j < 4; ++j) flip[j] = of_quarter(a.flipw[j], a.flipw[4 + j], a.flipw[8 + j], a.flipw[12 + j]);
-        const float gn = k_unit_codes<BITS, LUT>(q, ss, 1.0f, thr0, thr_lo, coef, flip, zero_word, a.norm_correction, nullptr, g);
+        const float gn = k_unit_codes<BITS, LUT>(q, ss, rowscale, thr0, thr_lo, coef, flip, zero_word, a.norm_correction, nullptr, g);
         if (t >= n_old) {
 #pragma unroll
             for (int j = 0; j < BITS; ++j) *reinterpret_cast<uint32_t *>(block + j * 2048 + t * 16 + kq * 4) = g[j];
@@ -2104,7 +2160,7 @@ __device__ __forceinline__ void append_units(const __half *x, uint8_t *packed, c
         }
     } else {
         uint32_t w[4] = {0, 0, 0, 0}, zero_tokens = 0, zm[4] = {0, 0, 0, 0};
-        const float gn = v_subtile_codes<BITS, false, LUT>(q, gram, n16, kq, thr0, thr_lo, coef, a.norm_correction, nullptr, w, zero_tokens, zm);
+        const float gn = v_subtile_codes<BITS, F32, LUT>(q, gram, n16, kq, thr0, thr_lo, coef, a.norm_correction, nullptr, w, zero_tokens, zm);
         // field 4 hf + i of a word is token i's code of dim half hf
         constexpr uint32_t CM = (1u << BITS) - 1u, SB = 1u << (BITS - 1);
         if constexpr (AS_STORE) {  // (else a token of zeros has nothing but zero values)
@@ -2148,8 +2204,8 @@ __device__ __forceinline__ void append_units(const __half *x, uint8_t *packed, c
     }
 }
 
-template <int BITS, int KIND>
-__global__ __launch_bounds__(APPEND_THREADS, 4) void k_append_units(const __half *x, uint8_t *packed, AppendUnitArgs a) {
+template <int BITS, int KIND, typename TI>
+__global__ __launch_bounds__(APPEND_THREADS, sizeof(TI) == 4 ? 3 : 4) void k_append_units(const TI *x, uint8_t *packed, AppendUnitArgs a) {
     append_units<BITS, KIND, false>(x, packed, a, blockIdx.x);
 }
 
@@ -3152,12 +3208,12 @@ template <int SIDE> struct AppendSide { using Args = std::conditional_t<SIDE == 
 template <int SIDE, int KIND, typename TI>
 __device__ __forceinline__ void append_side(const TI *x, uint8_t *packed, typename AppendSide<SIDE>::Args &a, const unsigned wg) {
     if constexpr (SIDE == 0) q8_0_append_block<TI, KIND>(x, packed, a, wg);
-    else if constexpr (SIDE > UNITS) append_units<SIDE % UNITS, KIND, (SIDE > UNITS_AS_STORE)>(x, packed, a, wg);
+    else if constexpr (SIDE > UNITS) append_units<SIDE % UNITS, KIND, (SIDE > UNITS_AS_STORE), TI>(x, packed, a, wg);
     else if (resolve_append(a, wg)) append_block<SIDE, TI>(x, packed, a, wg);
 }
 static_assert(APPEND_THREADS == Q8A_THREADS, "both kinds of rows run in one launch");
 template <int KB, int VB, typename TI>
-__global__ __launch_bounds__(APPEND_THREADS, (KB > UNITS || VB > UNITS) ? 4 : 1) void k_append_kv(const TI *xk, uint8_t *pk, typename AppendSide<KB>::Args ka, const TI *xv,
+__global__ __launch_bounds__(APPEND_THREADS, (KB > UNITS || VB > UNITS) ? (sizeof(TI) == 4 ? 3 : 4) : 1) void k_append_kv(const TI *xk, uint8_t *pk, typename AppendSide<KB>::Args ka, const TI *xv,
                                                               uint8_t *pv, typename AppendSide<VB>::Args va) {
     const unsigned half = gridDim.x >> 1;
     if (blockIdx.x < half) append_side<KB, TQ_KIND_K, TI>(xk, pk, ka, blockIdx.x);
@@ -4353,9 +4409,8 @@ static Q8AppendArgs make_q8_append_args(const void *x, int64_t pos, const int64_
     return a;
 }
 
-// Rows that append_units takes: fp16, whose products with the +-1 factor are exact on the matrix cores, of the codebooks that
-// the matrix-core store takes.  (fp32 rows stay with the butterfly: the store's two fp16 terms per value are 22 bits.)
-static bool append_units_ok(const tq_handle *h, int in_dtype) { return in_dtype == TQ_F16 && store_fast_ok(h, in_dtype, 0); }
+// Rows that append_units takes: fp16 and fp32, of the codebooks that the matrix-core store takes.
+static bool append_units_ok(const tq_handle *h, int in_dtype) { return store_fast_ok(h, in_dtype, 0); }
 
 static AppendUnitArgs make_append_unit_args(const tq_handle *h, int64_t pos, const int64_t *pos_dev, int64_t n_new, int64_t capacity,
                                             uint32_t *overrun) {
@@ -4394,7 +4449,7 @@ static AppendUnitArgs make_append_unit_args(const tq_handle *h, int64_t pos, con
 
 // K and V through append_units (both turbo sides fit for it, one at least); false: no kernel for this pair
 static bool launch_units_kv(const tq_handle *hk, const tq_handle *hv, const void *k, const void *v, int64_t n_seqs, int64_t pos,
-                            int64_t n_new, int64_t capacity, bool as_store, void *packed_k, void *packed_v, hipStream_t s,
+                            int64_t n_new, int64_t capacity, int in_dtype, bool as_store, void *packed_k, void *packed_v, hipStream_t s,
                             const int64_t *pos_dev, uint32_t *overrun) {
     const Q8AppendArgs qk = make_q8_append_args(k, pos, pos_dev, n_new, capacity, pos_dev ? overrun : nullptr);
     const Q8AppendArgs qv = make_q8_append_args(v, pos, pos_dev, n_new, capacity, nullptr);  // the K half reports
@@ -4404,7 +4459,9 @@ static bool launch_units_kv(const tq_handle *hk, const tq_handle *hv, const void
     const unsigned grid = 2u * (unsigned)(n_seqs * qk.n_touched);
     const int kb = hk ? hk->bits : 0, vb = hv ? hv->bits : 0;
     bool one_launch = true;
-    if (as_store) TQ_APPEND_PAIRS(UNITS_AS_STORE, __half)
+    if (as_store && in_dtype == TQ_F32) TQ_APPEND_PAIRS(UNITS_AS_STORE, float)
+    else if (as_store) TQ_APPEND_PAIRS(UNITS_AS_STORE, __half)
+    else if (in_dtype == TQ_F32) TQ_APPEND_PAIRS(UNITS, float)
     else TQ_APPEND_PAIRS(UNITS, __half)
     return one_launch;
 }
@@ -4418,7 +4475,7 @@ int tqk_append_kv(const tq_handle *hk, const tq_handle *hv, const void *k, const
     const bool ku = hk && append_units_ok(hk, in_dtype), vu = hv && append_units_ok(hv, in_dtype);
     bool one_launch = true;
     if ((ku || vu) && (ku || !hk) && (vu || !hv)) {
-        one_launch = launch_units_kv(hk, hv, k, v, n_seqs, pos, n_new, capacity, false, packed_k, packed_v, s, pos_dev, overrun);
+        one_launch = launch_units_kv(hk, hv, k, v, n_seqs, pos, n_new, capacity, in_dtype, false, packed_k, packed_v, s, pos_dev, overrun);
     } else if (ku || vu) {
         one_launch = false;  // one side's codebook is for the butterfly
     } else {
@@ -4451,15 +4508,19 @@ int tqk_append(const tq_handle *h, const void *x, int64_t n_seqs, int64_t pos, i
     const unsigned grid = (unsigned)(n_seqs * a.n_touched);
     if (append_units_ok(h, in_dtype)) {
         const AppendUnitArgs u = make_append_unit_args(h, pos, pos_dev, n_new, capacity, overrun);
-#define TQ_UNITS(B)                                                                                                          \
-    if (kind == TQ_KIND_K) k_append_units<B, TQ_KIND_K><<<grid, APPEND_THREADS, 0, s>>>((const __half *)x, (uint8_t *)packed, u); \
-    else k_append_units<B, TQ_KIND_V><<<grid, APPEND_THREADS, 0, s>>>((const __half *)x, (uint8_t *)packed, u)
+#define TQ_UNITS_T(B, T)                                                                                                     \
+    if (kind == TQ_KIND_K) k_append_units<B, TQ_KIND_K, T><<<grid, APPEND_THREADS, 0, s>>>((const T *)x, (uint8_t *)packed, u);   \
+    else k_append_units<B, TQ_KIND_V, T><<<grid, APPEND_THREADS, 0, s>>>((const T *)x, (uint8_t *)packed, u)
+#define TQ_UNITS(B)                             \
+    if (in_dtype == TQ_F32) { TQ_UNITS_T(B, float); } \
+    else { TQ_UNITS_T(B, __half); }
         switch (h->bits) {
         case 2: TQ_UNITS(2); break;
         case 3: TQ_UNITS(3); break;
         default: TQ_UNITS(4); break;
         }
 #undef TQ_UNITS
+#undef TQ_UNITS_T
         return tq_check_launch("append_units");
     }
 #define TQ_APPEND_BITS(B) \
@@ -4474,11 +4535,12 @@ int tqk_append(const tq_handle *h, const void *x, int64_t n_seqs, int64_t pos, i
     return tq_check_launch("append");
 }
 
-// fp16 prompts up to this many blocks take a wavefront per 16 tokens (append_units) instead of the persistent store, where a
+// fp16 and fp32 prompts up to this many blocks take a wavefront per 16 tokens (append_units) instead of the persistent store, where a
 // V tile of 64 is one wavefront's chain of 4 to 8 us however few there are.  Two workgroups per CU: beyond, the store's queue
 // and prefetch are the better ones for the wide formats (kernel, us, store / units: turbo3 8 x 777 tokens 7.8 / 4.6, 256
 // blocks 8.9 / 7.4, 384 10.5 / 9.9, 448 11.6 / 12.6; turbo4 8.7 / 5.2, 10.0 / 8.4, 11.0 / 11.5, 12.5 / 14.3; turbo2 6.5 / 4.1,
-// 7.3 / 6.3, 8.8 / 8.7, 9.7 / 9.6).  The bytes are the same.
+// 7.3 / 6.3, 8.8 / 8.7, 9.7 / 9.6; fp32 rows, turbo3 10.8 / 6.8, 256 blocks 13.5 / 10.8, and turbo4 K with turbo2 V, two
+// launches of the store, 13.4 / 6.4 and 17.4 / 10.7).  The bytes are the same.
 constexpr int64_t SHORT_PROMPT_BLOCKS = 256;
 // capacity > 0: the packed buffers are caches laid out for `capacity` tokens per sequence (tq_append's layout) and the
 // `tokens` tokens of every sequence go to its first blocks; 0: sequences follow each other at blocks_for(tokens)
@@ -4493,8 +4555,8 @@ int tqk_store_kv(const tq_handle *hk, const tq_handle *hv, const void *k, const 
         const int rc = tqk_store(hk, k, n_seqs, tokens, in_dtype, TQ_KIND_K, packed_k, nullptr, nullptr, s);
         return rc ? rc : tqk_store(hv, v, n_seqs, tokens, in_dtype, TQ_KIND_V, packed_v, nullptr, nullptr, s);
     }
-    if (in_dtype == TQ_F16 && n_blocks <= SHORT_PROMPT_BLOCKS &&
-        launch_units_kv(hk, hv, k, v, n_seqs, 0, tokens, out_bps * TQ_ROWS_PER_BLOCK, true, packed_k, packed_v, s, nullptr, nullptr))
+    if (n_blocks <= SHORT_PROMPT_BLOCKS &&
+        launch_units_kv(hk, hv, k, v, n_seqs, 0, tokens, out_bps * TQ_ROWS_PER_BLOCK, in_dtype, true, packed_k, packed_v, s, nullptr, nullptr))
         return tq_check_launch("store_kv (short)");
     StoreKArgs ka = make_k_args(hk, tokens, bps, n_blocks);
     StoreVArgs va = make_v_args(hv, tokens, bps, n_blocks);
@@ -4548,8 +4610,7 @@ int tqk_store_kv(const tq_handle *hk, const tq_handle *hv, const void *k, const 
 
 // Prompt of a layer of any two formats (hk / hv NULL: q8_0-style rows) into caches laid out for `capacity` tokens, one launch.
 // fp16 rows of a long prompt (512 blocks) have the turbo side's bytes from tq_store's arithmetic, all others from the
-// append's.  fp32 rows stay with the butterfly: the matrix cores would take them as two fp16 terms, which drop what lies
-// below 2^-22 of a value (split8).
+// append's (fp32 rows at every length: tq_store's two fp16 terms drop what lies below 2^-22 of a value).
 // (Two launches, the 8-bit side's append and the persistent store, took (kernels, us; 8-bit K with turbo3 V, fp16) 21.0 for 528
 // blocks, 23.2 for 752 and 44.5 for 2048; in one launch 13.9, 16.4 and 40.7; turbo4 V 22.4, 24.8 and 46.4 against 15.5, 18.0 and
 // 44.8; turbo3 K with 8-bit V 16.7, 19.4 and 42.2 against 12.5, 15.7 and 38.2.)
@@ -4561,7 +4622,7 @@ int tqk_store_layer(const tq_handle *hk, const tq_handle *hv, const void *k, con
     const int64_t n_blocks = n_seqs * blocks_for(tokens), out_bps = blocks_for(capacity);
     if (!h || in_dtype != TQ_F16 || n_blocks < AS_STORE_BLOCKS || !store_fast_ok(h, in_dtype, n_blocks) || out_bps * n_seqs >= (1ll << 28))
         return tqk_append_kv(hk, hv, k, v, n_seqs, 0, tokens, capacity, in_dtype, packed_k, packed_v, s);
-    launch_units_kv(hk, hv, k, v, n_seqs, 0, tokens, capacity, true, packed_k, packed_v, s, nullptr, nullptr);
+    launch_units_kv(hk, hv, k, v, n_seqs, 0, tokens, capacity, in_dtype, true, packed_k, packed_v, s, nullptr, nullptr);
     return tq_check_launch("store_layer");
 }
 
