@@ -215,13 +215,13 @@ struct AttnArgs {
     const int64_t *tokens_dev;  // NULL, or where the step's context length is read from (<= tokens, which then is the maximum)
     int n_groups, n_splits, tiles_per_split, n_tiles;
     int q_group, head_off;  // query heads per KV head; first of the heads that this launch's first pass works on
-    int pass_heads;         // heads per pass; blockIdx.y numbers the passes of a launch, whose partials and counters follow each other
     int d256;               // heads of 256 dims: a token is two 128-value rows (2 token + half) of the K and V caches
     int gpw;                // (batch, kv head) groups per workgroup: 1, or wavefronts per workgroup / n_splits when a group's
                             // splits are fewer than a workgroup's wavefronts (short contexts: the groups share the decode tables)
     int gw_shift;           // gpw > 1: log2(n_splits), a power of two then
     int wgs_per_group;      // gpw == 1: n_splits / wavefronts per workgroup
     float tau;
+    int pass_heads;         // heads per pass; blockIdx.y numbers the passes of a launch, whose partials and counters follow each other
 };
 
 constexpr int KFMT_TURBO = 0, KFMT_Q8 = 1;

@@ -2076,71 +2076,64 @@ __device__ __forceinline__ void append_units(const TI *x, uint8_t *packed, const
     if constexpr (KIND == TQ_KIND_K) build_k_fragments(fr, of_quarter(a.s1neg[0], a.s1neg[1], a.s1neg[2], a.s1neg[3]), lane);
     else build_v_fragments(fr, a.s1neg, lane);
     const bool fresh = t >= n_old && t < n_end;
-#pragma unroll
-    for (int i = 0; i < NX; ++i) xb[i] = fresh ? xb[i] : make_uint4(0, 0, 0, 0);
-
     float4_t gram = {0.f, 0.f, 0.f, 0.f};  // of token 4 kq + i: element i of column 4 kq + i
     float ss = 0.0f, rowscale = 1.0f;      // of token n16
-    if constexpr (AS_STORE && F32) {
-        float s0 = 0.0f, s1 = 0.0f;
-#pragma unroll
-        for (int ks = 0; ks < 4; ks += 2) {
-            s0 = sumsq8(xb[2 * ks], xb[2 * ks + 1], s0);
-            s1 = sumsq8(xb[2 * ks + 2], xb[2 * ks + 3], s1);
-        }
-        ss = s0 + s1;
+    // a norm goes over the four lanes that share the token, in short sums: closer than the matrix cores' X X^T (AS_STORE)
+    auto over_lanes = [&] {
         ss += xor_lane<16>(ss);
         ss += xor_lane<32>(ss);
         gram = float4_t{ss, ss, ss, ss};
-        rowscale = row_pow2_scale(__builtin_amdgcn_sqrtf(ss));
-    } else if constexpr (AS_STORE) {
-#pragma unroll
-        for (int ks = 0; ks < 4; ++ks)
-            gram = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8_t, xb[ks]), __builtin_bit_cast(half8_t, xb[ks]), gram, 0, 0, 0);
-    } else {
-        // over the four lanes that share the token, in four short sums: closer than the matrix cores' X X^T
-        float part[4];
-#pragma unroll
-        for (int ks = 0; ks < 4; ++ks) {
-            if constexpr (F32) {
-                part[ks] = sumsq8(xb[2 * ks], xb[2 * ks + 1], 0.0f);
-            } else {
-                const half8_t h = __builtin_bit_cast(half8_t, xb[ks]);
-                part[ks] = 0.0f;
-#pragma unroll
-                for (int e = 0; e < 8; ++e) part[ks] = fmaf((float)h[e], (float)h[e], part[ks]);
-            }
-        }
-        ss = (part[0] + part[1]) + (part[2] + part[3]);
-        ss += xor_lane<16>(ss);
-        ss += xor_lane<32>(ss);
-        gram = float4_t{ss, ss, ss, ss};
-        if constexpr (F32) rowscale = row_pow2_scale(sqrtf(ss));
-    }
+    };
     auto product = [&](half8_t f, half8_t v, float4_t c) {
         return KIND == TQ_KIND_K ? __builtin_amdgcn_mfma_f32_16x16x32_f16(f, v, c, 0, 0, 0) : __builtin_amdgcn_mfma_f32_16x16x32_f16(v, f, c, 0, 0, 0);
     };
     const float4_t none = {0.f, 0.f, 0.f, 0.f};
     float4_t q[2][4];
+    if constexpr (F32) {
+        float part[4];
 #pragma unroll
-    for (int ks = 0; ks < 4; ++ks) {
-        if constexpr (AS_STORE && F32) {
-            half8_t hi, mid;
-            split8(xb[2 * ks], xb[2 * ks + 1], rowscale, hi, mid);
+        for (int i = 0; i < NX; ++i) xb[i] = fresh ? xb[i] : make_uint4(0, 0, 0, 0);
 #pragma unroll
-            for (int h = 0; h < 2; ++h) q[h][ks] = product(fr[h * 4 + ks], hi, product(fr[h * 4 + ks], mid, none));
-        } else if constexpr (F32) {
+        for (int ks = 0; ks < 4; ++ks)  // AS_STORE: two sums of sixteen, the store's
+            part[ks] = sumsq8(xb[2 * ks], xb[2 * ks + 1], AS_STORE && ks >= 2 ? part[ks - 2] : 0.0f);
+        ss = AS_STORE ? part[2] + part[3] : (part[0] + part[1]) + (part[2] + part[3]);
+        over_lanes();
+        rowscale = row_pow2_scale(AS_STORE ? __builtin_amdgcn_sqrtf(ss) : sqrtf(ss));
+#pragma unroll
+        for (int ks = 0; ks < 4; ++ks) {
             half8_t hi, mid, lo;
-            split8(xb[2 * ks], xb[2 * ks + 1], rowscale, hi, mid, lo);
+            if constexpr (AS_STORE) split8(xb[2 * ks], xb[2 * ks + 1], rowscale, hi, mid);
+            else split8(xb[2 * ks], xb[2 * ks + 1], rowscale, hi, mid, lo);
 #pragma unroll
-            for (int h = 0; h < 2; ++h)  // the small terms apart: large ones that cancel leave them whole
-                q[h][ks] = product(fr[h * 4 + ks], hi, none) + product(fr[h * 4 + ks], mid, product(fr[h * 4 + ks], lo, none));
-        } else {
-#pragma unroll
-            for (int h = 0; h < 2; ++h) q[h][ks] = product(fr[h * 4 + ks], __builtin_bit_cast(half8_t, xb[ks]), none);
+            for (int h = 0; h < 2; ++h) {
+                const half8_t f = fr[h * 4 + ks];
+                if constexpr (AS_STORE) q[h][ks] = product(f, hi, product(f, mid, none));
+                else q[h][ks] = product(f, hi, none) + product(f, mid, product(f, lo, none));  // large ones that cancel leave the small ones whole
+            }
         }
+    } else {
+        half8_t xh[4];
+#pragma unroll
+        for (int ks = 0; ks < 4; ++ks) xh[ks] = __builtin_bit_cast(half8_t, fresh ? xb[ks] : make_uint4(0, 0, 0, 0));
+        if constexpr (AS_STORE) {
+#pragma unroll
+            for (int ks = 0; ks < 4; ++ks) gram = __builtin_amdgcn_mfma_f32_16x16x32_f16(xh[ks], xh[ks], gram, 0, 0, 0);
+        } else {
+            float part[4];
+#pragma unroll
+            for (int ks = 0; ks < 4; ++ks) {
+                part[ks] = 0.0f;
+#pragma unroll
+                for (int e = 0; e < 8; ++e) part[ks] = fmaf((float)xh[ks][e], (float)xh[ks][e], part[ks]);
+            }
+            ss = (part[0] + part[1]) + (part[2] + part[3]);
+            over_lanes();
+        }
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+#pragma unroll
+            for (int ks = 0; ks < 4; ++ks) q[h][ks] = product(fr[h * 4 + ks], xh[ks], none);
     }
-
     settle_matrix_results();  // what follows may be compiled to branches
     if constexpr (KIND == TQ_KIND_K) {
         if constexpr (AS_STORE && !F32) {
