@@ -8,7 +8,8 @@
 //                  16 lanes per vector (8 values each): three in-lane stages and
 //                  four DPP row stages; a workgroup owns one 128-token block,
 //                  stages the codes in LDS and writes the block coalesced.
-//   k_store_qjl_mfma  float64 variant that also sketches the residual (1-bit QJL), projection on fp64 MFMAs.
+//   k_append_units, append_units  rows appended to a growing cache and short prompts, a wavefront per 16 tokens.
+//   k_store_qjl_mfma  float64 variant that also sketches the residual (1-bit QJL), projection on fp16 MFMAs.
 //   k_load         packed block -> values (rotated or original domain).
 //   k_unpack_codes packed block -> uint8 indices + fp32 norms.
 //   k_q8_0_store   32-value int8 blocks with fp16 scale, 128-token block layout.
@@ -1993,7 +1994,7 @@ __global__ __launch_bounds__(APPEND_THREADS) void k_append(const TI *x, uint8_t 
 // (5.4 / 5.4 / 6.2e-5).
 // Bound: vector instructions (650 to 1230 for 16 tokens; the butterfly needs about 300 for each four, and its codes go
 // through LDS).  64 x 2048 tokens, K and V: turbo2 35.0 -> 21.0 us, turbo3 45.6 -> 25.8, turbo4 47.3 -> 29.4, 8-bit K with
-// turbo3 V 39.0 -> 26.8 (copies of these bytes: 15 to 18 us).  fp32 rows (copies: 29 us): 41.4 -> 37.0, 47.8 -> 39.6, 54.2 ->
+// turbo3 V 39.0 -> 25.4 (copies of these bytes: 15 to 18 us).  fp32 rows (copies: 29 us): 41.4 -> 37.0, 47.8 -> 39.6, 54.2 ->
 // 43.4 us; shares off, norms over four decades, 2 / 3 / 4 bits: codes 3.5 / 8.0 / 16.9e-8 (butterfly 6.0 / 13.2 / 25.3e-8), norms
 // 4.9 / 5.1 / 5.6e-5 (5.2 / 5.7 / 6.1e-5).
 struct AppendUnitArgs {
@@ -3259,8 +3260,8 @@ int tqk_rotate128(const tq_handle *h, const void *x, void *y, int64_t n, int in_
     DISPATCH_T(in_dtype, TI, return launch_wht128<TI>(x, y, n, out_dtype, sa, sb, s));
 }
 
-// fp16 input with a sign-symmetric codebook: rotation on the matrix cores, codes packed in
-// registers.  The butterfly kernel serves every other case (fp32 / fp64 input, asymmetric codebooks).
+// fp16 and fp32 input with a sign-symmetric codebook: rotation on the matrix cores, codes packed in
+// registers.  The butterfly kernel serves every other case (fp64 input, asymmetric codebooks).
 static bool store_fast_ok(const tq_handle *h, int in_dtype, int64_t n_blocks) {
     return (in_dtype == TQ_F16 || in_dtype == TQ_F32) && h->symmetric && h->bits >= 2 && h->bits <= 4 &&
            (h->bits != 4 || h->quant_lut_ok) && n_blocks < (1ll << 28);
