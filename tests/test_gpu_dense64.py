@@ -51,6 +51,29 @@ def test_dense_products_at_tile_edges(n, d, dtype):
     assert np.all(np.abs(q.dequantize(s, rn) - qo.dequantize(s, rn)) <= 4 * bound(d) * np.sqrt(d) * q.scale * rn[:, None] + 1e-300)
 
 
+# the tile that a launch's workgroups are done first with: 1 x 1 past sixteen vectors (one column block a tile, seven or fewer
+# and more than seven of them; several row groups a workgroup), 1 x 2, 2 x 2 and 2 x 3 with whole and cut tiles on both sides
+@pytest.mark.parametrize("n,d", [(17, 16), (900, 23), (33, 250), (300, 300), (600, 128), (325, 601), (1200, 127), (400, 384), (513, 381),
+                                 (1024, 384), (1023, 200), (2300, 128), (210, 1100), (137, 2048)])
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+def test_dense_products_in_every_tile(n, d, dtype):
+    test_dense_products_at_tile_edges(n, d, dtype)
+
+
+@pytest.mark.parametrize("n,d", [(450, 64), (325, 601), (1000, 383), (256, 1100)])
+def test_tiles_do_not_change_a_vector_s_results(n, d):
+    """A vector's bits are those it has alone, in a single tile."""
+    x = np.random.default_rng(n).standard_normal((n, d))
+    tq = tqa.TurboQuant(d, 3)
+    whole = tq.quantize(x)
+    back = tq.dequantize(whole)
+    for at in (0, 15, 16, n // 2, n - 1):
+        part = tq.quantize(x[at:at + 1])
+        for name in ("mse_indices", "vector_norms", "qjl_signs", "residual_norms"):
+            assert np.array_equal(getattr(part, name), getattr(whole, name)[at:at + 1]), (name, at)
+        assert np.array_equal(tq.dequantize(part), back[at:at + 1])
+
+
 @pytest.mark.parametrize("bits", [1, 5, 8])
 def test_level_search_at_every_width(bits):
     """The level of a value is the number of midpoints below it."""

@@ -8,6 +8,8 @@
 // 128 threads per VB = 8 vectors (4 or 2 for dimensions above 1024 / 2048), in
 // the reference's stage order, which makes the float64 WHT results
 // bit-identical to NumPy's.
+#include <algorithm>
+
 #include "tq_internal.h"
 #include "tq_device64.h"
 
@@ -28,7 +30,7 @@ __device__ __forceinline__ int level_of(double v, const double *bounds, int bits
 // ---- dense products: out[row][j] = sum_k f(in[row][k]) M[k][j], float64 matrix cores -----------------------------
 // One thread per (output, vector) read the whole matrix from L2 once per VB vectors and an LDS operand per multiply:
 // 1.56 ms per product for 256 vectors of 1536 (0.8 of 75 TFLOP/s), 92 us for 32 768 of 128.  Here a wavefront owns RT x
-// CT tiles of 16 x 16 outputs of v_mfma_f64_16x16x4_f64 and a slice of the contraction or all of it: 39 and 39 us.  What
+// CT tiles of 16 x 16 outputs of v_mfma_f64_16x16x4_f64 and a slice of the contraction or all of it: 28 and 39 us.  What
 // bounds it is the matrix instruction (64 clocks; 22 and 20 us of them at the 1.7 GHz the part holds here), then the
 // uneven last round of workgroups.  The order of the contraction is free, so in a chunk of 16 values lane quarter q takes
 // values 4q .. 4q+3 for the chunk's four steps: the A operand of four steps is one vector load, the B operand of a step
@@ -329,20 +331,40 @@ void launch_dense_tiles(DenseArgs a, int slices, hipStream_t s) {
 //   not SPLIT where whole tiles fill the chip - from 1536 tiles of 2 x 2 below 512 dimensions, where a slice is short beside
 //   the exchange of its tiles (32 768 vectors of 128: 55 / 39; 4096 of 384: 50 / 43; 8192 of 128, 1024 tiles: 17 / 22), from
 //   4096 above (4096 of 768, 3072 tiles: 117 / 141; 4096 of 1536, 6144 tiles: equal);
-//   fewer than 256 tiles of 2 x 2: tiles of 1 x 2, so that more CUs get a workgroup (100 of 768: 10.5 against 13.5);
-//   up to 16 vectors: single tiles (one vector of 1536: 8.0 against 11.5; sixteen: 12.7 against 15.3).
+//   up to 16 vectors: single tiles (one vector of 1536: 8.0 against 11.5; sixteen: 12.7 against 15.3);
+//   else the tiles of 1 x 1, 1 x 2, 2 x 2 or 2 x 3 whose workgroups are done first, where the launch takes as long as the CU
+//   with the most of them and a workgroup as long as split_cost's last argument, to scale (a matrix operand is loaded per row
+//   tile and a vector's per column tile, so small tiles cost more than their share).  256 of 1536, 1.5 workgroups of 2 x 2 per
+//   CU or one of 2 x 3: 32.5 to 37.3 / 26.8 to 27.4; 200 of 1536 the same; 1000 of 384: 12.6 to 13.3 / 10.6 to 11.9; 325 of 768,
+//   2 x 2 / 1 x 2: 18.2 / 13.9; 100 of 1536, 1 x 2 / 2 x 2: 21.9 to 25.1 / 19.5 to 20.6; 20 of 1536, 1 x 2 / 1 x 1: 13.6 / 10.6.
+//   Not 1 x 1 or 1 x 2 from the fourth workgroup of a CU on (325 of 1536, 2 x 2 / 1 x 2: 47 / 38 to 49), nor 2 x 3 for less than a
+//   tenth (2300 of 1536: 204 to 235 / 230) or where fewer than eight slices leave a workgroup short (5000 of 100: 12.2 / 12.8).
 // A count of slices that follows the work as well (16 / 8 / 4 / 2 / none) is up to a tenth faster for many vectors (32 768 of
 // 128: 37.9 us, of 256: 106 for 116, 1000 of 1536: 102 for 114) and differs in the last place between a batch and its vectors
 // one by one.
+// Workgroups of rt x ct tiles, shared by `slices` wavefronts each, on the busiest of the 256 CUs (of the 32 of an XCD where the
+// columns are dealt to those), times the time of one; none if they are more than `most`.
+inline int64_t split_cost(const DenseArgs &a, int slices, int rt, int ct, int64_t most, int cost) {
+    const int64_t rows = 8 / slices * rt * 16, n_row = (a.n + rows - 1) / rows, n_col = (a.d + 16 * ct - 1) / (16 * ct);
+    const int64_t wgs = n_col >= 8 ? (n_row * ((n_col + 7) / 8) + 31) / 32 : (n_row * n_col + 255) / 256;
+    return wgs > most ? INT64_MAX : wgs * cost;
+}
+
 template <DenseOp OP, typename TI, typename TO>
 int launch_dense(const DenseArgs &a, const char *what, hipStream_t s) {
     const int64_t tiles = ((a.n + 31) / 32) * ((a.d + 31) / 32);
     int slices = 8;
     while (slices > 1 && 16 * slices > a.d) slices >>= 1;
-    if (a.n <= 16) launch_dense_tiles<OP, TI, TO, 1, 1, true>(a, slices, s);
-    else if (tiles < 256) launch_dense_tiles<OP, TI, TO, 1, 2, true>(a, slices, s);
-    else if (slices == 1 || tiles < (a.d < 512 ? 1536 : 4096)) launch_dense_tiles<OP, TI, TO, 2, 2, true>(a, slices, s);
-    else launch_dense_tiles<OP, TI, TO, 2, 2, false>(a, slices, s);
+    if (slices > 1 && tiles >= (a.d < 512 ? 1536 : 4096)) {
+        launch_dense_tiles<OP, TI, TO, 2, 2, false>(a, slices, s);
+        return tq_check_launch(what);
+    }
+    const int64_t c11 = split_cost(a, slices, 1, 1, 3, 63), c12 = split_cost(a, slices, 1, 2, 3, 88),
+                  c22 = split_cost(a, slices, 2, 2, INT64_MAX, 145), c23 = split_cost(a, slices, 2, 3, slices == 8 ? INT64_MAX : 0, 245);
+    if (a.n <= 16 || c11 < std::min({c12, c22, c23})) launch_dense_tiles<OP, TI, TO, 1, 1, true>(a, slices, s);
+    else if (c12 < std::min(c22, c23)) launch_dense_tiles<OP, TI, TO, 1, 2, true>(a, slices, s);
+    else if (c22 <= c23) launch_dense_tiles<OP, TI, TO, 2, 2, true>(a, slices, s);
+    else launch_dense_tiles<OP, TI, TO, 2, 3, true>(a, slices, s);
     return tq_check_launch(what);
 }
 
