@@ -1,6 +1,8 @@
 """Appends whose first and last token fall on, before and behind the edges of the append kernels' units: the 16-token
 groups of a V tile (a thread per row and group), the four tokens of a 16-lane row, the 128-token block.  The oracle is the
 store of the whole sequence with the same arithmetic (float64 rows for the turbo formats), byte for byte."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -247,3 +249,36 @@ def test_codebooks_that_the_matrix_cores_do_not_take(dtype, which):
         mid = (codec.centroids[1:] + codec.centroids[:-1]) / 2
         lo, hi = ((mid[None, None] < (y + e)[..., None]).sum(-1) for e in (-1e-6, 1e-6))
         assert ((idx >= lo) & (idx <= hi)).all()
+
+
+def launches(call):
+    """Kernels of a call, as the nodes of its captured graph."""
+    tt = L.torch()
+    call()
+    graph = tt.cuda.CUDAGraph(keep_graph=True)
+    with tt.cuda.graph(graph):
+        call()
+    n = C.c_size_t(0)
+    assert L.lib().hipGraphGetNodes(C.c_void_p(graph.raw_cuda_graph()), None, C.byref(n)) == 0
+    return n.value
+
+
+@pytest.mark.parametrize("dtype", ["float16", "float32", "float64"])
+@pytest.mark.parametrize("pair", [(2, 2), (3, 3), (4, 4), (4, 2), (4, 3), (3, 2)])
+@pytest.mark.parametrize("asymmetric", ["", "k", "v", "kv"])
+def test_a_step_is_one_launch(asymmetric, pair, dtype):
+    """Whichever codebooks of a layer the matrix cores take: K and V are appended in one launch, with the bytes of an append
+    per side."""
+    tt = L.torch()
+    cent = {b: np.sort(np.random.default_rng(2).uniform(-0.25, 0.3, 1 << b)) for b in pair}
+    kc, vc = (tqa.TurboCodec(b, seed=s, centroids=cent[b] if side in asymmetric else None) for b, s, side in zip(pair, (3, 503), "kv"))
+    k, v = (tt.randn((N_SEQS, 200, D), generator=tt.Generator("cuda").manual_seed(s), device="cuda").to(getattr(tt, dtype)) for s in (1, 2))
+    one, two = ([tt.zeros(tqa.packed_bytes(b, N_SEQS, CAPACITY), dtype=tt.uint8, device="cuda") for b in pair] for _ in range(2))
+    for pos, n_new in ((0, 200), (200, 1), (201, 70)):
+        kn, vn = k[:, :n_new].contiguous(), v[:, :n_new].contiguous()
+        assert launches(lambda: kc.append_kv(vc, kn, vn, *one, pos, CAPACITY)) == 1
+        kc.append_kv(vc, kn, vn, *one, pos, CAPACITY)
+        kc.append(kn, two[0], pos, CAPACITY, kind="k")
+        vc.append(vn, two[1], pos, CAPACITY, kind="v")
+        for a, b in zip(one, two):
+            assert tt.equal(a, b), (pos, n_new)

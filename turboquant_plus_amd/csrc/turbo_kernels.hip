@@ -4420,43 +4420,41 @@ static AppendUnitArgs make_append_unit_args(const tq_handle *h, int64_t pos, con
     return u;
 }
 
-// The widths that have a kernel for K and V in one launch (0: q8_0-style rows); U: 0, or what append_side says is added to a
-// turbo side.  `one_launch` becomes false where there is none (turbo V wider than turbo K).
+// The widths that have a kernel for K and V in one launch (0: q8_0-style rows); UK, UV: 0, or what append_side says is added to
+// a turbo side.  `one_launch` becomes false where there is none (turbo V wider than turbo K).
 #define TQ_APPEND_KV(KB, VB, TI, KA, VA)                                                                                     \
     k_append_kv<KB, VB, TI><<<grid, APPEND_THREADS, 0, s>>>((const TI *)k, (uint8_t *)packed_k, KA, (const TI *)v, (uint8_t *)packed_v, VA)
-#define TQ_APPEND_PAIRS(U, TI)                                              \
+#define TQ_APPEND_PAIRS(UK, UV, TI, KA, VA)                                 \
     switch (8 * kb + vb) {                                                  \
-    case 8 * 3 + 3: TQ_APPEND_KV(U + 3, U + 3, TI, ka, va); break;          \
-    case 8 * 4 + 4: TQ_APPEND_KV(U + 4, U + 4, TI, ka, va); break;          \
-    case 8 * 2 + 2: TQ_APPEND_KV(U + 2, U + 2, TI, ka, va); break;          \
-    case 8 * 4 + 2: TQ_APPEND_KV(U + 4, U + 2, TI, ka, va); break;          \
-    case 8 * 3 + 2: TQ_APPEND_KV(U + 3, U + 2, TI, ka, va); break;          \
-    case 8 * 4 + 3: TQ_APPEND_KV(U + 4, U + 3, TI, ka, va); break;          \
-    case 2: TQ_APPEND_KV(0, U + 2, TI, qk, va); break;                      \
-    case 3: TQ_APPEND_KV(0, U + 3, TI, qk, va); break;                      \
-    case 4: TQ_APPEND_KV(0, U + 4, TI, qk, va); break;                      \
-    case 8 * 2: TQ_APPEND_KV(U + 2, 0, TI, ka, qv); break;                  \
-    case 8 * 3: TQ_APPEND_KV(U + 3, 0, TI, ka, qv); break;                  \
-    case 8 * 4: TQ_APPEND_KV(U + 4, 0, TI, ka, qv); break;                  \
+    case 8 * 3 + 3: TQ_APPEND_KV(UK + 3, UV + 3, TI, KA, VA); break;        \
+    case 8 * 4 + 4: TQ_APPEND_KV(UK + 4, UV + 4, TI, KA, VA); break;        \
+    case 8 * 2 + 2: TQ_APPEND_KV(UK + 2, UV + 2, TI, KA, VA); break;        \
+    case 8 * 4 + 2: TQ_APPEND_KV(UK + 4, UV + 2, TI, KA, VA); break;        \
+    case 8 * 3 + 2: TQ_APPEND_KV(UK + 3, UV + 2, TI, KA, VA); break;        \
+    case 8 * 4 + 3: TQ_APPEND_KV(UK + 4, UV + 3, TI, KA, VA); break;        \
+    case 2: TQ_APPEND_KV(0, UV + 2, TI, qk, VA); break;                     \
+    case 3: TQ_APPEND_KV(0, UV + 3, TI, qk, VA); break;                     \
+    case 4: TQ_APPEND_KV(0, UV + 4, TI, qk, VA); break;                     \
+    case 8 * 2: TQ_APPEND_KV(UK + 2, 0, TI, KA, qv); break;                 \
+    case 8 * 3: TQ_APPEND_KV(UK + 3, 0, TI, KA, qv); break;                 \
+    case 8 * 4: TQ_APPEND_KV(UK + 4, 0, TI, KA, qv); break;                 \
     default: one_launch = false;                                            \
     }
 
-// K and V through append_units (both turbo sides fit for it, one at least); false: no kernel for this pair
-static bool launch_units_kv(const tq_handle *hk, const tq_handle *hv, const void *k, const void *v, int64_t n_seqs, int64_t pos,
-                            int64_t n_new, int64_t capacity, int in_dtype, bool as_store, void *packed_k, void *packed_v, hipStream_t s,
-                            const int64_t *pos_dev, uint32_t *overrun) {
-    const Q8AppendArgs qk = make_q8_append_args(k, pos, pos_dev, n_new, capacity, pos_dev ? overrun : nullptr);
-    const Q8AppendArgs qv = make_q8_append_args(v, pos, pos_dev, n_new, capacity, nullptr);  // the K half reports
-    AppendUnitArgs ka{}, va{};
-    if (hk) ka = make_append_unit_args(hk, pos, pos_dev, n_new, capacity, overrun);
-    if (hv) va = make_append_unit_args(hv, pos, pos_dev, n_new, capacity, nullptr);
+// A prompt's K and V through append_units with the bytes of tq_store (both turbo sides fit for it, one at least); false: no
+// kernel for this pair
+static bool launch_prompt_units(const tq_handle *hk, const tq_handle *hv, const void *k, const void *v, int64_t n_seqs, int64_t tokens,
+                                int64_t capacity, int in_dtype, void *packed_k, void *packed_v, hipStream_t s) {
+    const Q8AppendArgs qk = make_q8_append_args(k, 0, nullptr, tokens, capacity, nullptr);
+    const Q8AppendArgs qv = make_q8_append_args(v, 0, nullptr, tokens, capacity, nullptr);
+    AppendUnitArgs uk{}, uv{};
+    if (hk) uk = make_append_unit_args(hk, 0, nullptr, tokens, capacity, nullptr);
+    if (hv) uv = make_append_unit_args(hv, 0, nullptr, tokens, capacity, nullptr);
     const unsigned grid = 2u * (unsigned)(n_seqs * qk.n_touched);
     const int kb = hk ? hk->bits : 0, vb = hv ? hv->bits : 0;
     bool one_launch = true;
-    if (as_store && in_dtype == TQ_F32) TQ_APPEND_PAIRS(UNITS_AS_STORE, float)
-    else if (as_store) TQ_APPEND_PAIRS(UNITS_AS_STORE, __half)
-    else if (in_dtype == TQ_F32) TQ_APPEND_PAIRS(UNITS, float)
-    else TQ_APPEND_PAIRS(UNITS, __half)
+    if (in_dtype == TQ_F32) TQ_APPEND_PAIRS(UNITS_AS_STORE, UNITS_AS_STORE, float, uk, uv)
+    else TQ_APPEND_PAIRS(UNITS_AS_STORE, UNITS_AS_STORE, __half, uk, uv)
     return one_launch;
 }
 
@@ -4466,25 +4464,35 @@ int tqk_append_kv(const tq_handle *hk, const tq_handle *hv, const void *k, const
                   const int64_t *pos_dev, uint32_t *overrun) {
     if (n_seqs == 0 || n_new == 0) return TQ_OK;
     const int kb = hk ? hk->bits : 0, vb = hv ? hv->bits : 0;
-    const bool ku = hk && append_units_ok(hk, in_dtype), vu = hv && append_units_ok(hv, in_dtype);
+    const bool ku = !hk || append_units_ok(hk, in_dtype), vu = !hv || append_units_ok(hv, in_dtype);
+    const Q8AppendArgs qk = make_q8_append_args(k, pos, pos_dev, n_new, capacity, pos_dev ? overrun : nullptr);
+    const Q8AppendArgs qv = make_q8_append_args(v, pos, pos_dev, n_new, capacity, nullptr);  // the K half reports
+    AppendArgs ka{}, va{};
+    AppendUnitArgs uk{}, uv{};
+    if (hk && ku) uk = make_append_unit_args(hk, pos, pos_dev, n_new, capacity, overrun);
+    else if (hk) ka = make_append_args(hk, pos, pos_dev, n_new, capacity, TQ_KIND_K, overrun);
+    if (hv && vu) uv = make_append_unit_args(hv, pos, pos_dev, n_new, capacity, nullptr);
+    else if (hv) va = make_append_args(hv, pos, pos_dev, n_new, capacity, TQ_KIND_V);
+    const unsigned grid = 2u * (unsigned)(n_seqs * qk.n_touched);
     bool one_launch = true;
-    if ((ku || vu) && (ku || !hk) && (vu || !hv)) {
-        one_launch = launch_units_kv(hk, hv, k, v, n_seqs, pos, n_new, capacity, in_dtype, false, packed_k, packed_v, s, pos_dev, overrun);
-    } else if (ku || vu) {
-        one_launch = false;  // one side's codebook is for the butterfly
+    // Every side as in an append of its own, in one launch also where the matrix cores take only one of two codebooks (kernels, us,
+    // 3-bit fp16 rows, asymmetric K: a launch per side / one: 8 x 1 token 8.8 / 5.2, 32 x 512 13.9 / 9.0, 64 x 2048 39.1 / 35.6;
+    // both sides on the butterfly 5.9, 10.1, 44.3).
+#define TQ_APPEND_SIDES(TI)                                        \
+    if (ku && vu) TQ_APPEND_PAIRS(UNITS, UNITS, TI, uk, uv)        \
+    else if (ku) TQ_APPEND_PAIRS(UNITS, 0, TI, uk, va)             \
+    else if (vu) TQ_APPEND_PAIRS(0, UNITS, TI, ka, uv)             \
+    else TQ_APPEND_PAIRS(0, 0, TI, ka, va)
+    if (!hk && !hv) {
+        DISPATCH_T(in_dtype, TI, (TQ_APPEND_KV(0, 0, TI, qk, qv)));
+    } else if (in_dtype == TQ_F16) {
+        TQ_APPEND_SIDES(__half)
+    } else if (in_dtype == TQ_F32) {
+        TQ_APPEND_SIDES(float)
     } else {
-        const Q8AppendArgs qk = make_q8_append_args(k, pos, pos_dev, n_new, capacity, pos_dev ? overrun : nullptr);
-        const Q8AppendArgs qv = make_q8_append_args(v, pos, pos_dev, n_new, capacity, nullptr);
-        AppendArgs ka{}, va{};
-        if (hk) ka = make_append_args(hk, pos, pos_dev, n_new, capacity, TQ_KIND_K, overrun);
-        if (hv) va = make_append_args(hv, pos, pos_dev, n_new, capacity, TQ_KIND_V);
-        const unsigned grid = 2u * (unsigned)(n_seqs * qk.n_touched);
-        if (!hk && !hv) {
-            DISPATCH_T(in_dtype, TI, (TQ_APPEND_KV(0, 0, TI, qk, qv)));
-        } else {
-            DISPATCH_T(in_dtype, TI, TQ_APPEND_PAIRS(0, TI));
-        }
+        DISPATCH_T(in_dtype, TI, TQ_APPEND_PAIRS(0, 0, TI, ka, va));
     }
+#undef TQ_APPEND_SIDES
     if (!one_launch) {
         if (!hk || !hv) { tq_set_error("tq_append_layer: bits must be 2, 3 or 4 (got %d and %d)", kb, vb); return TQ_ERR_UNSUPPORTED; }
         const int rc = tqk_append(hk, k, n_seqs, pos, n_new, capacity, in_dtype, TQ_KIND_K, packed_k, s, pos_dev, overrun);
@@ -4550,7 +4558,7 @@ int tqk_store_kv(const tq_handle *hk, const tq_handle *hv, const void *k, const 
         return rc ? rc : tqk_store(hv, v, n_seqs, tokens, in_dtype, TQ_KIND_V, packed_v, nullptr, nullptr, s);
     }
     if (n_blocks <= SHORT_PROMPT_BLOCKS &&
-        launch_units_kv(hk, hv, k, v, n_seqs, 0, tokens, out_bps * TQ_ROWS_PER_BLOCK, in_dtype, true, packed_k, packed_v, s, nullptr, nullptr))
+        launch_prompt_units(hk, hv, k, v, n_seqs, tokens, out_bps * TQ_ROWS_PER_BLOCK, in_dtype, packed_k, packed_v, s))
         return tq_check_launch("store_kv (short)");
     StoreKArgs ka = make_k_args(hk, tokens, bps, n_blocks);
     StoreVArgs va = make_v_args(hv, tokens, bps, n_blocks);
@@ -4616,7 +4624,7 @@ int tqk_store_layer(const tq_handle *hk, const tq_handle *hv, const void *k, con
     const int64_t n_blocks = n_seqs * blocks_for(tokens), out_bps = blocks_for(capacity);
     if (!h || in_dtype != TQ_F16 || n_blocks < AS_STORE_BLOCKS || !store_fast_ok(h, in_dtype, n_blocks) || out_bps * n_seqs >= (1ll << 28))
         return tqk_append_kv(hk, hv, k, v, n_seqs, 0, tokens, capacity, in_dtype, packed_k, packed_v, s);
-    launch_units_kv(hk, hv, k, v, n_seqs, 0, tokens, capacity, in_dtype, true, packed_k, packed_v, s, nullptr, nullptr);
+    launch_prompt_units(hk, hv, k, v, n_seqs, tokens, capacity, in_dtype, packed_k, packed_v, s);
     return tq_check_launch("store_layer");
 }
 
