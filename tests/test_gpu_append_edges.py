@@ -282,3 +282,28 @@ def test_a_step_is_one_launch(asymmetric, pair, dtype):
         vc.append(vn, two[1], pos, CAPACITY, kind="v")
         for a, b in zip(one, two):
             assert tt.equal(a, b), (pos, n_new)
+
+
+@pytest.mark.parametrize("fmt", [("q8_0", "turbo2"), ("q8_0", "turbo3"), ("q8_0", "turbo4"), ("turbo2", "q8_0"), ("turbo3", "q8_0"),
+                                 ("turbo4", "q8_0")])
+@pytest.mark.parametrize("blocks", [2047, 2048, 3583, 3584])
+def test_long_prompt_of_a_layer_with_8_bit_rows(fmt, blocks):
+    """The 8-bit side and the turbo side of a long prompt take a launch each from the lengths on where that is the faster, and
+    the bytes of a store per side in either way, into caches with room behind them."""
+    tt = L.torch()
+    layer = tqa.LayerKV(tqa.LayerFormat(*fmt))
+    n, per = next((blocks // m, m) for m in (32, 89, 3583) if blocks % m == 0)
+    tokens, capacity = 128 * per - 3, 128 * (per + 1)
+    gen = tt.Generator("cuda").manual_seed(blocks)
+    k, v = (tt.randn((n, tokens, D), generator=gen, device="cuda", dtype=tt.float16) for _ in range(2))
+    caches = [b.fill_(0xA5) for b in layer.new_cache(n, capacity)]
+    bits = int(max(fmt)[-1])
+    assert launches(lambda: layer.prefill(k, v, *caches, capacity)) == (2 if bits == 4 and blocks >= 2048 or bits == 3 and blocks >= 3584 else 1)
+    for b in caches:
+        b.fill_(0xA5)
+    layer.prefill(k, v, *caches, capacity)
+    for codec, x, cache, kind in ((layer.k_codec, k, caches[0], "k"), (layer.v_codec, v, caches[1], "v")):
+        want = tqa.q8_0_store(x, kind=kind)[0] if codec is None else codec.store(x, kind=kind)
+        got = cache.view(n, per + 1, -1)
+        assert tt.equal(got[:, :per], want.view(n, per, -1)), kind
+        assert bool((got[:, per:] == 0xA5).all()), kind

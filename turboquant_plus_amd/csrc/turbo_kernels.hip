@@ -4610,13 +4610,16 @@ int tqk_store_kv(const tq_handle *hk, const tq_handle *hv, const void *k, const 
     return tq_check_launch("store_kv");
 }
 
-// Prompt of a layer of any two formats (hk / hv NULL: q8_0-style rows) into caches laid out for `capacity` tokens, one launch.
+// Prompt of a layer of any two formats (hk / hv NULL: q8_0-style rows) into caches laid out for `capacity` tokens.
 // fp16 rows of a long prompt (512 blocks) have the turbo side's bytes from tq_store's arithmetic, all others from the
 // append's (fp32 rows at every length: tq_store's two fp16 terms drop what lies below 2^-22 of a value).
-// (Two launches, the 8-bit side's append and the persistent store, took (kernels, us; 8-bit K with turbo3 V, fp16) 21.0 for 528
-// blocks, 23.2 for 752 and 44.5 for 2048; in one launch 13.9, 16.4 and 40.7; turbo4 V 22.4, 24.8 and 46.4 against 15.5, 18.0 and
-// 44.8; turbo3 K with 8-bit V 16.7, 19.4 and 42.2 against 12.5, 15.7 and 38.2.)
+// One launch of the units, whose K and V workgroups overlap, or two, the 8-bit side's append and the persistent store, whose
+// units cost fewer vector instructions (the table of 4-bit levels most of all) and whose second launch is paid once.  Layers, us,
+// one / two launches, 8-bit K, then 8-bit V: turbo4 1536 blocks 40.5 / 40.5, 36.8 / 36.8, 2048 52.8 / 52.0, 50.3 / 47.7, 4096 95.6 /
+// 89.7, 91.5 / 82.4, 16384 321 / 289, 313 / 278; turbo3 2048 47.7 / 49.4, 44.5 / 46.1, 3072 67.8 / 67.6, 64.2 / 63.2, 3584 78.9 / 75.8,
+// 74.9 / 72.3, 12288 223 / 224, 216 / 207; turbo2 4096 73.4 / 79.6, 67.9 / 71.9, 16384 262 / 287, 261 / 260.
 constexpr int64_t AS_STORE_BLOCKS = 512;
+static int64_t two_launch_blocks(int bits) { return bits == 4 ? 2048 : bits == 3 ? 3584 : INT64_MAX; }
 int tqk_store_layer(const tq_handle *hk, const tq_handle *hv, const void *k, const void *v, int64_t n_seqs, int64_t tokens,
                     int64_t capacity, int in_dtype, void *packed_k, void *packed_v, hipStream_t s) {
     if (hk && hv) return tqk_store_kv(hk, hv, k, v, n_seqs, tokens, capacity, in_dtype, packed_k, packed_v, s);
@@ -4624,8 +4627,15 @@ int tqk_store_layer(const tq_handle *hk, const tq_handle *hv, const void *k, con
     const int64_t n_blocks = n_seqs * blocks_for(tokens), out_bps = blocks_for(capacity);
     if (!h || in_dtype != TQ_F16 || n_blocks < AS_STORE_BLOCKS || !store_fast_ok(h, in_dtype, n_blocks) || out_bps * n_seqs >= (1ll << 28))
         return tqk_append_kv(hk, hv, k, v, n_seqs, 0, tokens, capacity, in_dtype, packed_k, packed_v, s);
-    launch_prompt_units(hk, hv, k, v, n_seqs, tokens, capacity, in_dtype, packed_k, packed_v, s);
-    return tq_check_launch("store_layer");
+    if (n_blocks < two_launch_blocks(h->bits)) {
+        launch_prompt_units(hk, hv, k, v, n_seqs, tokens, capacity, in_dtype, packed_k, packed_v, s);
+        return tq_check_launch("store_layer");
+    }
+    const int rc = hk ? tqk_q8_0_append(v, n_seqs, 0, tokens, capacity, in_dtype, TQ_KIND_V, packed_v, s, nullptr, nullptr)
+                      : tqk_q8_0_append(k, n_seqs, 0, tokens, capacity, in_dtype, TQ_KIND_K, packed_k, s, nullptr, nullptr);
+    if (rc) return rc;
+    return hk ? store_one(hk, k, n_seqs, tokens, out_bps, in_dtype, TQ_KIND_K, packed_k, s)
+              : store_one(hv, v, n_seqs, tokens, out_bps, in_dtype, TQ_KIND_V, packed_v, s);
 }
 
 // K and V of a layer to fp16 in the original domain.  One launch when both handles hold the fragments of the

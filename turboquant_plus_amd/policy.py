@@ -140,8 +140,8 @@ class LayerKV:
     def prefill(self, k, v, k_cache, v_cache, capacity: int):
         """The prompt's K and V [n_seqs, tokens, 128] into caches laid out for `capacity` tokens, from position 0:
         turbo K with turbo V through the fused store (TurboCodec.store_kv(capacity=...), the matrix-core kernels for
-        fp16 and fp32 rows), layers with 8-bit rows in one launch of the append kernel (a long prompt's turbo side in fp16
-        has the fused store's bytes there)."""
+        fp16 and fp32 rows), layers with 8-bit rows in one launch of the append kernel, the turbo side of a long fp16 prompt with
+        the fused store's bytes and, where that is the faster, in a launch of its own."""
         if self.k_codec is not None and self.v_codec is not None:
             self.k_codec.store_kv(self.v_codec, k, v, out_k=k_cache, out_v=v_cache, capacity=capacity)
             return k_cache, v_cache
