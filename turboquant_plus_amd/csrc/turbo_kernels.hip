@@ -4424,14 +4424,16 @@ static AppendUnitArgs make_append_unit_args(const tq_handle *h, int64_t pos, con
 // a turbo side.  `one_launch` becomes false where there is none (turbo V wider than turbo K).
 #define TQ_APPEND_KV(KB, VB, TI, KA, VA)                                                                                     \
     k_append_kv<KB, VB, TI><<<grid, APPEND_THREADS, 0, s>>>((const TI *)k, (uint8_t *)packed_k, KA, (const TI *)v, (uint8_t *)packed_v, VA)
-#define TQ_APPEND_PAIRS(UK, UV, TI, KA, VA)                                 \
-    switch (8 * kb + vb) {                                                  \
+#define TQ_TURBO_PAIRS(UK, UV, TI, KA, VA)                                  \
     case 8 * 3 + 3: TQ_APPEND_KV(UK + 3, UV + 3, TI, KA, VA); break;        \
     case 8 * 4 + 4: TQ_APPEND_KV(UK + 4, UV + 4, TI, KA, VA); break;        \
     case 8 * 2 + 2: TQ_APPEND_KV(UK + 2, UV + 2, TI, KA, VA); break;        \
     case 8 * 4 + 2: TQ_APPEND_KV(UK + 4, UV + 2, TI, KA, VA); break;        \
     case 8 * 3 + 2: TQ_APPEND_KV(UK + 3, UV + 2, TI, KA, VA); break;        \
-    case 8 * 4 + 3: TQ_APPEND_KV(UK + 4, UV + 3, TI, KA, VA); break;        \
+    case 8 * 4 + 3: TQ_APPEND_KV(UK + 4, UV + 3, TI, KA, VA); break;
+#define TQ_APPEND_PAIRS(UK, UV, TI, KA, VA)                                 \
+    switch (8 * kb + vb) {                                                  \
+    TQ_TURBO_PAIRS(UK, UV, TI, KA, VA)                                      \
     case 2: TQ_APPEND_KV(0, UV + 2, TI, qk, VA); break;                     \
     case 3: TQ_APPEND_KV(0, UV + 3, TI, qk, VA); break;                     \
     case 4: TQ_APPEND_KV(0, UV + 4, TI, qk, VA); break;                     \
@@ -4441,8 +4443,8 @@ static AppendUnitArgs make_append_unit_args(const tq_handle *h, int64_t pos, con
     default: one_launch = false;                                            \
     }
 
-// A prompt's K and V through append_units with the bytes of tq_store (both turbo sides fit for it, one at least); false: no
-// kernel for this pair
+// A prompt's K and V through append_units with the bytes of tq_store (both turbo sides fit for it, one at least; fp32 rows:
+// both); false: no kernel for this pair
 static bool launch_prompt_units(const tq_handle *hk, const tq_handle *hv, const void *k, const void *v, int64_t n_seqs, int64_t tokens,
                                 int64_t capacity, int in_dtype, void *packed_k, void *packed_v, hipStream_t s) {
     const Q8AppendArgs qk = make_q8_append_args(k, 0, nullptr, tokens, capacity, nullptr);
@@ -4453,8 +4455,12 @@ static bool launch_prompt_units(const tq_handle *hk, const tq_handle *hv, const 
     const unsigned grid = 2u * (unsigned)(n_seqs * qk.n_touched);
     const int kb = hk ? hk->bits : 0, vb = hv ? hv->bits : 0;
     bool one_launch = true;
-    if (in_dtype == TQ_F32) TQ_APPEND_PAIRS(UNITS_AS_STORE, UNITS_AS_STORE, float, uk, uv)
-    else TQ_APPEND_PAIRS(UNITS_AS_STORE, UNITS_AS_STORE, __half, uk, uv)
+    if (in_dtype == TQ_F32) {
+        switch (8 * kb + vb) {
+        TQ_TURBO_PAIRS(UNITS_AS_STORE, UNITS_AS_STORE, float, uk, uv)
+        default: one_launch = false;
+        }
+    } else TQ_APPEND_PAIRS(UNITS_AS_STORE, UNITS_AS_STORE, __half, uk, uv)
     return one_launch;
 }
 
@@ -4501,6 +4507,7 @@ int tqk_append_kv(const tq_handle *hk, const tq_handle *hv, const void *k, const
     return tq_check_launch("append_kv");
 }
 #undef TQ_APPEND_PAIRS
+#undef TQ_TURBO_PAIRS
 #undef TQ_APPEND_KV
 
 int tqk_append(const tq_handle *h, const void *x, int64_t n_seqs, int64_t pos, int64_t n_new, int64_t capacity, int in_dtype,
@@ -4628,8 +4635,9 @@ int tqk_store_layer(const tq_handle *hk, const tq_handle *hv, const void *k, con
     if (!h || in_dtype != TQ_F16 || n_blocks < AS_STORE_BLOCKS || !store_fast_ok(h, in_dtype, n_blocks) || out_bps * n_seqs >= (1ll << 28))
         return tqk_append_kv(hk, hv, k, v, n_seqs, 0, tokens, capacity, in_dtype, packed_k, packed_v, s);
     if (n_blocks < two_launch_blocks(h->bits)) {
-        launch_prompt_units(hk, hv, k, v, n_seqs, tokens, capacity, in_dtype, packed_k, packed_v, s);
-        return tq_check_launch("store_layer");
+        if (launch_prompt_units(hk, hv, k, v, n_seqs, tokens, capacity, in_dtype, packed_k, packed_v, s)) return tq_check_launch("store_layer");
+        tq_set_error("tq_store_layer: bits must be 2, 3 or 4 (got %d)", h->bits);
+        return TQ_ERR_UNSUPPORTED;
     }
     const int rc = hk ? tqk_q8_0_append(v, n_seqs, 0, tokens, capacity, in_dtype, TQ_KIND_V, packed_v, s, nullptr, nullptr)
                       : tqk_q8_0_append(k, n_seqs, 0, tokens, capacity, in_dtype, TQ_KIND_K, packed_k, s, nullptr, nullptr);
