@@ -487,6 +487,11 @@ __device__ __forceinline__ float row_pow2_scale(float norm) {
     const uint32_t se = 263u - e;                              // 2^(9 - (e - 127)), biased
     return (e == 0u || e == 255u) ? 1.0f : __uint_as_float((se > 254u ? 254u : se) << 23);
 }
+// row_pow2_scale(sqrtf(ss)) without the root, which never carries ss to the next power of four
+__device__ __forceinline__ float row_pow2_scale_of_square(float ss) {
+    const int e = __builtin_amdgcn_frexp_expf(ss);  // ss = f 2^e, 1/2 <= f < 1
+    return ss > 0.0f && ss < INFINITY ? __uint_as_float((uint32_t)(136 - ((e - 1) >> 1)) << 23) : 1.0f;
+}
 __device__ __forceinline__ float pow2_reciprocal(float p) { return __uint_as_float(0x7F000000u - __float_as_uint(p)); }  // p = 2^k, |k| < 127
 // eight consecutive fp32 inputs (two 16-byte pieces) times sc -> their hi and mid terms as MFMA operands
 __device__ __forceinline__ void split8(uint4 a, uint4 b, float sc, half8_t &hi, half8_t &mid) {
@@ -650,7 +655,8 @@ __device__ __forceinline__ float k_unit_codes(const float4_t (&q)[2][4], float s
     constexpr bool EXACT = LUT == LUT_NONE, NORMALISED = BITS == 4 && !EXACT;
     // root of 1 ulp: scales boundaries (1e-7 relative) and the stored fp16 norm
     const float norm = EXACT ? sqrtf(ss) : __builtin_amdgcn_sqrtf(ss);
-    const float scale = norm > 0.0f ? (EXACT ? sqrtf(128.0f * (ss * rowscale * rowscale)) : norm * rowscale * 11.313708498984761f) : 1.0f;  // y' = sqrt(128) ||x|| y
+    // y' = sqrt(128) ||x|| y; the root behind the choice, or it becomes a branch
+    const float scale = EXACT ? sqrtf(norm > 0.0f ? 128.0f * (ss * rowscale * rowscale) : 1.0f) : norm > 0.0f ? norm * rowscale * 11.313708498984761f : 1.0f;
     float thr[NT];
 #pragma unroll
     for (int k = 0; k < NT; ++k) thr[k] = EXACT ? fmaf(thr0[k], scale, thr_lo[k] * scale) : thr0[k] * scale;
@@ -1135,12 +1141,13 @@ __device__ __forceinline__ float v_subtile_codes(const float4_t (&qq)[2][4], con
         const float ss = row16_sum(n16 == 4 * kq + i ? gram[i] : 0.0f);
         nrm[i] = EXACT ? ss : __builtin_amdgcn_sqrtf(ss);
         const bool nz = ss > 0.0f;
-        const float rowscale = F32 ? row_pow2_scale(EXACT ? sqrtf(ss) : nrm[i]) : 1.0f;  // the power of two the token's fp32 row was multiplied by
+        // the power of two the token's fp32 row was multiplied by
+        const float rowscale = !F32 ? 1.0f : EXACT ? row_pow2_scale_of_square(ss) : row_pow2_scale(nrm[i]);
         if constexpr (NORMALISED) {
             inv[i] = nz ? __builtin_amdgcn_rsqf(ss) * (0.08838834764831845f * pow2_reciprocal(rowscale)) : 1.0f;  // 1 / (||x|| sqrt(128))
         } else {
             inv[i] = 1.0f;
-            const float scale = nz ? (EXACT ? sqrtf(128.0f * (ss * rowscale * rowscale)) : nrm[i] * rowscale * 11.313708498984761f) : 1.0f;
+            const float scale = EXACT ? sqrtf(nz ? 128.0f * (ss * rowscale * rowscale) : 1.0f) : nz ? nrm[i] * rowscale * 11.313708498984761f : 1.0f;
 #pragma unroll
             for (int k = 0; k < NT; ++k) thr_tok[i][k] = EXACT ? fmaf(thr0[k], scale, thr_lo[k] * scale) : thr0[k] * scale;
         }
@@ -1996,7 +2003,9 @@ __global__ __launch_bounds__(APPEND_THREADS) void k_append(const TI *x, uint8_t 
 // through LDS).  64 x 2048 tokens, K and V: turbo2 35.0 -> 21.0 us, turbo3 45.6 -> 25.8, turbo4 47.3 -> 29.4, 8-bit K with
 // turbo3 V 39.0 -> 25.4 (copies of these bytes: 15 to 18 us).  fp32 rows (copies: 29 us): 41.4 -> 37.0, 47.8 -> 39.6, 54.2 ->
 // 43.4 us; shares off, norms over four decades, 2 / 3 / 4 bits: codes 3.5 / 8.0 / 16.9e-8 (butterfly 6.0 / 13.2 / 25.3e-8), norms
-// 4.9 / 5.1 / 5.6e-5 (5.2 / 5.7 / 6.1e-5).
+// 4.9 / 5.1 / 5.6e-5 (5.2 / 5.7 / 6.1e-5).  One token is a chain of these instructions whatever the lanes hold: without roots
+// for the powers of two and without branches round the others, 8 fp32 rows take 5.4 / 5.9 / 6.1 us (5.9 / 6.4 / 6.6 with them, the
+// butterfly 5.5 / 6.0 / 6.5).
 struct AppendUnitArgs {
     int64_t pos, n_new, capacity, blocks_per_seq, first_block;
     const int64_t *pos_dev;  // as in AppendArgs
@@ -2099,7 +2108,7 @@ __device__ __forceinline__ void append_units(const TI *x, uint8_t *packed, const
             part[ks] = sumsq8(xb[2 * ks], xb[2 * ks + 1], AS_STORE && ks >= 2 ? part[ks - 2] : 0.0f);
         ss = AS_STORE ? part[2] + part[3] : (part[0] + part[1]) + (part[2] + part[3]);
         over_lanes();
-        rowscale = row_pow2_scale(AS_STORE ? __builtin_amdgcn_sqrtf(ss) : sqrtf(ss));
+        rowscale = AS_STORE ? row_pow2_scale(__builtin_amdgcn_sqrtf(ss)) : row_pow2_scale_of_square(ss);
 #pragma unroll
         for (int ks = 0; ks < 4; ++ks) {
             half8_t hi, mid, lo;
