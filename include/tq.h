@@ -378,11 +378,13 @@ int tq_decode_attention(const tq_handle *hk, const tq_handle *hv, const tq_attn_
  * graph capture, tight serving loops, harnesses that forbid hipMalloc).  No counterpart in the reference.
  * Same arguments, kernels and results as tq_decode_attention; the split partials go to a workspace of
  * TQ_STATIC_WORKSPACE_BYTES that is built into the library's device code (every GPU the library runs on
- * holds one copy until the process ends), so the call allocates nothing; several passes run one after the
- * other.  Parameter sets one pass of which needs more than that (tq_attn_workspace_bytes() counts all; about 8000 workgroups: batch * n_kv_heads * n_splits / 16 of them
- * when n_splits is a multiple of 16) are rejected with TQ_ERR_UNSUPPORTED.  All calls on one GPU share the one workspace: calls that overlap in time on the same
- * GPU (different streams or threads) race; order them.  The workspace's address is looked up once per
- * device, in tq_create or in the first call on that device. */
+ * holds one copy until the process ends), so the call allocates nothing.  Several passes run in one launch
+ * where tq_attn_workspace_bytes(), which counts them all, is not more than that, else one after the other;
+ * parameter sets one pass of which needs more (one pass has room for about 8000 workgroups: batch *
+ * n_kv_heads * n_splits / 16 of them when n_splits is a multiple of 16) are rejected with TQ_ERR_UNSUPPORTED.
+ * All calls on one GPU share the one workspace: calls that overlap in time on the same GPU (different streams
+ * or threads) race; order them.  The workspace's address is looked up once per device, in tq_create or in the
+ * first call on that device. */
 #define TQ_STATIC_WORKSPACE_BYTES (16 * 1024 * 1024)
 int tq_decode_attention_static(const tq_handle *hk, const tq_handle *hv, const tq_attn_params *p, const void *q,
                                int q_dtype, const void *k, const void *v, const float *bias, float *out,

@@ -10,6 +10,7 @@ import pytest
 import tq_oracle as O
 import turboquant_plus_amd as tqa
 from turboquant_plus_amd import _lib as L
+from test_gpu_append_edges import launches
 
 pytestmark = pytest.mark.gpu
 D = 128
@@ -64,6 +65,36 @@ def test_static_workspace_entry_point_two_calls_in_a_row():
     run_pair(kc, vc, 1, 4, 1, 700, 2, 0.0, seed=2, with_bias=False)
     # and Sparse V again on a small shape (skip slots of the first call must not be counted)
     run_pair(kc, vc, 1, 8, 2, 300, 1, 1e-2, seed=3, with_bias=False)
+
+
+@pytest.mark.parametrize("Hq,head_dim", [(9, 128), (16, 128), (8, 256)])
+@pytest.mark.parametrize("fits", [True, False])
+def test_static_workspace_with_two_passes(Hq, head_dim, fits):
+    """Two passes share a launch where the built-in workspace holds the partials of both, and run one by one where it holds
+    those of one; the results are those of a workspace for both."""
+    tt = L.torch()
+    kc, vc = tqa.TurboCodec(3, seed=42), tqa.TurboCodec(2, seed=542)
+    B, n_splits = (2, 12) if fits else (24, 91)      # an odd split count: every split is a partial of its own
+    N, rows = 64 * n_splits + 5, head_dim // D
+    gen = tt.Generator("cuda").manual_seed(Hq)
+    k, v = (tt.randn((B, rows * N, D), generator=gen, device="cuda").half() for _ in range(2))
+    q = tt.randn((B, Hq, head_dim), generator=gen, device="cuda").half()
+    kp, vp = kc.store(k, kind="k"), vc.store(v, kind="v")
+    params = L.TQAttnParams(batch=B, n_q_heads=Hq, n_kv_heads=1, tokens=N, capacity=0, n_splits=n_splits, k_format=L.KFMT_TURBO,
+                            v_format=L.KFMT_TURBO, scale=head_dim ** -0.5, sparse_v_tau=0.0, head_dim=head_dim)
+    ws = tt.empty(int(L.lib().tq_attn_workspace_bytes(C.byref(params))), dtype=tt.uint8, device="cuda")
+    assert (ws.numel() <= 16 << 20) == fits and ws.numel() < 32 << 20
+    want, got = (tt.full((B, Hq, head_dim), float("nan"), dtype=tt.float32, device="cuda") for _ in range(2))
+    L.check(L.lib().tq_decode_attention(kc.handle.h, vc.handle.h, C.byref(params), L.ptr(q), L.TQ_F16, L.ptr(kp), None, L.ptr(vp),
+                                        None, L.ptr(want), None, L.ptr(ws), ws.numel(), L.stream_ptr()))
+
+    def call():
+        L.check(L.lib().tq_decode_attention_static(kc.handle.h, vc.handle.h, C.byref(params), L.ptr(q), L.TQ_F16, L.ptr(kp), L.ptr(vp),
+                                                   None, L.ptr(got), None, L.stream_ptr()))
+    assert launches(call) == (1 if fits else 2)
+    got.fill_(float("nan"))
+    call()
+    assert bool(tt.isfinite(got).all()) and tt.equal(got, want)
 
 
 def test_static_workspace_rejects_what_does_not_fit():
