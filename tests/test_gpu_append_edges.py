@@ -307,3 +307,38 @@ def test_long_prompt_of_a_layer_with_8_bit_rows(fmt, blocks):
         got = cache.view(n, per + 1, -1)
         assert tt.equal(got[:, :per], want.view(n, per, -1)), kind
         assert bool((got[:, per:] == 0xA5).all()), kind
+
+
+def near_halves(rng, rows):
+    """Rows of four 32-value groups: the literals of test_q8_0_literal_blocks, and per group a scale that is no power of two with
+    values on and next to the products that round at a half."""
+    x = np.zeros((rows, D), np.float32)
+    x[:, :16] = [-127.0, 0.5, -0.5, 1.5, -1.5, 2.5, -2.5, 126.5, -126.5, 0.49999997, -0.49999997, 0.50000006, 3.0, -0.0, 100.25, -100.75]
+    for g, amax in enumerate((np.float32(127) * np.float32(1 + 2.0 ** -12), np.float32(100.3), np.float32(0.037)), 1):
+        d = amax / np.float32(127)
+        half = ((rng.integers(0, 126, (rows, 31)) + 0.5) * float(d)).astype(np.float32)
+        half = (half.view(np.int32) + rng.integers(-2, 3, (rows, 31), dtype=np.int32)).view(np.float32)
+        x[:, 32 * g:32 * g + 31] = half * rng.choice(np.float32([-1, 1]), (rows, 31))
+        x[:, 32 * g + 31] = amax
+    return x
+
+
+@pytest.mark.parametrize("kind", ["k", "v"])
+@pytest.mark.parametrize("other", ["q8_0", "turbo3"])
+def test_q8_0_rounds_halves_away_from_zero(kind, other):
+    """Appends, one side and a layer of any kind, quantise ties and their neighbours as the store and the oracle do."""
+    tt = L.torch()
+    rows = near_halves(np.random.default_rng(1), 2 * 200).reshape(2, 200, D)
+    q, scale = O.q8_0_quantize(rows.reshape(-1, D))
+    assert q[0, :16].tolist() == [-127, 1, -1, 2, -2, 3, -3, 127, -127, 0, 0, 1, 3, 0, 100, -101]
+    x = tt.from_numpy(rows).cuda()
+    layer = tqa.LayerKV(tqa.LayerFormat(*(("q8_0", other) if kind == "k" else (other, "q8_0"))))
+    one, (ck, cv) = tt.zeros(2 * 256 * 136, dtype=tt.uint8, device="cuda"), layer.new_cache(2, 256)
+    for pos, n_new in ((0, 1), (1, 66), (67, 133)):
+        xn = x[:, pos:pos + n_new].contiguous()
+        tqa.q8_0_append(xn, one, pos, 256, kind=kind)
+        layer.append(xn, xn, ck, cv, pos, 256)
+    assert tt.equal(one, ck if kind == "k" else cv)
+    assert tt.equal(one, tqa.q8_0_store(x, kind=kind)[0])
+    got, s = (np_(a)[:, :200].reshape(400, -1) for a in tqa.q8_0_unpack(one, 2, 256, kind=kind))
+    assert np.array_equal(got, q) and np.array_equal(s.astype(np.float16), scale)
