@@ -342,3 +342,39 @@ def test_q8_0_rounds_halves_away_from_zero(kind, other):
     assert tt.equal(one, tqa.q8_0_store(x, kind=kind)[0])
     got, s = (np_(a)[:, :200].reshape(400, -1) for a in tqa.q8_0_unpack(one, 2, 256, kind=kind))
     assert np.array_equal(got, q) and np.array_equal(s.astype(np.float16), scale)
+
+
+@pytest.mark.parametrize("bits", [2, 3, 4])
+@pytest.mark.parametrize("kind", ["k", "v"])
+@pytest.mark.parametrize("dtype", ["float16", "float32"])
+def test_infinities_and_nan_stay_in_their_rows(bits, kind, dtype):
+    """Rows with an infinity or a NaN have a norm that is not finite; the codes and norms of the tokens that share a word, a
+    product or a sum with them are those they have beside ordinary rows, in appends, short prompts and the store."""
+    tt = L.torch()
+    codec = tqa.TurboCodec(bits, seed=3)
+    x = tt.randn((N_SEQS, 400, D), generator=tt.Generator("cuda").manual_seed(bits), device="cuda").to(getattr(tt, dtype))
+    bad = x.clone()
+    rows = {(0, 0): float("inf"), (0, 7): float("nan"), (0, 130): -float("inf"), (1, 66): float("inf"), (1, 67): float("nan"), (1, 399): -float("inf")}
+    for i, ((s, t), value) in enumerate(rows.items()):
+        bad[s, t, 37 * i % D] = value
+    bad[1, 66, :64], bad[1, 200] = -float("inf"), float("nan")
+    whole = np.ones((N_SEQS, 400), bool)
+    for s, t in list(rows) + [(1, 200)]:
+        whole[s, t] = False
+
+    def appended(r):
+        cache = tt.zeros(tqa.packed_bytes(bits, N_SEQS, CAPACITY), dtype=tt.uint8, device="cuda")
+        for pos, n_new in ((0, 1), (1, 65), (66, 2), (68, 332)):
+            codec.append(r[:, pos:pos + n_new], cache, pos, CAPACITY, kind=kind)
+        return codec.unpack_codes(cache, N_SEQS, CAPACITY, kind=kind)
+
+    def prompt(r):
+        packed = codec.store_kv(codec, r, r)[kind == "v"]
+        return codec.unpack_codes(packed, N_SEQS, 400, kind=kind)
+
+    def stored(r):
+        return codec.unpack_codes(codec.store(r, kind=kind), N_SEQS, 400, kind=kind)
+    for way in (appended, prompt, stored):
+        (codes, norms), (got, g) = ([np_(a)[:, :400] for a in way(r)] for r in (x, bad))
+        assert np.array_equal(got[whole], codes[whole]) and np.array_equal(g[whole], norms[whole]), way
+        assert not np.isfinite(g[~whole]).any(), way
