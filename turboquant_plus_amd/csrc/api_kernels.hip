@@ -30,7 +30,8 @@ __device__ __forceinline__ int level_of(double v, const double *bounds, int bits
 // ---- dense products: out[row][j] = sum_k f(in[row][k]) M[k][j], float64 matrix cores -----------------------------
 // One thread per (output, vector) read the whole matrix from L2 once per VB vectors and an LDS operand per multiply:
 // 1.56 ms per product for 256 vectors of 1536 (0.8 of 75 TFLOP/s), 92 us for 32 768 of 128.  Here a wavefront owns RT x
-// CT tiles of 16 x 16 outputs of v_mfma_f64_16x16x4_f64 and a slice of the contraction or all of it: 28 and 39 us.  What
+// CT tiles of 16 x 16 outputs of v_mfma_f64_16x16x4_f64 and a slice of the contraction or all of it: 28 to 32 and 34 to 43 us
+// by what is folded in (back to back and traced).  What
 // bounds it is the matrix instruction (64 clocks; 22 and 20 us of them at the 1.7 GHz the part holds here), then the
 // uneven last round of workgroups.  The order of the contraction is free, so in a chunk of 16 values lane quarter q takes
 // values 4q .. 4q+3 for the chunk's four steps: the A operand of four steps is one vector load, the B operand of a step
@@ -335,7 +336,7 @@ void launch_dense_tiles(DenseArgs a, int slices, hipStream_t s) {
 //   else the tiles of 1 x 1, 1 x 2, 2 x 2 or 2 x 3 whose workgroups are done first, where the launch takes as long as the CU
 //   with the most of them and a workgroup as long as split_cost's last argument, to scale (a matrix operand is loaded per row
 //   tile and a vector's per column tile, so small tiles cost more than their share).  256 of 1536, 1.5 workgroups of 2 x 2 per
-//   CU or one of 2 x 3: 32.5 to 37.3 / 26.8 to 27.4; 200 of 1536 the same; 1000 of 384: 12.6 to 13.3 / 10.6 to 11.9; 325 of 768,
+//   CU or one of 2 x 3: 33.5 to 34.1 / 27.7 to 28.4 back to back; 200 of 1536 the same; 1000 of 384: 12.6 to 13.3 / 10.6 to 11.9; 325 of 768,
 //   2 x 2 / 1 x 2: 18.2 / 13.9; 100 of 1536, 1 x 2 / 2 x 2: 21.9 to 25.1 / 19.5 to 20.6; 20 of 1536, 1 x 2 / 1 x 1: 13.6 / 10.6.
 //   Not 1 x 1 or 1 x 2 from the fourth workgroup of a CU on (325 of 1536, 2 x 2 / 1 x 2: 47 / 38 to 49), nor 2 x 3 for less than a
 //   tenth (2300 of 1536: 204 to 235 / 230) or where fewer than eight slices leave a workgroup short (5000 of 100: 12.2 / 12.8).

@@ -2017,8 +2017,9 @@ struct AppendUnitArgs {
     float thr[8], thr_lo[8], coef[8];       // boundaries: thr + thr_lo
 };
 // AS_STORE: a prompt's rows, whose bytes are those of tq_store (the store kernels' roots, table decisions and zeros).
-// TI = float: fp32 rows as three fp16 terms per value, which hold all of its bits (a term's sums are as good as exact), or in
-// the store's two.
+// TI = float: fp32 rows as three fp16 terms per value, or in the store's two.  Three hold all 24 bits of values above about 2^-10
+// of the row's norm and the others to 2^-34 of it (a row is scaled to a norm of 512 to 1024, where an fp16 term ends at 2^-24):
+// less than the 32-bit sums round.
 template <int BITS, int KIND, bool AS_STORE, typename TI>
 __device__ __forceinline__ void append_units(const TI *x, uint8_t *packed, const AppendUnitArgs &a, const unsigned wg) {
     constexpr bool F32 = sizeof(TI) == 4;
