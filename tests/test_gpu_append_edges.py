@@ -130,7 +130,7 @@ def test_layer_with_8_bit_rows(fmt, dtypes):
 @pytest.mark.parametrize("dtype", ["float16", "float32", "float64"])
 @pytest.mark.parametrize("tokens", [1023, 1025, 1152])
 def test_prompt_of_a_layer_with_8_bit_rows(fmt, dtype, tokens):
-    """64 sequences of 8 (one launch of the append kernel for K and V but for float16) and 9 blocks: the 8-bit side as
+    """64 sequences of 8 and 9 blocks, one launch of the append kernel for K and V: the 8-bit side as
     appended, the turbo side as stored (float16) or appended, sequence by sequence, and nothing past a sequence's last
     block.  (tq_store takes float32 rows as two fp16 terms: no oracle for rows that are computed in 32 bits.)"""
     tt = L.torch()
