@@ -41,192 +41,11 @@
 #include <type_traits>
 #include <utility>
 
-#include "tq_device.h"
+#include "tq_attn.h"
 
 namespace {
 
-using namespace tqd;
-
-constexpr float LOG2E = 1.4426950408889634f;
-constexpr float RSQRT128 = 0.08838834764831845f;
-
-template <typename T> __device__ inline float ldf(const T *p) { return (float)*p; }
-template <> __device__ inline float ldf<__half>(const __half *p) { return __half2float(*p); }
-
-template <int BITS> __device__ __forceinline__ uint32_t pair_off(const uint32_t (&w)[4 * BITS], int p) {
-    return pair_lut_offset<BITS>(w, p);
-}
-
-// TQ_PAIRTAB3 (tq_measure.h; measurement builds only): 3-bit codes decode through a pair table with one copy
-// per LDS bank (entry e of lane l at dword 64 e + l: no bank conflicts, two 4-byte reads per four values)
-// instead of the 4096-entry quad table (one 8-byte read per four values, about 1.6 conflicts per read).
-// bytes of the decode table of a codebook: quad entries for BITS <= 3, pair entries for 4
-__host__ __device__ constexpr int lut_bytes(int bits) {
-    if (TQ_PAIRTAB3 && bits == 3) return 64 * 64 * 4;
-    return bits == 8 ? 0 : bits <= 3 ? 8 << (4 * bits) : 4 << (2 * bits);  // 8: int8 rows, no table
-}
-
-// the four values of quad Q (pairs 2Q, 2Q+1) of a row as an MFMA operand
-template <int BITS> __device__ __forceinline__ half4_t quad_values(const uint32_t (&w)[4 * BITS], const char *lut, int Q) {
-    if constexpr (TQ_PAIRTAB3 && BITS == 3) {
-        // lut already points at this lane's bank (+ 4 * lane); a pair code selects the 256-byte row
-        const uint32_t o0 = pair_lut_offset<BITS>(w, 2 * Q) << 6, o1 = pair_lut_offset<BITS>(w, 2 * Q + 1) << 6;
-        const uint2 u = make_uint2(*reinterpret_cast<const uint32_t *>(lut + o0), *reinterpret_cast<const uint32_t *>(lut + o1));
-        return __builtin_bit_cast(half4_t, u);
-    } else if constexpr (BITS <= 3) {
-        return __builtin_bit_cast(half4_t, *reinterpret_cast<const uint2 *>(lut + quad_lut_offset<BITS>(w, Q)));
-    } else {
-        const uint2 u = make_uint2(*reinterpret_cast<const uint32_t *>(lut + pair_lut_offset<BITS>(w, 2 * Q)),
-                                   *reinterpret_cast<const uint32_t *>(lut + pair_lut_offset<BITS>(w, 2 * Q + 1)));
-        return __builtin_bit_cast(half4_t, u);
-    }
-}
-
-// build a codebook's decode table in LDS from its pair table (half2 per pair code) with n_waves wavefronts;
-// `mine` is pair entry tid % 64, fetched by the caller ahead of time (used by the 3-bit table only)
-template <int BITS>
-__device__ __forceinline__ void build_lut(char *dst, const uint32_t *pair_lut, uint32_t mine, int tid, int n_waves) {
-    constexpr int NP = 1 << (2 * BITS);
-    if constexpr (TQ_PAIRTAB3 && BITS == 3) {
-        uint32_t *t = reinterpret_cast<uint32_t *>(dst);
-        const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-        for (int e = wave; e < 64; e += n_waves) t[e * 64 + lane] = (uint32_t)__builtin_amdgcn_readlane((int)mine, e);
-    } else if constexpr (BITS == 3) {
-        // lane l holds pair entry l; wavefront w writes the rows hi = w, w + n_waves, ..
-        uint2 *t = reinterpret_cast<uint2 *>(dst);
-        const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-        for (int hi = wave; hi < 64; hi += n_waves)
-            t[hi * 64 + lane] = make_uint2(mine, (uint32_t)__builtin_amdgcn_readlane((int)mine, hi));
-    } else if constexpr (BITS == 2) {
-        for (int e = tid; e < 256; e += 64 * n_waves)
-            reinterpret_cast<uint2 *>(dst)[e] = make_uint2(pair_lut[e & 15], pair_lut[e >> 4]);
-    } else {
-        static_assert(NP == 256, "pair table of 256 entries");
-        for (int e = tid; e < 256; e += 64 * n_waves) reinterpret_cast<uint32_t *>(dst)[e] = pair_lut[e];
-    }
-}
-
-// raise a progress mark in LDS to `mine` and return what it held before (one atomic per wavefront)
-__device__ __forceinline__ uint32_t lead_progress(uint32_t *mark, uint32_t mine, int lane) {
-    uint32_t t = 0;
-    if (lane == 0) t = atomicMax(mark, mine);
-    return __builtin_amdgcn_readfirstlane(t);
-}
-
-template <int BITS> __device__ __forceinline__ void load_row(const uint8_t *block, int row, uint32_t (&w)[4 * BITS]) {
-#pragma unroll
-    for (int c = 0; c < BITS; ++c) {
-        const uint4 u = stream_load<STREAM_ATTN_ROWS>(reinterpret_cast<const uint4 *>(block + c * 2048 + row * 16));
-        w[4 * c] = u.x; w[4 * c + 1] = u.y; w[4 * c + 2] = u.z; w[4 * c + 3] = u.w;
-    }
-}
-
-__device__ __forceinline__ float4_t mfma4(half4_t a, half4_t b, float4_t c) {
-    return __builtin_amdgcn_mfma_f32_4x4x4f16(a, b, c, 0, 0, 0);
-}
-
-// 4x4x4 MFMA whose A operand is taken from block ABID and broadcast to all 16 blocks
-template <int ABID> __device__ __forceinline__ float4_t mfma4_bcast(half4_t a, half4_t b, float4_t c) {
-    return __builtin_amdgcn_mfma_f32_4x4x4f16(a, b, c, 4, ABID, 0);
-}
-
-// the same with the A operand taken from block ABID of each group of 8 blocks (lanes 0..31 and 32..63 apart)
-template <int ABID> __device__ __forceinline__ float4_t mfma4_bcast8(half4_t a, half4_t b, float4_t c) {
-    return __builtin_amdgcn_mfma_f32_4x4x4f16(a, b, c, 3, ABID, 0);
-}
-
-// four int8 of a dword as fp16, in the order 0, 2, 1, 3: 0x6400 | (x + 128) is the fp16 number 1024 + (x + 128),
-// exactly, so a byte permute builds two of them at once and one packed fp16 subtraction of 1152 leaves (x0, x2)
-// and (x1, x3)
-__device__ __forceinline__ half4_t int8x4_to_half_0213(uint32_t w) {
-    typedef _Float16 half2_t __attribute__((ext_vector_type(2)));
-    const uint32_t u = w ^ 0x80808080u;
-    const half2_t bias = {(_Float16)1152.0f, (_Float16)1152.0f};
-    const half2_t h02 = __builtin_bit_cast(half2_t, __builtin_amdgcn_perm(0x64646464u, u, 0x04020400u)) - bias;
-    const half2_t h13 = __builtin_bit_cast(half2_t, __builtin_amdgcn_perm(0x64646464u, u, 0x04030401u)) - bias;
-    half4_t kv;
-    kv[0] = h02[0];
-    kv[1] = h02[1];
-    kv[2] = h13[0];
-    kv[3] = h13[1];
-    return kv;
-}
-
-// transpose the 4x4 matrix held by a quad of lanes (element [lane%4][register]), two exchange stages
-__device__ __forceinline__ void quad_transpose(float (&r)[4], int lane) {
-    const bool b0 = lane & 1, b1 = lane & 2;
-#pragma unroll
-    for (int p = 0; p < 4; p += 2) {  // swap (even lane, odd reg) <-> (odd lane, even reg)
-        const float give = b0 ? r[p] : r[p + 1];
-        const float got = xor_lane<1>(give);
-        if (b0) r[p] = got;
-        else r[p + 1] = got;
-    }
-#pragma unroll
-    for (int p = 0; p < 2; ++p) {     // swap (lane bit1 clear, reg p+2) <-> (lane bit1 set, reg p)
-        const float give = b1 ? r[p] : r[p + 2];
-        const float got = xor_lane<2>(give);
-        if (b1) r[p] = got;
-        else r[p + 2] = got;
-    }
-}
-
-// sum over the 16 lanes that share lane%4 (blocks b = 0..15)
-__device__ __forceinline__ float sum_over_blocks(float v) {
-    v += xor_lane<4>(v);
-    v += xor_lane<8>(v);
-    v += xor_lane<16>(v);
-    v += xor_lane<32>(v);
-    return v;
-}
-__device__ __forceinline__ float max_over_blocks(float v) {
-    v = fmaxf(v, xor_lane<4>(v));
-    v = fmaxf(v, xor_lane<8>(v));
-    v = fmaxf(v, xor_lane<16>(v));
-    v = fmaxf(v, xor_lane<32>(v));
-    return v;
-}
-
-struct AttnArgs {
-    const void *q;       // [groups*4][128] queries in the original domain, q_dtype
-    int q_dtype;
-    const float *ks1, *ks2;  // K rotation signs (NULL: K is not rotated, q is only scaled)
-    float scale_log2e;       // logit scale * log2(e), folded into the fp16 query
-    const uint8_t *k, *v;
-    const uint32_t *klut, *vlut;  // pair tables (half2 per pair code)
-    const float *bias;            // [groups*4][tokens] natural-log units, or NULL
-    const int32_t *sbias_pos;     // sparse bias: [groups*q_group][sbias_n] positions, ascending within a head (entries that
-    const float *sbias_val;       // do not exist: any position >= tokens), and their values (natural-log units)
-    int sbias_n;                  // entries per head, 0 = no sparse bias
-    float *part_o;                // [groups][workgroups per group][4][128]
-    float *part_ml;               // [groups][workgroups per group][4][2]  (m in log2 units, l)
-    unsigned long long *skip_slots;  // Sparse V: [workgroup] nonce tag | (query, position) pairs it skipped; 0 after the count
-    // merge of the workgroups' partials by the last workgroup of a group to finish (see merge_group)
-    float *out;                      // [groups * q_group][128]
-    const float *vs1, *vs2;          // V rotation signs (NULL: V rows are stored unrotated)
-    unsigned long long *flags;       // [group][workgroups per group]; word 0 of a group is its arrival counter (tag | count), 0 after the merge
-    unsigned long long nonce;        // differs from call to call (and from whatever the workspace held before)
-    int poll_slots;                       // Sparse V: the merging workgroups add the slots up themselves
-    unsigned long long *pass_totals;      // Sparse V: [pass] skipped pairs of each four-head pass of this step
-    unsigned long long *skip_count;       // caller's {skipped, total} or NULL
-    unsigned long long total_pairs;
-    int pass;                             // head_off / pass_heads
-    int64_t tokens, blocks_per_seq;
-    const int64_t *tokens_dev;  // NULL, or where the step's context length is read from (<= tokens, which then is the maximum)
-    int n_groups, n_splits, tiles_per_split, n_tiles;
-    int q_group, head_off;  // query heads per KV head; first of the heads that this launch's first pass works on
-    int d256;               // heads of 256 dims: a token is two 128-value rows (2 token + half) of the K and V caches
-    int gpw;                // (batch, kv head) groups per workgroup: 1, or wavefronts per workgroup / n_splits when a group's
-                            // splits are fewer than a workgroup's wavefronts (short contexts: the groups share the decode tables)
-    int gw_shift;           // gpw > 1: log2(n_splits), a power of two then
-    int wgs_per_group;      // gpw == 1: n_splits / wavefronts per workgroup
-    float tau;
-    int pass_heads;         // heads per pass; blockIdx.y numbers the passes of a launch, whose partials and counters follow each other
-};
-
-constexpr int KFMT_TURBO = 0, KFMT_Q8 = 1;
-constexpr unsigned long long SKIP_COUNT_MASK = (1ull << 40) - 1ull;  // count bits of a Sparse-V slot; the rest is a nonce tag
-constexpr int MERGE_FLOATS = 520;  // LDS floats per wavefront for the end-of-kernel merge: out[4][128], m[4], l[4]
+using namespace tqattn;
 
 // QK over the 32 dim groups: B = this lane's K row (4 dims per group), A = q from block G % 16
 // (HG sets of four query heads share every dequantised operand: one table look-up, HG products)
@@ -355,201 +174,7 @@ __device__ __forceinline__ void pv_all_q8_d256(std::integer_sequence<int, T...>,
 // scales of those rows for the 32-dim block of this lane's dims of dim half hf (v[2 hf], v[2 hf + 1])
 template <int VBITS> struct VSide { uint2 v[VBITS == 8 ? 4 : 2]; };
 
-constexpr unsigned long long ARRIVAL_COUNT_MASK = 0xFFFFFFull;  // workgroups of a group (the tag of the call sits above)
 constexpr float Q8V_PRESCALE = 64.0f;  // keeps weight * scale products out of fp16's subnormals; 65504 / 64 > any scale
-
-// ---- merging the workgroups' partials inside the launch -------------------------------------
-// A group's partials are written by up to n_splits / wavefronts-per-workgroup workgroups that may run on
-// different dies, whose L2 caches are not coherent with each other for ordinary accesses.  Everything the
-// workgroups exchange therefore moves with device-scope atomic accesses (they go through to memory): a workgroup
-// stores its partial, waits for the stores to complete, and then increments the group's arrival counter with one
-// read-modify-write; the workgroup whose increment completes the count merges the group.  The counter carries a tag
-// of the call, so what a fresh workspace happens to contain is not mistaken for arrivals, and the merging workgroup
-// puts it back to zero, so a replay of a captured launch (same tag) starts clean.  No cache-wide write-back or
-// invalidate is involved, which is what made a merge behind device-scope fences cost more than the second launch it
-// saved.  (An earlier version raised a flag per workgroup and read the group's flags: two more trips to memory per
-// workgroup, and "somebody sees every flag" needed a store-to-load ordering argument where the counter needs none.)
-__device__ __forceinline__ void st_dev(float *p, float v) {
-    __hip_atomic_store(reinterpret_cast<uint32_t *>(p), __float_as_uint(v), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-__device__ __forceinline__ void st_dev(unsigned long long *p, unsigned long long v) {
-    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-__device__ __forceinline__ unsigned long long ld_dev(const unsigned long long *p) {
-    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-__device__ __forceinline__ float2 ld_dev2(const float *p) {  // 8-byte aligned pair
-    const unsigned long long u = ld_dev(reinterpret_cast<const unsigned long long *>(p));
-    return make_float2(__uint_as_float((uint32_t)u), __uint_as_float((uint32_t)(u >> 32)));
-}
-__device__ __forceinline__ void wait_stores() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
-
-// Log-sum-exp merge of a group's n_parts partials, transpose of the V rotation, output rows; one wavefront per
-// query head (the partials come straight from memory: every load of a head is issued before the first is used
-// when there are at most four).
-// The partials [p_lo, p_hi) of one head of a group, merged by one wavefront: running maximum M (log2 units), weight
-// sum L and this lane's two output dims, all relative to M.  Up to 16 partials have every load requested before the
-// first is used, so the merge costs one trip to memory (in batches of four, sixteen partials took four trips at the
-// very end of the launch).
-struct MergedPart {
-    float M, L, o0, o1;
-};
-__device__ __forceinline__ MergedPart merge_range(const float *ml0, const float *po0, int ML, int PO, int head, int p_lo, int p_hi,
-                                                  int lane) {
-    MergedPart r{-INFINITY, 0.0f, 0.0f, 0.0f};
-    const int n = p_hi - p_lo;
-    auto merge_few = [&](auto np_tag) {
-        constexpr int NP = decltype(np_tag)::value;
-        float2 ml[NP], v[NP];
-#pragma unroll
-        for (int p = 0; p < NP; ++p) {
-            const int pc = p_lo + (p < n ? p : 0);
-            ml[p] = ld_dev2(ml0 + pc * ML + head * 2);
-            v[p] = ld_dev2(po0 + (int64_t)pc * PO + head * 128 + 2 * lane);
-            if (p >= n) ml[p].y = 0.0f;
-        }
-#pragma unroll
-        for (int p = 0; p < NP; ++p)
-            if (ml[p].y > 0.0f) r.M = fmaxf(r.M, ml[p].x);
-#pragma unroll
-        for (int p = 0; p < NP; ++p) {
-            const float w = ml[p].y > 0.0f ? exp2f(ml[p].x - r.M) : 0.0f;
-            r.L = fmaf(ml[p].y, w, r.L);
-            r.o0 = fmaf(v[p].x, w, r.o0);
-            r.o1 = fmaf(v[p].y, w, r.o1);
-        }
-    };
-    if (n <= 0) return r;
-    if (n <= 4) {
-        merge_few(std::integral_constant<int, 4>{});
-    } else if (n <= 16) {
-        merge_few(std::integral_constant<int, 16>{});
-    } else {
-        for (int p0 = p_lo; p0 < p_hi; p0 += 64) {  // lane <-> partial: maximum, then weights
-            const int p = p0 + lane;
-            float m = -INFINITY;
-            if (p < p_hi) {
-                const float2 e = ld_dev2(ml0 + p * ML + head * 2);
-                if (e.y > 0.0f) m = e.x;
-            }
-            for (int o = 32; o > 0; o >>= 1) m = fmaxf(m, __shfl_xor(m, o));
-            r.M = fmaxf(r.M, m);
-        }
-        for (int p0 = p_lo; p0 < p_hi; p0 += 64) {
-            const int p = p0 + lane;
-            float w = 0.0f, l = 0.0f;
-            if (p < p_hi) {
-                const float2 e = ld_dev2(ml0 + p * ML + head * 2);
-                l = e.y;
-                w = l > 0.0f ? exp2f(e.x - r.M) : 0.0f;
-            }
-            float lw = l * w;
-            for (int o = 32; o > 0; o >>= 1) lw += __shfl_xor(lw, o);
-            r.L += lw;
-            const int cnt = min(64, p_hi - p0);
-            // eight partials per trip to memory (a lane exchange cannot sit in a loop that the compiler unrolls with
-            // a remainder, so the batches are written out: past the count the last partial is read again with weight 0)
-            for (int t0 = 0; t0 < cnt; t0 += 8) {
-                float2 v[8];
-                float wt[8];
-#pragma unroll
-                for (int k = 0; k < 8; ++k) {
-                    const int t = min(t0 + k, cnt - 1);
-                    v[k] = ld_dev2(po0 + (int64_t)(p0 + t) * PO + head * 128 + 2 * lane);
-                    wt[k] = t0 + k < cnt ? __shfl(w, t) : 0.0f;
-                }
-#pragma unroll
-                for (int k = 0; k < 8; ++k) {
-                    r.o0 = fmaf(v[k].x, wt[k], r.o0);
-                    r.o1 = fmaf(v[k].y, wt[k], r.o1);
-                }
-            }
-        }
-    }
-    return r;
-}
-
-// The group's partials -> output rows (log-sum-exp merge, then the V rotation's transpose).  A workgroup with at least
-// twice as many wavefronts as the pass has heads gives every head several wavefronts, each merging a share of the
-// partials, and joins their results through `lds` (free LDS of 132 floats per wavefront; unused otherwise): the merge
-// runs at the very end of the launch, so its trips to memory are the launch's tail.
-template <int HG>
-__device__ __forceinline__ void merge_group(const AttnArgs &a, int group, int pgroup, int head_off, int n_parts, int tid, int n_waves,
-                                            float *lds) {
-    constexpr int NH = 4 * HG, ML = 2 * NH, PO = 128 * NH;  // heads, (m, l) floats and output floats of one partial
-    const int lane = tid & 63, wave = tid >> 6;
-    const float *ml0 = a.part_ml + (int64_t)pgroup * n_parts * ML;
-    const float *po0 = a.part_o + (int64_t)pgroup * n_parts * PO;
-    auto finish = [&](int head, MergedPart r) {
-        // heads of 256 dims (HG = 2): partial row 4 dh + i is dims 128 dh .. 128 dh + 127 of head i
-        const int hq = a.d256 ? (head & 3) : head;
-        const int64_t r_out = a.d256 ? 2 * ((int64_t)group * a.q_group + head_off + hq) + (head >> 2)
-                                     : (int64_t)group * a.q_group + head_off + head;
-        const float invL = r.L > 0.0f ? 1.0f / r.L : 0.0f;
-        float o0 = r.o0, o1 = r.o1;
-        float2 res;
-        if (!a.vs1) {  // V rows were stored unrotated
-            res = make_float2(o0 * invL, o1 * invL);
-        } else {
-            const float2 s1v = *reinterpret_cast<const float2 *>(a.vs1 + 2 * lane);
-            const float2 s2v = *reinterpret_cast<const float2 *>(a.vs2 + 2 * lane);
-            o0 *= invL * s2v.x;
-            o1 *= invL * s2v.y;
-            wht128_wave(o0, o1, lane);
-            res = make_float2(o0 * (s1v.x * RSQRT128), o1 * (s1v.y * RSQRT128));
-        }
-        *reinterpret_cast<float2 *>(a.out + r_out * 128 + 2 * lane) = res;
-    };
-    // a repeated head of a group with fewer than four left is not written
-    auto head_exists = [&](int head) { return head_off + (a.d256 ? (head & 3) : head) < a.q_group; };
-    const int n_sub = lds && n_waves >= 2 * NH && n_parts > 4 ? n_waves / NH : 1;
-    if (n_sub == 1) {
-        for (int head = wave; head < NH; head += n_waves)
-            if (head_exists(head)) finish(head, merge_range(ml0, po0, ML, PO, head, 0, n_parts, lane));
-        return;
-    }
-    const int head = wave % NH, sub = wave / NH;
-    const int per = (n_parts + n_sub - 1) / n_sub;
-    const bool mine = sub < n_sub && head_exists(head);
-    MergedPart r{-INFINITY, 0.0f, 0.0f, 0.0f};
-    if (mine) r = merge_range(ml0, po0, ML, PO, head, min(sub * per, n_parts), min(sub * per + per, n_parts), lane);
-    float *slot = lds + (head * n_sub + (sub < n_sub ? sub : 0)) * 132;
-    if (mine) {
-        *reinterpret_cast<float2 *>(slot + 2 * lane) = make_float2(r.o0, r.o1);
-        if (lane == 0) {
-            slot[128] = r.M;
-            slot[129] = r.L;
-        }
-    }
-    __syncthreads();
-    if (mine && sub == 0) {
-        const float *s0 = lds + head * n_sub * 132;
-        float M = -INFINITY;
-        for (int k = 0; k < n_sub; ++k)
-            if (s0[k * 132 + 129] > 0.0f) M = fmaxf(M, s0[k * 132 + 128]);
-        MergedPart t{M, 0.0f, 0.0f, 0.0f};
-        for (int k = 0; k < n_sub; ++k) {
-            const float l = s0[k * 132 + 129];
-            const float w = l > 0.0f ? exp2f(s0[k * 132 + 128] - M) : 0.0f;
-            const float2 o = *reinterpret_cast<const float2 *>(s0 + k * 132 + 2 * lane);
-            t.L = fmaf(l, w, t.L);
-            t.o0 = fmaf(o.x, w, t.o0);
-            t.o1 = fmaf(o.y, w, t.o1);
-        }
-        finish(head, t);
-    }
-}
-
-
-// sum over the workgroup of one 64-bit value per thread (every thread gets the total); red: one shared word
-__device__ __forceinline__ unsigned long long block_sum(unsigned long long t, unsigned long long *red, int tid) {
-    if (tid == 0) *red = 0ull;
-    __syncthreads();
-    for (int o = 32; o > 0; o >>= 1) t += __shfl_xor(t, o);
-    if ((tid & 63) == 0 && t) atomicAdd(red, t);
-    __syncthreads();
-    return *red;
-}
 
 // SHARE: K and V decode through one table (same width, same centroids); table positions are
 // compile-time constants so that they fold into the LDS instructions' offset fields.
@@ -618,8 +243,8 @@ __global__ __launch_bounds__(64 * max_waves_per_workgroup(VBITS, HG, KFMT == KFM
     const int split = part * n_waves + wave_g;  // index of this wavefront's partial
     // dynamic LDS: the wavefronts' merge space (end of the split), then 1 KB per group and set of four heads that
     // stages the rotated queries
-    extern __shared__ float merge_s[];
-    char *q_stage = reinterpret_cast<char *>(merge_s) + (n_waves > 1 ? (size_t)n_waves * HG * MERGE_FLOATS * sizeof(float) : 0) +
+    extern __shared__ __attribute__((aligned(16))) float merge_s[];
+    char *q_stage = reinterpret_cast<char *>(merge_s) + (size_t)n_waves * HG * MERGE_FLOATS * sizeof(float) +
                     (size_t)gidx * (1024 * HG);
     // The context length: a kernel argument, or read from memory when the caller replays one captured launch at
     // changing lengths (the split geometry then follows the length; a.tokens stays the bias rows' stride).
@@ -694,6 +319,8 @@ __global__ __launch_bounds__(64 * max_waves_per_workgroup(VBITS, HG, KFMT == KFM
         }
         return r;
     };
+    unsigned long long arrivals_seen = 0ull;
+    if (wgs_per_group > 1 && tid == 0) arrivals_seen = ld_dev(arrival_counter(a, pgroup, wgs_per_group));
     uint2 kn = make_uint2(0u, 0u);
     VSide<VBITS> gvu;
 #pragma unroll
@@ -716,10 +343,6 @@ __global__ __launch_bounds__(64 * max_waves_per_workgroup(VBITS, HG, KFMT == KFM
     uint32_t kpair = 0, vpair = 0;
     if constexpr (KFMT == KFMT_TURBO && KBITS == 3) kpair = a.klut[lane];
     if constexpr (!SHARE && VBITS == 3) vpair = a.vlut[lane];
-
-    // one partial per workgroup: index (group, part), 4 HG heads each
-    float *po = a.part_o + ((int64_t)pgroup * wgs_per_group + part) * 4 * HG * 128;
-    float *pml = a.part_ml + ((int64_t)pgroup * wgs_per_group + part) * 4 * HG * 2;
 
     // A operand of QK, broadcast from one block per MFMA: lane (b, i) keeps q[head i] for the
     // dim groups g = b and g = b + 16 (4 dims each); MFMA g reads it from block g % 16.
@@ -818,6 +441,7 @@ __global__ __launch_bounds__(64 * max_waves_per_workgroup(VBITS, HG, KFMT == KFM
         qw[p0] = (_Float16)(x0 * qscale);
         qw[p1] = (_Float16)(x1 * qscale);
     }
+    if (wgs_per_group > 1 && tid == 0) install_tag(a, arrival_counter(a, pgroup, wgs_per_group), arrivals_seen);
     __syncthreads();
     half4_t qa[HG][2];
     half4_t qa4[4];   // 256-dim heads: dim groups b, b + 8, b + 16, b + 24 of this half-wavefront's half of the query
@@ -1168,150 +792,18 @@ __global__ __launch_bounds__(64 * max_waves_per_workgroup(VBITS, HG, KFMT == KFM
         l_tot[1] = l_tot[0];
         m_run[1] = m_run[0];
     }
-    if (gw == 1) {
+    auto slot = [&](int w) { return merge_s + w * (MERGE_FLOATS * HG); };
+    float *mine = slot(wave);
 #pragma unroll
-        for (int hg = 0; hg < HG; ++hg) {
+    for (int hg = 0; hg < HG; ++hg) {
 #pragma unroll
-            for (int hf = 0; hf < 2; ++hf)
+        for (int hf = 0; hf < 2; ++hf)
 #pragma unroll
-                for (int i = 0; i < 4; ++i)
-                    st_dev(po + (4 * hg + i) * 128 + 64 * hf + lane, acc_o[hg][hf][0][i] + acc_o[hg][hf][1][i]);
-            if (lane < 4) {
-                st_dev(pml + 2 * (4 * hg + j), m_run[hg]);
-                st_dev(pml + 2 * (4 * hg + j) + 1, l_tot[hg]);
-            }
-        }
-    } else {
-        // per wavefront and set of four heads: out[4][128], then m[4], l[4]; a group's wavefronts are wave0 .. wave0 + gw - 1
-        constexpr int MS = MERGE_FLOATS * HG;
-        float *mine = merge_s + wave * MS;
-#pragma unroll
-        for (int hg = 0; hg < HG; ++hg)
-            if (lane < 4) {
-                mine[hg * MERGE_FLOATS + 512 + j] = m_run[hg];
-                mine[hg * MERGE_FLOATS + 516 + j] = l_tot[hg];
-            }
-        __syncthreads();
-        float M[HG];
-#pragma unroll
-        for (int hg = 0; hg < HG; ++hg) {
-            // head j's maximum over the wavefronts that saw an unmasked position
-            M[hg] = -INFINITY;
-            const float *ml_g = merge_s + wave0 * MS + hg * MERGE_FLOATS;   // the group's first wavefront
-#pragma unroll 8
-            for (int w = 0; w < gw; ++w)
-                if (ml_g[w * MS + 516 + j] > 0.0f) M[hg] = fmaxf(M[hg], ml_g[w * MS + 512 + j]);
-            const float f = l_tot[hg] > 0.0f ? __builtin_amdgcn_exp2f(m_run[hg] - M[hg]) : 0.0f;
-            const float f4[4] = {dpp<0x00>(f), dpp<0x55>(f), dpp<0xAA>(f), dpp<0xFF>(f)};
-#pragma unroll
-            for (int hf = 0; hf < 2; ++hf)
-#pragma unroll
-                for (int i = 0; i < 4; ++i)
-                    mine[hg * MERGE_FLOATS + i * 128 + 64 * hf + lane] = (acc_o[hg][hf][0][i] + acc_o[hg][hf][1][i]) * f4[i];
-        }
-        __syncthreads();
-        for (int e = tid_g; e < 512 * HG; e += 64 * gw) {
-            const int src = (e >> 9) * MERGE_FLOATS + (e & 511);  // partial element e = head e / 128, dim e % 128
-            float sum = 0.0f;
-            const float *col = merge_s + wave0 * MS + src;
-#pragma unroll 8
-            for (int w = 0; w < gw; ++w) sum += col[w * MS];
-            st_dev(po + e, sum);
-        }
-        if (tid_g < 4) {  // lanes 0..3 of the group's first wavefront hold heads 0..3 of each set
-#pragma unroll
-            for (int hg = 0; hg < HG; ++hg) {
-                float L = 0.0f;
-                const float *ml_g = merge_s + wave0 * MS + hg * MERGE_FLOATS;
-#pragma unroll 8
-                for (int w = 0; w < gw; ++w) {
-                    const float lw = ml_g[w * MS + 516 + j];
-                    if (lw > 0.0f) L = fmaf(lw, __builtin_amdgcn_exp2f(ml_g[w * MS + 512 + j] - M[hg]), L);
-                }
-                st_dev(pml + 2 * (4 * hg + j), M[hg]);
-                st_dev(pml + 2 * (4 * hg + j) + 1, L);
-            }
-        }
+            for (int i = 0; i < 4; ++i) mine[hg * MERGE_FLOATS + i * 128 + 64 * hf + lane] = acc_o[hg][hf][0][i] + acc_o[hg][hf][1][i];
+        if (lane < 4) *reinterpret_cast<float2 *>(mine + hg * MERGE_FLOATS + 512 + 2 * j) = make_float2(m_run[hg], l_tot[hg]);
     }
-    if constexpr (SPARSE) {
-        // one slot per workgroup, added up by the merge kernel: thousands of wavefronts finishing together
-        // on one atomic would queue for longer than the kernel's own tail, and nothing needs clearing
-        if (lane == 0 && nskip) atomicAdd(&skipped, nskip);
-        __syncthreads();
-        if (tid == 0) st_dev(a.skip_slots + blockIdx.x, (a.nonce & ~SKIP_COUNT_MASK) | (unsigned long long)skipped);
-    }
-
-    // ---- the group's last workgroup merges the partials and writes the output rows -----------------
-    const int n_parts = wgs_per_group;
-    wait_stores();  // this lane's part of the partial (and the skip slot) is in memory
-    __syncthreads();
-    if (n_parts > 1) {
-        // Arrival counter of the group: the call's tag in the upper 40 bits, the number of workgroups whose partial is
-        // in memory in the lower 24.  One read-modify-write per workgroup; a word that does not carry the tag (whatever a
-        // fresh workspace held, or the zero a finished call leaves) counts as zero arrivals.  Read-modify-writes on one
-        // word happen one after the other, so exactly one workgroup brings the count to n_parts: it merges, and every
-        // other partial was complete in memory before its owner's increment, hence before this one's.
-        __shared__ int i_am_last;
-        if (tid == 0) {
-            unsigned long long *ctr = a.flags + (int64_t)pgroup * n_parts;
-            const unsigned long long tag = a.nonce & ~ARRIVAL_COUNT_MASK;
-            unsigned long long seen = ld_dev(ctr), count;
-            for (;;) {
-                if ((seen & ~ARRIVAL_COUNT_MASK) == tag) {
-                    // the word is this call's (it stays so until the merge): a plain increment, no retry however many
-                    // workgroups arrive together
-                    count = (__hip_atomic_fetch_add(ctr, 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) & ARRIVAL_COUNT_MASK) + 1ull;
-                    break;
-                }
-                // first arrival of the call: install the tag with a count of one, unless somebody else just did
-                if (__hip_atomic_compare_exchange_strong(ctr, &seen, tag | 1ull, __ATOMIC_RELAXED, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) {
-                    count = 1ull;
-                    break;
-                }
-            }
-            i_am_last = (int)count == n_parts;
-        }
-        __syncthreads();
-        if (!i_am_last) return;
-    }
-    // Sparse V: every workgroup's slot carries its count (40 bits: at most 4 heads x 2^31 positions) under 24 bits
-    // of the nonce.  A merging workgroup reads all slots of the launch now, so that the trip to memory overlaps
-    // the merge; the one that finds them all tagged (the merging workgroup of the group that finishes last does)
-    // writes the step's total.  Launches with more workgroups than one can poll are added up by a launch of their
-    // own (poll_slots == 0).
-    int all_in = 1;
-    unsigned long long counted = 0ull;
-    if constexpr (SPARSE) {
-        if (a.poll_slots) {
-            const unsigned long long tag = a.nonce & ~SKIP_COUNT_MASK;
-            for (int g = tid; g < (int)gridDim.x; g += (int)blockDim.x) {
-                const unsigned long long word = ld_dev(a.skip_slots + g);
-                all_in &= (word & ~SKIP_COUNT_MASK) == tag;
-                counted += word & SKIP_COUNT_MASK;
-            }
-        }
-    }
-    // the wavefronts' merge space is free again (every partial of this workgroup is in memory); with several groups
-    // per workgroup every group's wavefronts finish their own group (one partial: no exchange between them)
-    merge_group<HG>(a, group, pgroup, head_off, n_parts, tid_g, gw, n_waves > 1 && a.gpw <= 1 ? merge_s : nullptr);
-    if (n_parts > 1 && tid == 0) st_dev(a.flags + (int64_t)pgroup * n_parts, 0ull);  // a replay of a captured launch (same tag) starts from zero
-    if constexpr (SPARSE) {
-        if (a.poll_slots) {
-            if (!__syncthreads_and(all_in)) return;
-            __shared__ unsigned long long red;
-            const unsigned long long pass_total = block_sum(counted, &red, tid);
-            for (int g = tid; g < (int)gridDim.x; g += (int)blockDim.x) st_dev(a.skip_slots + g, 0ull);
-            if (tid == 0) {
-                // this pass's total is kept apart so that writing the step's total twice (two groups finishing
-                // together) gives the same value both times
-                st_dev(a.pass_totals + a.pass, pass_total);
-                unsigned long long sum = pass_total;
-                for (int k = 0; k < a.pass; ++k) sum += ld_dev(a.pass_totals + k);
-                a.skip_count[0] = sum;
-                a.skip_count[1] = a.total_pairs;
-            }
-        }
-    }
+    if (SPARSE && lane == 0 && nskip) atomicAdd(&skipped, nskip);
+    finish_group<HG, SPARSE>(a, slot, group, pgroup, head_off, wgs_per_group, part, tid, tid_g, gw, wave0, merge_s, &skipped);
 }
 
 // Sparse-V bookkeeping for launches with more groups than one workgroup polls (and for a caller that asks for the
@@ -1495,9 +987,8 @@ int tqk_decode_attention(const tq_handle *hk, const tq_handle *hv, const tq_attn
     const unsigned pass_wgs = (unsigned)((int64_t)groups * pl.n_parts / pl.gpw);
     const dim3 grid(pass_wgs, n_pass);
     const unsigned wg = 64u * (unsigned)wpw;
-    const int n_parts = pl.n_parts;  // partials per group: the wavefronts of a workgroup merge theirs in LDS
     // dynamic LDS: the wavefronts' merge space, then the staged queries of the workgroup's groups
-    const size_t merge_bytes = (wpw > 1 ? (size_t)wpw * hg * MERGE_FLOATS * sizeof(float) : 0) + (size_t)pl.gpw * 1024 * hg;
+    const size_t merge_bytes = (size_t)wpw * hg * MERGE_FLOATS * sizeof(float) + (size_t)pl.gpw * 1024 * hg;
     a.gpw = pl.gpw;
     a.gw_shift = 0;
     while ((1 << a.gw_shift) < p->n_splits) ++a.gw_shift;
@@ -1522,7 +1013,6 @@ int tqk_decode_attention(const tq_handle *hk, const tq_handle *hv, const tq_attn
     a.pass_totals = reinterpret_cast<unsigned long long *>((char *)ws + w.pass_totals);
     a.skip_count = skip_count;
     a.total_pairs = total_pairs;
-    (void)n_parts;
     (void)kb;
     for (a.head_off = 0; a.head_off < a.q_group; a.head_off += n_pass * a.pass_heads) {
         a.pass = a.head_off / a.pass_heads;
