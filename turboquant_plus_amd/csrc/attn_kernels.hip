@@ -1013,7 +1013,17 @@ int tqk_decode_attention(const tq_handle *hk, const tq_handle *hv, const tq_attn
     a.pass_totals = reinterpret_cast<unsigned long long *>((char *)ws + w.pass_totals);
     a.skip_count = skip_count;
     a.total_pairs = total_pairs;
-    (void)kb;
+    // A 4-bit side: k_decode_turbo, whose table of 64 KB has a copy per lane (16 x 8 groups at 32768 tokens, turbo4: 110 -> 97 us,
+    // eight heads 121 -> 90; turbo4 K with turbo2 V 87 -> 77 and 100 -> 78).  It has to leave the workgroups that share a CU room
+    // (25 x 8 groups at 3175 tokens in 1000 workgroups of four: 30.5 us against 28.4 here; turbo4 K with turbo3 V, 96 KB, 20 x 8
+    // groups of eight heads at 2500 tokens in 320: 32.0 against 25.7), and building it has to pay: three tiles per wavefront and
+    // four wavefronts (2 x 8 groups at 3000 tokens, three: 12.7 us against 13.2 here; 8 at 4000, two: 11.7 against 11.5; one at
+    // 300, two wavefronts: 12.1 against 11.5).  Four heads with a bias list have no registers for it (16 x 9000 tokens with 64
+    // entries: 41.4 against 38.8, with Sparse V 47.6 against 43.0), and dense bias rows keep the general variants.
+    const int tables = tqk_decode_turbo_lds(kb, vb, share) + pl.gpw * 1024 * hg;
+    const int per_cu = std::min((int)(((int64_t)pass_wgs * n_pass + 255) / 256), std::max(1, (hg == 2 ? 12 : 16) / wpw));
+    const bool lane_tables = (kb == 4 || vb == 4) && per_cu * tables <= 160 * 1024 && a.tiles_per_split >= 3 && wpw >= 4 &&
+                             !bias && (hg == 2 || !a.sbias_n);
     for (a.head_off = 0; a.head_off < a.q_group; a.head_off += n_pass * a.pass_heads) {
         a.pass = a.head_off / a.pass_heads;
         a.nonce = next_nonce();
@@ -1066,7 +1076,8 @@ int tqk_decode_attention(const tq_handle *hk, const tq_handle *hv, const tq_attn
     else if (share) TQ_ATTN_ONE(KFMT_TURBO, B, B, false, true)        \
     else if (sparse) TQ_ATTN_ONE(KFMT_TURBO, B, B, true, false)       \
     else TQ_ATTN_ONE(KFMT_TURBO, B, B, false, false)
-    if (turbo_k && kb == 3 && vb == 3) { TQ_ATTN_SAME(3); }
+    if (turbo_k && turbo_v && lane_tables && tqk_launch_decode_turbo(a, kb, vb, share, 4 * hg, sparse, grid, wpw, s)) {}
+    else if (turbo_k && kb == 3 && vb == 3) { TQ_ATTN_SAME(3); }
     else if (turbo_k && kb == 4 && vb == 4) { TQ_ATTN_SAME(4); }
     else if (turbo_k && kb == 2 && vb == 2) { TQ_ATTN_SAME(2); }
     else if (turbo_k && kb == 4 && vb == 2) { TQ_ATTN(KFMT_TURBO, 4, 2); }

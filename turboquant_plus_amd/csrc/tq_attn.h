@@ -564,3 +564,9 @@ __device__ __forceinline__ void finish_group(const AttnArgs &a, Slot slot, int g
 }
 
 }  // namespace tqattn
+
+// attn_turbo_kernels.hip: turbo K and V rows of 128-dim heads, 4-bit on one side or both, n_heads (4 or 8) query heads per pass;
+// false: another pair; and the static LDS of a workgroup
+int tqk_decode_turbo_lds(int kb, int vb, bool share);
+bool tqk_launch_decode_turbo(const tqattn::AttnArgs &a, int kb, int vb, bool share, int n_heads, bool sparse, dim3 grid, int waves,
+                             hipStream_t s);
