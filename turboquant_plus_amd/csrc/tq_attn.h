@@ -565,8 +565,11 @@ __device__ __forceinline__ void finish_group(const AttnArgs &a, Slot slot, int g
 
 }  // namespace tqattn
 
-// attn_turbo_kernels.hip: turbo K and V rows of 128-dim heads, 4-bit on one side or both, n_heads (4 or 8) query heads per pass;
-// false: another pair; and the static LDS of a workgroup
-int tqk_decode_turbo_lds(int kb, int vb, bool share);
+// Launchers of the kernel files; kb, vb: code widths (8: q8_0-style rows), hg: sets of four heads per pass; false: no such pair.
+// attn_turbo_kernels.hip: 128-dim heads, turbo rows, 4-bit on one side or both; n_heads 4 or 8; and a workgroup's static LDS
 bool tqk_launch_decode_turbo(const tqattn::AttnArgs &a, int kb, int vb, bool share, int n_heads, bool sparse, dim3 grid, int waves,
                              hipStream_t s);
+int tqk_decode_turbo_lds(int kb, int vb, bool share);
+bool tqk_launch_decode_q8(const tqattn::AttnArgs &a, int kb, int vb, int hg, bool sparse, dim3 grid, unsigned wg, size_t lds, hipStream_t s);
+bool tqk_launch_decode_256(const tqattn::AttnArgs &a, int kb, int vb, bool share, bool sparse, dim3 grid, unsigned wg, size_t lds,
+                           hipStream_t s);
