@@ -9,7 +9,8 @@ import ctypes as C
 import math
 import os
 import threading
-from concurrent.futures import Future, ThreadPoolExecutor
+from concurrent.futures import ThreadPoolExecutor
+from contextlib import contextmanager, nullcontext
 
 import numpy as np
 
@@ -39,6 +40,20 @@ class TQAttnParams(C.Structure):
                 ("scale", C.c_float), ("sparse_v_tau", C.c_float), ("tokens_dev", C.c_void_p),
                 ("bias_entries", C.c_int32), ("bias_pos", C.c_void_p), ("bias_val", C.c_void_p),
                 ("head_dim", C.c_int32)]
+
+
+HOST_SLOTS = 8
+HOST_FETCH, HOST_WIDEN, HOST_UPLOAD, HOST_NARROW = 0, 1, 2, 3
+
+
+class TQHostJob(C.Structure):
+    _fields_ = [("kind", C.c_int64), ("n", C.c_int64), ("n_pieces", C.c_int64), ("piece", C.c_int64), ("host", C.c_void_p),
+                ("other", C.c_void_p), ("slots", C.c_void_p), ("seen", C.c_int64), ("next", C.c_int64), ("ready", C.c_int64),
+                ("done", C.c_int64), ("slot_done", C.c_int32 * HOST_SLOTS)]
+
+
+class TQHostSession(C.Structure):
+    _fields_ = [("job", C.c_void_p), ("users", C.c_int64), ("bell", C.c_int32), ("closed", C.c_int32)]
 
 
 _P, _I, _L, _D = C.c_void_p, C.c_int, C.c_int64, C.c_double
@@ -92,6 +107,9 @@ PROTOTYPES = {
     "tq_attn_workspace_bytes": (_L, [C.POINTER(TQAttnParams)]),
     "tq_decode_attention": (_I, [_P, _P, C.POINTER(TQAttnParams), _P, _I, _P, _P, _P, _P, _P, _P, _P, _L, _P]),
     "tq_decode_attention_static": (_I, [_P, _P, C.POINTER(TQAttnParams), _P, _I, _P, _P, _P, _P, _P, _P]),
+    "tq_host_serve": (None, [C.POINTER(TQHostSession)]),
+    "tq_host_close": (None, [C.POINTER(TQHostSession)]),
+    "tq_host_drive": (_I, [C.POINTER(TQHostSession), C.POINTER(TQHostJob), _P, _P]),
     "tq_score_tile": (_I, [_P, _P, _I, _L, _P, _P, _P, _L, _P, _I, _P, _L, _P]),
 }
 
@@ -181,7 +199,7 @@ def to_device(x, float_ok=(np.float16, np.float32, np.float64)):
     a = np.asarray(x)
     if a.dtype not in [np.dtype(f) for f in float_ok]:
         a = a.astype(np.float64)
-    return tt.from_numpy(np.ascontiguousarray(a)).to(require_gpu())
+    return _upload_one(np.ascontiguousarray(a), require_gpu())
 
 
 # ---- results of the NumPy classes: device buffers and their way into host arrays -----------------------------------
@@ -208,13 +226,14 @@ def device_block(*specs):
 # A block up to this size travels as one pageable copy (a copy costs 14 us before its first byte).  64 rows of 384: 0.23 ms, 0.25
 # with 128 KiB; a cache of 2 x 4 x 512 x 128: 1.44 and 1.55.
 ONE_COPY = 1 << 19
-# Bytes of the result that one pinned staging slot holds, and threads that empty it.  Both ways through the classes, ms, with
-# slots of 1 / 4 / 8 / 16 MiB and with three / eight threads: a cache of 2 x 4 x 4096 x 128 in float32 15.3 / 14.2 / 9.3 / 9.4 and
-# 10.0 / 10.5, in float64 16.7 / 15.5 / 10.8 / 10.8 and 11.3 / 11.6; 20 000 rows of 384 in float32 14.3 / 13.2 / 9.2 / 8.1 and 10.0 /
-# 10.0, 4096 of 1536 in float64 18.8 / 21.3 / 9.9 / 9.5 and 11.3 / 10.5; 256 rows of 1536 and a cache of 2 x 4 x 512 x 128 alike with
-# all of them.  On one host with 16 CPUs; with fewer the threads are the limit.
-STAGE = 8 << 20
-COPY_THREADS = 6
+# Bytes of the host array that a thread takes at a time (no two threads clear the same huge page), and the threads beside the
+# caller's.  A cache of 2 x 4 x 4096 x 128 in float32, both ways, ms, with pieces of 1 / 2 / 4 MiB: four threads 9.6 / 8.6 / 8.5, six
+# 8.9 / 8.6 / 8.0, eight 9.1 / 7.8 / 7.6, eleven 9.1 / 8.4 / 7.9 (16 CPUs); through the interpreter, which handed a share of each slot to six
+# threads, 9.4 - 11.0, 16 000 rows of 128 10.1 (now 4.5 - 5.4), 2 x 4 x 2048 x 256 in float64 11.9 - 13.7 (9.0).
+STAGE = 4 << 20
+COPY_THREADS = 8
+# Host arrays from this size on are worked on by several threads: below, handing the work over costs more.
+SHARED = 4 << 20
 _copiers = None
 _copiers_lock = threading.Lock()
 
@@ -236,94 +255,85 @@ def _forget_copiers():
 os.register_at_fork(after_in_child=_forget_copiers)
 
 
-def _hand_over(fn, *args):
-    """A future of fn(*args), run on the copy threads or, where those take no more work (the interpreter is ending, no
-    thread can be started), here.  A submit that fails may have queued the work all the same: who comes first runs it."""
-    done, claim = Future(), threading.Lock()
+_helping = threading.local()     # .session: this thread's, while it has one
 
-    def run():
-        if claim.acquire(blocking=False):
-            try:
-                done.set_result(fn(*args))
-            except BaseException as e:
-                done.set_exception(e)
+
+_alone = nullcontext()
+
+
+def helpers(nbytes):
+    """A context in which the copy threads help with this thread's host arrays where those are large (`nbytes`: the largest
+    one's): one handing over for all the arrays of a call.  Where there are no threads (the ending interpreter takes no more work, a
+    forked child starts its own) the caller's does it all."""
+    return _alone if nbytes <= SHARED or getattr(_helping, "session", None) is not None else _helped()
+
+
+@contextmanager
+def _helped():
+    session = TQHostSession()
+    serve = lib().tq_host_serve
     try:
-        _copy_pool().submit(run)
-    except RuntimeError:
-        run()
-    return done
+        try:
+            for _ in range(COPY_THREADS):
+                _copy_pool().submit(serve, session)     # the queue keeps the session's memory as long as it may be looked at
+        except RuntimeError:
+            pass
+        _helping.session = session
+        yield
+    finally:
+        _helping.session = None
+        lib().tq_host_close(session)
 
 
-def _shares(n, item_bytes):
-    """(start, stop) shares of n elements for the copy threads: one per MiB, at most COPY_THREADS.  Up to 4 MiB one
-    thread does it all: handing the work over costs more (256 vectors of 1536 both ways: 0.8 against 1.4 ms)."""
-    k = min(COPY_THREADS, n * item_bytes >> 20) if n * item_bytes > 4 << 20 else 1
-    return [(n * i // k, n * (i + 1) // k) for i in range(k)]
-
-
-def _fetch_staged(t, out):
-    """A large contiguous device tensor into the NumPy array `out` (same shape; a wider integer type is filled by
-    conversion).  Fresh host memory costs more than the transfer (64 MiB: 9.3 ms by one pageable copy, 1.2 ms of them
-    PCIe): the bytes come through two pinned slots while the copy threads empty them into `out`."""
-    tt = torch()
-    src, dst = t.reshape(-1), out.reshape(-1)
-    step = max(min(STAGE, out.nbytes // 4), 1 << 18) // out.itemsize
-    slots = [tt.empty(step, dtype=t.dtype, pin_memory=True) for _ in range(2)]
-    host = [s.numpy() for s in slots]
-    done = [tt.cuda.Event() for _ in slots]
-    work = [[], []]
-    n = src.numel()
-
-    def empty_slot(i, at, count):
-        done[i].synchronize()
-        shares = _shares(count, dst.itemsize)
-        if len(shares) == 1:
-            np.copyto(dst[at:at + count], host[i][:count])
-        else:
-            work[i] = [_hand_over(np.copyto, dst[at + a:at + b], host[i][a:b]) for a, b in shares]
-
-    last = None
-    for k, at in enumerate(range(0, n, step)):
-        i, count = k & 1, min(step, n - at)
-        for w in work[i]:
-            w.result()
-        work[i] = []
-        slots[i][:count].copy_(src[at:at + count], non_blocking=True)
-        done[i].record()
-        if last is not None:
-            empty_slot(*last)
-        last = (i, at, count)
-    if last is not None:
-        empty_slot(*last)
-    for w in work[0] + work[1]:
-        w.result()
+def _host_job(kind, n, host, *, other=None, device=None):
+    """A job of n elements (include/tq.h) on the contiguous array `host`: with pinned slots to or from the device tensor
+    `device`, or into the array `other`.  Returns the bits that HOST_NARROW saw."""
+    each = 8 if kind in (HOST_WIDEN, HOST_NARROW) else 1       # host bytes of an element; one on the other side
+    piece = max(min(STAGE, n * each // 4), 1 << 18) // each
+    pieces = -(-n // piece)
+    job = TQHostJob(kind=kind, n=n, n_pieces=pieces, piece=piece, host=host.ctypes.data, other=None if other is None else other.ctypes.data)
+    stream = None
+    if device is not None:
+        slots = torch().empty(min(HOST_SLOTS, pieces) * piece, dtype=torch().uint8, pin_memory=True)
+        job.slots, stream = slots.data_ptr(), stream_ptr()
+    if n * each <= SHARED:
+        check(lib().tq_host_drive(None, job, ptr(device), stream))
+    else:
+        with helpers(n * each):
+            check(lib().tq_host_drive(_helping.session, job, ptr(device), stream))
+    return job.seen
 
 
 def narrow_indices(indices, n_centroids):
     """Codebook indices of any type as contiguous uint8; ValueError if one is outside 0 .. n_centroids - 1 (a power of
-    two).  int64 ones, what the classes return, are checked and narrowed in one go by the copy threads."""
-    def refuse():
-        raise ValueError("indices out of range for this codebook")
+    two).  int64 ones, what the classes return, are checked and narrowed in one go."""
     if indices.dtype != np.int64 or not indices.flags.c_contiguous:
         if indices.size and (indices.min() < 0 or indices.max() >= n_centroids):
-            refuse()
+            _refuse_indices()
         return np.ascontiguousarray(indices, dtype=np.uint8)
     out = np.empty(indices.shape, np.uint8)
-    src, dst = indices.reshape(-1), out.reshape(-1)
-
-    def share(a, b):
-        np.copyto(dst[a:b], src[a:b], casting="unsafe")
-        return int(np.bitwise_or.reduce(src[a:b])) if b > a else 0     # a bit above the codebook's: some index is outside
-    shares = _shares(src.size, 8)
-    if len(shares) == 1:
-        seen = share(*shares[0])
+    if indices.nbytes > SHARED:
+        seen = _host_job(HOST_NARROW, indices.size, indices, other=out)
     else:
-        seen = 0
-        for w in [_hand_over(share, a, b) for a, b in shares]:
-            seen |= w.result()
-    if seen & ~(n_centroids - 1):
-        refuse()
+        np.copyto(out, indices, casting="unsafe")
+        seen = int(np.bitwise_or.reduce(indices, axis=None))
+    if seen & ~(n_centroids - 1):       # a bit above the codebook's: some index is outside
+        _refuse_indices()
     return out
+
+
+def _refuse_indices():
+    raise ValueError("indices out of range for this codebook")
+
+
+def upload_indices(indices, n_centroids, *others):
+    """Device tensors of codebook indices (uint8; checked as narrow_indices does) and of further arrays (upload)."""
+    if indices.dtype != np.int64 or not indices.flags.c_contiguous or indices.nbytes <= SHARED:
+        return upload(narrow_indices(indices, n_centroids), *others)
+    t = torch().empty(indices.shape, dtype=torch().uint8, device=require_gpu())
+    if _host_job(HOST_NARROW, indices.size, indices, device=t) & ~(n_centroids - 1):
+        _refuse_indices()
+    return [t, *upload(*others)]
 
 
 def fetch(buf, *wanted):
@@ -342,10 +352,12 @@ def fetch(buf, *wanted):
     res = []
     for t, dtype in wanted:
         a = np.empty(tuple(t.shape), dtype)
-        if t.nbytes > ONE_COPY:
-            _fetch_staged(t, a)
+        same = a.dtype == _NP_DTYPES[str(t.dtype)]
+        if t.nbytes > ONE_COPY and (same or (t.dtype == tt.uint8 and dtype == np.int64)):
+            # fresh host memory costs more than the transfer (64 MiB: 9.3 ms by one pageable copy, 1.2 ms of them the link)
+            _host_job(HOST_FETCH if same else HOST_WIDEN, a.nbytes if same else a.size, a, device=t)
         else:
-            src = a if a.dtype == _NP_DTYPES[str(t.dtype)] else np.empty(tuple(t.shape), _NP_DTYPES[str(t.dtype)])
+            src = a if same else np.empty(tuple(t.shape), _NP_DTYPES[str(t.dtype)])
             tt.from_numpy(src).copy_(t)
             if src is not a:
                 np.copyto(a, src)
@@ -355,7 +367,7 @@ def fetch(buf, *wanted):
 
 def _torch_dtype(dt):
     tt = torch()
-    return {"u1": tt.uint8, "i1": tt.int8, "f8": tt.float64}[dt.str[1:]]
+    return {"u1": tt.uint8, "i1": tt.int8, "f2": tt.float16, "f4": tt.float32, "f8": tt.float64}[dt.str[1:]]
 
 
 _NP_DTYPES = {"torch.uint8": np.dtype(np.uint8), "torch.int8": np.dtype(np.int8), "torch.float64": np.dtype(np.float64)}
@@ -369,12 +381,21 @@ def host_norms(norms, n):
     return a
 
 
+def _upload_one(a, dev):
+    tt = torch()
+    if a.nbytes < SHARED // 2:
+        return tt.from_numpy(a if a.flags.writeable else a.copy()).to(dev)   # torch warns of read-only memory
+    t = tt.empty(a.shape, dtype=_torch_dtype(a.dtype), device=dev)
+    _host_job(HOST_UPLOAD, a.nbytes, a, device=t)
+    return t
+
+
 def upload(*arrays):
     """Contiguous NumPy arrays -> device tensors; small ones in one copy."""
     tt = torch()
     dev = require_gpu()
     if sum(a.nbytes for a in arrays) > ONE_COPY:
-        return [tt.from_numpy(a if a.flags.writeable else a.copy()).to(dev) for a in arrays]   # torch warns of read-only memory
+        return [_upload_one(a, dev) for a in arrays]
     offs, total = [], 0
     for a in arrays:
         offs.append(total)

@@ -74,10 +74,11 @@ class KVCacheCompressor:
         k_rows, v_rows = np.asarray(k_cache).reshape(L * H * S, D), np.asarray(v_cache).reshape(L * H * S, D)
         if self._on_device():   # both tensors are on their way before the first results are waited for
             kq, vq = self.k_quantizer, self.v_quantizer.polar_quant
-            k_block = kq._launch_quantize(lib.to_device(k_rows))
-            v_block = vq._start_quantize(v_rows)
-            k_idx, k_nrm, k_sgn, k_rn = kq._fetch(k_block)
-            vi, vn = vq._fetch(v_block)
+            with lib.helpers(8 * k_rows.size):     # results of 8 bytes per value
+                k_block = kq._launch_quantize(lib.to_device(k_rows))
+                v_block = vq._start_quantize(v_rows)
+                k_idx, k_nrm, k_sgn, k_rn = kq._fetch(k_block)
+                vi, vn = vq._fetch(v_block)
         else:
             kc = self.k_quantizer.quantize(k_rows)
             k_idx, k_nrm, k_sgn, k_rn = kc.mse_indices, kc.vector_norms, kc.qjl_signs, kc.residual_norms
@@ -99,10 +100,11 @@ class KVCacheCompressor:
             return z, z.copy()
         kc = CompressedVector(_joined([c.mse_indices for c in flat]), _joined([c.vector_norms for c in flat]),
                               _joined([c.qjl_signs for c in flat]), _joined([c.residual_norms for c in flat]), self.k_bits)
-        k = self.k_quantizer.dequantize(kc).reshape(L, H, S, D)
         vi = _joined([compressed.v_indices[l][h] for l in range(L) for h in range(H)])
         vn = _joined([compressed.v_norms[l][h] for l in range(L) for h in range(H)])
-        v = self.v_quantizer.dequantize(vi, vn).reshape(L, H, S, D)
+        with lib.helpers(8 * L * H * S * D if self._on_device() else 0):
+            k = self.k_quantizer.dequantize(kc).reshape(L, H, S, D)
+            v = self.v_quantizer.dequantize(vi, vn).reshape(L, H, S, D)
         return k, v
 
     def memory_stats(self, seq_len: int, num_layers: int, num_heads: int) -> dict:

@@ -99,7 +99,7 @@ class PolarQuant:
             norms = np.array([norms])
         self._check(indices, "dequantize")
         tt = L.torch()
-        idx, nrm = L.upload(L.narrow_indices(indices, self.n_centroids), L.host_norms(norms, indices.shape[0]))
+        idx, nrm = L.upload_indices(indices, self.n_centroids, L.host_norms(norms, indices.shape[0]))
         buf, (out,) = L.device_block(((idx.shape[0], self.d), tt.float64))
         self._launch_dequantize(idx, nrm, out)
         out_h = L.fetch(buf, (out, np.float64))[0]
@@ -114,7 +114,7 @@ class PolarQuant:
         self._check(i2, "dequantize")
         self._check(x2, "quantize")
         xd = L.to_device(x2)
-        idx, nrm = L.upload(L.narrow_indices(i2, self.n_centroids), L.host_norms(norms, i2.shape[0]))
+        idx, nrm = L.upload_indices(i2, self.n_centroids, L.host_norms(norms, i2.shape[0]))
         buf, (res,) = L.device_block((tuple(i2.shape), tt.float64))
         self._launch_residual(xd, idx, nrm, res)
         res_h = L.fetch(buf, (res, np.float64))[0]

@@ -65,7 +65,8 @@ class TurboQuant:
             signs, rnorms = self.qjl.quantize(residual)
         else:
             self.polar_quant._check(x2, "quantize")
-            idx, norms, signs, rnorms = self._fetch(self._launch_quantize(L.to_device(x2)))
+            with L.helpers(8 * x2.size):
+                idx, norms, signs, rnorms = self._fetch(self._launch_quantize(L.to_device(x2)))
             if single:
                 idx, norms, signs, rnorms = idx[0], norms[0], signs[0], rnorms[0]
         return CompressedVector(mse_indices=idx, vector_norms=norms, qjl_signs=signs, residual_norms=rnorms,
@@ -82,12 +83,13 @@ class TurboQuant:
         self.polar_quant._check(idx, "dequantize")
         n = idx.shape[0]
         tt = L.torch()
-        idx_d, norms_d, signs_d, rnorms_d = L.upload(L.narrow_indices(idx, self.polar_quant.n_centroids), L.host_norms(norms, n),
-                                                     np.ascontiguousarray(signs, dtype=np.int8), L.host_norms(rnorms, n))
-        buf, (out,) = L.device_block(((n, self.d), tt.float64))
-        self.polar_quant._launch_dequantize(idx_d, norms_d, out)
-        self.qjl._launch_dequantize(signs_d, rnorms_d, shrinkage, out, add=True)
-        out_h = L.fetch(buf, (out, np.float64))[0]
+        with L.helpers(8 * idx.size):
+            idx_d, norms_d, signs_d, rnorms_d = L.upload_indices(idx, self.polar_quant.n_centroids, L.host_norms(norms, n),
+                                                                 np.ascontiguousarray(signs, dtype=np.int8), L.host_norms(rnorms, n))
+            buf, (out,) = L.device_block(((n, self.d), tt.float64))
+            self.polar_quant._launch_dequantize(idx_d, norms_d, out)
+            self.qjl._launch_dequantize(signs_d, rnorms_d, shrinkage, out, add=True)
+            out_h = L.fetch(buf, (out, np.float64))[0]
         return out_h[0] if single else out_h
 
     def compressed_size_bits(self, n_vectors: int) -> int:
