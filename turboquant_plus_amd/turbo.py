@@ -15,6 +15,7 @@ copied to the device first.
 from __future__ import annotations
 
 import ctypes as C
+import functools
 import math
 import os
 
@@ -494,6 +495,10 @@ class DecodeAttention:
                                                         sparse_v=sparse_v_tau > 0)
                 plain = own(False)      # a bias list changes the plan of eight heads on turbo K, and the rule for 8-bit V rows
                 self._own_splits = (plain, own(True) if k_codec is not None and (eight or v_codec is None) else plain)
+                if len(bits) == 2 and sparse_v_tau == 0:
+                    same = bits[0] == bits[1] and np.array_equal(k_codec.centroids, v_codec.centroids)
+                    self._own_splits = (turbo_splits(batch * n_kv_heads, tokens, plain, k_bits=bits[0], v_bits=bits[1], one_table=same,
+                                                     eight_heads=eight), self._own_splits[1])
             n_splits = self._own_splits[0]
         else:
             self._own_splits = (n_splits, n_splits)
@@ -712,3 +717,58 @@ def balanced_splits(n_groups: int, tokens: int, default: int, *, eight_heads: bo
         return default
     best = min(counts, key=estimate)
     return best if estimate(best) < (0.88 if turbo_v or not eight_heads else 0.82) * estimate(default) else default
+
+
+# What a step on turbo rows takes since its end became cheaper and 4-bit rows got tables with a copy per lane, in microseconds: a
+# constant, per tile on the busiest SIMD of the fullest CU (times four), per tile on the longest wavefront of each round of
+# workgroups, per partial of a group, per round, per partial beyond 16, per further round of workgroups of twelve.  Fitted to the
+# timings of 15 700 drawn shapes (1 to 300 groups, 512 to 131 072 tokens, up to nine counts each); ratios between counts of one shape
+# scatter by 7 - 9 %, 11 % for eight heads in the general kernel.
+_TURBO_COST = {  # by (more than four heads, widest code, table copies per lane)
+    (False, 2, False): (2.109, 0.189, 0.336, 0.106, 4.461, -0.033, 0.0),
+    (False, 3, False): (2.639, 0.225, 0.356, 0.116, 4.358, -0.048, 0.0),
+    (False, 4, False): (4.371, 0.352, -0.337, 0.096, 3.723, -0.024, 0.0),
+    (False, 4, True): (1.546, 0.219, 0.551, 0.143, 6.434, -0.073, 0.0),
+    (True, 4, False): (2.731, 0.313, 0.531, 0.227, 5.372, -0.07, 2.038),
+    (True, 4, True): (1.829, 0.206, 0.634, 0.258, 6.542, -0.104, 1.304),
+}
+
+
+@functools.lru_cache(maxsize=256)
+def turbo_splits(n_groups: int, tokens: int, current: int, *, k_bits: int, v_bits: int, one_table: bool, eight_heads: bool) -> int:
+    """The split count of a step on turbo K and V rows of 128-dim heads without a bias list or Sparse V: `current` (balanced_splits)
+    unless the estimate puts another count, down to one tile per wavefront, 12 % ahead (at 8 % up to 3 % of the shapes got more than
+    3 % slower).  Over the 15 700 shapes a quarter of the four-head steps with 4-bit rows change, which makes all of them 4.1 %
+    faster on average, a tenth of the others (turbo3 1.3 %, turbo2 0.9 %, eight heads with 4-bit rows 1.4 %); 0.2 to 0.8 % of them are
+    more than 3 % slower.  Eight heads without a 4-bit side keep `current` (the estimate is wrong by up to a third there); with
+    one, workgroups of three and six wavefronts and more than three per CU are left out, where it was wrong by 15 - 23 %."""
+    widest = max(k_bits, v_bits)
+    if (eight_heads, widest, False) not in _TURBO_COST:
+        return current
+    tiles, sets = max(1, (tokens + 63) // 64), 2 if eight_heads else 1
+    general, copied = _TURBO_COST[eight_heads, widest, False], _TURBO_COST.get((eight_heads, widest, True))
+    # LDS of a workgroup's tables: 2 and 3 bits, 4 bits (1 KB), 4 bits with a copy per lane (64 KB)
+    table = (0, 0, 2048, 32768, 1024)
+    lds_pair = table[k_bits] + (0 if one_table else table[v_bits])
+    lds_lane = 1024 + sum(65536 if b == 4 else table[b] for b in ((k_bits,) if one_table else (k_bits, v_bits)))
+    most = 12 if eight_heads else 16
+    best, best_time, now = current, math.inf, math.inf
+    for n in (current, *_SPLIT_COUNTS):
+        if now < math.inf and not (n <= tiles and 200 <= n * n_groups <= 8192):
+            continue
+        waves, parts, wgs = _workgroups(n, n_groups, eight_heads, True, True)
+        if now < math.inf and eight_heads and (waves in (3, 6) or wgs > 3 * 256):
+            continue
+        per_cu, deep, fit = -(-wgs // 256), -(-tiles // n), max(1, most // waves)
+        queries = max(1, waves // n) * _QUERY_BYTES * sets
+        cost, lds = general, lds_pair + sets * waves * _WAVE_MERGE_BYTES + queries
+        if copied and min(per_cu, fit) * (lds_lane + queries) <= _LDS_PER_CU and deep >= 3 and waves >= 4:      # the launcher's rule
+            cost, lds = copied, lds_lane + queries
+        rounds = -(-per_cu // max(1, min(fit, _LDS_PER_CU // lds)))
+        took = (cost[0] + cost[1] * per_cu * 4 * -(-waves // 4) * deep + cost[2] * rounds * deep + cost[3] * parts + cost[4] * rounds
+                + cost[5] * max(0, parts - 16) + (cost[6] * (rounds - 1) if waves == 12 else 0.0))
+        if now == math.inf:
+            now = took          # the first is `current`
+        if took < best_time:
+            best, best_time = n, took
+    return best if best_time < 0.88 * now else current
