@@ -729,6 +729,8 @@ _TURBO_COST = {  # by (more than four heads, widest code, table copies per lane)
     (False, 3, False): (2.639, 0.225, 0.356, 0.116, 4.358, -0.048, 0.0),
     (False, 4, False): (4.371, 0.352, -0.337, 0.096, 3.723, -0.024, 0.0),
     (False, 4, True): (1.546, 0.219, 0.551, 0.143, 6.434, -0.073, 0.0),
+    (True, 2, False): (6.872, 0.181, 0.718, 0.25, 0.349, -0.098, 6.371),
+    (True, 3, False): (7.115, 0.203, 0.857, 0.249, 0.644, -0.093, 6.953),
     (True, 4, False): (2.731, 0.313, 0.531, 0.227, 5.372, -0.07, 2.038),
     (True, 4, True): (1.829, 0.206, 0.634, 0.258, 6.542, -0.104, 1.304),
 }
@@ -737,13 +739,13 @@ _TURBO_COST = {  # by (more than four heads, widest code, table copies per lane)
 @functools.lru_cache(maxsize=256)
 def turbo_splits(n_groups: int, tokens: int, current: int, *, k_bits: int, v_bits: int, one_table: bool, eight_heads: bool) -> int:
     """The split count of a step on turbo K and V rows of 128-dim heads without a bias list or Sparse V: `current` (balanced_splits)
-    unless the estimate puts another count, down to one tile per wavefront, 12 % ahead (at 8 % up to 3 % of the shapes got more than
+    unless the estimate puts another count, down to one tile per wavefront, 12 % ahead (at 8 % up to 6 % of the shapes got more than
     3 % slower).  Over the 15 700 shapes a quarter of the four-head steps with 4-bit rows change, which makes all of them 4.1 %
-    faster on average, a tenth of the others (turbo3 1.3 %, turbo2 0.9 %, eight heads with 4-bit rows 1.4 %); 0.2 to 0.8 % of them are
-    more than 3 % slower.  Eight heads without a 4-bit side keep `current` (the estimate is wrong by up to a third there); with
-    one, workgroups of three and six wavefronts and more than three per CU are left out, where it was wrong by 15 - 23 %."""
+    faster on average, and a tenth of the others (turbo3 1.3 %, turbo2 0.9 %, eight heads 1.1 to 1.4 %); 0.1 to 0.8 % of them are more
+    than 3 % slower.  Eight heads leave out workgroups of three and six wavefronts, more than three per CU and more than 256
+    groups, where the estimate was wrong by 15 to 25 %."""
     widest = max(k_bits, v_bits)
-    if (eight_heads, widest, False) not in _TURBO_COST:
+    if eight_heads and n_groups > 256:
         return current
     tiles, sets = max(1, (tokens + 63) // 64), 2 if eight_heads else 1
     general, copied = _TURBO_COST[eight_heads, widest, False], _TURBO_COST.get((eight_heads, widest, True))
