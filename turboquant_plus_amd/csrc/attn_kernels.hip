@@ -245,7 +245,7 @@ int tqk_decode_attention(const tq_handle *hk, const tq_handle *hv, const tq_attn
     // entries: 41.4 against 38.8, with Sparse V 47.6 against 43.0), and dense bias rows keep the general variants.
     const int tables = tqk_decode_turbo_lds(kb, vb, share) + pl.gpw * 1024 * hg;
     const int per_cu = std::min((int)(((int64_t)pass_wgs * n_pass + 255) / 256), std::max(1, (hg == 2 ? 12 : 16) / wpw));
-    const bool lane_tables = turbo_k && turbo_v && (kb == 4 || vb == 4) && per_cu * tables <= 160 * 1024 && a.tiles_per_split >= 3 && wpw >= 4 &&
+    const bool lane_tables = !TQ_PAIRTAB3 && turbo_k && turbo_v && (kb == 4 || vb == 4) && per_cu * tables <= 160 * 1024 && a.tiles_per_split >= 3 && wpw >= 4 &&
                              !bias && (hg == 2 || !a.sbias_n);
     for (a.head_off = 0; a.head_off < a.q_group; a.head_off += n_pass * a.pass_heads) {
         a.pass = a.head_off / a.pass_heads;

@@ -6,7 +6,7 @@
 //
 //   TQ_KNOCKOUT=<bits>   fp16 store kernels with one phase removed (turbo_kernels.hip)
 //   TQ_TIMELINE          per-wavefront timestamps of the fused K+V store, read back with tq_dbg_read_timeline
-//   TQ_PAIRTAB3=1        3-bit decode attention through the conflict-free pair table (attn_kernels.hip)
+//   TQ_PAIRTAB3=1        3-bit decode attention through the conflict-free pair table (tq_attn.h)
 //   TQ_STREAM_SITES=<m>  non-temporal hints switched off per family of kernels (tq_device.h)
 #pragma once
 
