@@ -178,28 +178,31 @@ constexpr float Q8V_PRESCALE = 64.0f;  // keeps weight * scale products out of f
 // Two sets of four query heads per pass (HG = 2: GQA groups of more than four heads read K/V once per eight heads)
 // double the accumulators and the softmax state and run with at most 8 wavefronts too.
 // Wavefronts per workgroup that a variant is compiled for (its register budget follows: 16 -> 128, 12 -> 168, 8 -> 256).
-// wide12: eight heads per pass on turbo K and V rows of 128-dim heads without a bias list (dense rows or none) - 145-165 registers, so twelve
+// wide12: eight heads per pass on turbo K and V rows of 128-dim heads without a bias list - 134-164 registers, so twelve
 // wavefronts (three per SIMD) fit where two workgroups of eight do not.
 __host__ __device__ constexpr int max_waves_per_workgroup(int vbits, int hg, bool wide12 = false) {
     return vbits == 8 ? 8 : hg == 2 ? (wide12 ? 12 : 8) : 16;
 }
 
-// BIAS: none, a sparse logit bias, or dense rows with or without a list beside them.  A template parameter and not branches: the
-// list's cursor registers and per-tile test cost the eight-head variant 4 us per step when they were compiled in unconditionally,
+// BIAS: none, a sparse logit bias, dense rows, or both.  A template parameter and not branches: the list's cursor registers and
+// per-tile test cost the eight-head variant 4 us per step when they were compiled in unconditionally (in the variant of dense rows:
+// 8 to 68 bytes of scratch per lane with eight heads or 256 dims, and a wavefront per SIMD next to 8-bit rows; without them dense
+// rows of 8 x 8 groups at 8192 tokens, eight heads: turbo3 23.3 -> 21.4 us, turbo3 K with turbo4 V 28.2 -> 23.8, 8-bit K with turbo3
+// V 28.2 -> 25.6),
 // and a dense row's load that may or may not have been issued makes the compiler wait for the youngest loads, i.e. the V rows
 // just requested, at the top of every tile (4 x 20 000 tokens, turbo3, Sparse V 25.5 -> 23.4 us; 4 x 16 groups at 6000 tokens 15.1 ->
 // 14.6; one user at 4000 10.8 -> 10.5).
-constexpr int BIAS_NONE = 0, BIAS_LIST = 1, BIAS_DENSE = 2;
+constexpr int BIAS_NONE = 0, BIAS_LIST = 1, BIAS_DENSE = 2, BIAS_BOTH = BIAS_LIST | BIAS_DENSE;
 // D256: heads of 256 dims.  A token is rows 2 token and 2 token + 1 of caches that are
 // otherwise those of 128-dim heads with twice the tokens; a 64-row tile is 32 tokens.  The two sets of HG = 2 are
 // then the output's two halves of one set of four heads: one softmax, two accumulator sets.
 template <int KFMT, int KBITS, int VBITS, bool SPARSE, bool SHARE, int HG, int BIAS, bool D256 = false>
-__global__ __launch_bounds__(64 * max_waves_per_workgroup(VBITS, HG, KFMT == KFMT_TURBO && !D256 && BIAS != BIAS_LIST),
+__global__ __launch_bounds__(64 * max_waves_per_workgroup(VBITS, HG, KFMT == KFMT_TURBO && !D256 && !(BIAS & BIAS_LIST)),
                              D256 && KFMT == KFMT_TURBO && VBITS != 8 ? 4 : 1) void k_decode_attn(AttnArgs a) {
     // (256-dim heads on turbo K rows: four wavefronts per SIMD = two workgroups of eight per CU, i.e. at most 128 registers - the
     // variant sits at 119-136 without the bound, and one register over 128 halves its occupancy)
     static_assert(!D256 || HG == 2, "256-dim heads: two accumulator sets, the output's halves");
-    constexpr bool LIST = BIAS != BIAS_NONE, DENSE = BIAS == BIAS_DENSE;
+    constexpr bool LIST = (BIAS & BIAS_LIST) != 0, DENSE = (BIAS & BIAS_DENSE) != 0;
     constexpr int HQ = D256 ? 1 : HG;   // sets of four heads whose logits and softmax state the wavefront keeps
     constexpr int KROW_DW = KFMT == KFMT_TURBO ? 4 * KBITS : 32;
     constexpr int KBLOCK = KFMT == KFMT_TURBO ? TQ_ROWS_PER_BLOCK * (16 * KBITS + 2) : TQ_ROWS_PER_BLOCK * 136;
@@ -620,7 +623,7 @@ __global__ __launch_bounds__(64 * max_waves_per_workgroup(VBITS, HG, KFMT == KFM
             quad_transpose(sc[hg], lane);
             float s[4];
 #pragma unroll
-            for (int i = 0; i < 4; ++i) s[i] = LIST ? sc[hg][i] + bias4[hg][i] : sc[hg][i];
+            for (int i = 0; i < 4; ++i) s[i] = BIAS ? sc[hg][i] + bias4[hg][i] : sc[hg][i];
             if (n_valid < 64) {
 #pragma unroll
                 for (int i = 0; i < 4; ++i)
@@ -802,7 +805,8 @@ __global__ __launch_bounds__(64 * max_waves_per_workgroup(VBITS, HG, KFMT == KFM
 // by the bias that the call carries
 #define TQ_ATTN_LAUNCH(KF, KB, VB, SP, SH, HG, D256)                                                        \
     {                                                                                                      \
-        if (a.bias) k_decode_attn<KF, KB, VB, SP, SH, HG, BIAS_DENSE, D256><<<grid, wg, lds, s>>>(a);       \
+        if (a.bias && a.sbias_n) k_decode_attn<KF, KB, VB, SP, SH, HG, BIAS_BOTH, D256><<<grid, wg, lds, s>>>(a); \
+        else if (a.bias) k_decode_attn<KF, KB, VB, SP, SH, HG, BIAS_DENSE, D256><<<grid, wg, lds, s>>>(a);  \
         else if (a.sbias_n) k_decode_attn<KF, KB, VB, SP, SH, HG, BIAS_LIST, D256><<<grid, wg, lds, s>>>(a); \
         else k_decode_attn<KF, KB, VB, SP, SH, HG, BIAS_NONE, D256><<<grid, wg, lds, s>>>(a);               \
     }
