@@ -359,6 +359,20 @@ typedef struct tq_attn_params {
  * are turbo rows, which is the best shape for large steps: 256 workgroups of twelve). */
 int64_t tq_attn_workspace_bytes(const tq_attn_params *p);
 
+/* What tq_decode_attention launches for these parameters (host only: no GPU, no handles).  k_bits, v_bits: code widths of turbo rows;
+ * one_table: both sides have the same centroids; dense_bias: the call carries dense bias rows; workspace_bytes: as given to the call. */
+typedef struct {
+    int32_t passes;               /* over a KV head's rows, in one launch; a step has ceil(query heads per KV head / heads_per_pass) */
+    int32_t heads_per_pass;       /* 4 or 8 */
+    int32_t wavefronts;           /* of a workgroup */
+    int32_t partials;             /* of a KV head of one sequence, merged at the end */
+    int32_t groups_per_workgroup; /* KV heads of sequences that share a workgroup */
+    int32_t lane_tables;          /* 1: the kernel for 4-bit rows whose decode tables have a copy per lane; 0: the general one */
+    int64_t workgroups;           /* of a launch */
+} tq_attn_plan;
+int tq_decode_attention_plan(const tq_attn_params *p, int k_bits, int v_bits, int one_table, int dense_bias, int64_t workspace_bytes,
+                             tq_attn_plan *plan);
+
 /* softmax(scale * q k^T) v over packed K/V (tests/test_kv_cache.py:73-89,128-131
  * evaluated on stored codes; no reference kernel exists).
  *   q      [batch, n_q_heads, 128] q_dtype, in the ORIGINAL domain; the kernel

@@ -1,6 +1,7 @@
 """Decode steps with 4-bit rows on a side, where the look-up tables have a copy per lane: every pair of widths, four and eight
 heads per pass, Sparse V and bias lists, at the edges of the rule that takes them (three tiles per wavefront, four wavefronts
-per workgroup, room for the tables) against the oracle on the stored codes."""
+per workgroup, room for the tables) against the oracle on the stored codes.  Which of them run that kernel is checked in
+test_attention_plan.py."""
 import numpy as np
 import pytest
 
@@ -17,7 +18,7 @@ PAIRS = [(4, 4), (4, 2), (4, 3), (3, 4), (2, 4)]
 @pytest.mark.parametrize("kbits,vbits", PAIRS)
 def test_every_pair_of_widths(kbits, vbits, G):
     # tiles per wavefront: 3 with a ragged last tile, 2 (the general variant), 3 with splits that have no tile at all
-    for seed, (N, n_splits) in enumerate([(12 * 64 - 27, 4), (8 * 64, 4), (25 * 64 + 1, 12)]):
+    for seed, (N, n_splits) in enumerate([(12 * 64 - 27, 4), (8 * 64, 4), (17 * 64 + 1, 8)]):
         k, v, kc, vc, kp, vp = make_kv(2, 2, N, seed=10 * kbits + seed, kbits=kbits, vbits=vbits)
         q = np.random.default_rng(seed).standard_normal((2, 2 * G, D)).astype(np.float16)
         attn = tqa.DecodeAttention(kc, vc, 2, 2 * G, 2, N, n_splits=n_splits, poison_output=True)
@@ -71,7 +72,7 @@ def test_context_length_read_from_memory():
     k, v, kc, vc, kp, vp = make_kv(1, 2, N, seed=3, kbits=4, vbits=4)
     q = np.random.default_rng(5).standard_normal((1, 2 * G, D)).astype(np.float16)
     now = tt.zeros(1, dtype=tt.int64, device="cuda")
-    attn = tqa.DecodeAttention(kc, vc, 1, 2 * G, 2, N, n_splits=12, tokens_on_device=now, poison_output=True)
+    attn = tqa.DecodeAttention(kc, vc, 1, 2 * G, 2, N, n_splits=8, tokens_on_device=now, poison_output=True)
     for t in (N, N - 1, 700, 65, 1):
         now.fill_(t)
         ref, _, _ = reference_attention(q, kc, vc, kp, vp, 1, 2 * G, 2, t, 1 / np.sqrt(D), capacity=N)

@@ -42,6 +42,11 @@ class TQAttnParams(C.Structure):
                 ("head_dim", C.c_int32)]
 
 
+class TQAttnPlan(C.Structure):
+    _fields_ = [("passes", C.c_int32), ("heads_per_pass", C.c_int32), ("wavefronts", C.c_int32), ("partials", C.c_int32),
+                ("groups_per_workgroup", C.c_int32), ("lane_tables", C.c_int32), ("workgroups", C.c_int64)]
+
+
 HOST_SLOTS = 8
 HOST_FETCH, HOST_WIDEN, HOST_UPLOAD, HOST_NARROW = 0, 1, 2, 3
 
@@ -105,6 +110,7 @@ PROTOTYPES = {
     "tq_q8_0_unpack_v": (_I, [_P, _L, _L, _P, _P, _P]),
     "tq_q8_0_append": (_I, [_P, _L, _L, _L, _L, _I, _I, _P, _P]),
     "tq_attn_workspace_bytes": (_L, [C.POINTER(TQAttnParams)]),
+    "tq_decode_attention_plan": (_I, [C.POINTER(TQAttnParams), _I, _I, _I, _I, _L, C.POINTER(TQAttnPlan)]),
     "tq_decode_attention": (_I, [_P, _P, C.POINTER(TQAttnParams), _P, _I, _P, _P, _P, _P, _P, _P, _P, _L, _P]),
     "tq_decode_attention_static": (_I, [_P, _P, C.POINTER(TQAttnParams), _P, _I, _P, _P, _P, _P, _P, _P]),
     "tq_host_serve": (None, [C.POINTER(TQHostSession)]),

@@ -117,7 +117,56 @@ WsLayout ws_layout(const tq_attn_params *p, int passes) {
     return w;
 }
 
+// What a call launches: workgroups, passes in one launch, and which kernel.  kb, vb: code widths, 8 for q8_0-style rows; share: K
+// and V decode through one table; dense: the call carries dense bias rows.
+struct StepPlan : AttnPlan {
+    int n_pass;        // passes of one launch
+    int64_t pass_wgs;  // workgroups of a pass
+    bool lane_tables;  // k_decode_turbo
+};
+StepPlan step_plan(const tq_attn_params *p, int kb, int vb, bool share, bool dense, int64_t ws_bytes) {
+    StepPlan pl;
+    // wavefronts per workgroup: the largest power of two up to 16 (8 for int8 V rows and for eight heads per pass)
+    // that divides the split count
+    static_cast<AttnPlan &>(pl) = attn_plan(p, p->bias_entries > 0);
+    // All passes in one launch where the workspace has room: each is a chain of its own (launch, first rows, merge), one of few
+    // groups leaves most of the chip idle, and they read the same rows.  Steps of two passes over 256-dim heads (us with the
+    // append, one pass after the other / together): 2 x 8 KV heads x 259 tokens turbo4 35.0 / 19.6, 4 x 8 x 4000 turbo3 50.5 / 32.8,
+    // 1 x 1 x 100 000 turbo2 169 / 95, 8 x 4 x 16 000 8-bit K with turbo3 V 86.2 / 82.4, 16 x 8 x 12 000 turbo4 180 / 174 to 178.
+    // Sparse V counts pass by pass.
+    pl.n_pass = p->sparse_v_tau > 0.0f ? 1 : passes_of(p);
+    if (pl.n_pass > 1 && ws_bytes < ws_layout(p, pl.n_pass).total) pl.n_pass = 1;
+    pl.pass_wgs = (int64_t)p->batch * p->n_kv_heads * pl.n_parts / pl.gpw;
+    // A 4-bit side: k_decode_turbo, whose table of 64 KB has a copy per lane (16 x 8 groups at 32768 tokens, turbo4: 110 -> 97 us,
+    // eight heads 121 -> 90; turbo4 K with turbo2 V 87 -> 77 and 100 -> 78).  It has to leave the workgroups that share a CU room
+    // (25 x 8 groups at 3175 tokens in 1000 workgroups of four: 30.5 us against 28.4 here; turbo4 K with turbo3 V, 96 KB, 20 x 8
+    // groups of eight heads at 2500 tokens in 320: 32.0 against 25.7), and building it has to pay: three tiles per wavefront and
+    // four wavefronts (2 x 8 groups at 3000 tokens, three: 12.7 us against 13.2 here; 8 at 4000, two: 11.7 against 11.5; one at
+    // 300, two wavefronts: 12.1 against 11.5).  Four heads with a bias list have no registers for it (16 x 9000 tokens with 64
+    // entries: 41.4 against 38.8, with Sparse V 47.6 against 43.0), and dense bias rows keep the general variants.
+    // A context length read from memory is taken at its largest: at short ones the tables cost nothing that shows (16 x 8 groups,
+    // turbo4, of 32 768 tokens 64 to 2048: 9.7 to 14.4 us, 10.1 to 19.0 in k_decode_attn; turbo3 K with turbo4 V 10.4 to 15.0, 10.3
+    // to 17.3).
+    const int tables = tqk_decode_turbo_lds(kb, vb, share) + pl.gpw * 1024 * pl.hg;
+    const int64_t per_cu = std::min<int64_t>((pl.pass_wgs * pl.n_pass + 255) / 256, std::max(1, (pl.hg == 2 ? 12 : 16) / pl.wpw));
+    const int64_t tiles = (p->tokens + 63) / 64, tiles_per_split = (tiles + p->n_splits - 1) / p->n_splits;
+    pl.lane_tables = !TQ_PAIRTAB3 && p->head_dim != 256 && kb != 8 && vb != 8 && (kb == 4 || vb == 4) && per_cu * tables <= 160 * 1024 &&
+                     tiles_per_split >= 3 && pl.wpw >= 4 && !dense && (pl.hg == 2 || !p->bias_entries);
+    return pl;
+}
+
 }  // namespace
+
+void tqk_attn_plan(const tq_attn_params *p, int kb, int vb, bool share, bool dense, int64_t ws_bytes, tq_attn_plan *out) {
+    const StepPlan pl = step_plan(p, kb, vb, share, dense, ws_bytes);
+    out->passes = pl.n_pass;
+    out->heads_per_pass = heads_per_pass(p);
+    out->wavefronts = pl.wpw;
+    out->partials = pl.n_parts;
+    out->groups_per_workgroup = pl.gpw;
+    out->lane_tables = pl.lane_tables;
+    out->workgroups = pl.pass_wgs * pl.n_pass;
+}
 
 int64_t tqk_attn_workspace_bytes(const tq_attn_params *p) { return ws_layout(p, p->sparse_v_tau > 0.0f ? 1 : passes_of(p)).total; }
 
@@ -125,13 +174,12 @@ int tqk_decode_attention(const tq_handle *hk, const tq_handle *hv, const tq_attn
                          const void *k, const void *k_aux, const void *v, const float *bias, float *out,
                          unsigned long long *skip_count, void *ws, int64_t ws_bytes, hipStream_t s) {
     (void)k_aux;
-    // All passes in one launch where the workspace has room: each is a chain of its own (launch, first rows, merge), one of few
-    // groups leaves most of the chip idle, and they read the same rows.  Steps of two passes over 256-dim heads (us with the
-    // append, one pass after the other / together): 2 x 8 KV heads x 259 tokens turbo4 35.0 / 19.6, 4 x 8 x 4000 turbo3 50.5 / 32.8,
-    // 1 x 1 x 100 000 turbo2 169 / 95, 8 x 4 x 16 000 8-bit K with turbo3 V 86.2 / 82.4, 16 x 8 x 12 000 turbo4 180 / 174 to 178.
-    // Sparse V counts pass by pass.
-    int n_pass = p->sparse_v_tau > 0.0f ? 1 : passes_of(p);
-    if (n_pass > 1 && ws_bytes < ws_layout(p, n_pass).total) n_pass = 1;
+    const bool turbo_k = p->k_format == TQ_KFMT_TURBO, turbo_v = p->v_format == TQ_KFMT_TURBO;
+    const int kb = turbo_k ? hk->bits : 8, vb = turbo_v ? hv->bits : 8;
+    const bool share = turbo_k && turbo_v && hk->bits == hv->bits &&
+                       std::memcmp(hk->pair_lut_host, hv->pair_lut_host, sizeof(hk->pair_lut_host)) == 0;
+    const StepPlan pl = step_plan(p, kb, vb, share, bias != nullptr, ws_bytes);
+    const int n_pass = pl.n_pass, wpw = pl.wpw, hg = pl.hg;
     const WsLayout w = ws_layout(p, n_pass);
     if (ws_bytes < w.total) {
         tq_set_error("tq_decode_attention: workspace %lld < %lld bytes", (long long)ws_bytes, (long long)w.total);
@@ -147,7 +195,6 @@ int tqk_decode_attention(const tq_handle *hk, const tq_handle *hv, const tq_attn
     const int64_t cache_rows = (d256 ? 2 : 1) * p->tokens;   // a 256-dim token is two rows of the caches
     float *part_o = reinterpret_cast<float *>((char *)ws + w.part_o);
     float *part_ml = reinterpret_cast<float *>((char *)ws + w.part_ml);
-    const bool turbo_k = p->k_format == TQ_KFMT_TURBO;
     const float sc = p->scale * LOG2E;
     const unsigned long long total_pairs = (unsigned long long)rows * (unsigned long long)p->tokens;
     int rc = TQ_OK;
@@ -165,11 +212,8 @@ int tqk_decode_attention(const tq_handle *hk, const tq_handle *hv, const tq_attn
     a.k = (const uint8_t *)k;
     a.v = (const uint8_t *)v;
     a.klut = turbo_k ? (const uint32_t *)hk->pair_lut : nullptr;
-    const bool turbo_v = p->v_format == TQ_KFMT_TURBO;
     a.vlut = turbo_v ? (const uint32_t *)hv->pair_lut : nullptr;
     const float *vs1 = turbo_v ? hv->s1_32 : nullptr, *vs2 = turbo_v ? hv->s2_32 : nullptr;
-    const bool share = turbo_k && turbo_v && hk->bits == hv->bits &&
-                       std::memcmp(hk->pair_lut_host, hv->pair_lut_host, sizeof(hk->pair_lut_host)) == 0;
     a.bias = bias;
     a.sbias_n = p->bias_entries;
     a.sbias_pos = p->bias_pos;
@@ -203,11 +247,7 @@ int tqk_decode_attention(const tq_handle *hk, const tq_handle *hv, const tq_attn
         tq_set_error("tq_decode_attention: sparse_v_tau > 0 needs skip_count");
         return TQ_ERR_ARG;
     }
-    // wavefronts per workgroup: the largest power of two up to 16 (8 for int8 V rows and for eight heads per pass)
-    // that divides the split count
-    const AttnPlan pl = attn_plan(p, p->bias_entries > 0);
-    const int wpw = pl.wpw, hg = pl.hg;
-    const unsigned pass_wgs = (unsigned)((int64_t)groups * pl.n_parts / pl.gpw);
+    const unsigned pass_wgs = (unsigned)pl.pass_wgs;
     const dim3 grid(pass_wgs, n_pass);
     const unsigned wg = 64u * (unsigned)wpw;
     // dynamic LDS: the wavefronts' merge space, then the staged queries of the workgroup's groups
@@ -216,8 +256,6 @@ int tqk_decode_attention(const tq_handle *hk, const tq_handle *hv, const tq_attn
     a.gw_shift = 0;
     while ((1 << a.gw_shift) < p->n_splits) ++a.gw_shift;
     a.wgs_per_group = pl.gpw > 1 ? 1 : p->n_splits / wpw;
-    const int vb = turbo_v ? hv->bits : 8;
-    const int kb = turbo_k ? hk->bits : 8;
     // The kernels work on four query heads of a KV head at a time (the 4-row MFMA block), or on eight (two sets
     // against the same dequantised rows) when a KV head serves more than four: a group of G heads takes
     // ceil(G / 8) passes over the same K/V; a last pass with fewer heads than it has rows repeats the group's
@@ -236,36 +274,25 @@ int tqk_decode_attention(const tq_handle *hk, const tq_handle *hv, const tq_attn
     a.pass_totals = reinterpret_cast<unsigned long long *>((char *)ws + w.pass_totals);
     a.skip_count = skip_count;
     a.total_pairs = total_pairs;
-    // A 4-bit side: k_decode_turbo, whose table of 64 KB has a copy per lane (16 x 8 groups at 32768 tokens, turbo4: 110 -> 97 us,
-    // eight heads 121 -> 90; turbo4 K with turbo2 V 87 -> 77 and 100 -> 78).  It has to leave the workgroups that share a CU room
-    // (25 x 8 groups at 3175 tokens in 1000 workgroups of four: 30.5 us against 28.4 here; turbo4 K with turbo3 V, 96 KB, 20 x 8
-    // groups of eight heads at 2500 tokens in 320: 32.0 against 25.7), and building it has to pay: three tiles per wavefront and
-    // four wavefronts (2 x 8 groups at 3000 tokens, three: 12.7 us against 13.2 here; 8 at 4000, two: 11.7 against 11.5; one at
-    // 300, two wavefronts: 12.1 against 11.5).  Four heads with a bias list have no registers for it (16 x 9000 tokens with 64
-    // entries: 41.4 against 38.8, with Sparse V 47.6 against 43.0), and dense bias rows keep the general variants.
-    const int tables = tqk_decode_turbo_lds(kb, vb, share) + pl.gpw * 1024 * hg;
-    const int per_cu = std::min((int)(((int64_t)pass_wgs * n_pass + 255) / 256), std::max(1, (hg == 2 ? 12 : 16) / wpw));
-    const bool lane_tables = !TQ_PAIRTAB3 && turbo_k && turbo_v && (kb == 4 || vb == 4) && per_cu * tables <= 160 * 1024 && a.tiles_per_split >= 3 && wpw >= 4 &&
-                             !bias && (hg == 2 || !a.sbias_n);
     for (a.head_off = 0; a.head_off < a.q_group; a.head_off += n_pass * a.pass_heads) {
         a.pass = a.head_off / a.pass_heads;
         a.nonce = next_nonce();
         const bool launched = d256 ? tqk_launch_decode_256(a, kb, vb, share, sparse, grid, wg, merge_bytes, s)
-                              : lane_tables ? tqk_launch_decode_turbo(a, kb, vb, share, 4 * hg, sparse, grid, wpw, s)
+                              : pl.lane_tables ? tqk_launch_decode_turbo(a, kb, vb, share, 4 * hg, sparse, grid, wpw, s)
                               : turbo_k && turbo_v ? launch_turbo(a, kb, vb, share, hg, sparse, grid, wg, merge_bytes, s)
                                                    : tqk_launch_decode_q8(a, kb, vb, hg, sparse, grid, wg, merge_bytes, s);
         if (!launched) {
             tq_set_error("tq_decode_attention: head_dim %d with K %d bits, V %d bits is not built", d256 ? 256 : 128, kb, vb);
             return TQ_ERR_UNSUPPORTED;
         }
-    rc = tq_check_launch("decode_attn");
-    if (rc) return rc;
-    if (skip_count && !a.poll_slots) {
-        // more groups than the finishing workgroups poll (or a dense step whose caller wants the counts)
-        k_skip_sum<<<1, 1024, 0, s>>>(a.skip_slots, sparse ? (int)pass_wgs : 0, skip_count, total_pairs, a.head_off > 0);
-        rc = tq_check_launch("skip_sum");
+        rc = tq_check_launch("decode_attn");
         if (rc) return rc;
-    }
+        if (skip_count && !a.poll_slots) {
+            // more groups than the finishing workgroups poll (or a dense step whose caller wants the counts)
+            k_skip_sum<<<1, 1024, 0, s>>>(a.skip_slots, sparse ? (int)pass_wgs : 0, skip_count, total_pairs, a.head_off > 0);
+            rc = tq_check_launch("skip_sum");
+            if (rc) return rc;
+        }
     }
     return TQ_OK;
 }

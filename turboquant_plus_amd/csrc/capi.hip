@@ -852,6 +852,18 @@ int64_t tq_attn_workspace_bytes(const tq_attn_params *p) {
     return tqk_attn_workspace_bytes(p);
 }
 
+int tq_decode_attention_plan(const tq_attn_params *p, int k_bits, int v_bits, int one_table, int dense_bias, int64_t workspace_bytes,
+                             tq_attn_plan *plan) {
+    int rc = check_attn(p);
+    if (rc) return rc;
+    REQUIRE(plan, TQ_ERR_ARG, "tq_decode_attention_plan: null plan");
+    const int kb = p->k_format == TQ_KFMT_TURBO ? k_bits : 8, vb = p->v_format == TQ_KFMT_TURBO ? v_bits : 8;
+    REQUIRE((kb == 8 || (kb >= 2 && kb <= 4)) && (vb == 8 || (vb >= 2 && vb <= 4)), TQ_ERR_ARG, "tq_decode_attention_plan: K %d bits, V %d bits", kb, vb);
+    REQUIRE(p->bias_entries >= 0, TQ_ERR_ARG, "tq_decode_attention_plan: bias_entries %d", (int)p->bias_entries);
+    tqk_attn_plan(p, kb, vb, one_table && kb == vb && kb != 8, dense_bias != 0, workspace_bytes, plan);
+    return TQ_OK;
+}
+
 int tq_decode_attention(const tq_handle *hk, const tq_handle *hv, const tq_attn_params *p, const void *q, int q_dtype,
                         const void *k, const void *k_aux, const void *v, const float *bias, float *out,
                         unsigned long long *skip_count, void *workspace, int64_t workspace_bytes, void *stream) {

@@ -111,6 +111,7 @@ int tqk_q8_0_store_v(const void *x, int64_t n_seqs, int64_t tokens, int in_dtype
 int tqk_q8_0_unpack(const void *packed, int64_t n_seqs, int64_t tokens, int8_t *q, float *scales, int kind, hipStream_t s);
 
 int64_t tqk_attn_workspace_bytes(const tq_attn_params *p);
+void tqk_attn_plan(const tq_attn_params *p, int kb, int vb, bool share, bool dense, int64_t ws_bytes, tq_attn_plan *out);
 int tqk_decode_attention(const tq_handle *hk, const tq_handle *hv, const tq_attn_params *p, const void *q, int q_dtype,
                          const void *k, const void *k_aux, const void *v, const float *bias, float *out,
                          unsigned long long *skip_count, void *ws, int64_t ws_bytes, hipStream_t s);
