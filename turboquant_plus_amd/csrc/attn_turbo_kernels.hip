@@ -560,10 +560,7 @@ bool tqk_launch_decode_turbo(const AttnArgs &a, int kb, int vb, bool share, int 
         launch_pair<4, 4, true>(a, n_heads, sparse, grid, waves, s);
         return true;
     }
-#ifndef TQ_FEW
-    TQ_PAIR(4, 4) TQ_PAIR(4, 2) TQ_PAIR(2, 4) TQ_PAIR(3, 4)
-#endif
-    TQ_PAIR(4, 3)
+    TQ_PAIR(4, 4) TQ_PAIR(4, 2) TQ_PAIR(2, 4) TQ_PAIR(3, 4) TQ_PAIR(4, 3)
 #undef TQ_PAIR
     return false;
 }
