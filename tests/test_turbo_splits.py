@@ -1,8 +1,11 @@
 """The split count of steps on turbo rows: the launch plan's counts, taken where they are clearly ahead."""
 import itertools
+import math
+import random
 
 import pytest
 
+from test_attention_plan import plan
 from turboquant_plus_amd import turbo as T
 
 
@@ -26,3 +29,36 @@ def test_shapes_that_were_timed():
     for bits in (2, 3, 4):
         assert T.turbo_splits(128, 32768, 32, k_bits=bits, v_bits=bits, one_table=True, **four) == 32
     assert T.turbo_splits(8, 32768, 256, k_bits=3, v_bits=3, one_table=True, **four) == 256
+
+
+def _shapes(eight):
+    rng = random.Random(11 + eight)
+    for _ in range(1500):
+        k, v = rng.choice([(2, 2), (3, 3), (4, 4), (4, 2), (3, 4), (4, 3), (2, 4)])
+        per_kv = rng.choice((5, 8, 12, 16, 24)) if eight else rng.choice((1, 3, 4))
+        yield (rng.choice((1, 2, 8)), int(math.exp(rng.uniform(0, math.log(300)))), per_kv, int(math.exp(rng.uniform(math.log(200), math.log(131072)))),
+               k, v, k == v and rng.random() < 0.7, rng.choice(T._SPLIT_COUNTS))
+
+
+@pytest.mark.parametrize("eight", [False, True])
+def test_estimates_are_made_for_the_kernel_that_is_launched(eight):
+    """The estimate's workgroups and its choice of a kernel are the launcher's, also where several passes share a launch."""
+    taken = 0
+    for kv_heads, batch, per_kv, tokens, k, v, one, n in _shapes(eight):
+        p = plan(k, v, batch, per_kv * kv_heads, kv_heads, tokens, n, one_table=one)
+        waves, parts, wgs = T._workgroups(n, batch * kv_heads, eight, True, True)
+        passes = -(-per_kv // 8) if eight else 1
+        assert (p.wavefronts, p.partials, p.workgroups, p.passes) == (waves, parts, wgs * passes, passes)
+        lds = T._lane_tables(k, v, one, eight, n, waves, wgs * passes, (tokens + 63) // 64)
+        assert bool(p.lane_tables) == bool(lds)
+        taken += bool(lds)
+    assert taken > 100
+
+
+def test_steps_of_several_passes():
+    """us with both counts, measured."""
+    turbo3 = dict(k_bits=3, v_bits=3, one_table=True, eight_heads=True)
+    assert T.turbo_splits(104, 1750, 8, passes=3, **turbo3) == 8      # 25.2; 28 splits 41.1
+    assert T.turbo_splits(96, 1769, 8, passes=2, **turbo3) < 28       # 8: 19.0; 28: 27.9
+    turbo4 = dict(k_bits=4, v_bits=4, one_table=True, eight_heads=True)
+    assert T.turbo_splits(20, 32768, 72, passes=2, **turbo4) != 80    # no room for the tables of both passes' workgroups

@@ -497,8 +497,9 @@ class DecodeAttention:
                 self._own_splits = (plain, own(True) if k_codec is not None and (eight or v_codec is None) else plain)
                 if len(bits) == 2 and sparse_v_tau == 0:
                     same = bits[0] == bits[1] and np.array_equal(k_codec.centroids, v_codec.centroids)
+                    passes = -(-n_q_heads // max(n_kv_heads, 1) // 8) if eight else 1
                     self._own_splits = (turbo_splits(batch * n_kv_heads, tokens, plain, k_bits=bits[0], v_bits=bits[1], one_table=same,
-                                                     eight_heads=eight), self._own_splits[1])
+                                                     eight_heads=eight, passes=passes), self._own_splits[1])
             n_splits = self._own_splits[0]
         else:
             self._own_splits = (n_splits, n_splits)
@@ -736,36 +737,53 @@ _TURBO_COST = {  # by (more than four heads, widest code, table copies per lane)
 }
 
 
+def _lane_tables(k_bits: int, v_bits: int, one_table: bool, eight_heads: bool, n: int, waves: int, workgroups: int, tiles: int) -> int:
+    """LDS of a workgroup in the kernel for 4-bit rows whose tables have a copy per lane, 0 where the launcher takes the general
+    one (step_plan in attn_kernels.hip; workgroups: of all passes of a launch)."""
+    if 4 not in (k_bits, v_bits) or -(-tiles // n) < 3 or waves < 4:
+        return 0
+    table = (0, 0, 2048, 32768, 65536)
+    shared = waves // n if n < waves else 1     # groups in a workgroup
+    lds = 1024 + table[k_bits] + (0 if one_table else table[v_bits]) + shared * _QUERY_BYTES * (2 if eight_heads else 1)
+    together = min(-(-workgroups // 256), max(1, (12 if eight_heads else 16) // waves))
+    return lds if together * lds <= _LDS_PER_CU else 0
+
+
 @functools.lru_cache(maxsize=256)
-def turbo_splits(n_groups: int, tokens: int, current: int, *, k_bits: int, v_bits: int, one_table: bool, eight_heads: bool) -> int:
+def turbo_splits(n_groups: int, tokens: int, current: int, *, k_bits: int, v_bits: int, one_table: bool, eight_heads: bool,
+                 passes: int = 1) -> int:
     """The split count of a step on turbo K and V rows of 128-dim heads without a bias list or Sparse V: `current` (balanced_splits)
     unless the estimate puts another count, down to one tile per wavefront, 12 % ahead (at 8 % up to 6 % of the shapes got more than
     3 % slower).  Over the 15 700 shapes a quarter of the four-head steps with 4-bit rows change, which makes all of them 4.1 %
     faster on average, and a tenth of the others (turbo3 1.3 %, turbo2 0.9 %, eight heads 1.1 to 1.4 %); 0.1 to 0.8 % of them are more
     than 3 % slower.  Eight heads leave out workgroups of three and six wavefronts, more than three per CU and more than 256
-    groups, where the estimate was wrong by 15 to 25 %."""
+    groups, where the estimate was wrong by 15 to 25 %.
+    passes: over a KV head's rows in one launch, whose workgroups share the CUs.  Counted as one pass they made 13 % of the changed
+    steps of two and three passes more than 3 % slower (104 groups of 24 heads at 1750 tokens, turbo3: 8 splits 25.2 us, 28 41.1);
+    of 10 600 changed with all of them counted 0.4 % are, at most 14 %, and the mean is 22 % faster."""
     widest = max(k_bits, v_bits)
-    if eight_heads and n_groups > 256:
+    if eight_heads and n_groups * passes > 256:
         return current
     tiles, sets = max(1, (tokens + 63) // 64), 2 if eight_heads else 1
     general, copied = _TURBO_COST[eight_heads, widest, False], _TURBO_COST.get((eight_heads, widest, True))
-    # LDS of a workgroup's tables: 2 and 3 bits, 4 bits (1 KB), 4 bits with a copy per lane (64 KB)
+    # LDS of a workgroup's tables: 2 and 3 bits, 4 bits (1 KB)
     table = (0, 0, 2048, 32768, 1024)
     lds_pair = table[k_bits] + (0 if one_table else table[v_bits])
-    lds_lane = 1024 + sum(65536 if b == 4 else table[b] for b in ((k_bits,) if one_table else (k_bits, v_bits)))
     most = 12 if eight_heads else 16
     best, best_time, now = current, math.inf, math.inf
     for n in (current, *_SPLIT_COUNTS):
-        if now < math.inf and not (n <= tiles and 200 <= n * n_groups <= 8192):
+        if now < math.inf and not (n <= tiles and 200 <= n * n_groups * passes <= 8192):
             continue
         waves, parts, wgs = _workgroups(n, n_groups, eight_heads, True, True)
+        wgs *= passes
         if now < math.inf and eight_heads and (waves in (3, 6) or wgs > 3 * 256):
             continue
         per_cu, deep, fit = -(-wgs // 256), -(-tiles // n), max(1, most // waves)
-        queries = max(1, waves // n) * _QUERY_BYTES * sets
-        cost, lds = general, lds_pair + sets * waves * _WAVE_MERGE_BYTES + queries
-        if copied and min(per_cu, fit) * (lds_lane + queries) <= _LDS_PER_CU and deep >= 3 and waves >= 4:      # the launcher's rule
-            cost, lds = copied, lds_lane + queries
+        lds_lane = _lane_tables(k_bits, v_bits, one_table, eight_heads, n, waves, wgs, tiles)
+        if lds_lane:
+            cost, lds = copied, lds_lane
+        else:
+            cost, lds = general, lds_pair + sets * waves * _WAVE_MERGE_BYTES + max(1, waves // n) * _QUERY_BYTES * sets
         rounds = -(-per_cu // max(1, min(fit, _LDS_PER_CU // lds)))
         took = (cost[0] + cost[1] * per_cu * 4 * -(-waves // 4) * deep + cost[2] * rounds * deep + cost[3] * parts + cost[4] * rounds
                 + cost[5] * max(0, parts - 16) + (cost[6] * (rounds - 1) if waves == 12 else 0.0))
