@@ -1,5 +1,5 @@
-"""Dense bias rows where their variants are short of registers: eight heads in workgroups of twelve wavefronts, 256-dim heads, and
-a list beside them."""
+"""Dense bias rows where their variants are short of registers (eight heads in workgroups of twelve wavefronts), with
+a list beside them, and with the split counts that an object takes by itself."""
 import numpy as np
 import pytest
 
@@ -37,3 +37,23 @@ def test_eight_heads_in_workgroups_of_twelve(kbits, vbits, sparse):
                                         n_splits=24, tau=tau, bias=bias[:, G * at.start:])
         assert_close(out[:, G * at.start:], ref)
         assert_close(both[:, G * at.start:], ref)
+
+
+def test_each_call_takes_its_own_split_count():
+    """One object, calls without a bias, with dense rows, with a list and with both, in turn: counts differ, the workspace has
+    room for each, results hold."""
+    tt = L.torch()
+    groups, G, N = 36, 4, 1731
+    k, v, kc, vc, kp, vp = make_kv(1, groups, N, seed=9, kbits=4, vbits=4)
+    rng = np.random.default_rng(1)
+    q = rng.standard_normal((1, G * groups, D)).astype(np.float16)
+    bias = np.where(rng.random((1, G * groups, N)) < 0.01, np.float32(3), np.float32(0))
+    bd, lists = tt.from_numpy(bias).cuda(), tqa.sparse_bias_from_dense(bias)
+    attn = tqa.DecodeAttention(kc, vc, 1, G * groups, groups, N, poison_output=True)
+    ref = [reference_attention(q, kc, vc, kp, vp, 1, G * groups, groups, N, 1 / np.sqrt(D), bias=b)[0] for b in (None, bias, 2 * bias)]
+    seen = []
+    for _ in range(2):
+        for kw, want in (({}, ref[0]), (dict(bias=bd), ref[1]), (dict(sparse_bias=lists), ref[1]), (dict(bias=bd, sparse_bias=lists), ref[2])):
+            assert_close(np_(attn(q, kp, vp, **kw)), want)
+            seen.append(attn.params.n_splits)
+    assert seen[:4] == seen[4:] == [*(attn._own_splits[i] for i in (0, 2, 1, 1))] and seen[0] != seen[1]

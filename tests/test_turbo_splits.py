@@ -2,7 +2,9 @@
 import itertools
 import math
 import random
+from types import SimpleNamespace
 
+import numpy as np
 import pytest
 
 from test_attention_plan import plan
@@ -62,3 +64,21 @@ def test_steps_of_several_passes():
     assert T.turbo_splits(96, 1769, 8, passes=2, **turbo3) < 28       # 8: 19.0; 28: 27.9
     turbo4 = dict(k_bits=4, v_bits=4, one_table=True, eight_heads=True)
     assert T.turbo_splits(20, 32768, 72, passes=2, **turbo4) != 80    # no room for the tables of both passes' workgroups
+
+
+def test_every_kind_of_call_has_its_own_count():
+    """Dense bias rows run in the general kernel; us with the counts, measured."""
+    codec = lambda bits, scale=1.0: SimpleNamespace(bits=bits, centroids=scale * np.arange(1 << bits))
+    four, three = codec(4), codec(3)
+    none, listed, dense = T.call_splits(four, three, 288, 4, 1246)
+    assert (none, listed, dense) == (20, 8, 8)                          # dense: 8 20.6, 20 26.0
+    assert T.call_splits(four, three, 40, 8, 41753)[2] == 36            # 36 71.7, 20 89.9
+    assert T.call_splits(four, codec(2), 128, 4, 38329)[2] == 32        # 32 98, 8 159
+    for k, v, per_kv, dim in itertools.product((None, three, four), (None, three, four), (1, 4, 8, 16), (128, 256)):
+        for groups, tokens in ((3, 900), (16, 1781), (40, 27600)):
+            for sparse in (False, True):
+                none, listed, dense = T.call_splits(k, v, groups, per_kv, tokens, head_dim=dim, sparse_v=sparse)
+                if sparse or dim == 256 or k is None or v is None:
+                    assert none == dense
+                elif k is v is four and per_kv <= 4:
+                    assert dense == listed

@@ -483,26 +483,11 @@ class DecodeAttention:
             raise ValueError(f"head_dim {head_dim}: the packed-cache kernels take 128 or 256")
         self.head_dim = head_dim
         if n_splits is None:
-            n_splits = default_splits(batch * n_kv_heads, tokens * (head_dim // HEAD_DIM),
-                                      eight_heads=head_dim == HEAD_DIM and n_q_heads // max(n_kv_heads, 1) > 4,
-                                      turbo_rows=k_codec is not None and v_codec is not None,
-                                      one_workgroup_per_cu=v_codec is None or (head_dim != HEAD_DIM and k_codec is None))
-            self._own_splits = (n_splits, n_splits)
-            if head_dim == HEAD_DIM:
-                eight, bits = n_q_heads // max(n_kv_heads, 1) > 4, [c.bits for c in (k_codec, v_codec) if c is not None]
-                own = lambda bias_list: balanced_splits(batch * n_kv_heads, tokens, n_splits, eight_heads=eight, turbo_k=k_codec is not None,
-                                                        turbo_v=v_codec is not None, three_bit=3 in bits, bias_list=bias_list,
-                                                        sparse_v=sparse_v_tau > 0)
-                plain = own(False)      # a bias list changes the plan of eight heads on turbo K, and the rule for 8-bit V rows
-                self._own_splits = (plain, own(True) if k_codec is not None and (eight or v_codec is None) else plain)
-                if len(bits) == 2 and sparse_v_tau == 0:
-                    same = bits[0] == bits[1] and np.array_equal(k_codec.centroids, v_codec.centroids)
-                    passes = -(-n_q_heads // max(n_kv_heads, 1) // 8) if eight else 1
-                    self._own_splits = (turbo_splits(batch * n_kv_heads, tokens, plain, k_bits=bits[0], v_bits=bits[1], one_table=same,
-                                                     eight_heads=eight, passes=passes), self._own_splits[1])
+            self._own_splits = call_splits(k_codec, v_codec, batch * n_kv_heads, n_q_heads // max(n_kv_heads, 1), tokens, head_dim=head_dim,
+                                           sparse_v=sparse_v_tau > 0)
             n_splits = self._own_splits[0]
         else:
-            self._own_splits = (n_splits, n_splits)
+            self._own_splits = (n_splits,) * 3
         self.params = L.TQAttnParams(batch=batch, n_q_heads=n_q_heads, n_kv_heads=n_kv_heads, tokens=tokens,
                                      capacity=capacity, n_splits=n_splits, k_format=L.KFMT_TURBO if k_codec is not None else L.KFMT_Q8_0,
                                      v_format=L.KFMT_TURBO if v_codec is not None else L.KFMT_Q8_0,
@@ -516,7 +501,7 @@ class DecodeAttention:
                 raise ValueError("Sparse V keeps no count for a context length read from device memory")
             self.params.tokens_dev = tokens_on_device.data_ptr()
         nbytes = 0
-        for self.params.n_splits in self._own_splits[::-1]:     # room for either kind of call; without a list comes last
+        for self.params.n_splits in self._own_splits[::-1]:     # room for every kind of call; without a bias comes last
             need = L.lib().tq_attn_workspace_bytes(C.byref(self.params))
             if need < 0:
                 L.check(L.ERR_ARG)
@@ -551,7 +536,7 @@ class DecodeAttention:
             params.bias_entries = 0
             params.bias_pos = params.bias_val = None
         if params.n_splits == self._splits_set:    # not where the caller has set another one
-            splits = self._own_splits[params.bias_entries > 0]
+            splits = self._own_splits[1 if params.bias_entries > 0 else 2 if bias is not None else 0]
             if splits != self._splits_set:
                 params.n_splits = self._splits_set = splits
         hk = self.k_codec.handle.h if self.k_codec is not None else None
@@ -638,6 +623,27 @@ def default_splits(n_groups: int, tokens: int, eight_heads: bool = False, turbo_
     if n >= 16:
         return n // 16 * 16
     return 1 << (n.bit_length() - 1)
+
+
+def call_splits(k_codec, v_codec, n_groups: int, per_kv: int, tokens: int, *, head_dim: int = HEAD_DIM, sparse_v: bool = False) -> tuple[int, int, int]:
+    """The split counts that DecodeAttention takes by itself: of calls without a bias, with a bias list, and with dense bias rows
+    alone.  per_kv: query heads per KV head; a codec of None: q8_0-style rows."""
+    eight = head_dim == HEAD_DIM and per_kv > 4
+    default = default_splits(n_groups, tokens * (head_dim // HEAD_DIM), eight_heads=eight, turbo_rows=k_codec is not None and v_codec is not None,
+                             one_workgroup_per_cu=v_codec is None or (head_dim != HEAD_DIM and k_codec is None))
+    if head_dim != HEAD_DIM:
+        return default, default, default
+    bits = [c.bits for c in (k_codec, v_codec) if c is not None]
+    own = lambda bias_list: balanced_splits(n_groups, tokens, default, eight_heads=eight, turbo_k=k_codec is not None, turbo_v=v_codec is not None,
+                                            three_bit=3 in bits, bias_list=bias_list, sparse_v=sparse_v)
+    plain = own(False)      # a bias list changes the plan of eight heads on turbo K, and the rule for 8-bit V rows
+    listed = own(True) if k_codec is not None and (eight or v_codec is None) else plain
+    if len(bits) < 2 or sparse_v:
+        return plain, listed, plain
+    same = bits[0] == bits[1] and np.array_equal(k_codec.centroids, v_codec.centroids)
+    none, dense = (turbo_splits(n_groups, tokens, plain, k_bits=bits[0], v_bits=bits[1], one_table=same, eight_heads=eight,
+                                passes=-(-per_kv // 8) if eight else 1, dense_rows=rows) for rows in (False, True))
+    return none, listed, dense
 
 
 def _workgroups(n: int, n_groups: int, eight_heads: bool, turbo_k: bool, turbo_v: bool) -> tuple[int, int, int]:
@@ -751,7 +757,7 @@ def _lane_tables(k_bits: int, v_bits: int, one_table: bool, eight_heads: bool, n
 
 @functools.lru_cache(maxsize=256)
 def turbo_splits(n_groups: int, tokens: int, current: int, *, k_bits: int, v_bits: int, one_table: bool, eight_heads: bool,
-                 passes: int = 1) -> int:
+                 passes: int = 1, dense_rows: bool = False) -> int:
     """The split count of a step on turbo K and V rows of 128-dim heads without a bias list or Sparse V: `current` (balanced_splits)
     unless the estimate puts another count, down to one tile per wavefront, 12 % ahead (at 8 % up to 6 % of the shapes got more than
     3 % slower).  Over the 15 700 shapes a quarter of the four-head steps with 4-bit rows change, which makes all of them 4.1 %
@@ -760,9 +766,14 @@ def turbo_splits(n_groups: int, tokens: int, current: int, *, k_bits: int, v_bit
     groups, where the estimate was wrong by 15 to 25 %.
     passes: over a KV head's rows in one launch, whose workgroups share the CUs.  Counted as one pass they made 13 % of the changed
     steps of two and three passes more than 3 % slower (104 groups of 24 heads at 1750 tokens, turbo3: 8 splits 25.2 us, 28 41.1);
-    of 10 600 changed with all of them counted 0.4 % are, at most 14 %, and the mean is 22 % faster."""
+    of 10 600 changed with all of them counted 0.4 % are, at most 14 %, and the mean is 22 % faster.
+    dense_rows: the call carries dense bias rows, which 4-bit rows meet in the general kernel: estimated for the other one, 19 % of
+    the changed four-head calls were more than 3 % slower (288 groups at 1246 tokens: 20.6 -> 26.0 us) and 15 % with eight heads.
+    Four heads on 4-bit rows keep `current`: their line of the general kernel is fitted to the few tiles that its users have there
+    (128 groups at 38 300 tokens: 32 splits 98 us, the line's 8 splits 159).  With eight heads 2 200 calls change, 17 % faster, none
+    slower; without 4-bit rows 2 100, 13 to 17 % faster, 2 to 3 % of them more than 3 % slower."""
     widest = max(k_bits, v_bits)
-    if eight_heads and n_groups * passes > 256:
+    if (n_groups * passes > 256) if eight_heads else (dense_rows and widest == 4):
         return current
     tiles, sets = max(1, (tokens + 63) // 64), 2 if eight_heads else 1
     general, copied = _TURBO_COST[eight_heads, widest, False], _TURBO_COST.get((eight_heads, widest, True))
@@ -779,7 +790,7 @@ def turbo_splits(n_groups: int, tokens: int, current: int, *, k_bits: int, v_bit
         if now < math.inf and eight_heads and (waves in (3, 6) or wgs > 3 * 256):
             continue
         per_cu, deep, fit = -(-wgs // 256), -(-tiles // n), max(1, most // waves)
-        lds_lane = _lane_tables(k_bits, v_bits, one_table, eight_heads, n, waves, wgs, tiles)
+        lds_lane = 0 if dense_rows else _lane_tables(k_bits, v_bits, one_table, eight_heads, n, waves, wgs, tiles)
         if lds_lane:
             cost, lds = copied, lds_lane
         else:
