@@ -73,6 +73,7 @@ def test_every_kind_of_call_has_its_own_count():
     none, listed, dense = T.call_splits(four, three, 288, 4, 1246)
     assert (none, listed, dense) == (20, 8, 8)                          # dense: 8 20.6, 20 26.0
     assert T.call_splits(four, three, 40, 8, 41753)[2] == 36            # 36 71.7, 20 89.9
+    assert T.call_splits(codec(2), codec(2), 192, 8, 4081)[2] < 32      # 8 32.1, 32 39.5
     assert T.call_splits(four, codec(2), 128, 4, 38329)[2] == 32        # 32 98, 8 159
     for k, v, per_kv, dim in itertools.product((None, three, four), (None, three, four), (1, 4, 8, 16), (128, 256)):
         for groups, tokens in ((3, 900), (16, 1781), (40, 27600)):

@@ -770,8 +770,9 @@ def turbo_splits(n_groups: int, tokens: int, current: int, *, k_bits: int, v_bit
     dense_rows: the call carries dense bias rows, which 4-bit rows meet in the general kernel: estimated for the other one, 19 % of
     the changed four-head calls were more than 3 % slower (288 groups at 1246 tokens: 20.6 -> 26.0 us) and 15 % with eight heads.
     Four heads on 4-bit rows keep `current`: their line of the general kernel is fitted to the few tiles that its users have there
-    (128 groups at 38 300 tokens: 32 splits 98 us, the line's 8 splits 159).  With eight heads 2 200 calls change, 17 % faster, none
-    slower; without 4-bit rows 2 100, 13 to 17 % faster, 2 to 3 % of them more than 3 % slower."""
+    (128 groups at 38 300 tokens: 32 splits 98 us, the line's 8 splits 159).  More than sixteen wavefronts per CU in workgroups of four or
+    eight are left out: the variants of dense rows hold 12 to 16 (192 groups of eight heads at 4081 tokens, turbo2: 8 splits 32.1 us, 32
+    splits 39.5; 38 % of such calls were more than 3 % slower).  Of 5 770 changed calls 0.6 % are, at most 14 %; the mean is 17 % faster."""
     widest = max(k_bits, v_bits)
     if (n_groups * passes > 256) if eight_heads else (dense_rows and widest == 4):
         return current
@@ -797,6 +798,8 @@ def turbo_splits(n_groups: int, tokens: int, current: int, *, k_bits: int, v_bit
             cost, lds = general, lds_pair + sets * waves * _WAVE_MERGE_BYTES + max(1, waves // n) * _QUERY_BYTES * sets
         rounds = -(-per_cu // max(1, min(fit, _LDS_PER_CU // lds)))
         took = (cost[0] + cost[1] * per_cu * 4 * -(-waves // 4) * deep + cost[2] * rounds * deep + cost[3] * parts + cost[4] * rounds
+        if now < math.inf and dense_rows and waves < 12 and waves * per_cu > 16:
+            continue
                 + cost[5] * max(0, parts - 16) + (cost[6] * (rounds - 1) if waves == 12 else 0.0))
         if now == math.inf:
             now = took          # the first is `current`
