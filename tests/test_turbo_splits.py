@@ -83,3 +83,21 @@ def test_every_kind_of_call_has_its_own_count():
                     assert none == dense
                 elif k is v is four and per_kv <= 4:
                     assert dense == listed
+
+
+def test_outside_of_what_was_fitted():
+    """us with both counts, measured."""
+    four = dict(eight_heads=False)
+    assert T.turbo_splits(831, 795, 2, k_bits=4, v_bits=2, one_table=False, **four) == 2        # 21.9; 8 splits 27.2
+    assert T.turbo_splits(853, 682, 2, k_bits=4, v_bits=4, one_table=True, **four) == 2         # 24.1; 8: 29.8
+    for tokens in (318860, 325710):
+        assert T.turbo_splits(1, tokens, 2048, k_bits=4, v_bits=4, one_table=True, eight_heads=True) == 2048    # 40; 256: 48
+    rng = random.Random(3)
+    for _ in range(2000):
+        groups, tokens = rng.randint(301, 1100), int(math.exp(rng.uniform(math.log(400), math.log(131072))))
+        k, v = rng.choice([(2, 2), (3, 3), (3, 2), (4, 4), (4, 2), (4, 3), (3, 4)])
+        now = T.balanced_splits(groups, tokens, T.default_splits(groups, tokens), turbo_k=True, turbo_v=True, three_bit=3 in (k, v), **four)
+        n = T.turbo_splits(groups, tokens, now, k_bits=k, v_bits=v, one_table=k == v, **four)
+        if n != now:    # few shapes of the others gained
+            p = plan(k, v, groups, 4, 1, tokens, n)
+            assert p.lane_tables and -(-tokens // 64) >= 5 * n + 1

@@ -763,7 +763,11 @@ def turbo_splits(n_groups: int, tokens: int, current: int, *, k_bits: int, v_bit
     3 % slower).  Over the 15 700 shapes a quarter of the four-head steps with 4-bit rows change, which makes all of them 4.1 %
     faster on average, and a tenth of the others (turbo3 1.3 %, turbo2 0.9 %, eight heads 1.1 to 1.4 %); 0.1 to 0.8 % of them are more
     than 3 % slower.  Eight heads leave out workgroups of three and six wavefronts, more than three per CU and more than 256
-    groups, where the estimate was wrong by 15 to 25 %.
+    groups, where the estimate was wrong by 15 to 25 %.  Behind the 300 groups of the fit four heads change only to counts of the kernel
+    with a copy per lane at six tiles per wavefront and more: of 1500 shapes of 301 to 1024 groups timed there with both counts, half of
+    the 2- and 3-bit ones had become more than 3 % slower, and of the 4-bit ones 95 % at two tiles, 54 % at three, 14 % at five, 0.5 %
+    from six on (831 groups at 795 tokens, 4|2: 2 splits 21.9 us, 8 splits 27.2); what is left is 18 % faster.  Counts
+    above the fit's 1024 stay (one group of eight heads at 325 000 tokens: 2048 splits 40 us, 256 splits 48).
     passes: over a KV head's rows in one launch, whose workgroups share the CUs.  Counted as one pass they made 13 % of the changed
     steps of two and three passes more than 3 % slower (104 groups of 24 heads at 1750 tokens, turbo3: 8 splits 25.2 us, 28 41.1);
     of 10 600 changed with all of them counted 0.4 % are, at most 14 %, and the mean is 22 % faster.
@@ -775,6 +779,9 @@ def turbo_splits(n_groups: int, tokens: int, current: int, *, k_bits: int, v_bit
     splits 39.5; 38 % of such calls were more than 3 % slower).  Of 5 770 changed calls 0.6 % are, at most 14 %; the mean is 17 % faster."""
     widest = max(k_bits, v_bits)
     if (n_groups * passes > 256) if eight_heads else (dense_rows and widest == 4):
+        return current
+    many = not eight_heads and n_groups > 300      # more than were fitted
+    if current > 1024 or (many and (widest < 4 or dense_rows)):
         return current
     tiles, sets = max(1, (tokens + 63) // 64), 2 if eight_heads else 1
     general, copied = _TURBO_COST[eight_heads, widest, False], _TURBO_COST.get((eight_heads, widest, True))
@@ -791,15 +798,17 @@ def turbo_splits(n_groups: int, tokens: int, current: int, *, k_bits: int, v_bit
         if now < math.inf and eight_heads and (waves in (3, 6) or wgs > 3 * 256):
             continue
         per_cu, deep, fit = -(-wgs // 256), -(-tiles // n), max(1, most // waves)
+        if now < math.inf and dense_rows and waves < 12 and waves * per_cu > 16:
+            continue
         lds_lane = 0 if dense_rows else _lane_tables(k_bits, v_bits, one_table, eight_heads, n, waves, wgs, tiles)
+        if now < math.inf and many and not (lds_lane and deep >= 6):
+            continue
         if lds_lane:
             cost, lds = copied, lds_lane
         else:
             cost, lds = general, lds_pair + sets * waves * _WAVE_MERGE_BYTES + max(1, waves // n) * _QUERY_BYTES * sets
         rounds = -(-per_cu // max(1, min(fit, _LDS_PER_CU // lds)))
         took = (cost[0] + cost[1] * per_cu * 4 * -(-waves // 4) * deep + cost[2] * rounds * deep + cost[3] * parts + cost[4] * rounds
-        if now < math.inf and dense_rows and waves < 12 and waves * per_cu > 16:
-            continue
                 + cost[5] * max(0, parts - 16) + (cost[6] * (rounds - 1) if waves == 12 else 0.0))
         if now == math.inf:
             now = took          # the first is `current`
