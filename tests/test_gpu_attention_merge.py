@@ -54,3 +54,30 @@ def test_steps_captured_in_a_graph_find_their_counters():
         if step % 2:
             attn.out.fill_(float("nan"))
             assert bool((attn(q, kp, vp) == want).all()), step
+
+
+@pytest.mark.parametrize("G,n_splits,bits", [(4, 4, 3), (4, 32, 3), (8, 4, 4), (8, 12, 3), (8, 32, 4)])
+def test_a_split_whose_sum_is_not_a_number(G, n_splits, bits):
+    """A logit of +inf (a K row whose norm is beyond fp16) makes the sum of its wavefront's weights NaN.  With Sparse V, which skips
+    weights that are not above the threshold, that wavefront has nothing to add, and its workgroup's others count as they do without it."""
+    tt = L.torch()
+    tiles, groups = 4 * n_splits, 3
+    N = 64 * tiles
+    k, v, kc, vc, kp, vp = make_kv(1, groups, N, seed=bits, kbits=bits, vbits=bits)
+    q = np.random.default_rng(7).standard_normal((1, G * groups, D)).astype(np.float16)
+    q[:] = q[:, :1]                                     # one query for all heads: the logit's sign is the same for each
+    big = k.astype(np.float32)
+    big[1, 0] = 1e6 * q[0, 0].astype(np.float32) / np.linalg.norm(q[0, 0].astype(np.float32))
+    assert np.linalg.norm(big[1, 0]) > np.finfo(np.float16).max
+    kp2 = kc.store(big, kind="k")
+    attn = tqa.DecodeAttention(kc, vc, 1, G * groups, groups, N, n_splits=n_splits, sparse_v_tau=1e-6, poison_output=True)
+    got = np_(attn(q, kp2, vp)).copy()
+    per_k, per_v = kp.numel() // groups, vp.numel() // groups
+    # the group without its first split: what the other wavefronts have
+    cut = 64 * 4
+    rest_k, rest_v = kc.store(k[1:2, cut:], kind="k"), vc.store(v[1:2, cut:], kind="v")
+    ref, _, _ = reference_attention(q[:, G:2 * G], kc, vc, rest_k, rest_v, 1, G, 1, N - cut, 1 / np.sqrt(D))
+    assert np.isfinite(got).all()
+    assert_close(got[:, G:2 * G], ref)
+    others = np_(attn(q, kc.store(k.astype(np.float32), kind="k"), vp))     # fp32 rows, as above
+    assert np.array_equal(got[:, :G], others[:, :G]) and np.array_equal(got[:, 2 * G:], others[:, 2 * G:])

@@ -426,8 +426,9 @@ __device__ __forceinline__ void combine_waves_of(Slot slot, int wave0, int tid_g
         vec_t sum = 0.0f;
 #pragma unroll
         for (int w = 0; w < W; ++w) {
-            const float f = ml[w].y > 0.0f ? __builtin_amdgcn_exp2f(ml[w].x - M) : 0.0f;
-            L = fmaf(ml[w].y, f, L);
+            const bool seen = ml[w].y > 0.0f;   // false for a sum that is not a number, too: it stays out of the others'
+            const float f = seen ? __builtin_amdgcn_exp2f(ml[w].x - M) : 0.0f;
+            L = seen ? fmaf(ml[w].y, f, L) : L;
 #pragma unroll
             for (int i = 0; i < VW; ++i) sum[i] = fmaf(v[w][i], f, sum[i]);
         }
