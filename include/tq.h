@@ -418,19 +418,18 @@ int tq_score_tile(const tq_handle *h, const void *q, int q_dtype, int64_t nq, co
                   void *workspace, int64_t workspace_bytes, void *stream);
 
 /* Large host arrays by several of the caller's threads.  A session and a job lie in the caller's memory, zeroed but for the
- * job's first eight fields.  Threads in tq_host_serve wait for the session's jobs until tq_host_close; the session's memory has to
+ * job's first seven fields.  Threads in tq_host_serve wait for the session's jobs until tq_host_close; the session's memory has to
  * outlive them.  tq_host_drive works on one job: an array of n elements in n_pieces pieces of `piece` elements, taken by the
  * session's threads and by itself (session may be NULL, and nobody need come); it returns when every piece is done, the stream
  * has finished with the slots and no thread looks at the job.  `slots`: pinned memory for min(TQ_HOST_SLOTS, n_pieces) pieces, one
- * byte per element, and `device` the array's other side, on `stream`'s device; or slots == NULL (TQ_HOST_NARROW only) and the other
- * side is `other`, in host memory.
+ * byte per element; `device`: the array's other side, on `stream`'s device.
  *   TQ_HOST_FETCH   n device bytes -> host            TQ_HOST_WIDEN   n device uint8 -> host int64
- *   TQ_HOST_UPLOAD  n host bytes -> device            TQ_HOST_NARROW  n host int64 -> uint8 (low byte); their bits or'ed in `seen` */
+ *   TQ_HOST_UPLOAD  n host bytes -> device            TQ_HOST_NARROW  n host int64 -> device uint8 (low byte); their bits or'ed in `seen` */
 #define TQ_HOST_SLOTS 8
 enum { TQ_HOST_FETCH = 0, TQ_HOST_WIDEN = 1, TQ_HOST_UPLOAD = 2, TQ_HOST_NARROW = 3 };
 typedef struct {
     int64_t kind, n, n_pieces, piece;
-    void *host, *other, *slots;
+    void *host, *slots;
     int64_t seen;
     int64_t next, ready, done;
     int32_t slot_done[TQ_HOST_SLOTS];

@@ -47,14 +47,17 @@ def test_scalar_norms_join():
 
 @pytest.mark.parametrize("when", ["after a fork", "at exit", "in a thread that outlives the main one"])
 def test_copy_threads_that_are_not_there(when):
-    """Large host arrays are handled where the copy threads are gone: in a forked child, and once the interpreter ends."""
+    """A call with large host arrays begins and ends where the copy threads are gone: in a forked child, and once the interpreter
+    ends."""
     code = """
 import atexit, os, sys, threading, time
 import numpy as np
 from turboquant_plus_amd import _lib as L
 i = np.random.default_rng(0).integers(0, 8, 700_000)
 def narrow():
-    assert np.array_equal(L.narrow_indices(i, 8), i)
+    with L.helpers(L.SHARED + 1), L.helpers(L.SHARED + 1):
+        assert np.array_equal(L.narrow_indices(i, 8), i)
+    assert getattr(L._helping, "session", None) is None
     print("done", flush=True)
 narrow()
 together = threading.Barrier(L.COPY_THREADS)

@@ -53,8 +53,8 @@ HOST_FETCH, HOST_WIDEN, HOST_UPLOAD, HOST_NARROW = 0, 1, 2, 3
 
 class TQHostJob(C.Structure):
     _fields_ = [("kind", C.c_int64), ("n", C.c_int64), ("n_pieces", C.c_int64), ("piece", C.c_int64), ("host", C.c_void_p),
-                ("other", C.c_void_p), ("slots", C.c_void_p), ("seen", C.c_int64), ("next", C.c_int64), ("ready", C.c_int64),
-                ("done", C.c_int64), ("slot_done", C.c_int32 * HOST_SLOTS)]
+                ("slots", C.c_void_p), ("seen", C.c_int64), ("next", C.c_int64), ("ready", C.c_int64), ("done", C.c_int64),
+                ("slot_done", C.c_int32 * HOST_SLOTS)]
 
 
 class TQHostSession(C.Structure):
@@ -291,17 +291,15 @@ def _helped():
         lib().tq_host_close(session)
 
 
-def _host_job(kind, n, host, *, other=None, device=None):
-    """A job of n elements (include/tq.h) on the contiguous array `host`: with pinned slots to or from the device tensor
-    `device`, or into the array `other`.  Returns the bits that HOST_NARROW saw."""
+def _host_job(kind, n, host, device):
+    """A job of n elements (include/tq.h) between the contiguous array `host` and the device tensor `device`.  Returns the bits
+    that HOST_NARROW saw."""
     each = 8 if kind in (HOST_WIDEN, HOST_NARROW) else 1       # host bytes of an element; one on the other side
     piece = max(min(STAGE, n * each // 4), 1 << 18) // each
     pieces = -(-n // piece)
-    job = TQHostJob(kind=kind, n=n, n_pieces=pieces, piece=piece, host=host.ctypes.data, other=None if other is None else other.ctypes.data)
-    stream = None
-    if device is not None:
-        slots = torch().empty(min(HOST_SLOTS, pieces) * piece, dtype=torch().uint8, pin_memory=True)
-        job.slots, stream = slots.data_ptr(), stream_ptr()
+    slots = torch().empty(min(HOST_SLOTS, pieces) * piece, dtype=torch().uint8, pin_memory=True)
+    job = TQHostJob(kind=kind, n=n, n_pieces=pieces, piece=piece, host=host.ctypes.data, slots=slots.data_ptr())
+    stream = stream_ptr()
     if n * each <= SHARED:
         check(lib().tq_host_drive(None, job, ptr(device), stream))
     else:
@@ -318,11 +316,8 @@ def narrow_indices(indices, n_centroids):
             _refuse_indices()
         return np.ascontiguousarray(indices, dtype=np.uint8)
     out = np.empty(indices.shape, np.uint8)
-    if indices.nbytes > SHARED:
-        seen = _host_job(HOST_NARROW, indices.size, indices, other=out)
-    else:
-        np.copyto(out, indices, casting="unsafe")
-        seen = int(np.bitwise_or.reduce(indices, axis=None))
+    np.copyto(out, indices, casting="unsafe")
+    seen = int(np.bitwise_or.reduce(indices, axis=None))
     if seen & ~(n_centroids - 1):       # a bit above the codebook's: some index is outside
         _refuse_indices()
     return out
@@ -337,7 +332,7 @@ def upload_indices(indices, n_centroids, *others):
     if indices.dtype != np.int64 or not indices.flags.c_contiguous or indices.nbytes <= SHARED:
         return upload(narrow_indices(indices, n_centroids), *others)
     t = torch().empty(indices.shape, dtype=torch().uint8, device=require_gpu())
-    if _host_job(HOST_NARROW, indices.size, indices, device=t) & ~(n_centroids - 1):
+    if _host_job(HOST_NARROW, indices.size, indices, t) & ~(n_centroids - 1):
         _refuse_indices()
     return [t, *upload(*others)]
 
@@ -361,7 +356,7 @@ def fetch(buf, *wanted):
         same = a.dtype == _NP_DTYPES[str(t.dtype)]
         if t.nbytes > ONE_COPY and (same or (t.dtype == tt.uint8 and dtype == np.int64)):
             # fresh host memory costs more than the transfer (64 MiB: 9.3 ms by one pageable copy, 1.2 ms of them the link)
-            _host_job(HOST_FETCH if same else HOST_WIDEN, a.nbytes if same else a.size, a, device=t)
+            _host_job(HOST_FETCH if same else HOST_WIDEN, a.nbytes if same else a.size, a, t)
         else:
             src = a if same else np.empty(tuple(t.shape), _NP_DTYPES[str(t.dtype)])
             tt.from_numpy(src).copy_(t)
@@ -392,7 +387,7 @@ def _upload_one(a, dev):
     if a.nbytes < SHARED // 2:
         return tt.from_numpy(a if a.flags.writeable else a.copy()).to(dev)   # torch warns of read-only memory
     t = tt.empty(a.shape, dtype=_torch_dtype(a.dtype), device=dev)
-    _host_job(HOST_UPLOAD, a.nbytes, a, device=t)
+    _host_job(HOST_UPLOAD, a.nbytes, a, t)
     return t
 
 

@@ -1,5 +1,4 @@
-// Host arrays of the NumPy classes: large ones on their way between host memory and the device, and index arrays narrowed, by
-// several threads of the caller's.
+// Large host arrays of the NumPy classes on their way between host memory and the device, by several threads of the caller's.
 //
 // A transfer is a job that lies in the caller's memory (tq_host_job).  Its array is cut into pieces, which the threads in
 // tq_host_serve take until none are left; the thread in tq_host_drive moves the pinned slots between the device and the pieces'
@@ -58,9 +57,7 @@ int host_bytes(const tq_host_job *j) { return j->kind == TQ_HOST_WIDEN || j->kin
 void do_piece(tq_host_job *j, int64_t p) {
     const int64_t at = p * j->piece, n = j->n - at < j->piece ? j->n - at : j->piece;
     char *host = (char *)j->host + at * host_bytes(j);
-    // without slots (narrowing on the host) the other side is an array of its own
-    char *slot = j->slots ? (char *)j->slots + (p % SLOTS) * j->piece
-                          : (char *)j->other + at;
+    char *slot = (char *)j->slots + (p % SLOTS) * j->piece;
     if (j->kind == TQ_HOST_WIDEN) {
         if (has_avx2()) widen_avx2((int64_t *)host, (const uint8_t *)slot, n);
         else widen_any((int64_t *)host, (const uint8_t *)slot, n);
@@ -113,14 +110,6 @@ void ring(tq_host_session *s) {
 // the stream's part of a job, and pieces in between
 hipError_t move(tq_host_job *j, char *device, hipStream_t s) {
     int idle = 0;
-    if (!j->slots) {   // host to host
-        __atomic_store_n(&j->ready, j->n_pieces, __ATOMIC_RELEASE);
-        while (load(&j->done) < j->n_pieces) {
-            if (take(j)) idle = 0;
-            else pause_for(idle);
-        }
-        return hipSuccess;
-    }
     const bool down = j->kind == TQ_HOST_WIDEN || j->kind == TQ_HOST_FETCH;
     hipEvent_t ev[SLOTS];
     hipError_t err = hipSuccess;
