@@ -417,11 +417,12 @@ int tq_score_tile(const tq_handle *h, const void *q, int q_dtype, int64_t nq, co
                   const uint8_t *sign_bits, const void *rnorms_f16, int64_t nk, void *logits, int out_dtype,
                   void *workspace, int64_t workspace_bytes, void *stream);
 
-/* Large host arrays by several of the caller's threads.  A session and a job lie in the caller's memory, zeroed but for the
- * job's first seven fields.  Threads in tq_host_serve wait for the session's jobs until tq_host_close; the session's memory has to
- * outlive them.  tq_host_drive works on one job: an array of n elements in n_pieces pieces of `piece` elements, taken by the
- * session's threads and by itself (session may be NULL, and nobody need come); it returns when every piece is done, the stream
- * has finished with the slots and no thread looks at the job.  `slots`: pinned memory for min(TQ_HOST_SLOTS, n_pieces) pieces, one
+/* Large host arrays by several of the caller's threads.  A board and a job lie in the caller's memory, zeroed but for the
+ * job's first seven fields.  Threads in tq_host_serve work on the jobs of a board, and sleep between them, until it is closed: while
+ * its count of users, which tq_host_enter(board, +1 or -1) changes and returns (0: wakes the threads), is not positive.  The
+ * board's memory has to outlive them.  tq_host_drive works on one job: an array of n elements in n_pieces pieces of `piece` elements, taken by the
+ * board's threads and by itself (board may be NULL, and nobody need come); it returns when every piece is done, the stream
+ * has finished with the slots and no thread looks at the job.  Any number of threads may drive jobs on one board.  `slots`: pinned memory for min(TQ_HOST_SLOTS, n_pieces) pieces, one
  * byte per element; `device`: the array's other side, on `stream`'s device.
  *   TQ_HOST_FETCH   n device bytes -> host            TQ_HOST_WIDEN   n device uint8 -> host int64
  *   TQ_HOST_UPLOAD  n host bytes -> device            TQ_HOST_NARROW  n host int64 -> device uint8 (low byte); their bits or'ed in `seen` */
@@ -434,14 +435,18 @@ typedef struct {
     int64_t next, ready, done;
     int32_t slot_done[TQ_HOST_SLOTS];
 } tq_host_job;
+#define TQ_HOST_DESKS 16   /* jobs that a board's threads know of at a time; the drivers of others work alone */
 typedef struct {
     tq_host_job *job;
-    int64_t users;
-    int32_t bell, closed;
-} tq_host_session;
-void tq_host_serve(tq_host_session *session);
-void tq_host_close(tq_host_session *session);
-int tq_host_drive(tq_host_session *session, tq_host_job *job, void *device, void *stream);
+    int64_t users, taken;
+} tq_host_desk;
+typedef struct {
+    tq_host_desk desk[TQ_HOST_DESKS];
+    int32_t bell, sleepers, open, unused;
+} tq_host_board;
+void tq_host_serve(tq_host_board *board);
+int tq_host_enter(tq_host_board *board, int by);
+int tq_host_drive(tq_host_board *board, tq_host_job *job, void *device, void *stream);
 
 #ifdef __cplusplus
 }

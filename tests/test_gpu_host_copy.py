@@ -1,6 +1,7 @@
 """Large host arrays on their way to and from the device in pieces: sizes around pieces, slots and the sharing threshold, from
 several threads on streams of their own, and where no thread helps."""
 import threading
+import time
 
 import numpy as np
 import pytest
@@ -63,3 +64,19 @@ def test_threads_with_streams_of_their_own(monkeypatch):
         for t in threads:
             t.join()
         assert bad == []
+
+
+def test_a_result_behind_other_work_costs_one_processor():
+    """While the stream works on something else nobody spins for a result but the thread that asked for it."""
+    tt = L.torch()
+    m = tt.randn((4096, 4096), device="cuda")
+    buf, (t,) = L.device_block(((1 << 21,), tt.float64))
+    t.fill_(1.5)
+    L.fetch(buf, (t, np.float64))
+    for _ in range(400):
+        m @ m
+    wall, cpu = time.perf_counter(), time.process_time()
+    out, = L.fetch(buf, (t, np.float64))
+    wall, cpu = time.perf_counter() - wall, time.process_time() - cpu
+    assert (out == 1.5).all()
+    assert cpu < 1.5 * wall + 0.05, (cpu, wall)

@@ -57,7 +57,7 @@ i = np.random.default_rng(0).integers(0, 8, 700_000)
 def narrow():
     with L.helpers(L.SHARED + 1), L.helpers(L.SHARED + 1):
         assert np.array_equal(L.narrow_indices(i, 8), i)
-    assert getattr(L._helping, "session", None) is None
+    assert getattr(L._helping, "board", None) is None
     print("done", flush=True)
 narrow()
 together = threading.Barrier(L.COPY_THREADS)

@@ -57,8 +57,12 @@ class TQHostJob(C.Structure):
                 ("slot_done", C.c_int32 * HOST_SLOTS)]
 
 
-class TQHostSession(C.Structure):
-    _fields_ = [("job", C.c_void_p), ("users", C.c_int64), ("bell", C.c_int32), ("closed", C.c_int32)]
+class TQHostDesk(C.Structure):
+    _fields_ = [("job", C.c_void_p), ("users", C.c_int64), ("taken", C.c_int64)]
+
+
+class TQHostBoard(C.Structure):
+    _fields_ = [("desk", TQHostDesk * 16), ("bell", C.c_int32), ("sleepers", C.c_int32), ("open", C.c_int32), ("unused", C.c_int32)]
 
 
 _P, _I, _L, _D = C.c_void_p, C.c_int, C.c_int64, C.c_double
@@ -113,9 +117,9 @@ PROTOTYPES = {
     "tq_decode_attention_plan": (_I, [C.POINTER(TQAttnParams), _I, _I, _I, _I, _L, C.POINTER(TQAttnPlan)]),
     "tq_decode_attention": (_I, [_P, _P, C.POINTER(TQAttnParams), _P, _I, _P, _P, _P, _P, _P, _P, _P, _L, _P]),
     "tq_decode_attention_static": (_I, [_P, _P, C.POINTER(TQAttnParams), _P, _I, _P, _P, _P, _P, _P, _P]),
-    "tq_host_serve": (None, [C.POINTER(TQHostSession)]),
-    "tq_host_close": (None, [C.POINTER(TQHostSession)]),
-    "tq_host_drive": (_I, [C.POINTER(TQHostSession), C.POINTER(TQHostJob), _P, _P]),
+    "tq_host_serve": (None, [C.POINTER(TQHostBoard)]),
+    "tq_host_enter": (_I, [C.POINTER(TQHostBoard), _I]),
+    "tq_host_drive": (_I, [C.POINTER(TQHostBoard), C.POINTER(TQHostJob), _P, _P]),
     "tq_score_tile": (_I, [_P, _P, _I, _L, _P, _P, _P, _L, _P, _I, _P, _L, _P]),
 }
 
@@ -235,13 +239,19 @@ ONE_COPY = 1 << 19
 # Bytes of the host array that a thread takes at a time (no two threads clear the same huge page), and the threads beside the
 # caller's.  A cache of 2 x 4 x 4096 x 128 in float32, both ways, ms, with pieces of 1 / 2 / 4 MiB: four threads 9.6 / 8.6 / 8.5, six
 # 8.9 / 8.6 / 8.0, eight 9.1 / 7.8 / 7.6, eleven 9.1 / 8.4 / 7.9 (16 CPUs); through the interpreter, which handed a share of each slot to six
-# threads, 9.4 - 11.0, 16 000 rows of 128 10.1 (now 4.5 - 5.4), 2 x 4 x 2048 x 256 in float64 11.9 - 13.7 (9.0).
+# threads, 9.4 - 11.0, 16 000 rows of 128 10.1 (now 4.5 - 5.4), 2 x 4 x 2048 x 256 in float64 11.9 - 13.7 (9.0).  Never more of them than
+# there are processors for beside the caller's.
 STAGE = 4 << 20
-COPY_THREADS = 8
+COPY_THREADS = max(1, min(8, len(os.sched_getaffinity(0)) - 1))
 # Host arrays from this size on are worked on by several threads: below, handing the work over costs more.
 SHARED = 4 << 20
 _copiers = None
 _copiers_lock = threading.Lock()
+# The copy threads work for every thread of the process that has large arrays under way, and go back to the pool when the last of
+# them is done: _serving counts those that were sent to the board and are not back.
+_board = TQHostBoard()
+_board_lock = threading.Lock()
+_serving = 0
 
 
 def _copy_pool():
@@ -253,15 +263,16 @@ def _copy_pool():
 
 
 def _forget_copiers():
-    """A forked child has none of the threads, and the lock as it happened to be held."""
-    global _copiers, _copiers_lock
+    """A forked child has none of the threads, and the locks and the board as they happened to be held."""
+    global _copiers, _copiers_lock, _board, _board_lock, _serving
     _copiers, _copiers_lock = None, threading.Lock()
+    _board, _board_lock, _serving = TQHostBoard(), threading.Lock(), 0
 
 
 os.register_at_fork(after_in_child=_forget_copiers)
 
 
-_helping = threading.local()     # .session: this thread's, while it has one
+_helping = threading.local()     # .board: where this thread's jobs are helped with, while it has any
 
 
 _alone = nullcontext()
@@ -271,24 +282,51 @@ def helpers(nbytes):
     """A context in which the copy threads help with this thread's host arrays where those are large (`nbytes`: the largest
     one's): one handing over for all the arrays of a call.  Where there are no threads (the ending interpreter takes no more work, a
     forked child starts its own) the caller's does it all."""
-    return _alone if nbytes <= SHARED or getattr(_helping, "session", None) is not None else _helped()
+    return _alone if nbytes <= SHARED or getattr(_helping, "board", None) is _board else _helped()
+
+
+def _serve(board, claim):
+    """A copy thread's work on the board, until nobody has arrays under way."""
+    global _serving
+    if not claim.acquire(blocking=False):
+        return      # counted out by the thread that could not submit it
+    while True:
+        lib().tq_host_serve(board)
+        with _board_lock:
+            if board.open <= 0:
+                _serving -= 1
+                return
+
+
+def _call_copiers(board):
+    """As many copy threads at the board as there are.  A submit that fails (the interpreter is ending, no thread can be started)
+    may have queued its work all the same: whoever claims it first counts it."""
+    global _serving
+    with _board_lock:
+        missing = COPY_THREADS - _serving
+        _serving += missing
+    while missing > 0:
+        claim = threading.Lock()
+        try:
+            _copy_pool().submit(_serve, board, claim)
+            missing -= 1
+        except RuntimeError:
+            with _board_lock:
+                _serving -= missing - 1 + claim.acquire(blocking=False)
+            return
 
 
 @contextmanager
 def _helped():
-    session = TQHostSession()
-    serve = lib().tq_host_serve
+    board, before = _board, getattr(_helping, "board", None)
+    lib().tq_host_enter(board, 1)
     try:
-        try:
-            for _ in range(COPY_THREADS):
-                _copy_pool().submit(serve, session)     # the queue keeps the session's memory as long as it may be looked at
-        except RuntimeError:
-            pass
-        _helping.session = session
+        _call_copiers(board)
+        _helping.board = board
         yield
     finally:
-        _helping.session = None
-        lib().tq_host_close(session)
+        lib().tq_host_enter(board, -1)
+        _helping.board = before
 
 
 def _host_job(kind, n, host, device):
@@ -304,7 +342,7 @@ def _host_job(kind, n, host, device):
         check(lib().tq_host_drive(None, job, ptr(device), stream))
     else:
         with helpers(n * each):
-            check(lib().tq_host_drive(_helping.session, job, ptr(device), stream))
+            check(lib().tq_host_drive(_board, job, ptr(device), stream))
     return job.seen
 
 

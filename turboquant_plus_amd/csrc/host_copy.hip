@@ -1,12 +1,20 @@
 // Large host arrays of the NumPy classes on their way between host memory and the device, by several threads of the caller's.
 //
 // A transfer is a job that lies in the caller's memory (tq_host_job).  Its array is cut into pieces, which the threads in
-// tq_host_serve take until none are left; the thread in tq_host_drive moves the pinned slots between the device and the pieces'
-// workers, takes pieces itself while it has nothing to move, and returns when every piece is done.  So a job needs no other thread
-// to end, and no thread belongs to this file.
+// tq_host_serve take; the thread in tq_host_drive moves the pinned slots between the device and the pieces' workers, takes pieces
+// itself while it has nothing to move, and returns when every piece is done.  So a job needs no other thread to end, and no thread
+// belongs to this file.
 //
-// What bounds it: the host's pages.  An int64 or float64 result of 32 MiB is fresh memory, which one thread fills at 14 - 23 GB/s
-// and six at 57 where the link gives 56; pieces are a few MiB of the host array, so that no two threads clear the same huge page.
+// The threads serve a board, on which every caller's job has a desk from the time that the stream is at it to its last piece; they go
+// round the desks a piece at a time.  A thread that finds nothing for a while (the time between two arrays of a call; a thread takes
+// longer to wake than a small array's piece to land) sleeps until the bell rings, which it does when a job comes and for every piece
+// that becomes ready while somebody sleeps.  The driver waits in the runtime until the stream is at its job: 0.43 s of other work in
+// front of a 32 MiB result, for which nine threads span 3.85 CPU-seconds, now take 0.43.
+//
+// What bounds it: fresh host pages, then the way through the slots.  A result of 32 to 64 MiB is fresh memory, which one thread fills
+// at 12 to 18 GB/s, six at 46 to 65 and eight at 77 to 86 (the link gives 56); with the transfer int64 results of 32 MiB come at 36 to
+// 45 GB/s of host bytes, float64 ones at 22 to 29, inputs go up at 30 to 34.  Pieces are a few MiB of the host array, so that no two
+// threads clear the same huge page.
 #include <hip/hip_runtime.h>
 #include <linux/futex.h>
 #include <sched.h>
@@ -85,36 +93,58 @@ bool take(tq_host_job *j) {
     return false;
 }
 
+constexpr int SPINS = 64;         // of the driver, before it sleeps until its next piece has landed
+constexpr int64_t SERVE_CYCLES = 500000;   // of a serving thread, before it sleeps: 0.15 to 0.25 ms
+
 void pause_for(int &idle) {
-    if (++idle < 64) __builtin_ia32_pause();
+    if (++idle < SPINS) __builtin_ia32_pause();
     else sched_yield();
 }
 
-}  // namespace
+// wakes at most n of the sleeping threads; they count themselves before they look at the bell for the last time
+void ring(tq_host_board *b, int n) {
+    __atomic_fetch_add(&b->bell, 1, __ATOMIC_SEQ_CST);
+    if (__atomic_load_n(&b->sleepers, __ATOMIC_SEQ_CST) > 0) syscall(SYS_futex, &b->bell, FUTEX_WAKE_PRIVATE, n, nullptr, nullptr, 0);
+}
 
-namespace {
-
-void work(tq_host_job *j) {
-    int idle = 0;
-    while (load(&j->next) < j->n_pieces) {   // the last piece taken: nothing is left for this thread
-        if (take(j)) idle = 0;
-        else pause_for(idle);
+// A job's place on the board while it lives.  Without a board, or where every desk is taken, the driver does the whole job.
+struct Desk {
+    tq_host_board *board;
+    tq_host_job *job;
+    tq_host_desk *at = nullptr;
+    void post() {   // others may look at the job from now on
+        for (int i = 0; board && !at && i < TQ_HOST_DESKS; ++i) {
+            int64_t free = 0;
+            if (!__atomic_compare_exchange_n(&board->desk[i].taken, &free, 1, false, __ATOMIC_ACQ_REL, __ATOMIC_RELAXED)) continue;
+            at = &board->desk[i];
+            __atomic_store_n(&at->job, job, __ATOMIC_SEQ_CST);
+        }
+        if (at) ring(board, (int)job->n_pieces);
     }
-}
-
-void ring(tq_host_session *s) {
-    __atomic_fetch_add(&s->bell, 1, __ATOMIC_RELEASE);
-    syscall(SYS_futex, &s->bell, FUTEX_WAKE_PRIVATE, 0x7FFFFFFF, nullptr, nullptr, 0);
-}
+    void allow(int64_t upto) {   // pieces below `upto` may be worked on
+        const int64_t was = job->ready, now = upto < job->n_pieces ? upto : job->n_pieces;
+        __atomic_store_n(&job->ready, now, __ATOMIC_RELEASE);
+        if (at && now > was) ring(board, (int)(now - was));
+    }
+    ~Desk() {
+        if (!at) return;
+        __atomic_store_n(&at->job, (tq_host_job *)nullptr, __ATOMIC_SEQ_CST);
+        int idle = 0;
+        while (__atomic_load_n(&at->users, __ATOMIC_SEQ_CST) > 0) pause_for(idle);
+        __atomic_store_n(&at->taken, 0, __ATOMIC_RELEASE);
+    }
+};
 
 // the stream's part of a job, and pieces in between
-hipError_t move(tq_host_job *j, char *device, hipStream_t s) {
+hipError_t move(tq_host_board *board, tq_host_job *j, char *device, hipStream_t s) {
+    Desk desk{board, j};
     int idle = 0;
     const bool down = j->kind == TQ_HOST_WIDEN || j->kind == TQ_HOST_FETCH;
-    hipEvent_t ev[SLOTS];
+    hipEvent_t ev[SLOTS + 1];   // of the slots' pieces, and one more
     hipError_t err = hipSuccess;
+    const int events = (j->n_pieces < SLOTS ? (int)j->n_pieces : SLOTS) + 1;
     int made = 0;
-    while (made < SLOTS && made < j->n_pieces && (err = hipEventCreateWithFlags(&ev[made], hipEventDisableTiming)) == hipSuccess) ++made;
+    while (made < events && (err = hipEventCreateWithFlags(&ev[made], hipEventDisableTiming)) == hipSuccess) ++made;
     // sent: pieces handed to the stream; landed: of those, the ones the stream is done with
     int64_t sent = 0, landed = 0;
     auto send = [&] {
@@ -124,33 +154,44 @@ hipError_t move(tq_host_job *j, char *device, hipStream_t s) {
         if (err == hipSuccess) err = hipEventRecord(ev[sent % SLOTS], s);
         ++sent;
     };
-    auto poll = [&] {   // one more piece landed?
+    auto poll = [&](bool wait) {   // one more piece landed?
         if (landed == sent) return false;
-        const hipError_t q = hipEventQuery(ev[landed % SLOTS]);
+        hipError_t q = hipEventQuery(ev[landed % SLOTS]);
         if (q == hipErrorNotReady) {
             (void)hipGetLastError();   // or the next launch's check would report it
-            return false;
+            if (!wait) return false;
+            q = hipEventSynchronize(ev[landed % SLOTS]);
         }
         if (q != hipSuccess) err = q;
         ++landed;
         return true;
     };
-    auto allow = [&](int64_t upto) { __atomic_store_n(&j->ready, upto < j->n_pieces ? upto : j->n_pieces, __ATOMIC_RELEASE); };
-    if (!down) allow(SLOTS);   // every slot is free
+    if (down) {
+        // the first pieces follow what the stream has before them; the threads wake up while they travel
+        if (err == hipSuccess) err = hipEventRecord(ev[made - 1], s);
+        while (err == hipSuccess && sent < SLOTS && sent < j->n_pieces) send();
+        if (err == hipSuccess) err = hipEventSynchronize(ev[made - 1]);
+    } else {
+        desk.allow(SLOTS);   // every slot is free
+    }
+    if (err == hipSuccess) desk.post();
     while (err == hipSuccess && (down ? load(&j->done) < j->n_pieces : landed < j->n_pieces)) {
         bool moved = false;
         // down: into a slot whose earlier piece is worked off; up: a slot that is filled, by the piece after the one that landed
-        if (sent < j->n_pieces && sent - SLOTS < landed && ((down && sent < SLOTS) || load(&j->slot_done[sent % SLOTS]))) {
+        if (sent < j->n_pieces && sent - SLOTS < landed && load(&j->slot_done[sent % SLOTS])) {
             if (down) __atomic_store_n(&j->slot_done[sent % SLOTS], 0, __ATOMIC_RELAXED);
             send();
             moved = true;
         }
-        if (err == hipSuccess && poll()) {
+        // with nothing else to do it sleeps until the next piece has landed: the stream has work of others before it, or is slower
+        // than the threads.  (With a slot to fill or empty there are pieces in work, whose workers do not wake it.)
+        const bool wait = !moved && idle >= SPINS && (down ? load(&j->done) == landed : load(&j->done) == sent);
+        if (err == hipSuccess && poll(wait)) {
             if (down) {
-                allow(landed);
+                desk.allow(landed);
             } else {   // that piece's slot may be filled again
                 __atomic_store_n(&j->slot_done[(landed - 1) % SLOTS], 0, __ATOMIC_RELAXED);
-                allow(landed + SLOTS);
+                desk.allow(landed + SLOTS);
             }
             moved = true;
         }
@@ -169,33 +210,43 @@ hipError_t move(tq_host_job *j, char *device, hipStream_t s) {
 
 }  // namespace
 
-extern "C" void tq_host_serve(tq_host_session *s) {
+extern "C" void tq_host_serve(tq_host_board *b) {
+    unsigned first = 0;
+    int64_t idle_since = 0;
     for (;;) {
-        const int32_t heard = load(&s->bell);
-        if (load(&s->closed)) return;
-        __atomic_fetch_add(&s->users, 1, __ATOMIC_SEQ_CST);   // before the look: tq_host_drive waits for users after it has taken the job away
-        if (tq_host_job *j = __atomic_load_n(&s->job, __ATOMIC_SEQ_CST)) work(j);
-        __atomic_fetch_sub(&s->users, 1, __ATOMIC_SEQ_CST);
-        syscall(SYS_futex, &s->bell, FUTEX_WAIT_PRIVATE, heard, nullptr, nullptr, 0);   // returns at once if it rang meanwhile
+        const int32_t heard = load(&b->bell);
+        if (load(&b->open) <= 0) return;
+        bool did = false;
+        for (int k = 0; k < TQ_HOST_DESKS; ++k) {
+            tq_host_desk *d = &b->desk[(first + k) % TQ_HOST_DESKS];
+            if (!load(&d->job)) continue;
+            __atomic_fetch_add(&d->users, 1, __ATOMIC_SEQ_CST);   // before the look that counts: the driver takes the job away and then waits for users
+            if (tq_host_job *j = __atomic_load_n(&d->job, __ATOMIC_SEQ_CST)) did |= take(j);
+            __atomic_fetch_sub(&d->users, 1, __ATOMIC_SEQ_CST);
+        }
+        ++first;
+        const int64_t now = (int64_t)__builtin_ia32_rdtsc();
+        if (did || !idle_since) {
+            idle_since = now;
+        } else if (now - idle_since < SERVE_CYCLES) {
+            __builtin_ia32_pause();
+        } else {
+            __atomic_fetch_add(&b->sleepers, 1, __ATOMIC_SEQ_CST);
+            syscall(SYS_futex, &b->bell, FUTEX_WAIT_PRIVATE, heard, nullptr, nullptr, 0);   // returns at once if it rang meanwhile
+            __atomic_fetch_sub(&b->sleepers, 1, __ATOMIC_SEQ_CST);
+            idle_since = 0;
+        }
     }
 }
 
-extern "C" void tq_host_close(tq_host_session *s) {
-    __atomic_store_n(&s->closed, 1, __ATOMIC_RELEASE);
-    ring(s);
+extern "C" int tq_host_enter(tq_host_board *b, int by) {
+    const int open = __atomic_add_fetch(&b->open, by, __ATOMIC_SEQ_CST);
+    if (open <= 0 || by == 0) ring(b, 0x7FFFFFFF);
+    return open;
 }
 
-extern "C" int tq_host_drive(tq_host_session *s, tq_host_job *j, void *device, void *stream) {
-    if (s) {
-        __atomic_store_n(&s->job, j, __ATOMIC_SEQ_CST);
-        ring(s);
-    }
-    const hipError_t err = move(j, (char *)device, (hipStream_t)stream);
-    if (s) {
-        __atomic_store_n(&s->job, (tq_host_job *)nullptr, __ATOMIC_SEQ_CST);
-        int idle = 0;
-        while (__atomic_load_n(&s->users, __ATOMIC_SEQ_CST) > 0) pause_for(idle);
-    }
+extern "C" int tq_host_drive(tq_host_board *b, tq_host_job *j, void *device, void *stream) {
+    const hipError_t err = move(b, j, (char *)device, (hipStream_t)stream);
     if (err == hipSuccess) return TQ_OK;
     tq_set_error("host copy: %s", hipGetErrorString(err));
     return TQ_ERR_HIP;
