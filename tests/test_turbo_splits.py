@@ -11,13 +11,66 @@ from test_attention_plan import plan
 from turboquant_plus_amd import turbo as T
 
 
-@pytest.mark.parametrize("eight", [False, True])
-@pytest.mark.parametrize("k,v", [(2, 2), (3, 3), (3, 2), (4, 4), (4, 2), (3, 4)])
-def test_counts(k, v, eight):
-    for groups, tokens, one in itertools.product((1, 2, 7, 40, 300, 5000), (1, 63, 64, 700, 5000, 90000, 3_000_000), {k == v, False}):
-        now = T.balanced_splits(groups, tokens, T.default_splits(groups, tokens, eight_heads=eight), eight_heads=eight, turbo_k=True, turbo_v=True)
-        n = T.turbo_splits(groups, tokens, now, k_bits=k, v_bits=v, one_table=one, eight_heads=eight)
-        assert n == now or (n in T._SPLIT_COUNTS and n <= (tokens + 63) // 64 and (not eight or groups <= 256))
+# steps timed with several counts: K bits, V bits, query heads per KV head, groups, tokens, dense bias rows, us by split count
+TIMED = [
+    (3, 3, 1, 1, 64230, False, {256: 16.9}),
+    (3, 3, 1, 3, 24338, False, {72: 16.7, 80: 15.5, 160: 14.1, 176: 14.5, 256: 14.4}),
+    (3, 3, 1, 16, 6682, False, {32: 12.7, 36: 12.0, 40: 12.0, 48: 11.9, 96: 13.7}),
+    (3, 4, 1, 93, 104190, False, {28: 228.4, 40: 224.0, 48: 258.2, 64: 209.5, 80: 186.2}),
+    (4, 2, 1, 326, 16472, False, {8: 123.0, 12: 115.5, 16: 128.3, 24: 106.8}),
+    (4, 4, 4, 1, 69520, False, {256: 20.0, 528: 23.9}),
+    (3, 3, 4, 2, 906, True, {4: 11.3}),
+    (3, 3, 4, 8, 837, True, {4: 11.1}),
+    (3, 3, 4, 24, 1650, True, {8: 13.6, 12: 12.3, 16: 11.0, 20: 11.3, 24: 11.6}),
+    (3, 4, 4, 68, 72610, False, {16: 183.8, 48: 129.4, 56: 120.0, 72: 132.9, 96: 112.1, 112: 105.0}),
+    (3, 3, 4, 291, 543, True, {4: 11.9, 8: 11.5}),
+    (3, 4, 4, 520, 3652, False, {4: 75.0, 8: 76.0, 12: 57.3}),
+    (4, 3, 8, 1, 36374, False, {256: 23.0, 272: 25.6}),
+    (4, 2, 8, 2, 12696, False, {96: 21.9, 112: 16.6, 128: 16.8, 160: 17.7, 192: 27.1}),
+    (4, 2, 8, 10, 6186, False, {28: 15.2, 32: 15.5, 48: 17.6, 56: 14.4, 64: 14.4, 80: 15.7}),
+    (2, 2, 8, 17, 34109, True, {64: 34.5, 112: 28.6, 128: 39.7, 256: 43.1}),
+    (4, 2, 8, 36, 20396, True, {8: 94.7, 28: 36.7, 56: 32.9, 96: 49.1, 192: 51.1}),
+    (4, 4, 8, 50, 2456, False, {8: 17.4, 12: 17.4, 16: 14.4, 24: 17.1}),
+    (4, 2, 8, 52, 28548, False, {8: 89.6, 32: 40.8, 36: 62.4, 112: 55.7, 128: 65.6}),
+    (4, 3, 8, 232, 38566, False, {8: 230.7, 12: 282.1, 16: 181.8, 20: 244.8, 24: 175.8}),
+    (3, 3, 12, 1, 106134, False, {128: 35.2, 160: 33.2, 192: 38.3, 256: 30.1}),
+    (4, 4, 12, 4, 95750, False, {40: 66.6, 48: 71.4, 72: 54.2, 128: 33.7, 192: 45.6, 512: 40.9}),
+    (4, 2, 12, 7, 24194, True, {20: 51.7, 56: 28.2, 72: 32.0, 96: 29.1, 128: 23.6}),
+    (2, 2, 12, 9, 4785, False, {16: 15.5, 24: 14.9, 32: 12.4, 40: 13.6, 72: 19.0}),
+    (4, 2, 12, 12, 65426, True, {32: 81.5, 48: 72.9, 56: 69.6, 128: 49.8, 160: 63.3, 192: 81.7}),
+    (3, 4, 12, 16, 31186, True, {24: 54.5, 56: 41.0, 64: 38.3, 112: 47.6, 128: 46.2, 160: 58.5}),
+    (2, 2, 12, 39, 3914, False, {16: 17.9, 28: 19.2, 32: 16.9, 36: 21.2, 56: 18.2}),
+    (3, 4, 16, 4, 71330, False, {28: 68.0, 56: 42.1, 128: 29.9, 192: 42.0, 256: 35.5, 512: 41.3}),
+    (3, 3, 16, 8, 598, False, {4: 10.5}),
+    (3, 3, 16, 16, 7091, False, {16: 20.1, 28: 15.7, 36: 23.0, 48: 21.0, 72: 24.0, 80: 21.2}),
+    (4, 4, 16, 21, 3638, False, {8: 21.8, 16: 16.2, 24: 19.0, 28: 17.5, 56: 19.9}),
+    (4, 2, 16, 40, 3769, False, {12: 22.4, 16: 19.1, 20: 17.5, 36: 25.4}),
+    (4, 3, 16, 48, 14357, True, {24: 51.4, 28: 53.0, 32: 50.3, 36: 87.7, 40: 65.4, 64: 68.5}),
+    (4, 2, 16, 100, 3099, False, {8: 25.6, 16: 34.3, 20: 31.0, 24: 55.2, 28: 33.4, 36: 38.3}),
+    (4, 4, 16, 125, 4462, True, {8: 45.8, 16: 58.4, 20: 57.0, 24: 73.5, 28: 57.0}),
+    (4, 2, 16, 179, 5421, True, {8: 61.5, 12: 94.6, 16: 81.6, 20: 79.1}),
+    (4, 3, 24, 3, 5110, False, {32: 13.8, 48: 16.4, 56: 15.0, 64: 14.8, 72: 19.3}),
+    (3, 4, 24, 17, 7807, True, {16: 28.5, 20: 26.8, 24: 29.2, 36: 32.6, 48: 38.2}),
+    (4, 4, 24, 33, 32020, False, {12: 122.0, 20: 74.5, 24: 118.2, 32: 115.9, 40: 101.9, 56: 109.7}),
+    (4, 2, 24, 38, 67284, False, {8: 200.0, 16: 138.5, 32: 195.9, 36: 217.0, 40: 186.1, 48: 192.2}),
+]
+
+
+def test_counts_beside_those_that_were_timed():
+    """Over drawn steps the count that a call gets is within 4 % of the fastest that was timed on average (balanced_splits': 12 %), and
+    hardly ever slower than balanced_splits'."""
+    own, plain = [], []
+    for k, v, per_kv, groups, tokens, dense, us in TIMED:
+        codecs = [SimpleNamespace(bits=b, centroids=np.arange(1 << b)) for b in (k, v)]
+        eight = per_kv > 4
+        before = T.balanced_splits(groups, tokens, T.default_splits(groups, tokens, eight_heads=eight), eight_heads=eight, turbo_k=True, turbo_v=True,
+                                   three_bit=3 in (k, v))
+        n = T.call_splits(*codecs, groups, per_kv, tokens)[2 if dense else 0]
+        if n in us and before in us:
+            own.append(us[n] / min(us.values()))
+            plain.append(us[before] / min(us.values()))
+    assert len(own) >= 32 and np.mean(own) < 1.04 and np.mean(plain) > 1.08
+    assert sum(o > 1.03 * p for o, p in zip(own, plain)) <= 1 and max(own) < 1.5
 
 
 def test_shapes_that_were_timed():

@@ -7,7 +7,9 @@
 // 10 007 tokens 27.5 -> 22.6.
 // Pairs of 2- and 3-bit codes stay with the general kernel: their quad tables (one 8-byte read per four values, 6.4 clocks) have no
 // room for copies, so only the matrix side would change, which is worth 8 us of 94 with eight heads, and costs 1 us of 80 with four
-// (28 swaps and 16 permutes per tile for 41 instructions of transposing); and a head must not depend on how many share its pass.
+// (28 swaps and 16 permutes per tile for 41 instructions of transposing).  Eight heads alone are not moved here either: a head on 2- and
+// 3-bit rows then has the same bits however many share its pass (where its splits are merged in one order), which it would lose.  (On rows with a 4-bit side it has them within
+// either kernel, but which one runs may depend on the number of heads: the room for the tables, a list beside four heads.)
 //
 // One wavefront owns one context split and walks it in tiles of 64 tokens.  Both products run on the 16x16x32 fp16 matrix
 // instructions with the packed side as the rows and the query heads as the columns:

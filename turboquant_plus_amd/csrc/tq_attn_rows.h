@@ -190,7 +190,7 @@ __host__ __device__ constexpr int max_waves_per_workgroup(int vbits, int hg, boo
 // rows of 8 x 8 groups at 8192 tokens, eight heads: turbo3 23.3 -> 21.4 us, turbo3 K with turbo4 V 28.2 -> 23.8, 8-bit K with turbo3
 // V 28.2 -> 25.6),
 // and a dense row's load that may or may not have been issued makes the compiler wait for the youngest loads, i.e. the V rows
-// just requested, at the top of every tile (4 x 20 000 tokens, turbo3, Sparse V 25.5 -> 23.4 us; 4 x 16 groups at 6000 tokens 15.1 ->
+// just requested, at the top of every tile (4 x 20 000 tokens, turbo3, Sparse V: kernel 24.6 -> 22.6 us; 4 x 16 groups at 6000 tokens 15.1 ->
 // 14.6; one user at 4000 10.8 -> 10.5).
 constexpr int BIAS_NONE = 0, BIAS_LIST = 1, BIAS_DENSE = 2, BIAS_BOTH = BIAS_LIST | BIAS_DENSE;
 // D256: heads of 256 dims.  A token is rows 2 token and 2 token + 1 of caches that are

@@ -728,7 +728,9 @@ def balanced_splits(n_groups: int, tokens: int, default: int, *, eight_heads: bo
 
 # What a step on turbo rows takes since its end became cheaper and 4-bit rows got tables with a copy per lane, in microseconds: a
 # constant, per tile on the busiest SIMD of the fullest CU (times four), per tile on the longest wavefront of each round of
-# workgroups, per partial of a group, per round, per partial beyond 16, per further round of workgroups of twelve.  Fitted to the
+# workgroups, per partial of a group, per round, per partial beyond 16, per further round of workgroups of twelve.  A line is one
+# regression: its coefficients share the time out between terms that go together (deep splits and many rounds, say), so that one by
+# itself is not the cost of its step, and some are negative; outside of the shapes below a line says nothing.  Fitted to the
 # timings of 15 700 drawn shapes (1 to 300 groups, 512 to 131 072 tokens, up to nine counts each); ratios between counts of one shape
 # scatter by 7 - 9 %, 11 % for eight heads in the general kernel.
 _TURBO_COST = {  # by (more than four heads, widest code, table copies per lane)
