@@ -6,10 +6,10 @@
 // belongs to this file.
 //
 // The threads serve a board, on which every caller's job has a desk from the time that the stream is at it to its last piece; they go
-// round the desks a piece at a time.  A thread that finds nothing for a while (the time between two arrays of a call; a thread takes
-// longer to wake than a small array's piece to land) sleeps until the bell rings, which it does when a job comes and for every piece
-// that becomes ready while somebody sleeps.  The driver waits in the runtime until the stream is at its job: 0.43 s of other work in
-// front of a 32 MiB result, for which nine threads span 3.85 CPU-seconds, now take 0.43.
+// round the desks a piece at a time.  A thread that finds nothing for a while (the time between two arrays of a call: it takes longer
+// to wake than a small piece to land) sleeps until the bell rings, which it does when a job comes and for every piece that becomes
+// ready while somebody sleeps.  The driver waits in the runtime until the stream is at its job: 0.43 s of other work in front of a
+// 32 MiB result, for which nine threads span 3.85 CPU-seconds, now take 0.43.
 //
 // What bounds it: fresh host pages, then the way through the slots.  A result of 32 to 64 MiB is fresh memory, which one thread fills
 // at 12 to 18 GB/s, six at 46 to 65 and eight at 77 to 86 (the link gives 56); with the transfer int64 results of 32 MiB come at 36 to
@@ -119,7 +119,7 @@ struct Desk {
             at = &board->desk[i];
             __atomic_store_n(&at->job, job, __ATOMIC_SEQ_CST);
         }
-        if (at) ring(board, (int)job->n_pieces);
+        if (at) ring(board, 0x7FFFFFFF);
     }
     void allow(int64_t upto) {   // pieces below `upto` may be worked on
         const int64_t was = job->ready, now = upto < job->n_pieces ? upto : job->n_pieces;
@@ -140,9 +140,9 @@ hipError_t move(tq_host_board *board, tq_host_job *j, char *device, hipStream_t 
     Desk desk{board, j};
     int idle = 0;
     const bool down = j->kind == TQ_HOST_WIDEN || j->kind == TQ_HOST_FETCH;
-    hipEvent_t ev[SLOTS + 1];   // of the slots' pieces, and one more
+    hipEvent_t ev[SLOTS + 1];   // of the slots' pieces, and with a board one more
     hipError_t err = hipSuccess;
-    const int events = (j->n_pieces < SLOTS ? (int)j->n_pieces : SLOTS) + 1;
+    const int events = (j->n_pieces < SLOTS ? (int)j->n_pieces : SLOTS) + (board ? 1 : 0);
     int made = 0;
     while (made < events && (err = hipEventCreateWithFlags(&ev[made], hipEventDisableTiming)) == hipSuccess) ++made;
     // sent: pieces handed to the stream; landed: of those, the ones the stream is done with
@@ -167,10 +167,11 @@ hipError_t move(tq_host_board *board, tq_host_job *j, char *device, hipStream_t 
         return true;
     };
     if (down) {
-        // the first pieces follow what the stream has before them; the threads wake up while they travel
-        if (err == hipSuccess) err = hipEventRecord(ev[made - 1], s);
+        // the first pieces follow what the stream has before them; the threads wake up while they travel (called ahead of that they
+        // were slower, 2 x 4 x 4096 x 128 both ways 7.7 ms against 7.2)
+        if (err == hipSuccess && board) err = hipEventRecord(ev[made - 1], s);
         while (err == hipSuccess && sent < SLOTS && sent < j->n_pieces) send();
-        if (err == hipSuccess) err = hipEventSynchronize(ev[made - 1]);
+        if (err == hipSuccess && board) err = hipEventSynchronize(ev[made - 1]);
     } else {
         desk.allow(SLOTS);   // every slot is free
     }
@@ -221,7 +222,16 @@ extern "C" void tq_host_serve(tq_host_board *b) {
             tq_host_desk *d = &b->desk[(first + k) % TQ_HOST_DESKS];
             if (!load(&d->job)) continue;
             __atomic_fetch_add(&d->users, 1, __ATOMIC_SEQ_CST);   // before the look that counts: the driver takes the job away and then waits for users
-            if (tq_host_job *j = __atomic_load_n(&d->job, __ATOMIC_SEQ_CST)) did |= take(j);
+            if (tq_host_job *j = __atomic_load_n(&d->job, __ATOMIC_SEQ_CST)) {
+                // some microseconds at a job whose next piece is not there yet: the threads' coming and going writes to the desk (without
+                // this 7.6 ms instead of 7.2)
+                bool took = take(j);
+                for (int spin = 0; !took && spin < SPINS && load(&j->next) < j->n_pieces; ++spin) {
+                    __builtin_ia32_pause();
+                    took = take(j);
+                }
+                did |= took;
+            }
             __atomic_fetch_sub(&d->users, 1, __ATOMIC_SEQ_CST);
         }
         ++first;
