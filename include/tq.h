@@ -418,9 +418,10 @@ int tq_score_tile(const tq_handle *h, const void *q, int q_dtype, int64_t nq, co
                   void *workspace, int64_t workspace_bytes, void *stream);
 
 /* Large host arrays by several of the caller's threads.  A board and a job lie in the caller's memory, zeroed but for the
- * job's first seven fields.  Threads in tq_host_serve work on the jobs of a board, and sleep between them, until it is closed: while
- * its count of users, which tq_host_enter(board, +1 or -1) changes and returns (0: wakes the threads), is not positive.  The
- * board's memory has to outlive them.  tq_host_drive works on one job: an array of n elements in n_pieces pieces of `piece` elements, taken by the
+ * job's first seven fields.  Threads in tq_host_serve work on the jobs of a board and sleep between them; they return some milliseconds
+ * after its last user has closed it.  tq_host_open(board, threads) counts a user and returns how many threads the caller has to send
+ * to tq_host_serve for there to be `threads` of them; tq_host_close(board, not_sent) counts the user out, and those of the threads
+ * that it could not send.  The board's memory has to outlive the threads.  tq_host_drive works on one job: an array of n elements in n_pieces pieces of `piece` elements, taken by the
  * board's threads and by itself (board may be NULL, and nobody need come); it returns when every piece is done, the stream
  * has finished with the slots and no thread looks at the job.  Any number of threads may drive jobs on one board.  `slots`: pinned memory for min(TQ_HOST_SLOTS, n_pieces) pieces, one
  * byte per element; `device`: the array's other side, on `stream`'s device.
@@ -442,10 +443,12 @@ typedef struct {
 } tq_host_desk;
 typedef struct {
     tq_host_desk desk[TQ_HOST_DESKS];
-    int32_t bell, sleepers, open, unused;
+    int64_t state;             /* users << 32 | threads */
+    int32_t bell, sleepers;
 } tq_host_board;
 void tq_host_serve(tq_host_board *board);
-int tq_host_enter(tq_host_board *board, int by);
+int tq_host_open(tq_host_board *board, int threads);
+void tq_host_close(tq_host_board *board, int not_sent);
 int tq_host_drive(tq_host_board *board, tq_host_job *job, void *device, void *stream);
 
 #ifdef __cplusplus

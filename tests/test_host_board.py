@@ -22,11 +22,11 @@ class Job:
     def post(self, board, at):
         board.desk[at].taken = 1
         board.desk[at].job = C.addressof(self.job)
-        L.lib().tq_host_enter(board, 0)
+        wake(board)
 
     def allow(self, board, upto):
         self.job.ready = upto
-        L.lib().tq_host_enter(board, 0)
+        wake(board)
 
     def wait(self, done, seconds=20):
         end = time.time() + seconds
@@ -41,7 +41,21 @@ class Job:
         board.desk[at].taken = 0
 
 
+def wake(board):
+    L.lib().tq_host_open(board, 0)
+    L.lib().tq_host_close(board, 0)
+
+
+def users(board):
+    return board.state >> 32
+
+
+def serving(board):
+    return board.state & 0xFFFFFFFF
+
+
 def serve(board, count):
+    assert L.lib().tq_host_open(board, count) == count
     threads = [threading.Thread(target=L.lib().tq_host_serve, args=(board,)) for _ in range(count)]
     for t in threads:
         t.start()
@@ -49,16 +63,16 @@ def serve(board, count):
 
 
 def close(board, threads):
-    assert L.lib().tq_host_enter(board, -1) == 0
+    L.lib().tq_host_close(board, 0)
     for t in threads:
         t.join(20)
         assert not t.is_alive()
+    assert board.state == 0
 
 
 def test_waiting_costs_no_processor_time():
     """A job whose pieces are not there yet (the stream has other work before them) and a board without jobs."""
     board, job = L.TQHostBoard(), Job(4)
-    assert L.lib().tq_host_enter(board, 1) == 1
     threads = serve(board, 6)
     for post in (False, True):
         if post:
@@ -78,7 +92,6 @@ def test_waiting_costs_no_processor_time():
 @pytest.mark.parametrize("count", [1, 3])
 def test_a_job_that_waits_keeps_nobody_from_another(count):
     board, stuck, other = L.TQHostBoard(), Job(3), Job(8)
-    L.lib().tq_host_enter(board, 1)
     stuck.post(board, 2)
     threads = serve(board, count)
     time.sleep(0.05)
@@ -99,7 +112,7 @@ def back_in_the_pool():
     for _ in range(L.COPY_THREADS):
         L._copy_pool().submit(together.wait)
     together.wait(20)
-    return L._serving == 0
+    return L._board.state == 0
 
 
 def test_two_callers_share_the_copy_threads():
@@ -134,26 +147,32 @@ def test_two_callers_share_the_copy_threads():
 
 
 def test_threads_that_cannot_be_had(monkeypatch):
-    """The count of threads at the board holds where a submit fails, also one that has queued its work."""
-    pool, left = L._copy_pool(), []
+    """The count of threads at the board holds where a submit fails, also one that has queued its work; without threads, too."""
+    pool, sent = L._copy_pool(), []
 
     class Ending:
         def submit(self, fn, *args):
-            if len(left) == 1:
-                pool.submit(fn, *args)
-            left.append(1)
-            if len(left) > 1:
-                raise RuntimeError("cannot schedule new futures after shutdown")
+            pool.submit(fn, *args)
+            sent.append(1)
+            if len(sent) == 2:
+                raise RuntimeError("can't start new thread")
     monkeypatch.setattr(L, "_copy_pool", Ending)
+    monkeypatch.setattr(L, "COPY_THREADS", 4)
     with L.helpers(L.SHARED + 1):
-        assert L._serving <= L.COPY_THREADS
+        assert len(sent) == 2 and users(L._board) == 1 and serving(L._board) == 4
+    assert serving(L._board) <= 2 and users(L._board) == 0
     monkeypatch.undo()
-    end = time.time() + 20
-    while L._serving != 1 and time.time() < end:    # the first of them was never run
-        time.sleep(0.001)
-    assert L._serving == 1
-    with L._board_lock:
-        L._serving -= 1
+    assert back_in_the_pool()
+
+
+def test_a_second_call_finds_the_threads_still_there():
+    """They leave some milliseconds after the last call, so that calls in a row do not send for them each time."""
+    with L.helpers(L.SHARED + 1):
+        pass
+    assert serving(L._board) == L.COPY_THREADS
+    before = L._copy_pool()._work_queue.qsize()
+    with L.helpers(L.SHARED + 1):
+        assert serving(L._board) == L.COPY_THREADS and L._copy_pool()._work_queue.qsize() <= before
     assert back_in_the_pool()
 
 

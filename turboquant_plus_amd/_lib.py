@@ -62,7 +62,7 @@ class TQHostDesk(C.Structure):
 
 
 class TQHostBoard(C.Structure):
-    _fields_ = [("desk", TQHostDesk * 16), ("bell", C.c_int32), ("sleepers", C.c_int32), ("open", C.c_int32), ("unused", C.c_int32)]
+    _fields_ = [("desk", TQHostDesk * 16), ("state", C.c_int64), ("bell", C.c_int32), ("sleepers", C.c_int32)]
 
 
 _P, _I, _L, _D = C.c_void_p, C.c_int, C.c_int64, C.c_double
@@ -118,7 +118,8 @@ PROTOTYPES = {
     "tq_decode_attention": (_I, [_P, _P, C.POINTER(TQAttnParams), _P, _I, _P, _P, _P, _P, _P, _P, _P, _L, _P]),
     "tq_decode_attention_static": (_I, [_P, _P, C.POINTER(TQAttnParams), _P, _I, _P, _P, _P, _P, _P, _P]),
     "tq_host_serve": (None, [C.POINTER(TQHostBoard)]),
-    "tq_host_enter": (_I, [C.POINTER(TQHostBoard), _I]),
+    "tq_host_open": (_I, [C.POINTER(TQHostBoard), _I]),
+    "tq_host_close": (None, [C.POINTER(TQHostBoard), _I]),
     "tq_host_drive": (_I, [C.POINTER(TQHostBoard), C.POINTER(TQHostJob), _P, _P]),
     "tq_score_tile": (_I, [_P, _P, _I, _L, _P, _P, _P, _L, _P, _I, _P, _L, _P]),
 }
@@ -247,11 +248,9 @@ COPY_THREADS = max(1, min(8, len(os.sched_getaffinity(0)) - 1))
 SHARED = 4 << 20
 _copiers = None
 _copiers_lock = threading.Lock()
-# The copy threads work for every thread of the process that has large arrays under way, and go back to the pool when the last of
-# them is done: _serving counts those that were sent to the board and are not back.
+# The copy threads work for every thread of the process that has large arrays under way, and go back to the pool some milliseconds
+# after the last of them is done.
 _board = TQHostBoard()
-_board_lock = threading.Lock()
-_serving = 0
 
 
 def _copy_pool():
@@ -263,10 +262,9 @@ def _copy_pool():
 
 
 def _forget_copiers():
-    """A forked child has none of the threads, and the locks and the board as they happened to be held."""
-    global _copiers, _copiers_lock, _board, _board_lock, _serving
-    _copiers, _copiers_lock = None, threading.Lock()
-    _board, _board_lock, _serving = TQHostBoard(), threading.Lock(), 0
+    """A forked child has none of the threads, and the lock and the board as they happened to be held."""
+    global _copiers, _copiers_lock, _board
+    _copiers, _copiers_lock, _board = None, threading.Lock(), TQHostBoard()
 
 
 os.register_at_fork(after_in_child=_forget_copiers)
@@ -285,47 +283,21 @@ def helpers(nbytes):
     return _alone if nbytes <= SHARED or getattr(_helping, "board", None) is _board else _helped()
 
 
-def _serve(board, claim):
-    """A copy thread's work on the board, until nobody has arrays under way."""
-    global _serving
-    if not claim.acquire(blocking=False):
-        return      # counted out by the thread that could not submit it
-    while True:
-        lib().tq_host_serve(board)
-        with _board_lock:
-            if board.open <= 0:
-                _serving -= 1
-                return
-
-
-def _call_copiers(board):
-    """As many copy threads at the board as there are.  A submit that fails (the interpreter is ending, no thread can be started)
-    may have queued its work all the same: whoever claims it first counts it."""
-    global _serving
-    with _board_lock:
-        missing = COPY_THREADS - _serving
-        _serving += missing
-    while missing > 0:
-        claim = threading.Lock()
-        try:
-            _copy_pool().submit(_serve, board, claim)
-            missing -= 1
-        except RuntimeError:
-            with _board_lock:
-                _serving -= missing - 1 + claim.acquire(blocking=False)
-            return
-
-
 @contextmanager
 def _helped():
     board, before = _board, getattr(_helping, "board", None)
-    lib().tq_host_enter(board, 1)
+    missing = lib().tq_host_open(board, COPY_THREADS)
     try:
-        _call_copiers(board)
+        try:
+            while missing > 0:
+                missing -= 1    # also where the submit fails: it may have queued its work all the same
+                _copy_pool().submit(lib().tq_host_serve, board)
+        except RuntimeError:    # the interpreter is ending, or no thread can be started
+            pass
         _helping.board = board
         yield
     finally:
-        lib().tq_host_enter(board, -1)
+        lib().tq_host_close(board, missing)
         _helping.board = before
 
 
