@@ -417,14 +417,16 @@ int tq_score_tile(const tq_handle *h, const void *q, int q_dtype, int64_t nq, co
                   const uint8_t *sign_bits, const void *rnorms_f16, int64_t nk, void *logits, int out_dtype,
                   void *workspace, int64_t workspace_bytes, void *stream);
 
-/* Large host arrays by several of the caller's threads.  A board and a job lie in the caller's memory, zeroed but for the
- * job's first seven fields.  Threads in tq_host_serve work on the jobs of a board and sleep between them; they return some milliseconds
- * after its last user has closed it.  tq_host_open(board, threads) counts a user and returns how many threads the caller has to send
- * to tq_host_serve for there to be `threads` of them; tq_host_close(board, not_sent) counts the user out, and those of the threads
- * that it could not send.  The board's memory has to outlive the threads.  tq_host_drive works on one job: an array of n elements in n_pieces pieces of `piece` elements, taken by the
- * board's threads and by itself (board may be NULL, and nobody need come); it returns when every piece is done, the stream
- * has finished with the slots and no thread looks at the job.  Any number of threads may drive jobs on one board.  `slots`: pinned memory for min(TQ_HOST_SLOTS, n_pieces) pieces, one
- * byte per element; `device`: the array's other side, on `stream`'s device.
+/* Large host arrays by several of the caller's threads.  A board and a job lie in the caller's memory, zeroed but for the job's
+ * first six fields (up to `slots`).
+ * Threads in tq_host_serve work on the jobs of a board and sleep between them; they return some milliseconds after its last user has
+ * closed it.  tq_host_open(board, threads) counts a user and returns how many threads the caller has to send to tq_host_serve for
+ * there to be `threads` of them; tq_host_close(board, not_sent) counts the user out, and those of the threads that it could not
+ * send.  The board's memory has to outlive the threads.
+ * tq_host_drive works on one job: an array of n elements in n_pieces pieces of `piece` elements, taken by the board's threads and by
+ * itself (board may be NULL, and nobody need come); it returns when every piece is done, the stream has finished with the slots and
+ * no thread looks at the job.  Any number of threads may drive jobs on one board.  `slots`: pinned memory for min(TQ_HOST_SLOTS,
+ * n_pieces) pieces, one byte per element; `device`: the array's other side, on `stream`'s device.
  *   TQ_HOST_FETCH   n device bytes -> host            TQ_HOST_WIDEN   n device uint8 -> host int64
  *   TQ_HOST_UPLOAD  n host bytes -> device            TQ_HOST_NARROW  n host int64 -> device uint8 (low byte); their bits or'ed in `seen` */
 #define TQ_HOST_SLOTS 8

@@ -95,7 +95,7 @@ bool take(tq_host_job *j) {
     return false;
 }
 
-constexpr int SPINS = 64;         // of the driver, before it sleeps until its next piece has landed
+constexpr int SPINS = 64;                  // of the driver, before it sleeps until its next piece has landed; of a serving thread, at a job
 constexpr int64_t SERVE_CYCLES = 500000;   // of a serving thread, before it sleeps: 0.15 to 0.25 ms
 
 void pause_for(int &idle) {
